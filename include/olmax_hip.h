@@ -96,7 +96,8 @@ int32_t olmax_qk_rope_bwd(olmax_stream_t stream, const void* dy, void* dx, const
 /* ---- Gated MLP input projection with the activation fused into the GEMM epilogue:
  * GatedMLP.forward, src/olmax/nn/mlp.py:69-73 (gate_proj, up_proj, act(gate) * up in one call).
  * W = [Wgate; Wup] ([2F, K], row stride ldw); act_out [M, F]; gu_out ([M, 2F], optional when
- * M % 256 == 0 and F % 128 == 0 and K % 64 == 0, required as scratch otherwise) receives gate|up
+ * M >= 256, F % 128 == 0, K % 64 == 0 and ceil(M / 256) * (F / 128) >= 128 with 16-byte aligned
+ * operands, required as scratch otherwise) receives gate|up
  * for the backward pass.  act: 0 = silu, 1 = tanh-approximated gelu.  Results equal
  * olmax_gemm_bf16 followed by olmax_glu_fwd bit for bit. */
 int32_t olmax_gemm_glu_bf16(olmax_stream_t stream, const void* X, const void* W, void* gu_out, void* act_out,
@@ -118,7 +119,7 @@ int32_t olmax_gemm_glu_bwd_bf16(olmax_stream_t stream, const void* X, const void
  * out[M, N] = X W^T with W = [Wq; Wk; Wv] ([N, K], row stride ldw); the first rope_heads heads of
  * 128 columns (q then k) leave rotated, position of row r = r % seq_len, cos/sin [seq_len, 64]
  * fp32.  Equals olmax_gemm_bf16 followed by olmax_qk_rope_fwd in place (the path taken when the
- * shape does not fit: M, N % 256, K % 64, rope_heads even, >= 128 tiles). */
+ * shape does not fit: M >= 256, N % 256, K % 64, rope_heads even, >= 128 tiles). */
 int32_t olmax_gemm_rope_bf16(olmax_stream_t stream, const void* X, const void* W, void* out, int32_t M, int32_t N,
                              int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, const float* cos_t,
                              const float* sin_t, int32_t seq_len, int32_t rope_heads);

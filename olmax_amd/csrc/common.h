@@ -158,3 +158,10 @@ __device__ __forceinline__ float act_gelu_grad(float g) {
 int olmax_adamw_grid(hipStream_t stream, float* p, const void* g, float* m, float* v, void* shadow_bf16, int64_t n,
                      int32_t grad_is_bf16, float lr, float b1, float b2, float eps, float wd, int64_t step,
                      float grad_scale, const float* grad_scale_dev, int grid_cap, const float* hyper_dev = nullptr);
+
+// gemm_small.hip: any M, N, K and alignment; `groups` (4 or 8) waves share a 64 x 64 tile's reduction
+void olmax_gemm_small(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N, int K, int64_t lda,
+                      int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, int groups);
+// gemm.hip: olmax_gemm_bf16 with an A whose rows are readable (and, k-contiguous, zero) up to a multiple of 8
+int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C, const bf16* r, int M, int N, int K,
+                      int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded);

@@ -40,6 +40,7 @@
 namespace {
 
 constexpr int BK = 64;
+typedef u32x4 __attribute__((aligned(2))) u32x4_u;  // 16 bytes at any element (ragged column edges)
 
 #ifndef GEMM_VGPR_CAP
 #define GEMM_VGPR_CAP
@@ -76,7 +77,14 @@ std::mutex g_prof_mu;
 // projection, as the separate RoPE kernel computes it); a wave's 64 columns are one half of a
 // head and its neighbour (wave ^ 1) holds the other, so the rotation reads both from the LDS
 // staging of the epilogue.  The position of a row is row % seq_len; cos/sin are [seq_len, 64] fp32.
-template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI = 0>
+//
+// RAG: 1 where M or N, 2 where K is not a multiple of the tile.  The last tile of a row or column is
+// moved back so that it ends with the matrix (the loop then reads nothing outside it and is the same
+// code) and stores only what no other tile stores.  The partial k-tile at the end of K is taken FIRST, ahead of
+// the loop, which then sees whole k-tiles only: it is fetched with per-lane addresses, and the wave
+// that fetched a chunk past the end overwrites it with zeros in LDS once its own fetches have landed,
+// before the barrier that publishes the stage.  Wants M >= BM, N >= BN, K >= 64 and 16-byte chunks that do not cross the end of a row (see olmax_gemm_padded).
+template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI = 0, int RAG = 0>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm_bf16_kernel(
     const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
     const bf16* __restrict__ R, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
@@ -140,7 +148,34 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
     tile_m = first_m + (pid % group_sz) % gm;
     tile_n = (pid % group_sz) / gm;
   }
-  const int m0 = tile_m * BM, n0 = tile_n * (GLU ? BN / 2 : BN);  // GLU: first feature of the block
+  constexpr bool KRAG = RAG == 2;
+  constexpr int BNC = GLU ? BN / 2 : BN;  // output columns of a block (GLU: features)
+  int m0 = tile_m * BM, n0 = tile_n * BNC;
+  // rows / columns of the block that this tile stores: all, or (RAG) those behind the previous tile's
+  int row_lo = 0, row_hi = BM, col_lo = 0;
+  if (RAG) {
+    m0 = min(m0, (A_KC ? M : (M + 7) & ~7) - BM);
+    n0 = min(n0, N - BNC);
+    row_lo = tile_m * BM - m0;
+    row_hi = M - m0;
+    col_lo = tile_n * BNC - n0;
+  }
+  // 8 output columns from column c of the block; c and the block's end are whole chunks except where
+  // N is not a multiple of 8 (then the chunk shared with the previous tile is stored by elements)
+  auto store8 = [&](bf16* dst, int c, const u32x4& v) {
+    if (!RAG) {
+      *reinterpret_cast<u32x4*>(dst) = v;
+    } else if (c >= col_lo) {
+      *reinterpret_cast<u32x4_u*>(dst) = v;
+    } else if (c + 8 > col_lo) {
+      Pack8 t;
+      t.u = v;
+#pragma unroll
+      for (int e = 1; e < 8; e++)
+        if (c + e >= col_lo) dst[e] = t.e[e];
+    }
+  };
+  auto stores_row = [&](int row) { return !RAG || (row >= row_lo && row < row_hi); };
 
   // swizzles (see the bank-geometry note at the top of the file)
   auto kswz = [](int row) { return (row >> 1) & 7; };                         // [rows][64] tiles
@@ -181,10 +216,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
   }
   const int64_t a_istep = (int64_t)A_IROWS * lda;  // elements between two instructions' sources
   const int64_t b_istep = (int64_t)(GLU ? 32 : B_IROWS) * ldb;
-  const bf16* a_panel = A_KC ? A + (int64_t)m0 * lda : A + m0;  // k-tile 0 of this block's rows
-  const bf16* b_panel = B_KC ? B + (int64_t)n0 * ldb : B + n0;
   const int64_t a_step = A_KC ? (int64_t)BK : (int64_t)BK * lda;
   const int64_t b_step = B_KC ? (int64_t)BK : (int64_t)BK * ldb;
+  // k-tile 0 of this block's rows (KRAG: of the loop's numbering, in which 1 is the first whole one)
+  const bf16* a_panel = (A_KC ? A + (int64_t)m0 * lda : A + m0) - (KRAG ? a_step : 0);
+  const bf16* b_panel = (B_KC ? B + (int64_t)n0 * ldb : B + n0) - (KRAG ? b_step : 0);
 
   f32x4 acc[TM][TN];
 #pragma unroll
@@ -194,7 +230,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
 #pragma unroll
       for (int r = 0; r < 4; r++) acc[i][j][r] = 0.f;
 
-  const int KT = K / BK;
+  const int KTF = K / BK;             // whole k-tiles
+  const int KT = KTF + (KRAG ? 1 : 0);
   const unsigned lds_base = lds_addr_of(smem);
   // issue DMA instructions [lo, hi) of the combined A+B list of k-tile kt into `stage`
   auto dma = [&](int kt, int stage, int lo, int hi) {
@@ -209,6 +246,54 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
         const int j = i - A_INS;
         dma16_s(b_panel + (int64_t)kt * b_step + j * b_istep, b_off, sb + (j * NW + wave) * 1024);
       }
+    }
+  };
+
+  // KRAG: source of DMA instruction i (of A, then of B) of the partial k-tile for this lane; chunks past
+  // the end are fetched from the row's start (k-contiguous) or from the last k-row and zeroed later
+  auto tail_src = [&](int i, bool& valid) -> const bf16* {
+    const int p = wave * 64 + lane;
+    if (i < A_INS) {
+      if (A_KC) {
+        const int row = i * A_IROWS + (p >> 3), k = KTF * BK + (((p & 7) ^ kswz(row)) << 3);
+        valid = k < K;
+        return A + (int64_t)(m0 + row) * lda + (valid ? k : 0);
+      }
+      constexpr int CPR = BM / 8;
+      const int kr = i * A_IROWS + p / CPR, k = KTF * BK + kr;
+      valid = k < K;
+      return A + (int64_t)(valid ? k : K - 1) * lda + m0 + (((p % CPR) ^ tswz(kr)) << 3);
+    }
+    const int j = i - A_INS;
+    if (B_KC) {
+      const int row = j * B_IROWS + (p >> 3), k = KTF * BK + (((p & 7) ^ kswz(row)) << 3);
+      valid = k < K;
+      return B + (int64_t)(n0 + row) * ldb + (valid ? k : 0);
+    }
+    constexpr int CPR = BN / 8;
+    const int kr = j * B_IROWS + p / CPR, k = KTF * BK + kr;
+    valid = k < K;
+    return B + (int64_t)(valid ? k : K - 1) * ldb + n0 + (((p % CPR) ^ tswz(kr)) << 3);
+  };
+  auto tail_lds = [&](int i, int stage) -> unsigned {
+    return i < A_INS ? lds_base + stage * A_BYTES + (i * NW + wave) * 1024
+                     : lds_base + 2 * A_BYTES + stage * B_BYTES + ((i - A_INS) * NW + wave) * 1024;
+  };
+  auto dma_tail = [&](int stage) {
+#pragma unroll 1
+    for (int i = 0; i < NINS; i++) {
+      bool valid;
+      const bf16* src = tail_src(i, valid);
+      dma16(src, tail_lds(i, stage));
+    }
+  };
+  auto zero_tail = [&](int stage) {  // only after this wave's own fetches have landed
+#pragma unroll 1
+    for (int i = 0; i < NINS; i++) {
+      bool valid;
+      (void)tail_src(i, valid);
+      if (!valid)
+        *reinterpret_cast<__attribute__((address_space(3))) u32x4*>((uintptr_t)(tail_lds(i, stage) + lane * 16)) = u32x4{0u, 0u, 0u, 0u};
     }
   };
 
@@ -319,13 +404,15 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
   static_assert(2 * NINS <= NM && NF + 1 <= NM && NINS + NF <= NM, "not enough MFMA slots for the loads");
   static_assert(ASB == 0 || (NM >= 3 * NINS - 2 && NM >= 4 * (TN + ND)), "slot layout of the single-buffered scheme");
   bf16x8 fas[ASB > 0 ? ASB : 1], fad[2][ND], fb[2][TN];
-  dma(0, 0, 0, NINS);
+  if (KRAG) dma_tail(0);
+  else dma(0, 0, 0, NINS);
   if (KT > 1) {
     dma(1, 1, 0, NINS);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NINS) : "memory");  // k-tile 0 has landed
   } else {
     dma_wait_all();
   }
+  if (KRAG) zero_tail(0);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < TM; i++) {
@@ -470,19 +557,20 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
 #pragma unroll
         for (int t = 0; t < 8; t++) {
           const int row = wave * 32 + t * 4 + (lane_e >> 4), c = lane_e & 15;
+          if (!stores_row(row)) continue;
           const int lrow = row & (WM - 1);
           const unsigned char* src = smem + ((row / WM) * WAVES_N + (c >> 2)) * REG + lrow * 64 + (((c & 3) ^ ((lrow >> 2) & 3)) << 4);
           if (pass == 0) {
-            *reinterpret_cast<u32x4*>(act + (int64_t)(m0 + row) * ldr + n0 + c * 8) = *reinterpret_cast<const u32x4*>(src);
+            store8(act + (int64_t)(m0 + row) * ldr + n0 + c * 8, c * 8, *reinterpret_cast<const u32x4*>(src));
           } else {
-            *reinterpret_cast<u32x4*>(gu + (int64_t)(m0 + row) * ldc + n0 + c * 8) = *reinterpret_cast<const u32x4*>(src);
-            *reinterpret_cast<u32x4*>(gu + (int64_t)(m0 + row) * ldc + N + n0 + c * 8) = *reinterpret_cast<const u32x4*>(src + 8 * REG);
+            store8(gu + (int64_t)(m0 + row) * ldc + n0 + c * 8, c * 8, *reinterpret_cast<const u32x4*>(src));
+            store8(gu + (int64_t)(m0 + row) * ldc + N + n0 + c * 8, c * 8, *reinterpret_cast<const u32x4*>(src + 8 * REG));
           }
         }
       }
       return;
     }
-    if (GLU_BWD) return;  // the backward form is only launched with whole-line stores
+    if (GLU_BWD || RAG) return;  // the backward form and ragged sizes are only launched with whole-line stores
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -549,6 +637,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
       for (int t = 0; t < 16; t++) {
         const int row = wave * 32 + t * 2 + (lane_e >> 5);      // row of the block
         const int c32 = lane_e & 31, chunk = c32 & 7;            // 16-byte chunk of the 512-byte row
+        if (!stores_row(row)) continue;
         const int lrow = row & (WM - 1);                         // row inside the staging region
         const unsigned char* own = smem + ((row / WM) * WAVES_N + (c32 >> 3)) * (WM * 128) + lrow * 128 + ((chunk ^ kswz(lrow)) << 4);
         const unsigned char* oth = smem + ((row / WM) * WAVES_N + ((c32 >> 3) ^ 1)) * (WM * 128) + lrow * 128 + ((chunk ^ kswz(lrow)) << 4);
@@ -575,16 +664,18 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
 #pragma unroll
       for (int t = 0; t < WM / 8; t++) {  // all residual lines requested before the first is needed
         const int row = t * 8 + (lane_e >> 3), chunk = lane_e & 7;
-        rr[t].u = *reinterpret_cast<const u32x4*>(R + (int64_t)(m0 + wm * WM + row) * ldr + n0 + wn * WN + chunk * 8);
+        if (!stores_row(wm * WM + row)) continue;
+        rr[t].u = *reinterpret_cast<const u32x4_u*>(R + (int64_t)(m0 + wm * WM + row) * ldr + n0 + wn * WN + chunk * 8);
       }
 #pragma unroll
       for (int t = 0; t < WM / 8; t++) {
         const int row = t * 8 + (lane_e >> 3), chunk = lane_e & 7;
+        if (!stores_row(wm * WM + row)) continue;
         Pack8 line, o;
         line.u = *reinterpret_cast<const u32x4*>(ws + row * 128 + ((chunk ^ kswz(row)) << 4));
 #pragma unroll
         for (int e = 0; e < 8; e++) o.e[e] = f2bf(bf2f(line.e[e]) + bf2f(rr[t].e[e]));
-        *reinterpret_cast<u32x4*>(C + (int64_t)(m0 + wm * WM + row) * ldc + n0 + wn * WN + chunk * 8) = o.u;
+        store8(C + (int64_t)(m0 + wm * WM + row) * ldc + n0 + wn * WN + chunk * 8, wn * WN + chunk * 8, o.u);
       }
       return;
     }
@@ -592,7 +683,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
     for (int t = 0; t < WM / 8; t++) {
       const int row = t * 8 + (lane_e >> 3), chunk = lane_e & 7;
       const u32x4 line = *reinterpret_cast<const u32x4*>(ws + row * 128 + ((chunk ^ kswz(row)) << 4));
-      *reinterpret_cast<u32x4*>(C + (int64_t)(m0 + wm * WM + row) * ldc + n0 + wn * WN + chunk * 8) = line;
+      if (stores_row(wm * WM + row)) store8(C + (int64_t)(m0 + wm * WM + row) * ldc + n0 + wn * WN + chunk * 8, wn * WN + chunk * 8, line);
     }
     return;
   }
@@ -602,9 +693,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
 #pragma unroll
     for (int j = 0; j < TN; j++) {
       const int64_t row = m0 + wm * WM + i * 16 + l16e;
+      if (!stores_row(wm * WM + i * 16 + l16e)) continue;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int col = n0 + wn * WN + j * 16 + g16e * 4 + r;
+        if (RAG && col < n0 + col_lo) continue;
         float v = acc[i][j][r];
         if (HAS_RES) v = (OUT_F32 ? v : bf2f(f2bf(v))) + bf2f(R[row * ldr + col]);  // bf16 output: round, add, round
         if (OUT_F32)
@@ -613,38 +706,6 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
           reinterpret_cast<bf16*>(Cv)[row * ldc + col] = f2bf(v);
       }
     }
-}
-
-// Bounds-checked scalar-FMA kernel for shapes the MFMA tiles do not divide
-// (the reference's own unit tests use d_model=16, seq=12). One 16x16 output tile per block.
-template <bool OUT_F32>
-__global__ __launch_bounds__(256) void gemm_generic_kernel(
-    const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
-    const bf16* __restrict__ R, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-    int64_t ldr, int a_kc, int b_kc) {
-  __shared__ float As[16][17], Bs[16][17];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int row = blockIdx.y * 16 + ty, col = blockIdx.x * 16 + tx;
-  float acc = 0.f;
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    {
-      const int m = blockIdx.y * 16 + ty, k = k0 + tx;
-      As[ty][tx] = (m < M && k < K) ? bf2f(a_kc ? A[(int64_t)m * lda + k] : A[(int64_t)k * lda + m]) : 0.f;
-      const int n = blockIdx.x * 16 + ty;
-      Bs[ty][tx] = (n < N && k < K) ? bf2f(b_kc ? B[(int64_t)n * ldb + k] : B[(int64_t)k * ldb + n]) : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; k++) acc += As[ty][k] * Bs[tx][k];
-    __syncthreads();
-  }
-  if (row < M && col < N) {
-    if (R) acc = (OUT_F32 ? acc : bf2f(f2bf(acc))) + bf2f(R[(int64_t)row * ldr + col]);
-    if (OUT_F32)
-      reinterpret_cast<float*>(Cv)[(int64_t)row * ldc + col] = acc;
-    else
-      reinterpret_cast<bf16*>(Cv)[(int64_t)row * ldc + col] = f2bf(acc);
-  }
 }
 
 std::atomic<int> g_order{0};  // diagnostic override of the tile order, process-wide: 0 automatic, -1 run order, > 0 that many strips
@@ -672,15 +733,15 @@ unsigned order_grid(int order, int tm, int tn) {
   return (unsigned)((nwin + 7) / 8 * 256);
 }
 
-template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32>
+template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int RAG>
 int launch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N,
                 int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr) {
   constexpr int NT = (BM / WM) * (BN / WN) * 64;
   constexpr int SMEM = 2 * (BM + BN) * BK * 2;
-  auto kern = gemm_bf16_kernel<BM, BN, WM, WN, A_KC, B_KC, HAS_RES, OUT_F32>;
+  auto kern = gemm_bf16_kernel<BM, BN, WM, WN, A_KC, B_KC, HAS_RES, OUT_F32, 0, RAG>;
   static std::once_flag attr_once;  // per instantiation
   std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM); });
-  const int tm = M / BM, tn = N / BN;
+  const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   ProfRec rec{};
   if (g_prof_on) {
     (void)hipEventCreate(&rec.e0);
@@ -688,7 +749,7 @@ int launch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16
     (void)hipEventRecord(rec.e0, s);
   }
   // vector epilogue: 16-byte stores to C, 16-byte loads from R
-  const int c_vec = aligned16(C) && ldc % 8 == 0 && (!R || (aligned16(R) && ldr % 8 == 0));
+  const int c_vec = RAG || (aligned16(C) && ldc % 8 == 0 && (!R || (aligned16(R) && ldr % 8 == 0)));
   const int order = tile_order(tm, tn, A_KC, B_KC, N, K);
   hipLaunchKernelGGL(kern, dim3(order_grid(order, tm, tn)), dim3(NT), SMEM, s, A, B, C, R, M, N, K, lda, ldb, ldc,
                      ldr, tm, tn, c_vec, (const float*)nullptr, (const float*)nullptr, 1, 0, order);
@@ -706,14 +767,14 @@ int launch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16
 }
 
 // EPI 1 / 2: forward form (gu optional); 4 / 5: backward form (dact given, gu = d gate | d up)
-template <int EPI>
+template <int EPI, int RAG>
 int launch_glu(hipStream_t s, const bf16* A, const bf16* B, bf16* gu, bf16* act, int M, int F, int K, int64_t lda,
                int64_t ldb, int64_t ldgu, int64_t ldact, const bf16* dact = nullptr, int64_t lddact = 0) {
   constexpr int SMEM = 2 * (256 + 256) * BK * 2;
-  auto kern = gemm_bf16_kernel<256, 256, 128, 64, true, true, false, false, EPI>;
+  auto kern = gemm_bf16_kernel<256, 256, 128, 64, true, true, false, false, EPI, RAG>;
   static std::once_flag attr_once;  // per instantiation
   std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM); });
-  const int tm = M / 256, tn = F / 128;
+  const int tm = (M + 255) / 256, tn = (F + 127) / 128;
   ProfRec rec{};
   if (g_prof_on) {
     (void)hipEventCreate(&rec.e0);
@@ -742,11 +803,11 @@ int launch_glu(hipStream_t s, const bf16* A, const bf16* B, bf16* gu, bf16* act,
 template <bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32>
 int dispatch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N,
                   int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, int tile) {
-  if (tile == 256)
-    return launch_tile<256, 256, 128, 64, A_KC, B_KC, HAS_RES, OUT_F32>(s, A, B, C, R, M, N, K, lda,
-                                                                        ldb, ldc, ldr);
-  return launch_tile<128, 128, 64, 64, A_KC, B_KC, HAS_RES, OUT_F32>(s, A, B, C, R, M, N, K, lda,
-                                                                     ldb, ldc, ldr);
+  const bool rag = M % tile || N % tile;
+#define TILE(T, W, RAG) launch_tile<T, T, W, 64, A_KC, B_KC, HAS_RES, OUT_F32, RAG>(s, A, B, C, R, M, N, K, lda, ldb, ldc, ldr)
+  if (tile == 256) return K % BK ? TILE(256, 128, 2) : rag ? TILE(256, 128, 1) : TILE(256, 128, 0);
+  return K % BK ? TILE(128, 64, 2) : rag ? TILE(128, 64, 1) : TILE(128, 64, 0);
+#undef TILE
 }
 
 std::atomic<int> g_force_tile{0};  // diagnostic override, process-wide
@@ -828,30 +889,53 @@ static int device_cu_count() {
   return v;
 }
 
-extern "C" int32_t olmax_gemm_bf16(hipStream_t stream, const void* A, const void* B, void* C,
-                                   const void* R, int32_t M, int32_t N, int32_t K, int64_t lda,
-                                   int64_t ldb, int64_t ldc, int64_t ldr, int32_t a_layout,
-                                   int32_t b_layout, int32_t out_f32) {
-  OLMAX_CHECK(A && B && C, OLMAX_ERR_ARG, "olmax_gemm_bf16: null operand");
-  OLMAX_CHECK(M > 0 && N > 0 && K > 0, OLMAX_ERR_SHAPE, "olmax_gemm_bf16: M,N,K must be positive (got %d,%d,%d)", M, N, K);
-  OLMAX_CHECK((a_layout == 0 || a_layout == 1) && (b_layout == 0 || b_layout == 1), OLMAX_ERR_ARG,
-              "olmax_gemm_bf16: layout flags must be 0 (reduction-contiguous) or 1");
-  const bool a_kc = a_layout == 0, b_kc = b_layout == 0;
-  OLMAX_CHECK(lda >= (a_kc ? K : M) && ldb >= (b_kc ? K : N) && ldc >= N && (!R || ldr >= N),
-              OLMAX_ERR_SHAPE, "olmax_gemm_bf16: leading dimension smaller than row length");
-  const bf16* a = (const bf16*)A;
-  const bf16* b = (const bf16*)B;
-  const bf16* r = (const bf16*)R;
-  const bool vec_ok = aligned16(A) && aligned16(B) && (lda % 8 == 0) && (ldb % 8 == 0);
+// Estimated time (us) of each kernel on a problem of kt k-tiles, from measurements at 16 to 8192 rows
+// and 256 to 11008 columns (every layout; within about 15 %).  A k-tile costs a 256 tile 1.05 us with
+// few tiles in flight and 1.52 us with one on every CU (both bound by operand delivery), a 128 tile
+// 0.57 us alone, 0.83 us with one on every CU and 1.08 us with the two that fit, a 64 tile 0.22 us
+// per round.
+static float cost_128(int64_t n, int kt) {
+  auto part = [&](int64_t r) {
+    float f = r <= 64 ? 0.57f : r <= 256 ? 0.57f + 0.26f * (r - 64) / 192.f : 0.83f + 0.25f * (r - 256) / 256.f;
+    if (kt <= 32 && r <= 256) f = 0.6f;
+    return f * kt + 4.f;
+  };
+  return (n / 512) * (1.08f * kt + 4.f) + (n % 512 ? part(n % 512) : 0.f);
+}
+static float cost_256(int64_t n, int kt) {
+  const int64_t r = n % 256;
+  // (a last round that fills less than half of the CUs is cut off and runs as 128 tiles)
+  const float last = r == 0 ? 0.f : (1.05f + 0.47f * r / 256.f) * kt + 6.f;
+  return (n / 256) * (1.52f * kt + 6.f) + (n > 256 && r < 128 && cost_128(4 * r, kt) < last ? cost_128(4 * r, kt) : last);
+}
+static float cost_small(int64_t n, int kt) { return ((n + 255) / 256) * (0.22f * kt + 1.2f) + 2.4f; }
+
+// Which kernel takes a problem.  0: gemm_small (any size and alignment), else the edge of the
+// direct-to-LDS kernel's tiles.
+static int pick_tile(int M, int N, int K, bool direct_ok) {
+  if (!direct_ok || M < 128 || N < 128 || K < BK) return 0;
+  const int kt = (K + BK - 1) / BK;
+  auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
+  float best = cost_small(tiles(64), kt);
   int tile = 0;
+  if (const float c = cost_128(tiles(128), kt); c < best) best = c, tile = 128;
+  if (M >= 256 && N >= 256 && cost_256(tiles(256), kt) < best) tile = 256;
+  return tile;
+}
+
+// olmax_gemm_bf16 behind its argument checks.  a_padded: rows of A may be read up to the next multiple
+// of 8 elements (row stride permitting), and for a k-contiguous A those elements are zeros: what
+// lets an operand whose row length is not a multiple of 8 use 16-byte fetches.
+int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C, const bf16* r, int M, int N, int K,
+                      int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded) {
+  // whole 16-byte chunks everywhere: aligned rows, and a chunk never crosses the end of a row
+  const bool direct_ok = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 && (a_padded || (a_kc ? K : M) % 8 == 0) &&
+                         (b_kc ? K : N) % 8 == 0 && (a_kc || !b_kc);
+  int tile = pick_tile(M, N, K, direct_ok);
   const int force_tile = g_force_tile.load(std::memory_order_relaxed);
-  if (vec_ok && K % BK == 0) {
-    if (M % 256 == 0 && N % 256 == 0 && (int64_t)(M / 256) * (N / 256) >= 128) tile = 256;
-    else if (M % 128 == 0 && N % 128 == 0) tile = 128;
-  }
   if (force_tile && tile) {
-    if (force_tile == 256 && M % 256 == 0 && N % 256 == 0) tile = 256;
-    if (force_tile == 128) tile = 128;
+    if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
+    if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;
   }
   // Wave quantisation: with one 256x256 tile per CU per round, a last round that fills less
   // than half of the CUs (e.g. 1376 tiles = 5.375 rounds on 256 CUs) costs a whole round.
@@ -859,7 +943,7 @@ extern "C" int32_t olmax_gemm_bf16(hipStream_t stream, const void* A, const void
   // rounds and a remainder that goes through this function again (and gets smaller tiles).
   if (tile == 256 && !force_tile) {
     const int ncu = device_cu_count();
-    const int tm = M / 256, tn = N / 256;
+    const int tm = (M + 255) / 256, tn = (N + 255) / 256;
     const int64_t tiles = (int64_t)tm * tn;
     const int rem = (int)(tiles % ncu);
     if (tiles > ncu && rem > 0 && rem * 2 < ncu) {
@@ -869,30 +953,26 @@ extern "C" int32_t olmax_gemm_bf16(hipStream_t stream, const void* A, const void
       const size_t esz = out_f32 ? 4 : 2;
       if (rm > 0 && (int64_t)rm * tn >= (int64_t)cn * tm) {
         const int m1 = rm * 256;
-        int rc = olmax_gemm_bf16(stream, A, B, C, R, m1, N, K, lda, ldb, ldc, ldr, a_layout, b_layout, out_f32);
+        int rc = olmax_gemm_padded(stream, a, b, C, r, m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
         if (rc) return rc;
         const bf16* a2 = a_kc ? a + (int64_t)m1 * lda : a + m1;
-        return olmax_gemm_bf16(stream, a2, B, (char*)C + (int64_t)m1 * ldc * esz, r ? r + (int64_t)m1 * ldr : nullptr,
-                               M - m1, N, K, lda, ldb, ldc, ldr, a_layout, b_layout, out_f32);
+        return olmax_gemm_padded(stream, a2, b, (char*)C + (int64_t)m1 * ldc * esz, r ? r + (int64_t)m1 * ldr : nullptr,
+                                 M - m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
       }
       if (cn > 0) {
         const int n1 = cn * 256;
-        int rc = olmax_gemm_bf16(stream, A, B, C, R, M, n1, K, lda, ldb, ldc, ldr, a_layout, b_layout, out_f32);
+        int rc = olmax_gemm_padded(stream, a, b, C, r, M, n1, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
         if (rc) return rc;
         const bf16* b2 = b_kc ? b + (int64_t)n1 * ldb : b + n1;
-        return olmax_gemm_bf16(stream, A, b2, (char*)C + (int64_t)n1 * esz, r ? r + n1 : nullptr, M, N - n1, K, lda,
-                               ldb, ldc, ldr, a_layout, b_layout, out_f32);
+        return olmax_gemm_padded(stream, a, b2, (char*)C + (int64_t)n1 * esz, r ? r + n1 : nullptr, M, N - n1, K, lda,
+                                 ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
       }
     }
   }
   if (tile == 0) {
-    dim3 grid((N + 15) / 16, (M + 15) / 16);
-    if (out_f32)
-      hipLaunchKernelGGL(gemm_generic_kernel<true>, grid, dim3(256), 0, stream, a, b, C, r, M, N, K,
-                         lda, ldb, ldc, ldr, (int)a_kc, (int)b_kc);
-    else
-      hipLaunchKernelGGL(gemm_generic_kernel<false>, grid, dim3(256), 0, stream, a, b, C, r, M, N,
-                         K, lda, ldb, ldc, ldr, (int)a_kc, (int)b_kc);
+    olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32,
+                     // eight waves share a tile while there are not more tiles than CUs, else two workgroups fit a CU
+                     (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 256 ? 8 : 4);
     OLMAX_LAUNCH_CHECK();
     return OLMAX_OK;
   }
@@ -907,10 +987,24 @@ extern "C" int32_t olmax_gemm_bf16(hipStream_t stream, const void* A, const void
     }                                                                                            \
   } while (0)
   if (a_kc && b_kc) GO(true, true);
-  if (a_kc && !b_kc) GO(true, false);
-  if (!a_kc && !b_kc) GO(false, false);
-  GO(false, true);
+  if (a_kc) GO(true, false);
+  GO(false, false);
 #undef GO
+}
+
+extern "C" int32_t olmax_gemm_bf16(hipStream_t stream, const void* A, const void* B, void* C,
+                                   const void* R, int32_t M, int32_t N, int32_t K, int64_t lda,
+                                   int64_t ldb, int64_t ldc, int64_t ldr, int32_t a_layout,
+                                   int32_t b_layout, int32_t out_f32) {
+  OLMAX_CHECK(A && B && C, OLMAX_ERR_ARG, "olmax_gemm_bf16: null operand");
+  OLMAX_CHECK(M > 0 && N > 0 && K > 0, OLMAX_ERR_SHAPE, "olmax_gemm_bf16: M,N,K must be positive (got %d,%d,%d)", M, N, K);
+  OLMAX_CHECK((a_layout == 0 || a_layout == 1) && (b_layout == 0 || b_layout == 1), OLMAX_ERR_ARG,
+              "olmax_gemm_bf16: layout flags must be 0 (reduction-contiguous) or 1");
+  const bool a_kc = a_layout == 0, b_kc = b_layout == 0;
+  OLMAX_CHECK(lda >= (a_kc ? K : M) && ldb >= (b_kc ? K : N) && ldc >= N && (!R || ldr >= N),
+              OLMAX_ERR_SHAPE, "olmax_gemm_bf16: leading dimension smaller than row length");
+  return olmax_gemm_padded(stream, (const bf16*)A, (const bf16*)B, C, (const bf16*)R, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc,
+                           out_f32 != 0, false);
 }
 
 extern "C" int32_t olmax_qk_rope_fwd(hipStream_t stream, const void* x, void* y, const void* w, const float* cos_t,
@@ -930,14 +1024,19 @@ extern "C" int32_t olmax_gemm_rope_bf16(hipStream_t stream, const void* X, const
               "olmax_gemm_rope_bf16: bad shape (M %d N %d K %d seq_len %d rope_heads %d)", M, N, K, seq_len, rope_heads);
   OLMAX_CHECK(ldx >= K && ldw >= K && ldo >= N, OLMAX_ERR_SHAPE, "olmax_gemm_rope_bf16: leading dimension smaller than row length");
   const bool fits = aligned16(X) && aligned16(W) && aligned16(out) && aligned16(cos_t) && aligned16(sin_t) && ldx % 8 == 0 &&
-                    ldw % 8 == 0 && ldo % 8 == 0 && K % BK == 0 && M % 256 == 0 && N % 256 == 0 && rope_heads % 2 == 0 &&
-                    (int64_t)(M / 256) * (N / 256) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
+                    ldw % 8 == 0 && ldo % 8 == 0 && K % BK == 0 && M >= 256 && N % 256 == 0 && rope_heads % 2 == 0 &&
+                    (int64_t)((M + 255) / 256) * (N / 256) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
   if (fits) {
     constexpr int SMEM = 2 * (256 + 256) * BK * 2;
-    auto kern = gemm_bf16_kernel<256, 256, 128, 64, true, true, false, false, 3>;
-    static std::once_flag attr_once;  // per instantiation
-    std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM); });
-    const int tm = M / 256, tn = N / 256;
+    auto whole = gemm_bf16_kernel<256, 256, 128, 64, true, true, false, false, 3>;
+    auto ragged = gemm_bf16_kernel<256, 256, 128, 64, true, true, false, false, 3, 1>;
+    static std::once_flag attr_once;
+    std::call_once(attr_once, [&] {
+      (void)hipFuncSetAttribute((const void*)whole, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+      (void)hipFuncSetAttribute((const void*)ragged, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+    });
+    auto kern = M % 256 ? ragged : whole;
+    const int tm = (M + 255) / 256, tn = N / 256;
     ProfRec rec{};
     if (g_prof_on) {
       (void)hipEventCreate(&rec.e0);
@@ -979,11 +1078,15 @@ extern "C" int32_t olmax_gemm_glu_bf16(hipStream_t stream, const void* X, const 
   OLMAX_CHECK(act == 0 || act == 1, OLMAX_ERR_ARG, "olmax_gemm_glu_bf16: act must be 0 (silu) or 1 (gelu-tanh)");
   OLMAX_CHECK(ldx >= K && ldw >= K && ldact >= F && (!gu_out || ldgu >= 2 * (int64_t)F), OLMAX_ERR_SHAPE,
               "olmax_gemm_glu_bf16: leading dimension smaller than row length");
-  const bool fits = aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && K % BK == 0 && M % 256 == 0 &&
-                    F % 128 == 0 && (int64_t)(M / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
-  if (fits) {
-    if (act == 0) return launch_glu<1>(stream, (const bf16*)X, (const bf16*)W, (bf16*)gu_out, (bf16*)act_out, M, F, K, ldx, ldw, ldgu, ldact);
-    return launch_glu<2>(stream, (const bf16*)X, (const bf16*)W, (bf16*)gu_out, (bf16*)act_out, M, F, K, ldx, ldw, ldgu, ldact);
+  const bool fits = aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && K % BK == 0 && M >= 256 && F % 128 == 0 &&
+                    (int64_t)((M + 255) / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
+  // ragged rows leave through the whole-line stores only
+  const bool lines = aligned16(act_out) && ldact % 8 == 0 && (!gu_out || (aligned16(gu_out) && ldgu % 8 == 0));
+  if (fits && (M % 256 == 0 || lines)) {
+#define GLU(E, RAG) launch_glu<E, RAG>(stream, (const bf16*)X, (const bf16*)W, (bf16*)gu_out, (bf16*)act_out, M, F, K, ldx, ldw, ldgu, ldact)
+    if (act == 0) return M % 256 ? GLU(1, 1) : GLU(1, 0);
+    return M % 256 ? GLU(2, 1) : GLU(2, 0);
+#undef GLU
   }
   OLMAX_CHECK(gu_out, OLMAX_ERR_ARG, "olmax_gemm_glu_bf16: this shape needs gu_out as scratch for the unfused path");
   int rc = olmax_gemm_bf16(stream, X, W, gu_out, nullptr, M, 2 * F, K, ldx, ldw, ldgu, 0, 0, 0, 0);
@@ -1008,16 +1111,17 @@ extern "C" int32_t olmax_gemm_glu_bwd_bf16(hipStream_t stream, const void* X, co
   OLMAX_CHECK(act == 0 || act == 1, OLMAX_ERR_ARG, "olmax_gemm_glu_bwd_bf16: act must be 0 (silu) or 1 (gelu-tanh)");
   OLMAX_CHECK(ldx >= K && ldw >= K && ldact >= F && lddact >= F && lddgu >= 2 * (int64_t)F, OLMAX_ERR_SHAPE,
               "olmax_gemm_glu_bwd_bf16: leading dimension smaller than row length");
-  const bool fits = aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && K % BK == 0 && M % 256 == 0 &&
-                    F % 128 == 0 && (int64_t)(M / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed) &&
+  const bool fits = aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && K % BK == 0 && M >= 256 &&
+                    F % 128 == 0 && (int64_t)((M + 255) / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed) &&
                     aligned16(act_out) && ldact % 8 == 0 && aligned16(dgu_out) && lddgu % 8 == 0 &&
                     ((((uintptr_t)dact) & 7) == 0) && lddact % 4 == 0 && lddact < (1ll << 31);
   if (fits) {
-    if (act == 0)
-      return launch_glu<4>(stream, (const bf16*)X, (const bf16*)W, (bf16*)dgu_out, (bf16*)act_out, M, F, K, ldx, ldw, lddgu, ldact,
-                           (const bf16*)dact, lddact);
-    return launch_glu<5>(stream, (const bf16*)X, (const bf16*)W, (bf16*)dgu_out, (bf16*)act_out, M, F, K, ldx, ldw, lddgu, ldact,
-                         (const bf16*)dact, lddact);
+#define GLU(E, RAG)                                                                                                               \
+  launch_glu<E, RAG>(stream, (const bf16*)X, (const bf16*)W, (bf16*)dgu_out, (bf16*)act_out, M, F, K, ldx, ldw, lddgu, ldact,     \
+                     (const bf16*)dact, lddact)
+    if (act == 0) return M % 256 ? GLU(4, 1) : GLU(4, 0);
+    return M % 256 ? GLU(5, 1) : GLU(5, 0);
+#undef GLU
   }
   // unfused: gate | up into dgu_out, then the elementwise backward in place over it
   int rc = olmax_gemm_glu_bf16(stream, X, W, dgu_out, act_out, M, F, K, ldx, ldw, lddgu, ldact, act);

@@ -12,11 +12,6 @@
 // Optional final-logit soft-cap z = c*tanh(x/c) is applied on the fly in both passes.
 #include "common.h"
 
-extern "C" int32_t olmax_gemm_bf16(hipStream_t stream, const void* A, const void* B, void* C,
-                                   const void* R, int32_t M, int32_t N, int32_t K, int64_t lda,
-                                   int64_t ldb, int64_t ldc, int64_t ldr, int32_t a_layout,
-                                   int32_t b_layout, int32_t out_f32);
-
 namespace {
 
 __global__ __launch_bounds__(256) void ce_count_kernel(const int32_t* __restrict__ labels, int64_t T,
@@ -68,7 +63,7 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
     const T* __restrict__ logits, T* __restrict__ dlogits, const int32_t* __restrict__ labels,
     float* __restrict__ row_loss, float* __restrict__ lse_out, const int32_t* __restrict__ n_counted,
     int64_t rows, int V, int64_t ld, int64_t ldd, int32_t ignore_index, float cap, float dloss,
-    int vec_ok, const float* __restrict__ drow, int mean) {
+    int vec_ok, const float* __restrict__ drow, int mean, int pad) {
   constexpr int VEC = Io<T>::VEC;
   __shared__ float red[4];
   __shared__ float label_logit;
@@ -158,13 +153,15 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
     if (i == label) p -= 1.f;
     Io<T>::st1(dr + i, p * scale * chain);
   }
+  for (int i = V + threadIdx.x; i < V + pad; i += 256) Io<T>::st1(dr + i, 0.f);
 }
 
 // The same row computation for bf16 rows short enough to keep in registers between the two
 // passes (THREADS x MAXV vectors of 8): the logits are read from memory once and the gradient
 // written once, 4 B per logit instead of 6.  Max and sum-exp are two plain block reductions (no
-// online rescaling needed when the whole row is at hand).
-template <bool CAP, int THREADS, int MAXV>
+// online rescaling needed when the whole row is at hand).  PAD: V is not a multiple of 8 and the rows
+// have room up to the next one; those logits are left out and their gradient is written as zero.
+template <bool CAP, int THREADS, int MAXV, bool PAD>
 __global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
     const bf16* __restrict__ logits, bf16* __restrict__ dlogits, const int32_t* __restrict__ labels,
     float* __restrict__ row_loss, float* __restrict__ lse_out, const int32_t* __restrict__ n_counted,
@@ -177,7 +174,7 @@ __global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
   const bf16* zr = logits + row * ld;
   const int label = labels[row];
   const float inv_cap = CAP ? 1.f / cap : 0.f;
-  const int nvec = V / 8;
+  const int nvec = PAD ? (V + 7) / 8 : V / 8;
   const bool counted = label != ignore_index;
   const bool inrange = label >= 0 && label < V;
   // label logit into LDS before the first barrier (see ce_row_kernel): nothing reads the row
@@ -205,7 +202,8 @@ __global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
   for (int i = 0; i < MAXV; i++)
     if (i * THREADS + threadIdx.x < nvec) {
 #pragma unroll
-      for (int e = 0; e < 8; e++) mx = fmaxf(mx, value(c[i].e[e]));
+      for (int e = 0; e < 8; e++)
+        if (!PAD || (i * THREADS + (int)threadIdx.x) * 8 + e < V) mx = fmaxf(mx, value(c[i].e[e]));
     }
   const float gmx = block_max<NW>(mx, red);
   float sm = 0.f;
@@ -213,7 +211,8 @@ __global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
   for (int i = 0; i < MAXV; i++)
     if (i * THREADS + threadIdx.x < nvec) {
 #pragma unroll
-      for (int e = 0; e < 8; e++) sm += __expf(value(c[i].e[e]) - gmx);
+      for (int e = 0; e < 8; e++)
+        if (!PAD || (i * THREADS + (int)threadIdx.x) * 8 + e < V) sm += __expf(value(c[i].e[e]) - gmx);
     }
   const float gsm = block_sum<NW>(sm, red);
   const float lse = gmx + __logf(gsm);
@@ -240,7 +239,7 @@ __global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
         }
         float p = __expf(z - lse);
         if (idx * 8 + e == label) p -= 1.f;
-        o.e[e] = f2bf(p * scale * chain);
+        o.e[e] = f2bf(!PAD || idx * 8 + e < V ? p * scale * chain : 0.f);
       }
       *(reinterpret_cast<u32x4*>(dr) + idx) = o.u;
     }
@@ -269,11 +268,12 @@ extern "C" int64_t olmax_cross_entropy_workspace_bytes(int64_t T) { return ((T *
 // device array dloss_rows when given); lse_out (optional, [T]) <- log-normaliser *
 // (label != ignore_index)  (the reference's fused_cross_entropy_loss second output,
 // src/olmax/nn/functional.py:94-121).  reduction: 0 "mean", 1 "sum", 2 "none" (functional.py:84-91).
-extern "C" int32_t olmax_cross_entropy_reduce(hipStream_t stream, const void* logits, void* dlogits,
-                                              const int32_t* labels, float* loss, float* lse_out,
-                                              const float* dloss_rows, void* workspace, int64_t workspace_bytes,
-                                              int64_t T, int32_t V, int64_t ld, int64_t ldd, int32_t logits_f32,
-                                              int32_t ignore_index, float softcap, float dloss, int32_t reduction) {
+// padded (in place, bf16): the rows have room up to the next multiple of 8 logits, which may be read
+// and is written with zeros.
+static int cross_entropy(hipStream_t stream, const void* logits, void* dlogits, const int32_t* labels, float* loss, float* lse_out,
+                         const float* dloss_rows, void* workspace, int64_t workspace_bytes, int64_t T, int32_t V, int64_t ld,
+                         int64_t ldd, int32_t logits_f32, int32_t ignore_index, float softcap, float dloss, int32_t reduction,
+                         bool padded) {
   OLMAX_CHECK(logits && labels && loss && workspace, OLMAX_ERR_ARG, "olmax_cross_entropy: null pointer");
   OLMAX_CHECK(T > 0 && V > 0 && ld >= V && (!dlogits || ldd >= V), OLMAX_ERR_SHAPE, "olmax_cross_entropy: bad shape T=%ld V=%d", (long)T, V);
   OLMAX_CHECK(reduction >= 0 && reduction <= 2, OLMAX_ERR_ARG, "olmax_cross_entropy: reduction must be 0 (mean), 1 (sum) or 2 (none)");
@@ -291,11 +291,13 @@ extern "C" int32_t olmax_cross_entropy_reduce(hipStream_t stream, const void* lo
 #define CE_GO(TY, CAPV)                                                                          \
   hipLaunchKernelGGL((ce_row_kernel<TY, CAPV>), grid, dim3(256), 0, stream, (const TY*)logits,   \
                      (TY*)dlogits, labels, row_loss, lse_out, n_counted, T, V, ld, ldd,          \
-                     ignore_index, softcap, dloss, vec_ok, dloss_rows, mean)
-#define CE_REGS(CAPV, TH, MV)                                                                              \
-  hipLaunchKernelGGL((ce_row_regs_kernel<CAPV, TH, MV>), grid, dim3(TH), 0, stream, (const bf16*)logits,   \
+                     ignore_index, softcap, dloss, vec_ok, dloss_rows, mean, padded ? (8 - V % 8) % 8 : 0)
+#define CE_REGS_P(CAPV, TH, MV, PADV)                                                                          \
+  hipLaunchKernelGGL((ce_row_regs_kernel<CAPV, TH, MV, PADV>), grid, dim3(TH), 0, stream, (const bf16*)logits, \
                      (bf16*)dlogits, labels, row_loss, lse_out, n_counted, V, ld, ldd, ignore_index, softcap, dloss, dloss_rows, mean)
-  const bool regs_ok = !logits_f32 && vec_ok && V % 8 == 0;
+#define CE_REGS(CAPV, TH, MV)                                                                                  \
+  do { if (V % 8) CE_REGS_P(CAPV, TH, MV, true); else CE_REGS_P(CAPV, TH, MV, false); } while (0)
+  const bool regs_ok = !logits_f32 && vec_ok && (V % 8 == 0 || padded);
   if (logits_f32) {
     if (cap) CE_GO(float, true); else CE_GO(float, false);
   } else if (regs_ok && V <= 512 * 8 * 26) {  // up to 106496 logits: 8 waves holding 26 vectors each
@@ -307,9 +309,19 @@ extern "C" int32_t olmax_cross_entropy_reduce(hipStream_t stream, const void* lo
   }
 #undef CE_GO
 #undef CE_REGS
+#undef CE_REGS_P
   if (reduction != 2) hipLaunchKernelGGL(ce_finalize_kernel, dim3(1), dim3(256), 0, stream, row_loss, T, n_counted, loss, mean);
   OLMAX_LAUNCH_CHECK();
   return OLMAX_OK;
+}
+
+extern "C" int32_t olmax_cross_entropy_reduce(hipStream_t stream, const void* logits, void* dlogits,
+                                              const int32_t* labels, float* loss, float* lse_out,
+                                              const float* dloss_rows, void* workspace, int64_t workspace_bytes,
+                                              int64_t T, int32_t V, int64_t ld, int64_t ldd, int32_t logits_f32,
+                                              int32_t ignore_index, float softcap, float dloss, int32_t reduction) {
+  return cross_entropy(stream, logits, dlogits, labels, loss, lse_out, dloss_rows, workspace, workspace_bytes, T, V, ld, ldd,
+                       logits_f32, ignore_index, softcap, dloss, reduction, false);
 }
 
 // reduction "mean": what the benchmark's loss_fun and the fused LM head use
@@ -322,9 +334,14 @@ extern "C" int32_t olmax_cross_entropy(hipStream_t stream, const void* logits, v
                                     ldd, logits_f32, ignore_index, softcap, dloss, 0);
 }
 
-// Workspace for the fused LM head: bf16 logits [T, V] + the CE workspace.
+// Row stride of the LM head's own logits: whole 128-byte lines, so that the three GEMMs around the
+// cross entropy fetch 16-byte chunks whatever the vocabulary (100278 logits are rows of 2-byte
+// alignment when packed).
+static int64_t logits_stride(int32_t V) { return ((int64_t)V + 63) / 64 * 64; }
+
+// Workspace for the fused LM head: bf16 logits [T, logits_stride(V)] + the CE workspace.
 extern "C" int64_t olmax_lmhead_ce_workspace_bytes(int64_t T, int32_t V) {
-  return ((T * (int64_t)V * 2 + 255) / 256) * 256 + olmax_cross_entropy_workspace_bytes(T);
+  return ((T * logits_stride(V) * 2 + 255) / 256) * 256 + olmax_cross_entropy_workspace_bytes(T);
 }
 
 // Fused LM head + cross entropy, forward and backward in one call:
@@ -340,20 +357,22 @@ extern "C" int32_t olmax_lmhead_ce(hipStream_t stream, const void* h, const void
   OLMAX_CHECK(T > 0 && d > 0 && V > 0 && T < (1LL << 31), OLMAX_ERR_SHAPE, "olmax_lmhead_ce: bad shape");
   OLMAX_CHECK(workspace_bytes >= olmax_lmhead_ce_workspace_bytes(T, V) && (((uintptr_t)workspace) & 255) == 0, OLMAX_ERR_WORKSPACE,
               "olmax_lmhead_ce: workspace needs %ld bytes, 256-byte aligned", (long)olmax_lmhead_ce_workspace_bytes(T, V));
-  void* logits = workspace;
-  void* ce_ws = (char*)workspace + ((T * (int64_t)V * 2 + 255) / 256) * 256;
-  int rc = olmax_gemm_bf16(stream, h, W, logits, nullptr, (int)T, V, d, d, d, V, 0, 0, 0, 0);
+  const int64_t ldl = logits_stride(V);
+  bf16* logits = (bf16*)workspace;
+  void* ce_ws = (char*)workspace + ((T * ldl * 2 + 255) / 256) * 256;
+  const bf16 *hp = (const bf16*)h, *wp = (const bf16*)W;
+  int rc = olmax_gemm_padded(stream, hp, wp, logits, nullptr, (int)T, V, d, d, d, ldl, 0, true, true, false, false);
   if (rc) return rc;
   const bool need_grad = dh || dW;
-  rc = olmax_cross_entropy(stream, logits, need_grad ? logits : nullptr, labels, loss, nullptr, ce_ws,
-                           olmax_cross_entropy_workspace_bytes(T), T, V, V, V, 0, ignore_index, softcap, 1.f);
+  rc = cross_entropy(stream, logits, need_grad ? logits : nullptr, labels, loss, nullptr, nullptr, ce_ws,
+                     olmax_cross_entropy_workspace_bytes(T), T, V, ldl, ldl, 0, ignore_index, softcap, 1.f, 0, true);
   if (rc) return rc;
   if (dh) {
-    rc = olmax_gemm_bf16(stream, logits, W, dh, nullptr, (int)T, d, V, V, d, d, 0, 0, 1, 0);
+    rc = olmax_gemm_padded(stream, logits, wp, dh, nullptr, (int)T, d, V, ldl, d, d, 0, true, false, false, true);
     if (rc) return rc;
   }
   if (dW) {
-    rc = olmax_gemm_bf16(stream, logits, h, dW, nullptr, V, d, (int)T, V, d, d, 0, 1, 1, dw_f32);
+    rc = olmax_gemm_padded(stream, logits, hp, dW, nullptr, V, d, (int)T, ldl, d, d, 0, false, false, dw_f32 != 0, true);
     if (rc) return rc;
   }
   return OLMAX_OK;

@@ -162,7 +162,7 @@ def gated_mlp_in(x, w_gate_up, act: str = "silu", gate_up_out=None, save_gate_up
     F = w_gate_up.shape[0] // 2
     if out is None:
         out = torch.empty(T, F, device=x.device, dtype=BF16)
-    fits = T % 256 == 0 and F % 128 == 0 and d % 64 == 0 and (T // 256) * (F // 128) >= 128
+    fits = T >= 256 and F % 128 == 0 and d % 64 == 0 and -(-T // 256) * (F // 128) >= 128
     if gate_up_out is None and (save_gate_up or not fits):
         gate_up_out = torch.empty(T, 2 * F, device=x.device, dtype=BF16)
     check(_L().olmax_gemm_glu_bf16(stream_ptr(), ptr(x), ptr(w_gate_up), ptr(gate_up_out), ptr(out), i32(T), i32(F),
