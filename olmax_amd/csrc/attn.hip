@@ -1,4 +1,4 @@
-// Causal GQA flash attention for gfx950, head_dim 128, BSHD layout, bf16 in/out, fp32
+// Causal GQA flash attention for gfx950, head_dim 128 or 64 (D), BSHD layout, bf16 in/out, fp32
 // softmax statistics, optional sliding window and tanh logit soft-cap.
 //
 // Replaces the cuDNN fused-attention custom call that
@@ -36,37 +36,39 @@ __device__ __forceinline__ float cap_tanh(float raw, float c1) {
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LN2 = 0.6931471805599453f;
 
-// 16-byte chunk swizzle of the [rows][128] tiles (256 B rows = one line of the 64 LDS banks).
-// ds_read_b128 serves the lane groups {0-3,12-15,20-23,24-27} / {4-7,8-11,16-19,28-31} (one
-// row per lane, same logical chunk) per clock and the transposing ds_read_b64 serves lanes
-// 0-31 (4 consecutive rows x 4 chunks); this mask gives 16 distinct chunks in both cases.
-__device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+// 16-byte chunk swizzle of the [rows][D] tiles.  ds_read_b128 serves the lane groups
+// {0-3,12-15,20-23,24-27} / {4-7,8-11,16-19,28-31} (one row per lane, same logical chunk) per clock
+// and the transposing ds_read_b64 serves lanes 0-31 (4 consecutive rows x 4 chunks); these masks give
+// 16 distinct chunks modulo the 256-byte line of the 64 banks in both cases.  D = 128: a row is a
+// line; D = 64: two rows share one, so the row's lowest bit already separates them, and bit 1 moves
+// the transposed read's other two rows to the other half of their own.
+template <int D>
+__device__ __forceinline__ int swz(int row) {
+  return D == 128 ? ((row & 3) << 2) | ((row >> 2) & 3) : ((row & 2) << 1) | ((row >> 2) & 3);
+}
 
-// byte offset of 16B chunk `c` (0..15) of row `row` in a [rows][128] bf16 tile
-__device__ __forceinline__ int tile_off(int row, int c) { return row * 256 + ((c ^ swz(row)) << 4); }
-
-// Per-lane byte offsets of the operand fragments inside a [rows][128] tile.  The swizzle only
+// Per-lane byte offsets of the operand fragments inside a [rows][D] tile.  The swizzle only
 // looks at row bits 0-3, so stepping rows by 16 or 32 is a plain immediate offset and the
-// eight (k-contiguous) plus eight (transposed) lane-dependent offsets are loop invariant.
+// D/16 (k-contiguous) plus D/16 (transposed) lane-dependent offsets are loop invariant.
 // LEAN: the k-contiguous offsets are formed at each read from the first one (kc[s] = kc[0] ^ 32 s:
-// the k-step only enters the XOR-swizzled chunk index) instead of living in eight registers, for a
+// the k-step only enters the XOR-swizzled chunk index) instead of living in registers, for a
 // kernel that would otherwise spill them.
-template <bool LEAN = false>
-struct FragAddrT {
-  int kc[LEAN ? 1 : 8];  // row (lane % 32), k-step s
-  int tr[4][2];          // column tile dt, half h of the transposed read
+template <int D, bool LEAN = false>
+struct FragAddr {
+  int kc[LEAN ? 1 : D / 16];  // row (lane % 32), k-step s
+  int tr[D / 32][2];          // column tile dt, half h of the transposed read
   __device__ __forceinline__ void init(int lane) {
     const int l32 = lane & 31, lhi = lane >> 5;
 #pragma unroll
-    for (int s = 0; s < (LEAN ? 1 : 8); s++) kc[s] = l32 * 256 + (((2 * s + lhi) ^ swz(l32)) << 4);
+    for (int s = 0; s < (LEAN ? 1 : D / 16); s++) kc[s] = l32 * (2 * D) + (((2 * s + lhi) ^ swz<D>(l32)) << 4);
     const int j16 = lane & 15, g16 = lane >> 4;
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         const int col = dt * 32 + ((g16 & 1) << 4) + ((j16 & 3) << 2);
         const int row = ((g16 >> 1) << 2) + (h << 3) + (j16 >> 2);
-        tr[dt][h] = row * 256 + (((col >> 3) ^ swz(row)) << 4) + ((col & 7) << 1);
+        tr[dt][h] = row * (2 * D) + (((col >> 3) ^ swz<D>(row)) << 4) + ((col & 7) << 1);
       }
   }
   // k-contiguous fragment: rows row0 + lane%32 (row0 multiple of 16), k-step s
@@ -76,55 +78,32 @@ struct FragAddrT {
       asm volatile("" : "+v"(off));  // keeps the XOR at the read: hoisted out of the loop it is a register again
       off ^= s << 5;
     }
-    return *reinterpret_cast<const bf16x8*>(tile + off + row0 * 256);
+    return *reinterpret_cast<const bf16x8*>(tile + off + row0 * (2 * D));
   }
   // transposed fragment: MFMA rows = storage columns dt*32 + lane%32, k = storage rows r0 + {..}
   __device__ __forceinline__ bf16x8 load_tr(const unsigned char* tile, int r0, int dt) const {
     Pack8 p;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-      s16x4 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + tr[dt][h] + r0 * 256));
+      s16x4 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + tr[dt][h] + r0 * (2 * D)));
       p.u[h * 2 + 0] = ((u32x2&)t)[0];
       p.u[h * 2 + 1] = ((u32x2&)t)[1];
     }
     return p.v;
   }
 };
-typedef FragAddrT<false> FragAddr;
 
-// A/B operand fragment with the k index contiguous in storage: row `row`, k-step s (16 wide)
-__device__ __forceinline__ bf16x8 frag_kc(const unsigned char* tile, int row, int s, int lhi) {
-  return *reinterpret_cast<const bf16x8*>(tile + tile_off(row, 2 * s + lhi));
-}
-
-// A operand fragment read transposed: rows of the MFMA = storage columns col0 + (lane % 32),
-// k index = storage rows {r0 + 4*kg + 0..3, r0 + 8 + 4*kg + 0..3}
-__device__ __forceinline__ bf16x8 frag_tr(const unsigned char* tile, int r0, int col0, int lane) {
-  const int j16 = lane & 15, g16 = lane >> 4;
-  const int col = col0 + ((g16 & 1) << 4) + ((j16 & 3) << 2);
-  Pack8 p;
-#pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const int row = r0 + ((g16 >> 1) << 2) + (h << 3) + (j16 >> 2);
-    const int off = row * 256 + ((((col >> 3)) ^ swz(row)) << 4) + ((col & 7) << 1);
-    s16x4 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + off));
-    p.u[h * 2 + 0] = ((u32x2&)t)[0];
-    p.u[h * 2 + 1] = ((u32x2&)t)[1];
-  }
-  return p.v;
-}
-
-// Stream ROWS rows of 128 bf16 (global row r0 + i, clamped to S-1, row stride ld) into the
-// swizzled LDS tile at lds_addr: ROWS/4 DMA instructions of 1 KB (4 rows) shared by 4 waves.
-template <int ROWS>
+// Stream ROWS rows of D bf16 (global row r0 + i, clamped to S-1, row stride ld) into the
+// swizzled LDS tile at lds_addr: DMA instructions of 1 KB (512/D rows) shared by 4 waves.
+template <int ROWS, int D>
 __device__ __forceinline__ void dma_tile(const bf16* base, int64_t ld, int r0, int S, unsigned lds_addr, int wave, int lane) {
 #pragma unroll
-  for (int i = 0; i < ROWS / 16; i++) {
+  for (int i = 0; i < ROWS * D / 2048; i++) {
     const int blk = i * 4 + wave;
     const int p = blk * 64 + lane;
-    const int row = p >> 4, ph = p & 15;
+    const int row = p / (D / 8), ph = p % (D / 8);
     const int gr = min(r0 + row, S - 1);
-    dma16(base + (int64_t)gr * ld + ((ph ^ swz(row)) << 3), lds_addr + blk * 1024);
+    dma16(base + (int64_t)gr * ld + ((ph ^ swz<D>(row)) << 3), lds_addr + blk * 1024);
   }
 }
 
@@ -152,24 +131,24 @@ __device__ __forceinline__ WgCoord decode_wg(int id, int ngroups, int rep) {
 }
 
 // The same tile transfer with everything lane-dependent hoisted out of the loop: a lane's byte
-// offset (row * ld + swizzled chunk) inside a 16-row group is computed once, and since the
-// swizzle only looks at row bits 0-3 the ROWS/16 DMA instructions of a transfer differ by a
-// wave-uniform 16 * ld elements, which goes into the scalar base: one vector register per
+// offset (row * ld + swizzled chunk) inside the rows of one instruction of the four waves is computed
+// once, and since the swizzle only looks at row bits 0-3 the DMA instructions of a transfer differ by
+// a wave-uniform 2048/D rows, which go into the scalar base: one vector register per
 // operand whatever the tile height.  Only for tiles that lie entirely inside the sequence (no
 // row clamping).
-template <int ROWS>
+template <int ROWS, int D>
 struct TileDma {
   unsigned off;
   int64_t step;
   __device__ __forceinline__ void init(int64_t ld, int wave, int lane) {
     const int p = wave * 64 + lane;
-    const int row = p >> 4, ph = p & 15;
-    off = (unsigned)((row * ld + ((ph ^ swz(row)) << 3)) * 2);
-    step = 16 * ld;
+    const int row = p / (D / 8), ph = p % (D / 8);
+    off = (unsigned)((row * ld + ((ph ^ swz<D>(row)) << 3)) * 2);
+    step = (2048 / D) * ld;
   }
   __device__ __forceinline__ void issue(const bf16* row0, unsigned lds_addr, int wave) const {
 #pragma unroll
-    for (int i = 0; i < ROWS / 16; i++) dma16_s(row0 + i * step, off, lds_addr + (i * 4 + wave) * 1024);
+    for (int i = 0; i < ROWS * D / 2048; i++) dma16_s(row0 + i * step, off, lds_addr + (i * 4 + wave) * 1024);
   }
 };
 
@@ -192,12 +171,13 @@ __device__ __forceinline__ bf16x8 pack_bf16x8(const f32x16& a, int base) {
 // ---------------------------------------------------------------------------------------
 // Forward.  grid = ceil(S/128)*H*B workgroups (see decode_wg); 256 threads; wave w owns queries i0+32w .. +31.
 // ---------------------------------------------------------------------------------------
-template <bool CAP>
+template <int D, bool CAP>
 __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     bf16* __restrict__ O, float* __restrict__ LSE, int S, int H, int KH, int64_t ldq, int64_t ldk,
     int64_t ldv, int64_t ldo, float scale, int window, float cap) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [2][K 16K | V 16K]
+  constexpr int TILE = 64 * D * 2;  // bytes of a K or V tile of 64 keys
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [2][K | V]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
   const int l32 = lane & 31, lhi = lane >> 5;
@@ -211,42 +191,42 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
   const int qi = iw0 + l32;        // this lane's query
   const int qic = min(qi, S - 1);
 
-  bf16x8 qf[8];
+  bf16x8 qf[D / 16];
   {
-    const bf16* qp = Q + ((int64_t)b * S + qic) * ldq + h * 128 + lhi * 8;
+    const bf16* qp = Q + ((int64_t)b * S + qic) * ldq + h * D + lhi * 8;
 #pragma unroll
-    for (int s = 0; s < 8; s++) qf[s] = *reinterpret_cast<const bf16x8*>(qp + s * 16);
+    for (int s = 0; s < D / 16; s++) qf[s] = *reinterpret_cast<const bf16x8*>(qp + s * 16);
   }
   const int j_lo = window >= 0 ? max(0, i0 - window) : 0;
   const int t_lo = j_lo >> 6;
   const int t_hi = min(i0 + 127, S - 1) >> 6;  // inclusive
 
-  f32x16 o[4];
+  f32x16 o[D / 32];
 #pragma unroll
-  for (int dt = 0; dt < 4; dt++)
+  for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
     for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
   float m = -INFINITY, lsum = 0.f;
 
-  const bf16* kbase = K + (int64_t)b * S * ldk + kh * 128;
-  const bf16* vbase = V + (int64_t)b * S * ldv + kh * 128;
+  const bf16* kbase = K + (int64_t)b * S * ldk + kh * D;
+  const bf16* vbase = V + (int64_t)b * S * ldv + kh * D;
   const unsigned lds0 = lds_addr_of(smem);
   const int wv = __builtin_amdgcn_readfirstlane(wave);
-  TileDma<64> dk, dv;
+  TileDma<64, D> dk, dv;
   dk.init(ldk, wv, lane);
   dv.init(ldv, wv, lane);
   auto load_kv = [&](int t, int stage) {
     if (t * 64 + 64 <= S) {
-      dk.issue(kbase + (int64_t)t * 64 * ldk, lds0 + stage * 32768, wv);
-      dv.issue(vbase + (int64_t)t * 64 * ldv, lds0 + stage * 32768 + 16384, wv);
+      dk.issue(kbase + (int64_t)t * 64 * ldk, lds0 + stage * (2 * TILE), wv);
+      dv.issue(vbase + (int64_t)t * 64 * ldv, lds0 + stage * (2 * TILE) + TILE, wv);
     } else {
-      dma_tile<64>(kbase, ldk, t * 64, S, lds0 + stage * 32768, wv, lane);
-      dma_tile<64>(vbase, ldv, t * 64, S, lds0 + stage * 32768 + 16384, wv, lane);
+      dma_tile<64, D>(kbase, ldk, t * 64, S, lds0 + stage * (2 * TILE), wv, lane);
+      dma_tile<64, D>(vbase, ldv, t * 64, S, lds0 + stage * (2 * TILE) + TILE, wv, lane);
     }
   };
   const float sc2 = scale * LOG2E;
   const float cap_c1 = CAP ? 2.f * sc2 / cap : 0.f, cap_l2 = cap * LOG2E;  // soft-cap: see cap_tanh
-  FragAddr fa;
+  FragAddr<D> fa;
   fa.init(lane);
 
   load_kv(t_lo, 0);
@@ -259,15 +239,15 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
     // skip tiles this wave cannot see at all
     const bool visible = (j0 <= iw0 + 31) && (window < 0 || j0 + 63 >= iw0 - window);
     if (visible) {
-      const unsigned char* sk = smem + cur * 32768;
-      const unsigned char* sv = sk + 16384;
+      const unsigned char* sk = smem + cur * (2 * TILE);
+      const unsigned char* sv = sk + TILE;
       f32x16 st[2];
 #pragma unroll
       for (int jt = 0; jt < 2; jt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) st[jt][r] = 0.f;
 #pragma unroll
-      for (int s = 0; s < 8; s++)
+      for (int s = 0; s < D / 16; s++)
 #pragma unroll
         for (int jt = 0; jt < 2; jt++)
           st[jt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sk, jt * 32, s), qf[s], st[jt], 0, 0, 0);
@@ -307,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
         lsum *= alpha;
         m = m_new;
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++)
+        for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
           for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
       }
@@ -320,10 +300,16 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
       bf16x8 pb[4];
 #pragma unroll
       for (int u = 0; u < 4; u++) pb[u] = pack_bf16x8(st[u >> 1], (u & 1) * 8);
-      // row sum of the probabilities AS THE P.V PRODUCT SEES THEM (bf16), two per instruction
+      // Row sum.  D = 128: of the probabilities AS THE P.V PRODUCT SEES THEM (bf16), two per instruction
       // (v_dot2c_f32_bf16 against a pair of ones, two accumulators): numerator and denominator
-      // of the softmax then carry the same rounding
-      {
+      // of the softmax then carry the same rounding.  D = 64: in fp32, as the one-wave-per-query kernel that
+      // took this head_dim before sums them (LSE to 4e-8 instead of 3e-5; the kernel has registers and issue slots to spare).
+      if constexpr (D == 64) {
+        float ps0 = 0.f, ps1 = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) { ps0 += st[0][r]; ps1 += st[1][r]; }
+        lsum += ps0 + ps1;
+      } else {
         float ps0 = 0.f, ps1 = 0.f;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -337,7 +323,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
 #pragma unroll
       for (int u = 0; u < 4; u++)
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++)
+        for (int dt = 0; dt < D / 32; dt++)
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_tr(sv, u * 16, dt), pb[u], o[dt], 0, 0, 0);
     }
     dma_wait_all();
@@ -346,9 +332,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
   const float ltot = half_swap_sum(lsum);
   const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
   if (qi < S) {
-    bf16* op = O + ((int64_t)b * S + qi) * ldo + h * 128;
+    bf16* op = O + ((int64_t)b * S + qi) * ldo + h * D;
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
       for (int g = 0; g < 4; g++) {
         Pack4 pk;
@@ -363,12 +349,13 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
 // ---------------------------------------------------------------------------------------
 // dQ.  Same tiling and grid as the forward; K/V tiles stream through LDS.
 // ---------------------------------------------------------------------------------------
-template <bool CAP>
+template <int D, bool CAP>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     const bf16* __restrict__ O, const bf16* __restrict__ dO, const float* __restrict__ LSE,
     float* __restrict__ DELTA, bf16* __restrict__ dQ, int S, int H, int KH, int64_t ldq, int64_t ldk,
     int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, float scale, int window, float cap) {
+  constexpr int TILE = 64 * D * 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
@@ -383,17 +370,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const int qi = iw0 + l32;
   const int qic = min(qi, S - 1);
 
-  bf16x8 qf[8], dof[8];
+  bf16x8 qf[D / 16], dof[D / 16];
   // delta[b,h,i] = sum_d dO[i,h,d] * O[i,h,d]: the two lanes of a query each hold half of its dO
   // row already, so the row sum costs one pass over O here; it is also written out for the dK/dV
   // kernel, which runs after this one.
   float dlt = 0.f;
   {
-    const bf16* qp = Q + ((int64_t)b * S + qic) * ldq + h * 128 + lhi * 8;
-    const bf16* dp = dO + ((int64_t)b * S + qic) * lddo + h * 128 + lhi * 8;
-    const bf16* op = O + ((int64_t)b * S + qic) * ldo + h * 128 + lhi * 8;
+    const bf16* qp = Q + ((int64_t)b * S + qic) * ldq + h * D + lhi * 8;
+    const bf16* dp = dO + ((int64_t)b * S + qic) * lddo + h * D + lhi * 8;
+    const bf16* op = O + ((int64_t)b * S + qic) * ldo + h * D + lhi * 8;
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
+    for (int s = 0; s < D / 16; s++) {
       qf[s] = *reinterpret_cast<const bf16x8*>(qp + s * 16);
       dof[s] = *reinterpret_cast<const bf16x8*>(dp + s * 16);
       const bf16x8 of = *reinterpret_cast<const bf16x8*>(op + s * 16);
@@ -410,32 +397,32 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const int t_lo = j_lo >> 6;
   const int t_hi = min(i0 + 127, S - 1) >> 6;
 
-  f32x16 dq[4];
+  f32x16 dq[D / 32];
 #pragma unroll
-  for (int dt = 0; dt < 4; dt++)
+  for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
     for (int r = 0; r < 16; r++) dq[dt][r] = 0.f;
 
-  const bf16* kbase = K + (int64_t)b * S * ldk + kh * 128;
-  const bf16* vbase = V + (int64_t)b * S * ldv + kh * 128;
+  const bf16* kbase = K + (int64_t)b * S * ldk + kh * D;
+  const bf16* vbase = V + (int64_t)b * S * ldv + kh * D;
   const unsigned lds0 = lds_addr_of(smem);
   const int wv = __builtin_amdgcn_readfirstlane(wave);
-  TileDma<64> dk, dv;
+  TileDma<64, D> dk, dv;
   dk.init(ldk, wv, lane);
   dv.init(ldv, wv, lane);
   auto load_kv = [&](int t, int stage) {
     if (t * 64 + 64 <= S) {
-      dk.issue(kbase + (int64_t)t * 64 * ldk, lds0 + stage * 32768, wv);
-      dv.issue(vbase + (int64_t)t * 64 * ldv, lds0 + stage * 32768 + 16384, wv);
+      dk.issue(kbase + (int64_t)t * 64 * ldk, lds0 + stage * (2 * TILE), wv);
+      dv.issue(vbase + (int64_t)t * 64 * ldv, lds0 + stage * (2 * TILE) + TILE, wv);
     } else {
-      dma_tile<64>(kbase, ldk, t * 64, S, lds0 + stage * 32768, wv, lane);
-      dma_tile<64>(vbase, ldv, t * 64, S, lds0 + stage * 32768 + 16384, wv, lane);
+      dma_tile<64, D>(kbase, ldk, t * 64, S, lds0 + stage * (2 * TILE), wv, lane);
+      dma_tile<64, D>(vbase, ldv, t * 64, S, lds0 + stage * (2 * TILE) + TILE, wv, lane);
     }
   };
   const float sc2 = scale * LOG2E;
   const float cap_c1 = CAP ? 2.f * sc2 / cap : 0.f, cap_l2 = cap * LOG2E;  // soft-cap: see cap_tanh
 
-  FragAddrT<CAP> fa;  // the soft-cap variant is the one short of registers
+  FragAddr<D, CAP && D == 128> fa;  // the soft-cap variant is the one short of registers
   fa.init(lane);
 
   load_kv(t_lo, 0);
@@ -447,8 +434,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     const int j0 = t * 64;
     const bool visible = (j0 <= iw0 + 31) && (window < 0 || j0 + 63 >= iw0 - window);
     if (visible) {
-      const unsigned char* sk = smem + cur * 32768;
-      const unsigned char* sv = sk + 16384;
+      const unsigned char* sk = smem + cur * (2 * TILE);
+      const unsigned char* sv = sk + TILE;
       const bool need_mask = (j0 + 63 > iw0) || (window >= 0 && j0 < iw0 + 31 - window);
       // dS of one 32-key half from its scores and dP, packed as the B operand of the dQ product
       bf16x8 dsb[4];
@@ -479,7 +466,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
 #pragma unroll
         for (int r = 0; r < 16; r++) { st[jt][r] = 0.f; dpt[jt][r] = 0.f; }
 #pragma unroll
-        for (int s = 0; s < 8; s++) {
+        for (int s = 0; s < D / 16; s++) {
           st[jt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sk, jt * 32, s), qf[s], st[jt], 0, 0, 0);
           dpt[jt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sv, jt * 32, s), dof[s], dpt[jt], 0, 0, 0);
         }
@@ -494,16 +481,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
 #pragma unroll
       for (int u = 0; u < 4; u++)
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++)
+        for (int dt = 0; dt < D / 32; dt++)
           dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_tr(sk, u * 16, dt), dsb[u], dq[dt], 0, 0, 0);
     }
     dma_wait_all();
     __syncthreads();
   }
   if (qi < S) {
-    bf16* op = dQ + ((int64_t)b * S + qi) * lddq + h * 128;
+    bf16* op = dQ + ((int64_t)b * S + qi) * lddq + h * D;
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
       for (int g = 0; g < 4; g++) {
         Pack4 pk;
@@ -517,9 +504,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
 // ---------------------------------------------------------------------------------------
 // dK/dV.  grid = ceil(S/128)*KH*B workgroups; wave w owns keys j0+32w..+31 (K and V fragments stay in
 // registers); loops over the query heads of its group and over 32-row Q/dO tiles from the
-// diagonal downwards.  LDS: 2 stages of (Q 8K | dO 8K | lse 128 B | delta 128 B) + V tile 32K.
+// diagonal downwards.  LDS: 2 stages of (Q | dO | lse 128 B | delta 128 B) + V tile of 128 keys.
 // ---------------------------------------------------------------------------------------
-template <bool CAP>
+template <int D, bool CAP>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     const bf16* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ DELTA,
@@ -527,7 +514,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     int64_t ldv, int64_t lddo, int64_t lddk, int64_t lddv, float scale, int window, float cap) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int QT = 32;                   // query rows per iteration
-  constexpr int STAGE = 2 * QT * 256 + 256;  // Q | dO | lse, delta
+  constexpr int TILE = QT * D * 2;
+  constexpr int STAGE = 2 * TILE + 256;  // Q | dO | lse, delta
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
   const int l32 = lane & 31, lhi = lane >> 5;
@@ -543,15 +531,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 
   // K fragments of this wave's 32 keys stay in registers; the V tile of the whole workgroup
   // (128 keys) is parked in LDS behind the two stages and re-read as B operand every iteration
-  bf16x8 kf[8];
+  bf16x8 kf[D / 16];
   {
-    const bf16* kp = K + ((int64_t)b * S + kjc) * ldk + kh * 128 + lhi * 8;
+    const bf16* kp = K + ((int64_t)b * S + kjc) * ldk + kh * D + lhi * 8;
 #pragma unroll
-    for (int s = 0; s < 8; s++) kf[s] = *reinterpret_cast<const bf16x8*>(kp + s * 16);
+    for (int s = 0; s < D / 16; s++) kf[s] = *reinterpret_cast<const bf16x8*>(kp + s * 16);
   }
-  f32x16 dk[4], dv[4];
+  f32x16 dk[D / 32], dv[D / 32];
 #pragma unroll
-  for (int dt = 0; dt < 4; dt++)
+  for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
     for (int r = 0; r < 16; r++) { dk[dt][r] = 0.f; dv[dt][r] = 0.f; }
 
@@ -566,7 +554,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   const int wv = __builtin_amdgcn_readfirstlane(wave);
 
   float sreg = 0.f;
-  TileDma<QT> tq, tdo;
+  TileDma<QT, D> tq, tdo;
   tq.init(ldq, wv, lane);
   tdo.init(lddo, wv, lane);
   // (head, tile) of the next tile to load; heads of the K/V group outermost
@@ -578,11 +566,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
       ++ld_h;
     }
     if (t * QT + QT <= S) {
-      tq.issue(Q + ((int64_t)b * S + t * QT) * ldq + hq * 128, lds0 + stage * STAGE, wv);
-      tdo.issue(dO + ((int64_t)b * S + t * QT) * lddo + hq * 128, lds0 + stage * STAGE + QT * 256, wv);
+      tq.issue(Q + ((int64_t)b * S + t * QT) * ldq + hq * D, lds0 + stage * STAGE, wv);
+      tdo.issue(dO + ((int64_t)b * S + t * QT) * lddo + hq * D, lds0 + stage * STAGE + TILE, wv);
     } else {
-      dma_tile<QT>(Q + (int64_t)b * S * ldq + hq * 128, ldq, t * QT, S, lds0 + stage * STAGE, wv, lane);
-      dma_tile<QT>(dO + (int64_t)b * S * lddo + hq * 128, lddo, t * QT, S, lds0 + stage * STAGE + QT * 256, wv, lane);
+      dma_tile<QT, D>(Q + (int64_t)b * S * ldq + hq * D, ldq, t * QT, S, lds0 + stage * STAGE, wv, lane);
+      dma_tile<QT, D>(dO + (int64_t)b * S * lddo + hq * D, lddo, t * QT, S, lds0 + stage * STAGE + TILE, wv, lane);
     }
     if (tid < 2 * QT) {
       const int ii = min(t * QT + (tid & (QT - 1)), S - 1);
@@ -593,13 +581,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   // (the log2 scaling of LSE happens here, not at the load: touching the loaded value there
   // would make wave 0 wait out the memory latency at the top of every iteration)
   auto store_stats = [&](int stage) {
-    if (tid < 2 * QT) reinterpret_cast<float*>(smem + stage * STAGE + 2 * QT * 256)[tid] = tid < QT ? sreg * LOG2E : sreg;
+    if (tid < 2 * QT) reinterpret_cast<float*>(smem + stage * STAGE + 2 * TILE)[tid] = tid < QT ? sreg * LOG2E : sreg;
   };
 
-  FragAddr fa;
+  FragAddr<D> fa;
   fa.init(lane);
-  const unsigned char* svt = smem + 2 * STAGE;  // [128 keys][128] V tile
-  dma_tile<128>(V + (int64_t)b * S * ldv + kh * 128, ldv, j0, S, lds0 + 2 * STAGE, wv, lane);
+  const unsigned char* svt = smem + 2 * STAGE;  // [128 keys][D] V tile
+  dma_tile<128, D>(V + (int64_t)b * S * ldv + kh * D, ldv, j0, S, lds0 + 2 * STAGE, wv, lane);
   load_tile(0);
   store_stats(0);
   dma_wait_all();
@@ -614,8 +602,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     const bool visible = (ib + QT - 1 >= jw0) && (window < 0 || ib <= jw0 + 31 + window);
     if (visible) {
       const unsigned char* sq = smem + CUR * STAGE;
-      const unsigned char* so = sq + QT * 256;
-      const float* slse = reinterpret_cast<const float*>(sq + 2 * QT * 256);
+      const unsigned char* so = sq + TILE;
+      const float* slse = reinterpret_cast<const float*>(sq + 2 * TILE);
       const float* sdel = slse + QT;
       // every (query, key) pair of the tile is visible unless the tile touches the diagonal, the
       // window edge or the end of the sequence
@@ -630,7 +618,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
         for (int e = 0; e < 4; e++) { sa[g * 4 + e] = 0.f; dpa[g * 4 + e] = d4[e]; }
       }
 #pragma unroll
-      for (int s = 0; s < 8; s++) {
+      for (int s = 0; s < D / 16; s++) {
         sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sq, 0, s), kf[s], sa, 0, 0, 0);
         dpa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(so, 0, s), fa.load_kc(svt, wave * 32, s), dpa, 0, 0, 0);
       }
@@ -667,7 +655,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 #pragma unroll
       for (int u = 0; u < 2; u++)
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
+        for (int dt = 0; dt < D / 32; dt++) {
           dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_tr(so, u * 16, dt), pb[u], dv[dt], 0, 0, 0);
           dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_tr(sq, u * 16, dt), dsb[u], dk[dt], 0, 0, 0);
         }
@@ -688,10 +676,10 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     }
   }
   if (kj < S) {
-    bf16* kp = dK + ((int64_t)b * S + kj) * lddk + kh * 128;
-    bf16* vp = dV + ((int64_t)b * S + kj) * lddv + kh * 128;
+    bf16* kp = dK + ((int64_t)b * S + kj) * lddk + kh * D;
+    bf16* vp = dV + ((int64_t)b * S + kj) * lddv + kh * D;
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
       for (int g = 0; g < 4; g++) {
         Pack4 pk, pv;
@@ -708,7 +696,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 
 // ---------------------------------------------------------------------------------------
 // Any head_dim (<= 256): one wave per (batch, head, query); scores staged in LDS.
-// Used by the small shapes of unit tests and the CPU-sized reference configuration.
+// Takes what the MFMA kernels do not: other head_dims and unaligned views.
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void attn_fwd_generic(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
@@ -807,48 +795,78 @@ __global__ void strided_cast_f32_bf16(const float* __restrict__ in, bf16* __rest
   out[(i / cols) * ldo + i % cols] = f2bf(in[i]);
 }
 
-bool fast_ok(int D, const void* q, const void* k, const void* v, const void* o, int64_t ldq,
+// What the MFMA kernels take: head_dim 128, or 64 at lengths the one-wave-per-query kernels take too (the two
+// head_dims of the configurations that train; any other one, and unaligned views, stay on those kernels, which
+// hold a row of scores in LDS), 16-byte aligned operands.  head_dim 64, 4 heads, 4 sequences of 512: forward 620 -> 19 us,
+// backward 1850 -> 40 us; 8 heads over 2, 2 sequences of 2048: 6740 -> 36 us, 21100 -> 310 us.
+bool fast_ok(int D, int S, int max_s, const void* q, const void* k, const void* v, const void* o, int64_t ldq,
              int64_t ldk, int64_t ldv, int64_t ldo) {
-  return D == 128 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) && ldq % 8 == 0 &&
+  return (D == 128 || (D == 64 && S <= max_s)) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) && ldq % 8 == 0 &&
          ldk % 8 == 0 && ldv % 8 == 0 && ldo % 8 == 0;
 }
+constexpr int GENERIC_MAX_S_FWD = 16384, GENERIC_MAX_S_BWD = 8192;  // 64 KB of LDS: one, two floats per key
 
 bool bwd_fast_ok(const void* q, const void* k, const void* v, const void* o, const void* d_o, const void* dq, const void* dk,
-                 const void* dv, int D, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq,
+                 const void* dv, int S, int D, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq,
                  int64_t lddk, int64_t lddv) {
-  return fast_ok(D, q, k, v, o, ldq, ldk, ldv, ldo) && aligned16(d_o) && aligned16(dq) && aligned16(dk) && aligned16(dv) &&
-         lddo % 8 == 0 && lddq % 8 == 0 && lddk % 8 == 0 && lddv % 8 == 0;
+  return fast_ok(D, S, GENERIC_MAX_S_BWD, q, k, v, o, ldq, ldk, ldv, ldo) && aligned16(d_o) && aligned16(dq) && aligned16(dk) &&
+         aligned16(dv) && lddo % 8 == 0 && lddq % 8 == 0 && lddk % 8 == 0 && lddv % 8 == 0;
 }
 
-constexpr int SM_KV = 2 * (2 * 32 * 256 + 256) + 128 * 256;
+constexpr int smem_q(int D) { return 2 * 2 * 64 * D * 2; }                          // forward, dQ
+constexpr int smem_kv(int D) { return 2 * (2 * 32 * D * 2 + 256) + 128 * D * 2; }  // dK/dV
+
 // dynamic-LDS limits of the backward kernels, set once per process
+template <int D>
+void bwd_fast_attributes_d() {
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
+}
 void bwd_fast_attributes() {
   static std::once_flag once;
   std::call_once(once, [] {
-    (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SM_KV);
-    (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, SM_KV);
-    (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536);
-    (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536);
+    bwd_fast_attributes_d<128>();
+    bwd_fast_attributes_d<64>();
   });
 }
 
-// The two MFMA kernels of the backward pass (head_dim 128); delta: fp32 [B, H, S] scratch, fully
+// The two MFMA kernels of the backward pass; delta: fp32 [B, H, S] scratch, fully
 // written by the dQ kernel (each workgroup computes the entries of its own queries) before the
 // dK/dV kernel, launched after it, reads them.
+template <int D>
 void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const bf16* vp, const bf16* op, const float* lse,
                      const bf16* gop, bf16* dq, bf16* dk, bf16* dv, float* delta, int B, int S, int H, int KH, int64_t ldq,
                      int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, int64_t lddk, int64_t lddv, int window,
                      float softcap) {
-  const float scale = 1.f / sqrtf(128.f);
+  const float scale = 1.f / sqrtf((float)D);
   dim3 gkv((unsigned)(((S + 127) / 128) * KH * B)), gq((unsigned)(((S + 127) / 128) * H * B));
   bwd_fast_attributes();
-  if (softcap > 0.f) {
-    hipLaunchKernelGGL(attn_bwd_dq_kernel<true>, gq, dim3(256), 65536, stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
-    hipLaunchKernelGGL(attn_bwd_dkv_kernel<true>, gkv, dim3(256), SM_KV, stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap);
-  } else {
-    hipLaunchKernelGGL(attn_bwd_dq_kernel<false>, gq, dim3(256), 65536, stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
-    hipLaunchKernelGGL(attn_bwd_dkv_kernel<false>, gkv, dim3(256), SM_KV, stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap);
-  }
+  auto go = [&](auto cap) {
+    constexpr bool CAP = decltype(cap)::value;
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<D, CAP>), gq, dim3(256), smem_q(D), stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
+    hipLaunchKernelGGL((attn_bwd_dkv_kernel<D, CAP>), gkv, dim3(256), smem_kv(D), stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap);
+  };
+  if (softcap > 0.f) go(std::true_type());
+  else go(std::false_type());
+}
+
+template <int D>
+void launch_fwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const bf16* vp, bf16* o, float* lse, int B, int S, int H,
+                     int KH, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int window, float softcap) {
+  const float scale = 1.f / sqrtf((float)D);
+  dim3 grid((unsigned)(((S + 127) / 128) * H * B));
+  static std::once_flag once;  // per head_dim
+  std::call_once(once, [] {
+    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
+    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
+  });
+  auto go = [&](auto cap) {
+    hipLaunchKernelGGL((attn_fwd_kernel<D, decltype(cap)::value>), grid, dim3(256), smem_q(D), stream, qp, kp, vp, o, lse, S, H, KH, ldq, ldk, ldv, ldo, scale, window, softcap);
+  };
+  if (softcap > 0.f) go(std::true_type());
+  else go(std::false_type());
 }
 
 }  // namespace
@@ -865,20 +883,11 @@ extern "C" int32_t olmax_attn_fwd(hipStream_t stream, const void* q, const void*
   OLMAX_CHECK(ldq >= (int64_t)H * D && ldo >= (int64_t)H * D && ldk >= (int64_t)KH * D && ldv >= (int64_t)KH * D, OLMAX_ERR_SHAPE, "olmax_attn_fwd: row stride smaller than heads*head_dim");
   const float scale = 1.f / sqrtf((float)D);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k, *vp = (const bf16*)v;
-  if (fast_ok(D, q, k, v, o, ldq, ldk, ldv, ldo)) {
-    dim3 grid((unsigned)(((S + 127) / 128) * H * B));
-    static std::once_flag once;
-    std::call_once(once, [] {
-      (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536);
-      (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536);
-    });
-    if (softcap > 0.f) {
-      hipLaunchKernelGGL(attn_fwd_kernel<true>, grid, dim3(256), 65536, stream, qp, kp, vp, (bf16*)o, lse, S, H, KH, ldq, ldk, ldv, ldo, scale, window, softcap);
-    } else {
-      hipLaunchKernelGGL(attn_fwd_kernel<false>, grid, dim3(256), 65536, stream, qp, kp, vp, (bf16*)o, lse, S, H, KH, ldq, ldk, ldv, ldo, scale, window, softcap);
-    }
+  if (fast_ok(D, S, GENERIC_MAX_S_FWD, q, k, v, o, ldq, ldk, ldv, ldo)) {
+    auto go = D == 128 ? launch_fwd_fast<128> : launch_fwd_fast<64>;
+    go(stream, qp, kp, vp, (bf16*)o, lse, B, S, H, KH, ldq, ldk, ldv, ldo, window, softcap);
   } else {
-    OLMAX_CHECK(D <= 256 && (size_t)S * 4 <= 65536, OLMAX_ERR_SHAPE, "olmax_attn_fwd: generic path supports head_dim <= 256 and seq_len <= 16384");
+    OLMAX_CHECK(D <= 256 && S <= GENERIC_MAX_S_FWD, OLMAX_ERR_SHAPE, "olmax_attn_fwd: generic path supports head_dim <= 256 and seq_len <= 16384");
     hipLaunchKernelGGL(attn_fwd_generic, dim3(S, H, B), dim3(64), (size_t)S * 4, stream, qp, kp, vp, (bf16*)o, lse, S, H, KH, D, ldq, ldk, ldv, ldo, scale, window, softcap);
   }
   OLMAX_LAUNCH_CHECK();
@@ -911,14 +920,15 @@ extern "C" int32_t olmax_attn_bwd(hipStream_t stream, const void* q, const void*
   const float scale = 1.f / sqrtf((float)D);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k, *vp = (const bf16*)v, *op = (const bf16*)o, *gop = (const bf16*)d_o;
   float* delta = (float*)workspace;
-  if (bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv)) {
-    launch_bwd_fast(stream, qp, kp, vp, op, lse, gop, (bf16*)dq, (bf16*)dk, (bf16*)dv, delta, B, S, H, KH, ldq, ldk, ldv, ldo, lddo,
-                    lddq, lddk, lddv, window, softcap);
+  if (bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, S, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv)) {
+    auto go = D == 128 ? launch_bwd_fast<128> : launch_bwd_fast<64>;
+    go(stream, qp, kp, vp, op, lse, gop, (bf16*)dq, (bf16*)dk, (bf16*)dv, delta, B, S, H, KH, ldq, ldk, ldv, ldo, lddo,
+       lddq, lddk, lddv, window, softcap);
   } else {
-    OLMAX_CHECK(D <= 256 && (size_t)S * 8 <= 65536, OLMAX_ERR_SHAPE, "olmax_attn_bwd: generic path supports head_dim <= 256 and seq_len <= 8192");
+    OLMAX_CHECK(D <= 256 && S <= GENERIC_MAX_S_BWD, OLMAX_ERR_SHAPE, "olmax_attn_bwd: generic path supports head_dim <= 256 and seq_len <= 8192");
     const int64_t accb = attn_acc_bytes(B, S, KH, D);
     OLMAX_CHECK(workspace_bytes >= attn_delta_bytes(B, S, H) + 2 * accb, OLMAX_ERR_WORKSPACE,
-                "olmax_attn_bwd: the generic path (head_dim != 128, or operands not 16-byte aligned) needs %ld workspace bytes",
+                "olmax_attn_bwd: the generic path (head_dim not 128 or 64, or operands not 16-byte aligned) needs %ld workspace bytes",
                 (long)(attn_delta_bytes(B, S, H) + 2 * accb));
     float* dkf = (float*)((char*)workspace + attn_delta_bytes(B, S, H));
     float* dvf = (float*)((char*)dkf + accb);
@@ -995,7 +1005,7 @@ extern "C" int32_t olmax_attn_bwd_noalloc(hipStream_t stream, const void* q, con
   OLMAX_CHECK((int64_t)B * H * S <= ATTN_SCRATCH_FLOATS, OLMAX_ERR_WORKSPACE,
               "olmax_attn_bwd_noalloc: batch*heads*seq_len = %ld exceeds the built-in scratch of %ld rows; use olmax_attn_bwd with a workspace",
               (long)((int64_t)B * H * S), (long)ATTN_SCRATCH_FLOATS);
-  OLMAX_CHECK(bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv), OLMAX_ERR_ALIGN,
+  OLMAX_CHECK(D == 128 && bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, S, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv), OLMAX_ERR_ALIGN,
               "olmax_attn_bwd_noalloc: needs head_dim 128, 16-byte aligned pointers and row strides that are multiples of 8; use olmax_attn_bwd otherwise");
   float* delta = nullptr;
   {
@@ -1005,7 +1015,7 @@ extern "C" int32_t olmax_attn_bwd_noalloc(hipStream_t stream, const void* q, con
     int rc = scratch_for_current_device(&delta, !capturing);
     if (rc) return rc;
   }
-  launch_bwd_fast(stream, (const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)o, lse, (const bf16*)d_o, (bf16*)dq, (bf16*)dk,
+  launch_bwd_fast<128>(stream, (const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)o, lse, (const bf16*)d_o, (bf16*)dq, (bf16*)dk,
                   (bf16*)dv, delta, B, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv, window, softcap);
   OLMAX_LAUNCH_CHECK();
   return OLMAX_OK;

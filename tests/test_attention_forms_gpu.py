@@ -1,0 +1,57 @@
+"""GPU parity tests of the MFMA attention kernels' head_dim-64 form at the edges of their 128-row blocks,
+64-key and 32-query tiles."""
+import math
+
+import pytest
+import torch
+
+from oracle import ref
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+
+def rnd(*shape, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(*shape, device="cuda", generator=g).to(BF)
+
+
+def rel(got, want):
+    got, want = got.double().cpu(), want.double().cpu()
+    return ((got - want).norm() / (want.norm() + 1e-300)).item()
+
+
+def check(B, S, H, KH, D, window, softcap, strided=False):
+    """Every output against the float64 oracle.  P and dS are rounded to bf16 (2^-9 each) before the second products
+    and the results once more: 2-norm errors of 0.3 % at most; bounds are three times that."""
+    from olmax_amd import ops
+
+    print(f"[case] attn B{B} S{S} H{H} KH{KH} D{D} w{window} cap{softcap}", flush=True)
+    if strided:  # q | k | v columns of one projection
+        qkv = rnd(B * S, (H + 2 * KH) * D, seed=S + D)
+        q, k, v = qkv[:, :H * D], qkv[:, H * D:(H + KH) * D], qkv[:, (H + KH) * D:]
+    else:
+        q, k, v = rnd(B * S, H * D, seed=1), rnd(B * S, KH * D, seed=2), rnd(B * S, KH * D, seed=3)
+    do = rnd(B * S, H * D, seed=4)
+    kw = dict(B=B, S=S, H=H, KH=KH, D=D, window=window, softcap=softcap)
+    guard = torch.full((B * S + 2, H * D), 7.0, device="cuda", dtype=BF)  # nothing outside the output rows is written
+    o, lse = ops.attn_fwd(q, k, v, out=guard[1:-1], **kw)
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+    dq, dk, dv = ops.attn_bwd(q, k, v, o, lse, do, **kw)
+    q4, k4, v4, d4 = (t.cpu().double().reshape(B, S, -1, D) for t in (q, k, v, do))
+    wo, wlse = ref.attention_fwd(q4, k4, v4, window=window, softcap=softcap)
+    assert rel(o, wo.reshape(B * S, -1)) < 1e-2
+    assert (lse.cpu().double() - wlse).abs().max() < 2e-3
+    want = ref.attention_bwd(q4, k4, v4, wo, wlse, d4, window=window, softcap=softcap)
+    for name, got, w in zip(("dq", "dk", "dv"), (dq, dk, dv), want):
+        if w.norm() < 1e-12 * math.sqrt(w.numel()):  # S = 1: dS is exactly zero, what remains is rounding
+            assert got.double().norm() < 1e-2 * math.sqrt(got.numel()), name
+        else:
+            assert rel(got, w.reshape(B * S, -1)) < 1e-2, name
+
+
+@pytest.mark.parametrize("S", [1, 31, 33, 63, 65, 127, 128, 129, 192, 321])
+@pytest.mark.parametrize("H,KH,window,softcap", [(4, 4, None, 0.0), (4, 2, 40, 0.0), (2, 1, None, 30.0)])
+def test_head_dim_64(S, H, KH, window, softcap):
+    check(2, S, H, KH, 64, window, softcap, strided=S % 2 == 1)
