@@ -502,12 +502,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// dK/dV.  grid = ceil(S/128)*KH*B workgroups; wave w owns keys j0+32w..+31 (K and V fragments stay in
-// registers); loops over the query heads of its group and over 32-row Q/dO tiles from the
-// diagonal downwards.  LDS: 2 stages of (Q | dO | lse 128 B | delta 128 B) + V tile of 128 keys.
+// dK/dV.  grid = ceil(S/(32 KW))*KH*B workgroups of KW x QS waves; wave (kw, qs) owns keys j0+32kw..+31
+// (K fragments stay in registers) and every QS-th of the iterations over the query heads of its
+// group and the 32-row Q/dO tiles from the diagonal downwards.  LDS: per query group 2 stages of
+// (Q | dO | lse 128 B | delta 128 B), then the V tile of 32 KW keys.
+// KW = 4, QS = 1: two workgroups per CU, no reduction; what a grid that fills the GPU takes.
+// KW = 2, QS = 4: one workgroup of eight waves per CU, half the keys and a quarter of the serial chain; the
+// four partial sums are added through LDS in group order.  See dkv_split.
 // ---------------------------------------------------------------------------------------
-template <int D, bool CAP>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
+template <int D, bool CAP, int KW, int QS>
+__global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     const bf16* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ DELTA,
     bf16* __restrict__ dK, bf16* __restrict__ dV, int S, int H, int KH, int64_t ldq, int64_t ldk,
@@ -516,21 +520,24 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   constexpr int QT = 32;                   // query rows per iteration
   constexpr int TILE = QT * D * 2;
   constexpr int STAGE = 2 * TILE + 256;  // Q | dO | lse, delta
+  constexpr int KT = KW * 32;            // keys of the workgroup
+  constexpr int TEAMS = KW * QS / 4;     // tiles are fetched by teams of 4 waves
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
   const int l32 = lane & 31, lhi = lane >> 5;
+  const int kw = wave % KW, qs = wave / KW;
   // key tile 0 is seen by every query: rank order is already longest first
-  const WgCoord wg = decode_wg(blockIdx.x, (int)(gridDim.x / ((S + 127) >> 7)), 1);
+  const WgCoord wg = decode_wg(blockIdx.x, (int)(gridDim.x / ((S + KT - 1) / KT)), 1);
   const int kt = wg.rank;
   const int b = wg.group / KH, kh = wg.group % KH;
   const int rep = H / KH;
-  const int j0 = kt * 128;
-  const int jw0 = j0 + wave * 32;
+  const int j0 = kt * KT;
+  const int jw0 = j0 + kw * 32;
   const int kj = jw0 + l32;  // this lane's key
   const int kjc = min(kj, S - 1);
 
   // K fragments of this wave's 32 keys stay in registers; the V tile of the whole workgroup
-  // (128 keys) is parked in LDS behind the two stages and re-read as B operand every iteration
+  // is parked in LDS behind the stages and re-read as B operand every iteration
   bf16x8 kf[D / 16];
   {
     const bf16* kp = K + ((int64_t)b * S + kjc) * ldk + kh * D + lhi * 8;
@@ -543,7 +550,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 #pragma unroll
     for (int r = 0; r < 16; r++) { dk[dt][r] = 0.f; dv[dt][r] = 0.f; }
 
-  const int i_hi = window >= 0 ? min(S - 1, j0 + 127 + window) : S - 1;
+  const int i_hi = window >= 0 ? min(S - 1, j0 + KT - 1 + window) : S - 1;
   const int t_lo = j0 / QT;
   const int t_hi = i_hi / QT;  // inclusive
   const int ntile = t_hi - t_lo + 1;
@@ -551,57 +558,79 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   const float sc2 = scale * LOG2E;
   const float cap_c1 = CAP ? 2.f * sc2 / cap : 0.f, cap_l2 = cap * LOG2E;  // soft-cap: see cap_tanh
   const unsigned lds0 = lds_addr_of(smem);
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const int wv = wave & 3, team = wave >> 2;
+  const unsigned char* sgrp = smem + qs * (2 * STAGE);  // this query group's stages
 
   float sreg = 0.f;
   TileDma<QT, D> tq, tdo;
   tq.init(ldq, wv, lane);
   tdo.init(lddo, wv, lane);
-  // (head, tile) of the next tile to load; heads of the K/V group outermost
-  int ld_h = kh * rep, ld_t = t_lo;
-  auto load_tile = [&](int stage) {
-    const int hq = ld_h, t = ld_t;
-    if (++ld_t > t_hi) {
-      ld_t = t_lo;
-      ++ld_h;
+  // (head, tile) of the next iteration to load of each query group this team fetches for, and of this
+  // wave's own group (its row statistics); heads of the K/V group outermost
+  struct Iter { int h, t; };
+  auto advance = [&](Iter& x, int n) {
+    x.t += n;
+    while (x.t > t_hi) {
+      x.t -= ntile;
+      ++x.h;
     }
-    if (t * QT + QT <= S) {
-      tq.issue(Q + ((int64_t)b * S + t * QT) * ldq + hq * D, lds0 + stage * STAGE, wv);
-      tdo.issue(dO + ((int64_t)b * S + t * QT) * lddo + hq * D, lds0 + stage * STAGE + TILE, wv);
-    } else {
-      dma_tile<QT, D>(Q + (int64_t)b * S * ldq + hq * D, ldq, t * QT, S, lds0 + stage * STAGE, wv, lane);
-      dma_tile<QT, D>(dO + (int64_t)b * S * lddo + hq * D, lddo, t * QT, S, lds0 + stage * STAGE + TILE, wv, lane);
+  };
+  Iter own{kh * rep, t_lo}, ld[QS / TEAMS];
+  advance(own, qs);
+#pragma unroll
+  for (int g = 0; g < QS / TEAMS; g++) {
+    ld[g] = Iter{kh * rep, t_lo};
+    advance(ld[g], g * TEAMS + team);
+  }
+  auto load_tile = [&](int round, int stage) {
+#pragma unroll
+    for (int g = 0; g < QS / TEAMS; g++) {
+      const int grp = g * TEAMS + team;
+      if (QS > 1 && round * QS + grp >= total) break;
+      const int hq = ld[g].h, t = ld[g].t;
+      advance(ld[g], QS);
+      const unsigned dst = lds0 + (grp * 2 + stage) * STAGE;
+      if (t * QT + QT <= S) {
+        tq.issue(Q + ((int64_t)b * S + t * QT) * ldq + hq * D, dst, wv);
+        tdo.issue(dO + ((int64_t)b * S + t * QT) * lddo + hq * D, dst + TILE, wv);
+      } else {
+        dma_tile<QT, D>(Q + (int64_t)b * S * ldq + hq * D, ldq, t * QT, S, dst, wv, lane);
+        dma_tile<QT, D>(dO + (int64_t)b * S * lddo + hq * D, lddo, t * QT, S, dst + TILE, wv, lane);
+      }
     }
-    if (tid < 2 * QT) {
-      const int ii = min(t * QT + (tid & (QT - 1)), S - 1);
-      const float* src = tid < QT ? LSE : DELTA;
-      sreg = src[((int64_t)b * H + hq) * S + ii];  // consumed by store_stats a whole iteration later
+    if (kw == 0 && (QS == 1 || round * QS + qs < total)) {
+      const int ii = min(own.t * QT + l32, S - 1);
+      const float* src = lane < QT ? LSE : DELTA;
+      sreg = src[((int64_t)b * H + own.h) * S + ii];  // consumed by store_stats a whole iteration later
     }
   };
   // (the log2 scaling of LSE happens here, not at the load: touching the loaded value there
   // would make wave 0 wait out the memory latency at the top of every iteration)
   auto store_stats = [&](int stage) {
-    if (tid < 2 * QT) reinterpret_cast<float*>(smem + stage * STAGE + 2 * TILE)[tid] = tid < QT ? sreg * LOG2E : sreg;
+    if (kw == 0) reinterpret_cast<float*>(smem + (qs * 2 + stage) * STAGE + 2 * TILE)[lane] = lane < QT ? sreg * LOG2E : sreg;
   };
 
   FragAddr<D> fa;
   fa.init(lane);
-  const unsigned char* svt = smem + 2 * STAGE;  // [128 keys][D] V tile
-  dma_tile<128, D>(V + (int64_t)b * S * ldv + kh * D, ldv, j0, S, lds0 + 2 * STAGE, wv, lane);
-  load_tile(0);
+  const unsigned char* svt = smem + QS * 2 * STAGE;  // [KT keys][D] V tile
+  if (team == 0) dma_tile<KT, D>(V + (int64_t)b * S * ldv + kh * D, ldv, j0, S, lds0 + QS * 2 * STAGE, wv, lane);
+  load_tile(0, 0);
   store_stats(0);
   dma_wait_all();
   __syncthreads();
-  // One iteration on the tile in stage CUR (a compile-time constant, so that every LDS address
-  // below is a loop-invariant register plus an immediate); `t` is the tile's query-tile index.
-  auto iteration = [&](auto cur_tag, int t, bool more) {
+  // One round on the tiles in stage CUR (a compile-time constant, so that every LDS address
+  // below is a loop-invariant register plus an immediate); `t` is the query-tile index of this wave's.
+  auto iteration = [&](auto cur_tag, int round, int t, bool more) {
     constexpr int CUR = decltype(cur_tag)::value;
-    if (more) load_tile(CUR ^ 1);
+    if (more) {
+      advance(own, QS);
+      load_tile(round + 1, CUR ^ 1);
+    }
     const int ib = t * QT;  // first query of the tile
     // this wave sees the tile iff some i in [ib, ib+QT) has j <= i <= j + window for its keys
-    const bool visible = (ib + QT - 1 >= jw0) && (window < 0 || ib <= jw0 + 31 + window);
+    const bool visible = (QS == 1 || round * QS + qs < total) && (ib + QT - 1 >= jw0) && (window < 0 || ib <= jw0 + 31 + window);
     if (visible) {
-      const unsigned char* sq = smem + CUR * STAGE;
+      const unsigned char* sq = sgrp + CUR * STAGE;
       const unsigned char* so = sq + TILE;
       const float* slse = reinterpret_cast<const float*>(sq + 2 * TILE);
       const float* sdel = slse + QT;
@@ -620,7 +649,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 #pragma unroll
       for (int s = 0; s < D / 16; s++) {
         sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sq, 0, s), kf[s], sa, 0, 0, 0);
-        dpa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(so, 0, s), fa.load_kc(svt, wave * 32, s), dpa, 0, 0, 0);
+        dpa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(so, 0, s), fa.load_kc(svt, kw * 32, s), dpa, 0, 0, 0);
       }
 #pragma unroll
       for (int g = 0; g < 4; g++) {
@@ -665,32 +694,60 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     __syncthreads();
   };
   {
-    int t = t_lo;  // query tile being consumed
-    for (int it = 0; it < total; it += 2) {
-      iteration(std::integral_constant<int, 0>(), t, it + 1 < total);
-      if (++t > t_hi) t = t_lo;
-      if (it + 1 < total) {
-        iteration(std::integral_constant<int, 1>(), t, it + 2 < total);
-        if (++t > t_hi) t = t_lo;
+    const int rounds = (total + QS - 1) / QS;
+    Iter cur{0, t_lo};  // query tile being consumed
+    advance(cur, qs);
+    for (int it = 0; it < rounds; it += 2) {
+      iteration(std::integral_constant<int, 0>(), it, cur.t, it + 1 < rounds);
+      advance(cur, QS);
+      if (it + 1 < rounds) {
+        iteration(std::integral_constant<int, 1>(), it + 1, cur.t, it + 2 < rounds);
+        advance(cur, QS);
       }
     }
   }
-  if (kj < S) {
-    bf16* kp = dK + ((int64_t)b * S + kj) * lddk + kh * D;
-    bf16* vp = dV + ((int64_t)b * S + kj) * lddv + kh * D;
+  bf16* kp = dK + ((int64_t)b * S + kjc) * lddk + kh * D;
+  bf16* vp = dV + ((int64_t)b * S + kjc) * lddv + kh * D;
+  auto store4 = [&](bf16* p, int dt, int g, const f32x4& v, float mul) {
+    Pack4 pk;
 #pragma unroll
-    for (int dt = 0; dt < D / 32; dt++)
+    for (int e = 0; e < 4; e++) pk.e[e] = f2bf(v[e] * mul);
+    *reinterpret_cast<u32x2*>(p + dt * 32 + g * 8 + lhi * 4) = pk.u;
+  };
+  if constexpr (QS == 1) {
+    if (kj < S) {
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        Pack4 pk, pv;
+      for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          pk.e[e] = f2bf(dk[dt][g * 4 + e] * scale);
-          pv.e[e] = f2bf(dv[dt][g * 4 + e]);
+        for (int g = 0; g < 4; g++) {
+          store4(kp, dt, g, f32x4{dk[dt][g * 4], dk[dt][g * 4 + 1], dk[dt][g * 4 + 2], dk[dt][g * 4 + 3]}, scale);
+          store4(vp, dt, g, f32x4{dv[dt][g * 4], dv[dt][g * 4 + 1], dv[dt][g * 4 + 2], dv[dt][g * 4 + 3]}, 1.f);
         }
-        *reinterpret_cast<u32x2*>(kp + dt * 32 + g * 8 + lhi * 4) = pk.u;
-        *reinterpret_cast<u32x2*>(vp + dt * 32 + g * 8 + lhi * 4) = pv.u;
+    }
+  } else {
+    // Partial sums through LDS (the stages are free: the last round ended in a barrier): a wave parks its
+    // accumulators as units of 4 floats per lane, [kw][qs][unit][lane], then adds its share of the units over the
+    // query groups.  dK first, then dV in the same space.
+    constexpr int UNITS = D / 8, MINE = UNITS / QS;
+    static_assert(UNITS % QS == 0, "units are dealt evenly to the query groups");
+    f32x4* park = reinterpret_cast<f32x4*>(smem) + kw * (QS * UNITS * 64) + lane;
+    auto reduce = [&](const f32x16 (&acc)[D / 32], bf16* p, float mul) {
+#pragma unroll
+      for (int u = 0; u < UNITS; u++)
+        park[(qs * UNITS + u) * 64] = f32x4{acc[u >> 2][(u & 3) * 4], acc[u >> 2][(u & 3) * 4 + 1], acc[u >> 2][(u & 3) * 4 + 2], acc[u >> 2][(u & 3) * 4 + 3]};
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < MINE; i++) {
+        const int u = qs * MINE + i;
+        f32x4 v = park[u * 64];
+#pragma unroll
+        for (int g = 1; g < QS; g++) v += park[(g * UNITS + u) * 64];
+        if (kj < S) store4(p, u >> 2, u & 3, v, mul);
       }
+    };
+    reduce(dk, kp, scale);
+    __syncthreads();
+    reduce(dv, vp, 1.f);
   }
 }
 
@@ -814,13 +871,19 @@ bool bwd_fast_ok(const void* q, const void* k, const void* v, const void* o, con
 }
 
 constexpr int smem_q(int D) { return 2 * 2 * 64 * D * 2; }                          // forward, dQ
-constexpr int smem_kv(int D) { return 2 * (2 * 32 * D * 2 + 256) + 128 * D * 2; }  // dK/dV
+// dK/dV: stages and V tile, or the parked partial sums
+constexpr int smem_kv(int D, int KW, int QS) {
+  const int run = QS * 2 * (2 * 32 * D * 2 + 256) + KW * 32 * D * 2, sums = QS > 1 ? KW * QS * 32 * D * 4 : 0;
+  return run > sums ? run : sums;
+}
 
 // dynamic-LDS limits of the backward kernels, set once per process
 template <int D>
 void bwd_fast_attributes_d() {
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D));
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, true, 4, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 4, 1));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, false, 4, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 4, 1));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, true, 2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 2, 4));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, false, 2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 2, 4));
   (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
   (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
 }
@@ -832,6 +895,19 @@ void bwd_fast_attributes() {
   });
 }
 
+// Whether dK/dV takes the split kernel.  One workgroup per key tile and K/V head is little parallel work when the
+// heads are few: 224 workgroups for 2 x 1777 tokens of 8 K/V heads leave the GPU waiting for those of the first key tile,
+// which walk the four query heads of 1777 tokens one 32-row tile at a time with one wave per SIMD.  Backward
+// (dQ included), us, plain -> split: 2 x 1777, 32 heads on 8: 453 -> 244; 1 x 4096: 962 -> 530; 1 x 300: 89 -> 47;
+// 3 x 1000, 8 on 8: 95 -> 71; 1 x 6000, 40 on 8 (376 workgroups): 1954 -> 1419.  From 512 workgroups on it depends on
+// the length of the chain: 32 tiles 111 -> 116, 64 tiles 189 -> 182, 256 tiles 606 -> 520, 628 tiles (640 workgroups)
+// 1647 -> 1541; a filled GPU is better off without the halved reuse of Q and dO (1024: 1213 -> 1279, 2048: 1029 -> 1136).
+bool dkv_split(int B, int S, int H, int KH, int window) {
+  const int64_t n = (int64_t)((S + 127) / 128) * KH * B;
+  const int64_t chain = (int64_t)(H / KH) * ((window >= 0 && window < S - 128 ? window + 128 : S) / 32);
+  return n < 512 || (n < 1024 && chain >= 64);
+}
+
 // The two MFMA kernels of the backward pass; delta: fp32 [B, H, S] scratch, fully
 // written by the dQ kernel (each workgroup computes the entries of its own queries) before the
 // dK/dV kernel, launched after it, reads them.
@@ -841,12 +917,17 @@ void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const b
                      int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, int64_t lddk, int64_t lddv, int window,
                      float softcap) {
   const float scale = 1.f / sqrtf((float)D);
-  dim3 gkv((unsigned)(((S + 127) / 128) * KH * B)), gq((unsigned)(((S + 127) / 128) * H * B));
+  dim3 gq((unsigned)(((S + 127) / 128) * H * B));
   bwd_fast_attributes();
+  const bool split = dkv_split(B, S, H, KH, window);
   auto go = [&](auto cap) {
     constexpr bool CAP = decltype(cap)::value;
     hipLaunchKernelGGL((attn_bwd_dq_kernel<D, CAP>), gq, dim3(256), smem_q(D), stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
-    hipLaunchKernelGGL((attn_bwd_dkv_kernel<D, CAP>), gkv, dim3(256), smem_kv(D), stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap);
+    auto kv = [&](auto kern, int kw, int nqs) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * kw - 1) / (32 * kw)) * KH * B)), dim3(kw * nqs * 64), smem_kv(D, kw, nqs), stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap);
+    };
+    if (split) kv(attn_bwd_dkv_kernel<D, CAP, 2, 4>, 2, 4);
+    else kv(attn_bwd_dkv_kernel<D, CAP, 4, 1>, 4, 1);
   };
   if (softcap > 0.f) go(std::true_type());
   else go(std::false_type());

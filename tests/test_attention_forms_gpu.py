@@ -1,5 +1,5 @@
-"""GPU parity tests of the MFMA attention kernels' head_dim-64 form at the edges of their 128-row blocks,
-64-key and 32-query tiles."""
+"""GPU parity tests of the MFMA attention kernels' head_dim-64 form and of their split forms at the edges of
+their 128-row blocks, 64-key and 32-query tiles."""
 import math
 
 import pytest
@@ -55,3 +55,10 @@ def check(B, S, H, KH, D, window, softcap, strided=False):
 @pytest.mark.parametrize("H,KH,window,softcap", [(4, 4, None, 0.0), (4, 2, 40, 0.0), (2, 1, None, 30.0)])
 def test_head_dim_64(S, H, KH, window, softcap):
     check(2, S, H, KH, 64, window, softcap, strided=S % 2 == 1)
+
+
+# iterations (query heads x 32-row tiles) that the four query groups share out unevenly, or that some go without
+@pytest.mark.parametrize("S,H,KH,window,softcap", [(1, 2, 2, None, 0.0), (32, 3, 1, None, 0.0), (33, 8, 2, None, 0.0), (65, 3, 1, 0, 0.0), (97, 5, 1, 31, 0.0),
+                                                   (160, 2, 2, None, 30.0), (257, 4, 1, None, 0.0), (450, 3, 3, 64, 0.0)])
+def test_key_gradients_split_over_query_groups(S, H, KH, window, softcap):
+    check(2, S, H, KH, 128, window, softcap, strided=S % 2 == 1)
