@@ -168,26 +168,54 @@ __device__ __forceinline__ bf16x8 pack_bf16x8(const f32x16& a, int base) {
 }
 
 
+// Sum over the GROUPS waves that hold partial accumulators of the same 32 columns (column block c): every wave parks its D/8 units of 4 floats per lane in LDS, [c][group][unit][lane], and after a
+// barrier adds its share of the units in group order and hands them to `out`.
+template <int D, int GROUPS, typename Out>
+__device__ __forceinline__ void add_partials(unsigned char* smem, const f32x16 (&acc)[D / 32], int c, int group, int lane, Out out) {
+  constexpr int UNITS = D / 8, MINE = UNITS / GROUPS;
+  static_assert(UNITS % GROUPS == 0, "units are dealt evenly to the groups");
+  f32x4* park = reinterpret_cast<f32x4*>(smem) + c * (GROUPS * UNITS * 64) + lane;
+#pragma unroll
+  for (int u = 0; u < UNITS; u++)
+    park[(group * UNITS + u) * 64] = f32x4{acc[u >> 2][(u & 3) * 4], acc[u >> 2][(u & 3) * 4 + 1], acc[u >> 2][(u & 3) * 4 + 2], acc[u >> 2][(u & 3) * 4 + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < MINE; i++) {
+    const int u = group * MINE + i;
+    f32x4 v = park[u * 64];
+#pragma unroll
+    for (int g = 1; g < GROUPS; g++) v += park[(g * UNITS + u) * 64];
+    out(u, v);
+  }
+}
+
 // ---------------------------------------------------------------------------------------
-// Forward.  grid = ceil(S/128)*H*B workgroups (see decode_wg); 256 threads; wave w owns queries i0+32w .. +31.
+// Forward.  grid = ceil(S/(32 QW))*H*B workgroups (see decode_wg) of QW x KS waves; wave (qw, ks) owns queries
+// i0+32qw .. +31 and every KS-th of their K/V tiles.
+// KS = 1 (QW = 4): two workgroups per CU, no merge; what a grid that fills the GPU takes.
+// KS > 1: one workgroup of eight waves per CU with 1/KS of the serial chain of tiles; the partial softmaxes
+// are merged through LDS in key-group order.  See q_split.
 // ---------------------------------------------------------------------------------------
-template <int D, bool CAP>
-__global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
+template <int D, bool CAP, int QW, int KS>
+__global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     bf16* __restrict__ O, float* __restrict__ LSE, int S, int H, int KH, int64_t ldq, int64_t ldk,
     int64_t ldv, int64_t ldo, float scale, int window, float cap) {
   constexpr int TILE = 64 * D * 2;  // bytes of a K or V tile of 64 keys
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [2][K | V]
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [KS][2][K | V], then (KS > 1) the merge's statistics
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
   const int l32 = lane & 31, lhi = lane >> 5;
-  const int nqt = (S + 127) >> 7;
+  const int qw = wave % QW, ks = wave / QW;
+  constexpr int QR = QW * 32;         // queries of the workgroup
+  constexpr int TEAMS = QW * KS / 4;  // tiles are fetched by teams of 4 waves
+  const int nqt = (S + QR - 1) / QR;
   const WgCoord wg = decode_wg(blockIdx.x, (int)(gridDim.x / (nqt * (H / KH))), H / KH);
   const int qt = nqt - 1 - wg.rank;  // longest rows first
   const int b = wg.group / KH, kh = wg.group % KH;
   const int h = kh * (H / KH) + wg.r;
-  const int i0 = qt * 128;
-  const int iw0 = i0 + wave * 32;  // first query of this wave
+  const int i0 = qt * QR;
+  const int iw0 = i0 + qw * 32;  // first query of this wave
   const int qi = iw0 + l32;        // this lane's query
   const int qic = min(qi, S - 1);
 
@@ -199,7 +227,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
   }
   const int j_lo = window >= 0 ? max(0, i0 - window) : 0;
   const int t_lo = j_lo >> 6;
-  const int t_hi = min(i0 + 127, S - 1) >> 6;  // inclusive
+  const int t_hi = min(i0 + QR - 1, S - 1) >> 6;  // inclusive
 
   f32x16 o[D / 32];
 #pragma unroll
@@ -211,17 +239,24 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
   const bf16* kbase = K + (int64_t)b * S * ldk + kh * D;
   const bf16* vbase = V + (int64_t)b * S * ldv + kh * D;
   const unsigned lds0 = lds_addr_of(smem);
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const int wv = wave & 3, team = wave >> 2;
   TileDma<64, D> dk, dv;
   dk.init(ldk, wv, lane);
   dv.init(ldv, wv, lane);
-  auto load_kv = [&](int t, int stage) {
-    if (t * 64 + 64 <= S) {
-      dk.issue(kbase + (int64_t)t * 64 * ldk, lds0 + stage * (2 * TILE), wv);
-      dv.issue(vbase + (int64_t)t * 64 * ldv, lds0 + stage * (2 * TILE) + TILE, wv);
-    } else {
-      dma_tile<64, D>(kbase, ldk, t * 64, S, lds0 + stage * (2 * TILE), wv, lane);
-      dma_tile<64, D>(vbase, ldv, t * 64, S, lds0 + stage * (2 * TILE) + TILE, wv, lane);
+  // K/V tiles of round r: tile t_lo + r KS + g for key group g
+  auto load_kv = [&](int round, int stage) {
+#pragma unroll
+    for (int g0 = 0; g0 < KS / TEAMS; g0++) {
+      const int g = g0 * TEAMS + team, t = t_lo + round * KS + g;
+      if (KS > 1 && t > t_hi) break;
+      const unsigned dst = lds0 + (g * 2 + stage) * (2 * TILE);
+      if (t * 64 + 64 <= S) {
+        dk.issue(kbase + (int64_t)t * 64 * ldk, dst, wv);
+        dv.issue(vbase + (int64_t)t * 64 * ldv, dst + TILE, wv);
+      } else {
+        dma_tile<64, D>(kbase, ldk, t * 64, S, dst, wv, lane);
+        dma_tile<64, D>(vbase, ldv, t * 64, S, dst + TILE, wv, lane);
+      }
     }
   };
   const float sc2 = scale * LOG2E;
@@ -229,17 +264,18 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
   FragAddr<D> fa;
   fa.init(lane);
 
-  load_kv(t_lo, 0);
+  load_kv(0, 0);
   dma_wait_all();
   __syncthreads();
-  for (int t = t_lo; t <= t_hi; t++) {
-    const int cur = (t - t_lo) & 1;
-    if (t < t_hi) load_kv(t + 1, cur ^ 1);
-    const int j0 = t * 64;
+  const int rounds = (t_hi - t_lo + KS) / KS;
+  for (int r0 = 0; r0 < rounds; r0++) {
+    const int cur = r0 & 1;
+    if (r0 + 1 < rounds) load_kv(r0 + 1, cur ^ 1);
+    const int t = t_lo + r0 * KS + ks, j0 = t * 64;
     // skip tiles this wave cannot see at all
-    const bool visible = (j0 <= iw0 + 31) && (window < 0 || j0 + 63 >= iw0 - window);
+    const bool visible = (KS == 1 || t <= t_hi) && (j0 <= iw0 + 31) && (window < 0 || j0 + 63 >= iw0 - window);
     if (visible) {
-      const unsigned char* sk = smem + cur * (2 * TILE);
+      const unsigned char* sk = smem + (ks * 2 + cur) * (2 * TILE);
       const unsigned char* sv = sk + TILE;
       f32x16 st[2];
 #pragma unroll
@@ -329,28 +365,60 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(
     dma_wait_all();
     __syncthreads();
   }
-  const float ltot = half_swap_sum(lsum);
-  const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-  if (qi < S) {
-    bf16* op = O + ((int64_t)b * S + qi) * ldo + h * D;
+  float ltot = half_swap_sum(lsum);
+  auto store4 = [&](int dt, int g, const f32x4& v, float mul) {
+    bf16* op = O + ((int64_t)b * S + qic) * ldo + h * D;
+    Pack4 pk;
+#pragma unroll
+    for (int e = 0; e < 4; e++) pk.e[e] = f2bf(v[e] * mul);
+    *reinterpret_cast<u32x2*>(op + dt * 32 + g * 8 + lhi * 4) = pk.u;
+  };
+  if constexpr (KS == 1) {
+    const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
+    if (qi < S) {
+#pragma unroll
+      for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          store4(dt, g, f32x4{o[dt][g * 4], o[dt][g * 4 + 1], o[dt][g * 4 + 2], o[dt][g * 4 + 3]}, inv);
+    }
+  } else {
+    // statistics of the key groups behind the stages, then the accumulators, scaled to the common maximum,
+    // in their place (the last round ended in a barrier)
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    f32x2* stats = reinterpret_cast<f32x2*>(smem + KS * 4 * TILE) + qw * (KS * 32) + l32;
+    if (lhi == 0) stats[ks * 32] = f32x2{m, ltot};
+    __syncthreads();
+    const float m_own = m;
+#pragma unroll
+    for (int g = 0; g < KS; g++) {
+      const f32x2 st = stats[g * 32];
+      m = g == 0 ? st[0] : fmaxf(m, st[0]);
+    }
+    const float m_use = (m == -INFINITY) ? 0.f : m;
+    ltot = 0.f;
+#pragma unroll
+    for (int g = 0; g < KS; g++) {
+      const f32x2 st = stats[g * 32];
+      ltot += st[1] * fexp2(st[0] - m_use);
+    }
+    const float alpha = fexp2(m_own - m_use), inv = ltot > 0.f ? 1.f / ltot : 0.f;
 #pragma unroll
     for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        Pack4 pk;
-#pragma unroll
-        for (int e = 0; e < 4; e++) pk.e[e] = f2bf(o[dt][g * 4 + e] * inv);
-        *reinterpret_cast<u32x2*>(op + dt * 32 + g * 8 + lhi * 4) = pk.u;
-      }
-    if (lhi == 0) LSE[((int64_t)b * H + h) * S + qi] = (m + log2f(ltot)) * LN2;
+      for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
+    add_partials<D, KS>(smem, o, qw, ks, lane, [&](int u, const f32x4& v) {
+      if (qi < S) store4(u >> 2, u & 3, v, inv);
+    });
   }
+  if (qi < S && lhi == 0 && ks == 0) LSE[((int64_t)b * H + h) * S + qi] = (m + log2f(ltot)) * LN2;
 }
 
 // ---------------------------------------------------------------------------------------
 // dQ.  Same tiling and grid as the forward; K/V tiles stream through LDS.
 // ---------------------------------------------------------------------------------------
-template <int D, bool CAP>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
+template <int D, bool CAP, int QW, int KS>
+__global__ __launch_bounds__(QW * KS * 64, 2) void attn_bwd_dq_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     const bf16* __restrict__ O, const bf16* __restrict__ dO, const float* __restrict__ LSE,
     float* __restrict__ DELTA, bf16* __restrict__ dQ, int S, int H, int KH, int64_t ldq, int64_t ldk,
@@ -360,13 +428,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
   const int l32 = lane & 31, lhi = lane >> 5;
-  const int nqt = (S + 127) >> 7;
+  const int qw = wave % QW, ks = wave / QW;
+  constexpr int QR = QW * 32;         // queries of the workgroup
+  constexpr int TEAMS = QW * KS / 4;  // tiles are fetched by teams of 4 waves
+  const int nqt = (S + QR - 1) / QR;
   const WgCoord wg = decode_wg(blockIdx.x, (int)(gridDim.x / (nqt * (H / KH))), H / KH);
   const int qt = nqt - 1 - wg.rank;  // longest rows first
   const int b = wg.group / KH, kh = wg.group % KH;
   const int h = kh * (H / KH) + wg.r;
-  const int i0 = qt * 128;
-  const int iw0 = i0 + wave * 32;
+  const int i0 = qt * QR;
+  const int iw0 = i0 + qw * 32;
   const int qi = iw0 + l32;
   const int qic = min(qi, S - 1);
 
@@ -391,11 +462,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   dlt = half_swap_sum(dlt);
   // stored NEGATED: the dK/dV kernel starts its dP accumulators from it, so that dP - delta
   // comes out of the MFMAs and costs that kernel no subtraction
-  if (lhi == 0 && qi < S) DELTA[((int64_t)b * H + h) * S + qi] = -dlt;
+  if (lhi == 0 && ks == 0 && qi < S) DELTA[((int64_t)b * H + h) * S + qi] = -dlt;
   const float lse2 = LSE[((int64_t)b * H + h) * S + qic] * LOG2E;
   const int j_lo = window >= 0 ? max(0, i0 - window) : 0;
   const int t_lo = j_lo >> 6;
-  const int t_hi = min(i0 + 127, S - 1) >> 6;
+  const int t_hi = min(i0 + QR - 1, S - 1) >> 6;
 
   f32x16 dq[D / 32];
 #pragma unroll
@@ -406,17 +477,24 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const bf16* kbase = K + (int64_t)b * S * ldk + kh * D;
   const bf16* vbase = V + (int64_t)b * S * ldv + kh * D;
   const unsigned lds0 = lds_addr_of(smem);
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const int wv = wave & 3, team = wave >> 2;
   TileDma<64, D> dk, dv;
   dk.init(ldk, wv, lane);
   dv.init(ldv, wv, lane);
-  auto load_kv = [&](int t, int stage) {
-    if (t * 64 + 64 <= S) {
-      dk.issue(kbase + (int64_t)t * 64 * ldk, lds0 + stage * (2 * TILE), wv);
-      dv.issue(vbase + (int64_t)t * 64 * ldv, lds0 + stage * (2 * TILE) + TILE, wv);
-    } else {
-      dma_tile<64, D>(kbase, ldk, t * 64, S, lds0 + stage * (2 * TILE), wv, lane);
-      dma_tile<64, D>(vbase, ldv, t * 64, S, lds0 + stage * (2 * TILE) + TILE, wv, lane);
+  // K/V tiles of round r: tile t_lo + r KS + g for key group g
+  auto load_kv = [&](int round, int stage) {
+#pragma unroll
+    for (int g0 = 0; g0 < KS / TEAMS; g0++) {
+      const int g = g0 * TEAMS + team, t = t_lo + round * KS + g;
+      if (KS > 1 && t > t_hi) break;
+      const unsigned dst = lds0 + (g * 2 + stage) * (2 * TILE);
+      if (t * 64 + 64 <= S) {
+        dk.issue(kbase + (int64_t)t * 64 * ldk, dst, wv);
+        dv.issue(vbase + (int64_t)t * 64 * ldv, dst + TILE, wv);
+      } else {
+        dma_tile<64, D>(kbase, ldk, t * 64, S, dst, wv, lane);
+        dma_tile<64, D>(vbase, ldv, t * 64, S, dst + TILE, wv, lane);
+      }
     }
   };
   const float sc2 = scale * LOG2E;
@@ -425,16 +503,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   FragAddr<D, CAP && D == 128> fa;  // the soft-cap variant is the one short of registers
   fa.init(lane);
 
-  load_kv(t_lo, 0);
+  load_kv(0, 0);
   dma_wait_all();
   __syncthreads();
-  for (int t = t_lo; t <= t_hi; t++) {
-    const int cur = (t - t_lo) & 1;
-    if (t < t_hi) load_kv(t + 1, cur ^ 1);
-    const int j0 = t * 64;
-    const bool visible = (j0 <= iw0 + 31) && (window < 0 || j0 + 63 >= iw0 - window);
+  const int rounds = (t_hi - t_lo + KS) / KS;
+  for (int r0 = 0; r0 < rounds; r0++) {
+    const int cur = r0 & 1;
+    if (r0 + 1 < rounds) load_kv(r0 + 1, cur ^ 1);
+    const int t = t_lo + r0 * KS + ks, j0 = t * 64;
+    const bool visible = (KS == 1 || t <= t_hi) && (j0 <= iw0 + 31) && (window < 0 || j0 + 63 >= iw0 - window);
     if (visible) {
-      const unsigned char* sk = smem + cur * (2 * TILE);
+      const unsigned char* sk = smem + (ks * 2 + cur) * (2 * TILE);
       const unsigned char* sv = sk + TILE;
       const bool need_mask = (j0 + 63 > iw0) || (window >= 0 && j0 < iw0 + 31 - window);
       // dS of one 32-key half from its scores and dP, packed as the B operand of the dQ product
@@ -487,17 +566,24 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     dma_wait_all();
     __syncthreads();
   }
-  if (qi < S) {
-    bf16* op = dQ + ((int64_t)b * S + qi) * lddq + h * D;
+  auto store4 = [&](int dt, int g, const f32x4& v) {
+    bf16* op = dQ + ((int64_t)b * S + qic) * lddq + h * D;
+    Pack4 pk;
 #pragma unroll
-    for (int dt = 0; dt < D / 32; dt++)
+    for (int e = 0; e < 4; e++) pk.e[e] = f2bf(v[e] * scale);
+    *reinterpret_cast<u32x2*>(op + dt * 32 + g * 8 + lhi * 4) = pk.u;
+  };
+  if constexpr (KS == 1) {
+    if (qi < S) {
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        Pack4 pk;
+      for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) pk.e[e] = f2bf(dq[dt][g * 4 + e] * scale);
-        *reinterpret_cast<u32x2*>(op + dt * 32 + g * 8 + lhi * 4) = pk.u;
-      }
+        for (int g = 0; g < 4; g++) store4(dt, g, f32x4{dq[dt][g * 4], dq[dt][g * 4 + 1], dq[dt][g * 4 + 2], dq[dt][g * 4 + 3]});
+    }
+  } else {
+    add_partials<D, KS>(smem, dq, qw, ks, lane, [&](int u, const f32x4& v) {
+      if (qi < S) store4(u >> 2, u & 3, v);
+    });
   }
 }
 
@@ -725,29 +811,14 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
         }
     }
   } else {
-    // Partial sums through LDS (the stages are free: the last round ended in a barrier): a wave parks its
-    // accumulators as units of 4 floats per lane, [kw][qs][unit][lane], then adds its share of the units over the
-    // query groups.  dK first, then dV in the same space.
-    constexpr int UNITS = D / 8, MINE = UNITS / QS;
-    static_assert(UNITS % QS == 0, "units are dealt evenly to the query groups");
-    f32x4* park = reinterpret_cast<f32x4*>(smem) + kw * (QS * UNITS * 64) + lane;
-    auto reduce = [&](const f32x16 (&acc)[D / 32], bf16* p, float mul) {
-#pragma unroll
-      for (int u = 0; u < UNITS; u++)
-        park[(qs * UNITS + u) * 64] = f32x4{acc[u >> 2][(u & 3) * 4], acc[u >> 2][(u & 3) * 4 + 1], acc[u >> 2][(u & 3) * 4 + 2], acc[u >> 2][(u & 3) * 4 + 3]};
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < MINE; i++) {
-        const int u = qs * MINE + i;
-        f32x4 v = park[u * 64];
-#pragma unroll
-        for (int g = 1; g < QS; g++) v += park[(g * UNITS + u) * 64];
-        if (kj < S) store4(p, u >> 2, u & 3, v, mul);
-      }
-    };
-    reduce(dk, kp, scale);
+    // the stages are free: the last round ended in a barrier; dK first, then dV in the same space
+    add_partials<D, QS>(smem, dk, kw, qs, lane, [&](int u, const f32x4& v) {
+      if (kj < S) store4(kp, u >> 2, u & 3, v, scale);
+    });
     __syncthreads();
-    reduce(dv, vp, 1.f);
+    add_partials<D, QS>(smem, dv, kw, qs, lane, [&](int u, const f32x4& v) {
+      if (kj < S) store4(vp, u >> 2, u & 3, v, 1.f);
+    });
   }
 }
 
@@ -870,31 +941,49 @@ bool bwd_fast_ok(const void* q, const void* k, const void* v, const void* o, con
          aligned16(dv) && lddo % 8 == 0 && lddq % 8 == 0 && lddk % 8 == 0 && lddv % 8 == 0;
 }
 
-constexpr int smem_q(int D) { return 2 * 2 * 64 * D * 2; }                          // forward, dQ
+// forward, dQ: stages (the parked partial sums fit in their place), statistics of the forward's merge
+constexpr int smem_q(int D, int QW, int KS) { return KS * 2 * 2 * 64 * D * 2 + (KS > 1 ? QW * KS * 32 * 8 : 0); }
 // dK/dV: stages and V tile, or the parked partial sums
 constexpr int smem_kv(int D, int KW, int QS) {
   const int run = QS * 2 * (2 * 32 * D * 2 + 256) + KW * 32 * D * 2, sums = QS > 1 ? KW * QS * 32 * D * 4 : 0;
   return run > sums ? run : sums;
 }
 
+// waves of the split forward and dQ kernels: what 160 KB of stages hold
+template <int D> constexpr int SPLIT_QW = D == 128 ? 4 : 2;
+template <int D> constexpr int SPLIT_KS = D == 128 ? 2 : 4;
+
 // dynamic-LDS limits of the backward kernels, set once per process
-template <int D>
-void bwd_fast_attributes_d() {
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, true, 4, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 4, 1));
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, false, 4, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 4, 1));
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, true, 2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 2, 4));
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, false, 2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv(D, 2, 4));
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
-  (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
+template <int D, bool CAP>
+void bwd_fast_attributes_of() {
+  constexpr int QW = SPLIT_QW<D>, KS = SPLIT_KS<D>;
+  constexpr auto ATTR = hipFuncAttributeMaxDynamicSharedMemorySize;
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, CAP, 4, 1>, ATTR, smem_kv(D, 4, 1));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, CAP, 2, 4>, ATTR, smem_kv(D, 2, 4));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, CAP, 4, 1>, ATTR, smem_q(D, 4, 1));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, CAP, QW, KS>, ATTR, smem_q(D, QW, KS));
 }
 void bwd_fast_attributes() {
   static std::once_flag once;
   std::call_once(once, [] {
-    bwd_fast_attributes_d<128>();
-    bwd_fast_attributes_d<64>();
+    bwd_fast_attributes_of<128, true>();
+    bwd_fast_attributes_of<128, false>();
+    bwd_fast_attributes_of<64, true>();
+    bwd_fast_attributes_of<64, false>();
   });
 }
 
+// Whether the forward and dQ take their split kernels: while the workgroups of 128 queries do not fill the CUs twice
+// over, a wave has a SIMD to itself and its chain of key tiles is what takes the time.  Forward | backward (dK/dV
+// included), us, plain -> split: 3 x 1000 tokens, 8 heads (192 workgroups): 25.2 -> 22.5 | 70 -> 62; 2 x 2000 (256):
+// 44.0 -> 36.5 | 122 -> 104; 1 x 6000 (376): 127 -> 101 | 382 -> 330; 1 x 1500, 32 heads (384): 38.6 -> 33.6 | 163 -> 152.  At
+// 512 workgroups the chain decides: 32 tiles 53.5 -> 49.5 | 181 -> 171, 16 tiles 32.3 -> 34.6 | 109 -> 111, 18 tiles in
+// a window 40.6 -> 50.2 | 148 -> 155.  Beyond, the plain kernels' two workgroups per CU keep the SIMDs busy by themselves.
+bool q_split(int B, int S, int H, int window) {
+  const int64_t n = (int64_t)((S + 127) / 128) * H * B;
+  const int tiles = (window >= 0 && window < S - 128 ? window + 128 : S + 63) / 64;
+  return n <= 256 || (n <= 512 && tiles >= 24);
+}
 // Whether dK/dV takes the split kernel.  One workgroup per key tile and K/V head is little parallel work when the
 // heads are few: 224 workgroups for 2 x 1777 tokens of 8 K/V heads leave the GPU waiting for those of the first key tile,
 // which walk the four query heads of 1777 tokens one 32-row tile at a time with one wave per SIMD.  Backward
@@ -917,16 +1006,19 @@ void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const b
                      int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, int64_t lddk, int64_t lddv, int window,
                      float softcap) {
   const float scale = 1.f / sqrtf((float)D);
-  dim3 gq((unsigned)(((S + 127) / 128) * H * B));
   bwd_fast_attributes();
-  const bool split = dkv_split(B, S, H, KH, window);
+  const bool split_q = q_split(B, S, H, window), split_kv = dkv_split(B, S, H, KH, window);
   auto go = [&](auto cap) {
     constexpr bool CAP = decltype(cap)::value;
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<D, CAP>), gq, dim3(256), smem_q(D), stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
+    auto qk = [&](auto kern, int qw, int ks) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * qw - 1) / (32 * qw)) * H * B)), dim3(qw * ks * 64), smem_q(D, qw, ks), stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
+    };
+    if (split_q) qk(attn_bwd_dq_kernel<D, CAP, SPLIT_QW<D>, SPLIT_KS<D>>, SPLIT_QW<D>, SPLIT_KS<D>);
+    else qk(attn_bwd_dq_kernel<D, CAP, 4, 1>, 4, 1);
     auto kv = [&](auto kern, int kw, int nqs) {
       hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * kw - 1) / (32 * kw)) * KH * B)), dim3(kw * nqs * 64), smem_kv(D, kw, nqs), stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap);
     };
-    if (split) kv(attn_bwd_dkv_kernel<D, CAP, 2, 4>, 2, 4);
+    if (split_kv) kv(attn_bwd_dkv_kernel<D, CAP, 2, 4>, 2, 4);
     else kv(attn_bwd_dkv_kernel<D, CAP, 4, 1>, 4, 1);
   };
   if (softcap > 0.f) go(std::true_type());
@@ -937,14 +1029,23 @@ template <int D>
 void launch_fwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const bf16* vp, bf16* o, float* lse, int B, int S, int H,
                      int KH, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int window, float softcap) {
   const float scale = 1.f / sqrtf((float)D);
-  dim3 grid((unsigned)(((S + 127) / 128) * H * B));
+  constexpr int QW = SPLIT_QW<D>, KS = SPLIT_KS<D>;
   static std::once_flag once;  // per head_dim
   std::call_once(once, [] {
-    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
-    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q(D));
+    constexpr auto ATTR = hipFuncAttributeMaxDynamicSharedMemorySize;
+    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, true, 4, 1>, ATTR, smem_q(D, 4, 1));
+    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, false, 4, 1>, ATTR, smem_q(D, 4, 1));
+    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, true, QW, KS>, ATTR, smem_q(D, QW, KS));
+    (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, false, QW, KS>, ATTR, smem_q(D, QW, KS));
   });
+  const bool split = q_split(B, S, H, window);
   auto go = [&](auto cap) {
-    hipLaunchKernelGGL((attn_fwd_kernel<D, decltype(cap)::value>), grid, dim3(256), smem_q(D), stream, qp, kp, vp, o, lse, S, H, KH, ldq, ldk, ldv, ldo, scale, window, softcap);
+    constexpr bool CAP = decltype(cap)::value;
+    auto run = [&](auto kern, int qw, int ks) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * qw - 1) / (32 * qw)) * H * B)), dim3(qw * ks * 64), smem_q(D, qw, ks), stream, qp, kp, vp, o, lse, S, H, KH, ldq, ldk, ldv, ldo, scale, window, softcap);
+    };
+    if (split) run(attn_fwd_kernel<D, CAP, QW, KS>, QW, KS);
+    else run(attn_fwd_kernel<D, CAP, 4, 1>, 4, 1);
   };
   if (softcap > 0.f) go(std::true_type());
   else go(std::false_type());

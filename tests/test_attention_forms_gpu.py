@@ -62,3 +62,11 @@ def test_head_dim_64(S, H, KH, window, softcap):
                                                    (160, 2, 2, None, 30.0), (257, 4, 1, None, 0.0), (450, 3, 3, 64, 0.0)])
 def test_key_gradients_split_over_query_groups(S, H, KH, window, softcap):
     check(2, S, H, KH, 128, window, softcap, strided=S % 2 == 1)
+
+
+# key tiles that the key groups of the forward and dQ share out unevenly, or that some go without
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S,H,KH,window,softcap", [(1, 2, 2, None, 0.0), (64, 2, 1, None, 0.0), (65, 2, 2, 0, 0.0), (130, 3, 1, None, 30.0), (200, 4, 2, 70, 0.0),
+                                                   (449, 2, 2, None, 0.0)])
+def test_queries_split_over_key_groups(S, H, KH, window, softcap, D):
+    check(3, S, H, KH, D, window, softcap, strided=S % 2 == 0)
