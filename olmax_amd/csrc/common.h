@@ -162,6 +162,16 @@ int olmax_adamw_grid(hipStream_t stream, float* p, const void* g, float* m, floa
 // gemm_small.hip: any M, N, K and alignment; `groups` (4 or 8) waves share a 64 x 64 tile's reduction
 void olmax_gemm_small(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N, int K, int64_t lda,
                       int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, int groups);
+// memory a GEMM may use for partial results until it is done; what it holds before and after does not matter
+struct GemmScratch {
+  void* p = nullptr;
+  int64_t bytes = 0;
+};
 // gemm.hip: olmax_gemm_bf16 with an A whose rows are readable (and, k-contiguous, zero) up to a multiple of 8
 int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C, const bf16* r, int M, int N, int K,
-                      int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded);
+                      int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded,
+                      GemmScratch scratch = GemmScratch());
+// lmhead_ce.hip: olmax_lmhead_ce, its two gradient products with scratch memory
+int olmax_lmhead_ce_scratch(hipStream_t stream, const void* h, const void* W, const int32_t* labels, float* loss, void* dh, void* dW,
+                            void* workspace, int64_t workspace_bytes, int64_t T, int32_t d, int32_t V, int32_t ignore_index,
+                            float softcap, int32_t dw_f32, GemmScratch scratch);

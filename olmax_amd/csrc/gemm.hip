@@ -78,6 +78,10 @@ std::mutex g_prof_mu;
 // head and its neighbour (wave ^ 1) holds the other, so the rotation reads both from the LDS
 // staging of the epilogue.  The position of a row is row % seq_len; cos/sin are [seq_len, 64] fp32.
 //
+// EPI == 6 is one part of a reduction that several workgroups share (see olmax_gemm_padded): blockIdx.y
+// takes k in [y * seq_len, (y + 1) * seq_len), the last one the rest, and the accumulators leave as they
+// are, 1 KB per instruction, to Cv[part][tile][wave][i][j][lane] for gemm_split_sum_kernel.
+//
 // RAG: 1 where M or N, 2 where K is not a multiple of the tile.  The last tile of a row or column is
 // moved back so that it ends with the matrix (the loop then reads nothing outside it and is the same
 // code) and stores only what no other tile stores.  The partial k-tile at the end of K is taken FIRST, ahead of
@@ -93,7 +97,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
   constexpr int GLU = (EPI == 1 || EPI == 2) ? EPI : (EPI == 4 ? 1 : (EPI == 5 ? 2 : 0));
   constexpr bool GLU_BWD = EPI == 4 || EPI == 5;
   constexpr bool ROPE = EPI == 3;
-  static_assert(EPI == 0 || (BN == 256 && WN == 64 && B_KC && !HAS_RES && !OUT_F32), "fused epilogues: 256-wide NT tiles only");
+  constexpr bool SPLIT = EPI == 6;
+  static_assert(EPI == 0 || SPLIT || (BN == 256 && WN == 64 && B_KC && !HAS_RES && !OUT_F32), "fused epilogues: 256-wide NT tiles only");
   constexpr int NW = (BM / WM) * (BN / WN);
   constexpr int TM = WM / 16, TN = WN / 16;  // accumulators of 16x16 per wave
   constexpr int WAVES_N = BN / WN;
@@ -147,6 +152,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
     const int gm = min(tiles_m - first_m, GM);
     tile_m = first_m + (pid % group_sz) % gm;
     tile_n = (pid % group_sz) / gm;
+  }
+  if (SPLIT) {
+    const int k_lo = blockIdx.y * seq_len;
+    A += A_KC ? (int64_t)k_lo : (int64_t)k_lo * lda;
+    B += B_KC ? (int64_t)k_lo : (int64_t)k_lo * ldb;
+    K = blockIdx.y + 1 == gridDim.y ? K - k_lo : seq_len;
   }
   constexpr bool KRAG = RAG == 2;
   constexpr int BNC = GLU ? BN / 2 : BN;  // output columns of a block (GLU: features)
@@ -496,6 +507,15 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
   asm volatile("" : "+v"(lane_e));
   const int l16e = lane_e & 15, g16e = lane_e >> 4;
 
+  if (SPLIT) {
+    float* part = reinterpret_cast<float*>(Cv) + ((((int64_t)blockIdx.y * tiles_m + tile_m) * tiles_n + tile_n) * NW + wave) * (NM * 256);
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) *reinterpret_cast<f32x4*>(part + ((i * TN + j) * 64 + lane_e) * 4) = acc[i][j];
+    return;
+  }
+
   // ---- epilogue.  The MFMAs ran with their operands swapped (B fragment as the instruction's A),
   // so each accumulator is a transposed 16x16 tile: lane -> row l16e, columns 4*g16e + r, i.e. four
   // consecutive columns of one row of C per lane.
@@ -812,6 +832,99 @@ int dispatch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf
 
 std::atomic<int> g_force_tile{0};  // diagnostic override, process-wide
 
+// C = sum of the parts, in their order (+ R), with the roundings of the kernels above.  A wave takes one
+// 16 x 64 strip of a wave tile; its loads are the 1 KB runs the accumulators were stored as.  Bound by
+// the reads of the parts (at most 64 MB a round of workgroups, out of the memory-side cache).
+__global__ __launch_bounds__(256) void gemm_split_sum_kernel(const float* __restrict__ parts, int nparts, void* __restrict__ Cv,
+                                                             const bf16* __restrict__ R, int M, int N, int64_t ldc, int64_t ldr,
+                                                             int m_edge, int tiles_n, int ntiles, int out_f32, int vec) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g16 = lane >> 4;
+  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);  // (tile, wave of it, i): 64 per tile
+  const int tile = unit >> 6, wave = (unit >> 3) & 7, i = unit & 7;
+  const int tile_m = tile / tiles_n, tile_n = tile % tiles_n;
+  const int64_t stride = (int64_t)ntiles * 65536;
+  const float* src = parts + (int64_t)unit * 1024 + lane * 4;
+  f32x4 v[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) v[j] = *reinterpret_cast<const f32x4*>(src + j * 256);
+#pragma unroll 4
+  for (int p = 1; p < nparts; p++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(src + p * stride + j * 256);
+#pragma unroll
+      for (int r = 0; r < 4; r++) v[j][r] += x[r];
+    }
+  // a tile moved back to end with the matrix stores only what the one before it does not
+  const int64_t row = min(tile_m * 256, m_edge - 256) + (wave >> 2) * 128 + i * 16 + l16;
+  if (row < tile_m * 256 || row >= M) return;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int col = min(tile_n * 256, N - 256) + (wave & 3) * 64 + j * 16 + g16 * 4, lo = tile_n * 256 - col;
+    const bool whole = vec && lo <= 0;
+    Pack4 rr;
+    if (R && whole) rr.u = *reinterpret_cast<const u32x2*>(R + row * ldr + col);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      if (r < lo) continue;
+      if (R) v[j][r] = (out_f32 ? v[j][r] : bf2f(f2bf(v[j][r]))) + bf2f(whole ? rr.e[r] : R[row * ldr + col + r]);
+      if (whole) continue;
+      if (out_f32) reinterpret_cast<float*>(Cv)[row * ldc + col + r] = v[j][r];
+      else reinterpret_cast<bf16*>(Cv)[row * ldc + col + r] = f2bf(v[j][r]);
+    }
+    if (!whole) continue;
+    if (out_f32) {
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(Cv) + row * ldc + col) = v[j];
+    } else {
+      Pack4 o;
+#pragma unroll
+      for (int r = 0; r < 4; r++) o.e[r] = f2bf(v[j][r]);
+      *reinterpret_cast<u32x2*>(reinterpret_cast<bf16*>(Cv) + row * ldc + col) = o.u;
+    }
+  }
+}
+
+template <bool A_KC, bool B_KC>
+int launch_split(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N, int K, int64_t lda, int64_t ldb,
+                 int64_t ldc, int64_t ldr, bool out_f32, int parts, float* scratch) {
+  constexpr int SMEM = 2 * (256 + 256) * BK * 2;
+  auto whole = gemm_bf16_kernel<256, 256, 128, 64, A_KC, B_KC, false, true, 6, 0>;
+  auto ragged = gemm_bf16_kernel<256, 256, 128, 64, A_KC, B_KC, false, true, 6, 1>;
+  auto kragged = gemm_bf16_kernel<256, 256, 128, 64, A_KC, B_KC, false, true, 6, 2>;
+  static std::once_flag attr_once;
+  std::call_once(attr_once, [&] {
+    for (auto k : {whole, ragged, kragged}) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+  });
+  auto kern = K % BK ? kragged : (M % 256 || N % 256) ? ragged : whole;
+  const int tm = (M + 255) / 256, tn = (N + 255) / 256;
+  const int chunk = (K / BK + parts - 1) / parts;  // whole k-tiles of a part; every part has at least one
+  parts = (K / BK + chunk - 1) / chunk;
+  ProfRec rec{};
+  if (g_prof_on) {
+    (void)hipEventCreate(&rec.e0);
+    (void)hipEventCreate(&rec.e1);
+    (void)hipEventRecord(rec.e0, s);
+  }
+  // (run order: a round of windows is 256 tiles, and here there are fewer)
+  hipLaunchKernelGGL(kern, dim3(tm * tn, parts), dim3(512), SMEM, s, A, B, (void*)scratch, (const bf16*)nullptr, M, N, K, lda,
+                     ldb, (int64_t)0, (int64_t)0, tm, tn, 1, (const float*)nullptr, (const float*)nullptr, chunk * BK, 0, 0);
+  const uintptr_t mask = out_f32 ? 15 : 7;
+  const int vec = N % 4 == 0 && ldc % 4 == 0 && !((uintptr_t)C & mask) && (!R || (ldr % 4 == 0 && !((uintptr_t)R & 7)));
+  hipLaunchKernelGGL(gemm_split_sum_kernel, dim3((unsigned)(tm * tn * 16)), dim3(256), 0, s, (const float*)scratch, parts, C, R, M, N, ldc,
+                     ldr, A_KC ? M : (M + 7) & ~7, tn, tm * tn, (int)out_f32, vec);
+  if (g_prof_on) {
+    (void)hipEventRecord(rec.e1, s);
+    rec.flops = 2.0 * M * N * K;
+    rec.bytes = 2.0 * ((double)M * K + (double)N * K + (double)M * N * (R ? 2 : 1) * (out_f32 ? 2 : 1));
+    rec.key = 256 | (A_KC << 12) | (B_KC << 13) | ((R != nullptr) << 14) | (out_f32 << 15);
+    rec.M = M; rec.N = N; rec.K = K;
+    std::lock_guard<std::mutex> lk(g_prof_mu);
+    g_prof.push_back(rec);
+  }
+  OLMAX_LAUNCH_CHECK();
+  return OLMAX_OK;
+}
+
 }  // namespace
 
 extern "C" void olmax_gemm_set_tile(int tile) { g_force_tile = tile; }
@@ -902,37 +1015,62 @@ static float cost_128(int64_t n, int kt) {
   };
   return (n / 512) * (1.08f * kt + 4.f) + (n % 512 ? part(n % 512) : 0.f);
 }
-static float cost_256(int64_t n, int kt) {
+// n tiles of 256, their reductions shared by s workgroups each; a part costs 256 KB written and read again
+static float cost_split(int64_t n, int kt, int s) {
+  const int64_t w = n * s, r = w % 256;
+  const int k = (kt + s - 1) / s;
+  return (w / 256) * (1.52f * k + 6.f) + (r ? (1.05f + 0.47f * r / 256.f) * k + 6.f : 0.f) + 6.f + 0.1f * w;
+}
+// The cheapest number of parts (1: whole reductions) that `bytes` of scratch hold.  A part has 8 k-tiles or more.
+static int pick_parts(int64_t n, int kt, int64_t bytes, float* cost) {
+  int best = 1;
+  for (int s = 2; s <= 64 && s * 8 <= kt && n * s <= 512 && n * s * 262144 <= bytes; s++)
+    if (const float c = cost_split(n, kt, s); c < *cost) *cost = c, best = s;
+  return best;
+}
+static float cost_256(int64_t n, int kt, int64_t bytes) {
   const int64_t r = n % 256;
-  // (a last round that fills less than half of the CUs is cut off and runs as 128 tiles)
-  const float last = r == 0 ? 0.f : (1.05f + 0.47f * r / 256.f) * kt + 6.f;
-  return (n / 256) * (1.52f * kt + 6.f) + (n > 256 && r < 128 && cost_128(4 * r, kt) < last ? cost_128(4 * r, kt) : last);
+  // (a last round that fills less than half of the CUs is cut off and runs as 128 tiles or shared reductions)
+  float last = r == 0 ? 0.f : (1.05f + 0.47f * r / 256.f) * kt + 6.f;
+  if (n > 256 && r > 0 && r < 128) {
+    last = cost_128(4 * r, kt) < last ? cost_128(4 * r, kt) : last;
+    (void)pick_parts(r, kt, bytes, &last);
+  }
+  return (n / 256) * (1.52f * kt + 6.f) + last;
 }
 static float cost_small(int64_t n, int kt) { return ((n + 255) / 256) * (0.22f * kt + 1.2f) + 2.4f; }
 
 // Which kernel takes a problem.  0: gemm_small (any size and alignment), else the edge of the
-// direct-to-LDS kernel's tiles.
-static int pick_tile(int M, int N, int K, bool direct_ok) {
+// direct-to-LDS kernel's tiles; *parts > 1: 256 tiles with that many workgroups to a reduction.
+static int pick_tile(int M, int N, int K, bool direct_ok, int64_t bytes, int* parts) {
+  *parts = 1;
   if (!direct_ok || M < 128 || N < 128 || K < BK) return 0;
   const int kt = (K + BK - 1) / BK;
   auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
   float best = cost_small(tiles(64), kt);
   int tile = 0;
   if (const float c = cost_128(tiles(128), kt); c < best) best = c, tile = 128;
-  if (M >= 256 && N >= 256 && cost_256(tiles(256), kt) < best) tile = 256;
-  return tile;
+  if (M < 256 || N < 256) return tile;
+  if (const float c = cost_256(tiles(256), kt, bytes); c < best) best = c, tile = 256;
+  *parts = pick_parts(tiles(256), K / BK, bytes, &best);
+  return *parts > 1 ? 256 : tile;
 }
 
 // olmax_gemm_bf16 behind its argument checks.  a_padded: rows of A may be read up to the next multiple
 // of 8 elements (row stride permitting), and for a k-contiguous A those elements are zeros: what
 // lets an operand whose row length is not a multiple of 8 use 16-byte fetches.
 int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C, const bf16* r, int M, int N, int K,
-                      int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded) {
+                      int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded,
+                      GemmScratch scratch) {
   // whole 16-byte chunks everywhere: aligned rows, and a chunk never crosses the end of a row
   const bool direct_ok = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 && (a_padded || (a_kc ? K : M) % 8 == 0) &&
                          (b_kc ? K : N) % 8 == 0 && (a_kc || !b_kc);
-  int tile = pick_tile(M, N, K, direct_ok);
   const int force_tile = g_force_tile.load(std::memory_order_relaxed);
+  int parts;
+  int tile = pick_tile(M, N, K, direct_ok, b_kc || force_tile || !aligned16(scratch.p) ? 0 : scratch.bytes, &parts);
+  if (parts > 1)
+    return (a_kc ? launch_split<true, false> : launch_split<false, false>)(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts,
+                                                                          (float*)scratch.p);
   if (force_tile && tile) {
     if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
     if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;
@@ -953,19 +1091,19 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
       const size_t esz = out_f32 ? 4 : 2;
       if (rm > 0 && (int64_t)rm * tn >= (int64_t)cn * tm) {
         const int m1 = rm * 256;
-        int rc = olmax_gemm_padded(stream, a, b, C, r, m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
+        int rc = olmax_gemm_padded(stream, a, b, C, r, m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
         if (rc) return rc;
         const bf16* a2 = a_kc ? a + (int64_t)m1 * lda : a + m1;
         return olmax_gemm_padded(stream, a2, b, (char*)C + (int64_t)m1 * ldc * esz, r ? r + (int64_t)m1 * ldr : nullptr,
-                                 M - m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
+                                 M - m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
       }
       if (cn > 0) {
         const int n1 = cn * 256;
-        int rc = olmax_gemm_padded(stream, a, b, C, r, M, n1, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
+        int rc = olmax_gemm_padded(stream, a, b, C, r, M, n1, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
         if (rc) return rc;
         const bf16* b2 = b_kc ? b + (int64_t)n1 * ldb : b + n1;
         return olmax_gemm_padded(stream, a, b2, (char*)C + (int64_t)n1 * esz, r ? r + n1 : nullptr, M, N - n1, K, lda,
-                                 ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded);
+                                 ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
       }
     }
   }

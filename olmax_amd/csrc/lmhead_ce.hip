@@ -349,10 +349,9 @@ extern "C" int64_t olmax_lmhead_ce_workspace_bytes(int64_t T, int32_t V) {
 //   dlogits overwrites logits in the workspace ; dh = dlogits W ; dW = dlogits^T h.
 // h [T, d] bf16, W [V, d] bf16, labels [T] int32.  dh [T, d] bf16 and dW [V, d] (bf16, or
 // fp32 when dw_f32 != 0) may be NULL to skip that product (forward-only when both are NULL).
-extern "C" int32_t olmax_lmhead_ce(hipStream_t stream, const void* h, const void* W,
-                                   const int32_t* labels, float* loss, void* dh, void* dW,
-                                   void* workspace, int64_t workspace_bytes, int64_t T, int32_t d,
-                                   int32_t V, int32_t ignore_index, float softcap, int32_t dw_f32) {
+int olmax_lmhead_ce_scratch(hipStream_t stream, const void* h, const void* W, const int32_t* labels, float* loss, void* dh, void* dW,
+                            void* workspace, int64_t workspace_bytes, int64_t T, int32_t d, int32_t V, int32_t ignore_index,
+                            float softcap, int32_t dw_f32, GemmScratch scratch) {
   OLMAX_CHECK(h && W && labels && loss && workspace, OLMAX_ERR_ARG, "olmax_lmhead_ce: null pointer");
   OLMAX_CHECK(T > 0 && d > 0 && V > 0 && T < (1LL << 31), OLMAX_ERR_SHAPE, "olmax_lmhead_ce: bad shape");
   OLMAX_CHECK(workspace_bytes >= olmax_lmhead_ce_workspace_bytes(T, V) && (((uintptr_t)workspace) & 255) == 0, OLMAX_ERR_WORKSPACE,
@@ -368,12 +367,20 @@ extern "C" int32_t olmax_lmhead_ce(hipStream_t stream, const void* h, const void
                      olmax_cross_entropy_workspace_bytes(T), T, V, ldl, ldl, 0, ignore_index, softcap, 1.f, 0, true);
   if (rc) return rc;
   if (dh) {
-    rc = olmax_gemm_padded(stream, logits, wp, dh, nullptr, (int)T, d, V, ldl, d, d, 0, true, false, false, true);
+    rc = olmax_gemm_padded(stream, logits, wp, dh, nullptr, (int)T, d, V, ldl, d, d, 0, true, false, false, true, scratch);
     if (rc) return rc;
   }
   if (dW) {
-    rc = olmax_gemm_padded(stream, logits, hp, dW, nullptr, V, d, (int)T, ldl, d, d, 0, false, false, dw_f32 != 0, true);
+    rc = olmax_gemm_padded(stream, logits, hp, dW, nullptr, V, d, (int)T, ldl, d, d, 0, false, false, dw_f32 != 0, true, scratch);
     if (rc) return rc;
   }
   return OLMAX_OK;
+}
+
+extern "C" int32_t olmax_lmhead_ce(hipStream_t stream, const void* h, const void* W,
+                                   const int32_t* labels, float* loss, void* dh, void* dW,
+                                   void* workspace, int64_t workspace_bytes, int64_t T, int32_t d,
+                                   int32_t V, int32_t ignore_index, float softcap, int32_t dw_f32) {
+  return olmax_lmhead_ce_scratch(stream, h, W, labels, loss, dh, dW, workspace, workspace_bytes, T, d, V, ignore_index, softcap, dw_f32,
+                                 GemmScratch());
 }

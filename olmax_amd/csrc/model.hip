@@ -86,6 +86,11 @@ struct Tmp {
   bf16 *dact, *dgu, *d1, *d2, *d_o, *dqkv, *dqkr;
   void* attn_ws;
   int64_t attn_ws_bytes;
+  // What a GEMM may use for partial results: the buffers of the attention part while the MLP part runs, and the other
+  // way round; all of it before the first block's backward.
+  GemmScratch in_mlp() const { return {d_o, (char*)attn_ws + attn_ws_bytes - (char*)d_o}; }
+  GemmScratch in_attn() const { return {dact, (char*)d1 - (char*)dact}; }
+  GemmScratch before() const { return {dact, (char*)attn_ws + attn_ws_bytes - (char*)dact}; }
 };
 Tmp carve_tmp(const olmax_model_config* c, Arena& a) {
   const Dims m = dims_of(c);
@@ -119,13 +124,13 @@ int lin_fwd(hipStream_t s, const bf16* x, int64_t ldx, const void* W, int in, in
 }
 // dx[T,in] = dy[T,out] W[out,in] (+ res)
 int lin_dx(hipStream_t s, const bf16* dy, int64_t lddy, const void* W, int in, int out, bf16* dx, int64_t lddx,
-           const bf16* res, int64_t ldres, int64_t T) {
-  return olmax_gemm_bf16(s, dy, W, dx, res, (int)T, in, out, lddy, in, lddx, ldres, 0, 1, 0);
+           const bf16* res, int64_t ldres, int64_t T, GemmScratch ws) {
+  return olmax_gemm_padded(s, dy, (const bf16*)W, dx, res, (int)T, in, out, lddy, in, lddx, ldres, true, false, false, false, ws);
 }
 // dW[out,in] = dy[T,out]^T x[T,in]
 int lin_dw(hipStream_t s, const bf16* dy, int64_t lddy, const bf16* x, int64_t ldx, int in, int out, void* dW,
-           int64_t T, int out_f32 = 0) {
-  return olmax_gemm_bf16(s, dy, x, dW, nullptr, out, in, (int)T, lddy, ldx, in, 0, 1, 1, out_f32);
+           int64_t T, GemmScratch ws) {
+  return olmax_gemm_padded(s, dy, x, dW, nullptr, out, in, (int)T, lddy, ldx, in, 0, false, false, false, false, ws);
 }
 
 // need_y == false (recompute before the backward): the block output itself is not an input of
@@ -221,8 +226,8 @@ int attn_backward(hipStream_t s, const olmax_model_config* c, const olmax_block_
                   const Acts& a, const Tmp& t) {
   const Dims m = dims_of(c);
   const float eps = c->eps;
-  RC(lin_dx(s, d_attn_out, m.d, w->wo, m.HD, m.d, t.d_o, m.HD, nullptr, 0, m.T));
-  RC(lin_dw(s, d_attn_out, m.d, a.o, m.HD, m.HD, m.d, g->wo, m.T));
+  RC(lin_dx(s, d_attn_out, m.d, w->wo, m.HD, m.d, t.d_o, m.HD, nullptr, 0, m.T, t.in_attn()));
+  RC(lin_dw(s, d_attn_out, m.d, a.o, m.HD, m.HD, m.d, g->wo, m.T, t.in_attn()));
   const bf16* vp = a.qkv + m.HD + m.KD;
   RC(hook_point(POINT_ATTN_BWD));
   if (c->qk_norm) {
@@ -248,8 +253,8 @@ int attn_backward(hipStream_t s, const olmax_model_config* c, const olmax_block_
     RC(olmax_qk_rope_bwd(s, t.dqkv, t.dqkv, nullptr, nullptr, nullptr, cos_t, sin_t, m.T, m.H + m.K, m.D, m.S, m.QKV,
                          m.QKV, 0, eps));
   }
-  RC(lin_dx(s, t.dqkv, m.QKV, w->wqkv, m.d, m.QKV, dxin, m.d, res_for_dx, m.d, m.T));
-  RC(lin_dw(s, t.dqkv, m.QKV, attn_in, m.d, m.d, m.QKV, g->wqkv, m.T));
+  RC(lin_dx(s, t.dqkv, m.QKV, w->wqkv, m.d, m.QKV, dxin, m.d, res_for_dx, m.d, m.T, t.in_attn()));
+  RC(lin_dw(s, t.dqkv, m.QKV, attn_in, m.d, m.d, m.QKV, g->wqkv, m.T, t.in_attn()));
   return OLMAX_OK;
 }
 
@@ -264,14 +269,14 @@ int mlp_backward(hipStream_t s, const olmax_model_config* c, const olmax_block_w
   if (deferred) {
     RC(olmax_gemm_glu_bwd_bf16(s, mlp_in, w->wgu, t.dact, a.act, t.dgu, (int)m.T, m.F, m.d, m.d, m.d, m.F, m.F, 2 * m.F, c->act));
   } else {
-    RC(lin_dx(s, d_mlp_out, m.d, w->wdown, m.F, m.d, t.dact, m.F, nullptr, 0, m.T));
+    RC(lin_dx(s, d_mlp_out, m.d, w->wdown, m.F, m.d, t.dact, m.F, nullptr, 0, m.T, t.in_mlp()));
   }
-  RC(lin_dw(s, d_mlp_out, m.d, a.act, m.F, m.F, m.d, g->wdown, m.T));
+  RC(lin_dw(s, d_mlp_out, m.d, a.act, m.F, m.F, m.d, g->wdown, m.T, t.in_mlp()));
   if (!deferred)
     RC(olmax_glu_bwd(s, a.gu, a.gu + m.F, t.dact, t.dgu, t.dgu + m.F, m.T, m.F, 2 * m.F, 2 * m.F, m.F, 2 * m.F, 2 * m.F,
                      c->act));
-  RC(lin_dx(s, t.dgu, 2 * m.F, w->wgu, m.d, 2 * m.F, dxin, m.d, res_for_dx, m.d, m.T));
-  RC(lin_dw(s, t.dgu, 2 * m.F, mlp_in, m.d, m.d, 2 * m.F, g->wgu, m.T));
+  RC(lin_dx(s, t.dgu, 2 * m.F, w->wgu, m.d, 2 * m.F, dxin, m.d, res_for_dx, m.d, m.T, t.in_mlp()));
+  RC(lin_dw(s, t.dgu, 2 * m.F, mlp_in, m.d, m.d, 2 * m.F, g->wgu, m.T, t.in_mlp()));
   return OLMAX_OK;
 }
 
@@ -489,11 +494,11 @@ int model_run(hipStream_t s, const olmax_model_config* c, const int32_t* windows
   }
   if (c->tied) {
     // head dW is written (fp32) straight into the embedding's accumulator; the scatter-add follows
-    RC(olmax_lmhead_ce(s, w.hn, Wout, labels, loss, w.da, grad_f32 + L.f_embedding, w.head_ws, w.head_ws_bytes, m.T, m.d,
-                       c->vocab, -100, c->final_softcap, 1));
+    RC(olmax_lmhead_ce_scratch(s, w.hn, Wout, labels, loss, w.da, grad_f32 + L.f_embedding, w.head_ws, w.head_ws_bytes, m.T,
+                               m.d, c->vocab, -100, c->final_softcap, 1, w.tmp.before()));
   } else {
-    RC(olmax_lmhead_ce(s, w.hn, Wout, labels, loss, w.da, G + L.lm_head, w.head_ws, w.head_ws_bytes, m.T, m.d, c->vocab,
-                       -100, c->final_softcap, 0));
+    RC(olmax_lmhead_ce_scratch(s, w.hn, Wout, labels, loss, w.da, G + L.lm_head, w.head_ws, w.head_ws_bytes, m.T, m.d,
+                               c->vocab, -100, c->final_softcap, 0, w.tmp.before()));
   }
   RC(olmax_rmsnorm_bwd(s, xl, P + L.final_norm, w.da, nullptr, w.db, grad_f32 + L.f_final_norm, m.T, m.d, m.d, m.d, 0,
                        m.d, c->eps));
@@ -518,7 +523,7 @@ int model_run(hipStream_t s, const olmax_model_config* c, const int32_t* windows
     // memory, no GLU backward kernel: 0.9 GB less traffic per 7B layer).
     const bool defer = !keep && c->layer_type == 0;
     if (defer) {
-      RC(lin_dx(s, dcur, m.d, bw.wdown, m.F, m.d, w.tmp.dact, m.F, nullptr, 0, m.T));
+      RC(lin_dx(s, dcur, m.d, bw.wdown, m.F, m.d, w.tmp.dact, m.F, nullptr, 0, m.T, w.tmp.in_mlp()));
       RC(hook_point(POINT_AFTER_DACT));
     }
     if (!keep) {
