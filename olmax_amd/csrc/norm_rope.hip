@@ -7,6 +7,7 @@
 //   head-wise QK-norm   src/olmax/nn/attention.py:293-296 (one [head_dim] weight for all heads)
 //   RoPE                src/olmax/nn/rope.py:62-65,99-115 (rotate_half pairing i <-> i + D/2)
 #include "common.h"
+#include <mutex>
 
 namespace {
 
@@ -89,7 +90,26 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_generic(const bf16* __restric
 // ------------------------------------------------------------------ RMSNorm backward
 // dx = r*g - x * r^3 * mean(x*g), g = w*dy;   dw[c] += sum_rows dy*x*r   (fp32 atomics)
 // Optional `dres` is added to dx (fused residual-gradient add).
-// Narrow rows (d <= 1024): LPR lanes of one wave own a row, which stays in registers between the
+// The column sums of a block's SLOTS rows in flight meet in LDS, every slot in its own row (one barrier; added
+// one after the other in the same place they took 2.5 of the 10.8 us of 2048 x 256), then one global atomic per
+// column and block.  Global fp32 atomics are resolved beyond the per-XCD L2s at about 50 G/s, so the launches use
+// few, fat blocks.
+__device__ __forceinline__ void park8(float* dst, const float (&v)[8]) {
+  *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+  *reinterpret_cast<f32x4*>(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
+}
+template <int SLOTS, int THREADS>
+__device__ __forceinline__ void add_slots(const float* sdw, float* __restrict__ dw, int d) {
+  __syncthreads();
+  for (int i = threadIdx.x; i < d; i += THREADS) {
+    float t = sdw[i];
+#pragma unroll
+    for (int s = 1; s < SLOTS; s++) t += sdw[s * d + i];
+    atomicAdd(&dw[i], t);
+  }
+}
+
+// Narrow rows (d <= 256): LPR lanes of one wave own a row, which stays in registers between the
 // two passes, and the lanes' columns sums live in registers until the end.
 template <int LPR, int MAXC, int THREADS>
 __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_kernel(
@@ -153,44 +173,22 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_kernel(
       }
   }
   if (dw) {
-    // Combine the RPB row-slots of this block in LDS, then one global atomic per column per
-    // block.  Global fp32 atomics are the expensive part (they are resolved beyond the per-XCD
-    // L2s, ~50 G/s), so the launch uses few, fat blocks; inside the block the slots add in turn
-    // (each lane owns its columns, so plain read-modify-write is enough).
-    extern __shared__ float sdw[];  // d floats
-#pragma unroll 1
-    for (int turn = 0; turn < RPB; turn++) {
-      if (rloc == turn) {
+    extern __shared__ float sdw[];  // RPB x d floats
 #pragma unroll
-        for (int i = 0; i < MAXC; i++)
-          if ((i * LPR + sub) * 8 < d) {
-            float* dst = &sdw[(i * LPR + sub) * 8];
-            f32x4 lo, hi;
-            if (turn == 0) {
-#pragma unroll
-              for (int e = 0; e < 4; e++) { lo[e] = dwacc[i][e]; hi[e] = dwacc[i][4 + e]; }
-            } else {
-              lo = *reinterpret_cast<f32x4*>(dst);
-              hi = *reinterpret_cast<f32x4*>(dst + 4);
-#pragma unroll
-              for (int e = 0; e < 4; e++) { lo[e] += dwacc[i][e]; hi[e] += dwacc[i][4 + e]; }
-            }
-            *reinterpret_cast<f32x4*>(dst) = lo;
-            *reinterpret_cast<f32x4*>(dst + 4) = hi;
-          }
-      }
-      __syncthreads();
-    }
-    for (int i = threadIdx.x; i < d; i += THREADS) atomicAdd(&dw[i], sdw[i]);
+    for (int i = 0; i < MAXC; i++)
+      if ((i * LPR + sub) * 8 < d) park8(sdw + rloc * d + (i * LPR + sub) * 8, dwacc[i]);
+    add_slots<RPB, THREADS>(sdw, dw, d);
   }
 }
 
-// Wide rows (2048 < d <= 8192).  WPR waves share one row, a lane owns MAXC chunks of 8 columns,
+// Wider rows (d <= 8192).  WPR waves share one row, a lane owns MAXC chunks of 8 columns,
 // so the row held between the two passes and the dw column sums take 12 * MAXC registers
 // instead of 128 + 64: sixteen waves fit on a CU, and for a kernel that only streams, waves in
 // flight are what sets the bandwidth.  The waves of a row exchange their partial sums through
 // LDS (two slots used in turn, one barrier per iteration); the next row's x, dy and dres are
 // already on their way while the current one is reduced.
+// d <= 1024 has a wave to itself per row (no exchange): 8192 x 1024 26 -> 21 us and 3000 x 1024 15 -> 12 us against
+// the narrow kernel's eight waves per CU without a row in flight (67 and 25 MB; the rest is latency and atomics).
 template <int WPR, int MAXC, int THREADS>
 __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_split_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ w, const bf16* __restrict__ dy,
@@ -200,7 +198,7 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_split_kernel(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rloc = wave / WPR, part = wave % WPR;
   __shared__ float red[2][RPB][WPR][2];
-  extern __shared__ float sdw[];  // d floats when dw is asked for
+  extern __shared__ float sdw[];  // RPB x d floats when dw is asked for
 
   int col[MAXC];
   bool on[MAXC];
@@ -257,23 +255,27 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_split_kernel(
       ss += __shfl_xor(ss, o, 64);
       sxg += __shfl_xor(sxg, o, 64);
     }
-    if (lane == 0) {
-      red[buf][rloc][part][0] = ss;
-      red[buf][rloc][part][1] = sxg;
+    if (WPR > 1) {
+      if (lane == 0) {
+        red[buf][rloc][part][0] = ss;
+        red[buf][rloc][part][1] = sxg;
+      }
+      __syncthreads();
     }
-    __syncthreads();
     // Keep the row packed across the barrier: without this the compiler carries the widened
     // floats of the first pass into the second and doubles the register count.
 #pragma unroll
     for (int i = 0; i < MAXC; i++) {
       asm volatile("" : "+v"(cx[i].u), "+v"(cg[i].u), "+v"(wv[i].u));
     }
-    ss = 0.f;
-    sxg = 0.f;
+    if (WPR > 1) {
+      ss = 0.f;
+      sxg = 0.f;
 #pragma unroll
-    for (int p = 0; p < WPR; p++) {
-      ss += red[buf][rloc][p][0];
-      sxg += red[buf][rloc][p][1];
+      for (int p = 0; p < WPR; p++) {
+        ss += red[buf][rloc][p][0];
+        sxg += red[buf][rloc][p][1];
+      }
     }
     if (row < rows) {
       const float r = rsqrtf(ss / (float)d + eps);
@@ -297,32 +299,10 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_split_kernel(
     }
   }
   if (dw) {
-    // The RPB row slots of the block add their column sums in LDS in turn (every column has one
-    // owner per slot), then one global atomic per column and block.
-#pragma unroll 1
-    for (int turn = 0; turn < RPB; turn++) {
-      if (rloc == turn) {
 #pragma unroll
-        for (int i = 0; i < MAXC; i++)
-          if (on[i]) {
-            float* dst = &sdw[col[i]];
-            f32x4 lo, hi;
-            if (turn == 0) {
-#pragma unroll
-              for (int e = 0; e < 4; e++) { lo[e] = dwacc[i][e]; hi[e] = dwacc[i][4 + e]; }
-            } else {
-              lo = *reinterpret_cast<f32x4*>(dst);
-              hi = *reinterpret_cast<f32x4*>(dst + 4);
-#pragma unroll
-              for (int e = 0; e < 4; e++) { lo[e] += dwacc[i][e]; hi[e] += dwacc[i][4 + e]; }
-            }
-            *reinterpret_cast<f32x4*>(dst) = lo;
-            *reinterpret_cast<f32x4*>(dst + 4) = hi;
-          }
-      }
-      __syncthreads();
-    }
-    for (int i = threadIdx.x; i < d; i += THREADS) atomicAdd(&dw[i], sdw[i]);
+    for (int i = 0; i < MAXC; i++)
+      if (on[i]) park8(sdw + rloc * d + col[i], dwacc[i]);
+    add_slots<RPB, THREADS>(sdw, dw, d);
   }
 }
 
@@ -638,22 +618,29 @@ extern "C" int32_t olmax_rmsnorm_bwd(hipStream_t stream, const void* x, const vo
                    (!dres || (aligned16(dres) && lddres % 8 == 0)) && ldx % 8 == 0 && lddy % 8 == 0 && lddx % 8 == 0;
   const bf16 *xp = (const bf16*)x, *wp = (const bf16*)w, *dyp = (const bf16*)dy, *drp = (const bf16*)dres;
   bf16* dxp = (bf16*)dx;
-  const size_t smem = dw ? (size_t)d * 4 : 0;
-#define OLMAX_NORM_BWD_ARGS smem, stream, xp, wp, dyp, drp, dxp, dw, rows, d, ldx, lddy, lddres, lddx, eps
+  // SLOTS rows in flight per block of THREADS; the LDS row of each (64 KB at most) holds its column sums
+#define OLMAX_NORM_BWD(SLOTS, THREADS, ...)                                                                                       \
+  do {                                                                                                                            \
+    auto kern = __VA_ARGS__;                                                                                                      \
+    static std::once_flag once;                                                                                                   \
+    std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 65536); }); \
+    hipLaunchKernelGGL(kern, dim3(grid_for(rows, SLOTS, 256)), dim3(THREADS), dw ? (size_t)SLOTS * d * 4 : 0, stream, xp, wp, dyp, drp, \
+                       dxp, dw, rows, d, ldx, lddy, lddres, lddx, eps);                                                           \
+  } while (0)
   if (vec && d % 8 == 0 && d <= 256) {
-    hipLaunchKernelGGL((rmsnorm_bwd_kernel<16, 2, 256>), dim3(grid_for(rows, 16, 256)), dim3(256), OLMAX_NORM_BWD_ARGS);
+    OLMAX_NORM_BWD(16, 256, rmsnorm_bwd_kernel<16, 2, 256>);
   } else if (vec && d % 8 == 0 && d <= 1024) {
-    hipLaunchKernelGGL((rmsnorm_bwd_kernel<64, 2, 512>), dim3(grid_for(rows, 8, 256)), dim3(512), OLMAX_NORM_BWD_ARGS);
+    OLMAX_NORM_BWD(16, 1024, rmsnorm_bwd_split_kernel<1, 2, 1024>);
   } else if (vec && d % 8 == 0 && d <= 2048) {
-    hipLaunchKernelGGL((rmsnorm_bwd_split_kernel<2, 2, 1024>), dim3(grid_for(rows, 8, 256)), dim3(1024), OLMAX_NORM_BWD_ARGS);
+    OLMAX_NORM_BWD(8, 1024, rmsnorm_bwd_split_kernel<2, 2, 1024>);
   } else if (vec && d % 8 == 0 && d <= 4096) {
-    hipLaunchKernelGGL((rmsnorm_bwd_split_kernel<4, 2, 1024>), dim3(grid_for(rows, 4, 256)), dim3(1024), OLMAX_NORM_BWD_ARGS);
+    OLMAX_NORM_BWD(4, 1024, rmsnorm_bwd_split_kernel<4, 2, 1024>);
   } else if (vec && d % 8 == 0 && d <= 8192) {
-    hipLaunchKernelGGL((rmsnorm_bwd_split_kernel<8, 2, 1024>), dim3(grid_for(rows, 2, 256)), dim3(1024), OLMAX_NORM_BWD_ARGS);
+    OLMAX_NORM_BWD(2, 1024, rmsnorm_bwd_split_kernel<8, 2, 1024>);
   } else {
     hipLaunchKernelGGL(rmsnorm_bwd_generic, dim3(grid_for(rows, 1, 1 << 16)), dim3(256), 0, stream, xp, wp, dyp, drp, dxp, dw, rows, d, ldx, lddy, lddres, lddx, eps);
   }
-#undef OLMAX_NORM_BWD_ARGS
+#undef OLMAX_NORM_BWD
   OLMAX_LAUNCH_CHECK();
   return OLMAX_OK;
 }
