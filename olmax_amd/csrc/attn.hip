@@ -1102,7 +1102,9 @@ extern "C" int32_t olmax_attn_bwd(hipStream_t stream, const void* q, const void*
   const float scale = 1.f / sqrtf((float)D);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k, *vp = (const bf16*)v, *op = (const bf16*)o, *gop = (const bf16*)d_o;
   float* delta = (float*)workspace;
-  if (bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, S, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv)) {
+  // (a workspace of delta alone is head_dim 128's: any other head_dim may meet an unaligned view)
+  if (bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, S, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv) &&
+      (D == 128 || workspace_bytes >= attn_delta_bytes(B, S, H) + 2 * attn_acc_bytes(B, S, KH, D))) {
     auto go = D == 128 ? launch_bwd_fast<128> : launch_bwd_fast<64>;
     go(stream, qp, kp, vp, op, lse, gop, (bf16*)dq, (bf16*)dk, (bf16*)dv, delta, B, S, H, KH, ldq, ldk, ldv, ldo, lddo,
        lddq, lddk, lddv, window, softcap);

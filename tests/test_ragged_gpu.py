@@ -94,6 +94,20 @@ def test_fused_gated_projection_on_ragged_rows(act, T, F, d):
     assert torch.equal(act_b, want) and torch.equal(dgu[:, :F], dg) and torch.equal(dgu[:, F:], du)
 
 
+@pytest.mark.parametrize("which", ["x", "w", "out"])
+def test_gated_projection_on_ragged_rows_of_unaligned_views(which):
+    """Views the fused GEMM cannot take get the two-step path, also when gate|up were not asked for."""
+    from olmax_amd import ops
+    print(f"[case] gated projection, unaligned {which}", flush=True)
+    T, F, d = 2049, 2048, 128
+    shift = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)  # noqa: E731
+    x, w, out = rnd(T, d, seed=1), rnd(2 * F, d, seed=2, scale=d ** -0.5), torch.empty(T, F, device="cuda", dtype=BF)
+    want, _ = ops.gated_mlp_in(x, w)
+    args = {k: shift(t) if k == which else t for k, t in (("x", x), ("w", w), ("out", out))}
+    got, _ = ops.gated_mlp_in(args["x"], args["w"], save_gate_up=False, out=args["out"])
+    assert rel(got, want) < 2 ** -8
+
+
 @pytest.mark.parametrize("B,S,heads,N,d", [(3, 1000, 24, 3072, 128), (1, 2049, 20, 6144, 64)])
 def test_fused_rope_projection_on_ragged_rows(B, S, heads, N, d):
     from olmax_amd import ops
