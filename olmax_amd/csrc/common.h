@@ -175,3 +175,23 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
 int olmax_lmhead_ce_scratch(hipStream_t stream, const void* h, const void* W, const int32_t* labels, float* loss, void* dh, void* dW,
                             void* workspace, int64_t workspace_bytes, int64_t T, int32_t d, int32_t V, int32_t ignore_index,
                             float softcap, int32_t dw_f32, GemmScratch scratch);
+// elementwise.hip: pieces of the flat buffers too small for a launch each; one launch takes a table of them.  off: first element in
+// parameter layout, goff: of its gradient in the bf16 or (g_f32) fp32 buffer
+struct FlatRange {
+  int64_t off, goff;
+  int32_t n, g_f32, decay, first;  // first workgroup
+};
+struct FlatRanges {
+  static constexpr int MAX = 32, CHUNK = 1024;  // ranges; elements of a workgroup
+  static constexpr int64_t MAX_N = 1 << 21;
+  FlatRange r[MAX];
+  int32_t count = 0, blocks = 0;
+  void add(int64_t off, int64_t goff, int64_t n, bool g_f32, bool decay) {
+    r[count++] = {off, goff, (int32_t)n, g_f32, decay, blocks};
+    blocks += (int32_t)((n + CHUNK - 1) / CHUNK);
+  }
+};
+int olmax_adamw_ranges(hipStream_t stream, const FlatRanges& t, float* p, const bf16* g, const float* gf, float* m, float* v, bf16* shadow,
+                       float lr, float b1, float b2, float eps, float wd, int64_t step, const float* grad_scale_dev,
+                       const float* hyper_dev);
+int olmax_grad_accumulate_ranges(hipStream_t stream, const FlatRanges& t, float* acc, const bf16* g, const float* gf, int mini_step);

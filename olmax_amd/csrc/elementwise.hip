@@ -94,11 +94,11 @@ __global__ void glu_bwd_scalar(const bf16* gate, const bf16* up, const bf16* dh,
 // Running mean over micro-batches, acc += (g - acc) / (k + 1) for the k-th (0-based) micro-batch
 // (optax.MultiSteps with use_grad_mean, which the reference wraps its optimizer in,
 // src/olmax/optim/config.py:153-154); k = 0 overwrites acc.
-template <bool G_BF16>
-__global__ __launch_bounds__(256) void grad_accum_kernel(float* __restrict__ acc, const void* __restrict__ gv, int64_t n,
-                                                         float inv, int first) {
-  const int64_t n4 = n / 4;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
+// [i, end) in vectors of 4 elements, `step` apart, and the ntail (< 4) elements behind vector n4
+template <bool G_BF16, typename Int>
+__device__ __forceinline__ void grad_accum_span(float* __restrict__ acc, const void* __restrict__ gv, Int i, Int end, Int step, Int n4,
+                                                int ntail, float inv, int first) {
+  for (; i < end; i += step) {
     float g[4];
     if (G_BF16) {
       Pack4 gp;
@@ -121,11 +121,46 @@ __global__ __launch_bounds__(256) void grad_accum_kernel(float* __restrict__ acc
     }
     reinterpret_cast<f32x4*>(acc)[i] = a;
   }
-  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
-    const int64_t i = n4 * 4 + threadIdx.x;
-    const float g = G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[i]) : reinterpret_cast<const float*>(gv)[i];
-    acc[i] = first ? g : acc[i] + (g - acc[i]) * inv;
+  if ((int)threadIdx.x < ntail) {
+    const Int j = n4 * 4 + (Int)threadIdx.x;
+    const float g = G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[j]) : reinterpret_cast<const float*>(gv)[j];
+    acc[j] = first ? g : acc[j] + (g - acc[j]) * inv;
   }
+}
+template <bool G_BF16>
+__global__ __launch_bounds__(256) void grad_accum_kernel(float* __restrict__ acc, const void* __restrict__ gv, int64_t n,
+                                                         float inv, int first) {
+  grad_accum_span<G_BF16>(acc, gv, (int64_t)blockIdx.x * 256 + threadIdx.x, n / 4, (int64_t)gridDim.x * 256, n / 4,
+                          blockIdx.x == 0 ? (int)(n & 3) : 0, inv, first);
+}
+
+// ------------------------------------------------------------------ ranges of the flat buffers
+// A model has two to six vectors of a few KB per layer (norm weights, gradients in fp32) between its matrices, and
+// a small one matrices of a few hundred KB: a launch for each is 3 to 5 us of latency and 2 us of gap.  One launch takes up to
+// 32 of them: CHUNK elements to a workgroup, one vector of 4 to a lane; a workgroup finds its range with one load per lane and a ballot.
+__device__ __forceinline__ int find_range(const FlatRanges& t) {
+  const int lane = threadIdx.x & 63;
+  const int first = lane < t.count ? t.r[lane & (FlatRanges::MAX - 1)].first : 0x7fffffff;
+  return __builtin_amdgcn_readfirstlane((int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(first <= (int)blockIdx.x)) - 1);
+}
+// a workgroup's part of a range: its first element, vectors of 4, and the elements (< 4) behind them
+struct RangeSpan {
+  int64_t at;
+  int n4, ntail;
+  __device__ __forceinline__ explicit RangeSpan(const FlatRange& r) {
+    const int skip = ((int)blockIdx.x - r.first) * FlatRanges::CHUNK, n = min(r.n - skip, FlatRanges::CHUNK);
+    at = skip;
+    n4 = n >> 2;
+    ntail = n & 3;
+  }
+};
+__global__ __launch_bounds__(256) void grad_accum_ranges_kernel(FlatRanges t, float* __restrict__ acc, const bf16* __restrict__ g,
+                                                                const float* __restrict__ gf, float inv, int first) {
+  const FlatRange r = t.r[find_range(t)];
+  const RangeSpan sp(r);
+  acc += r.off + sp.at;
+  if (r.g_f32) grad_accum_span<false>(acc, gf + r.goff + sp.at, (int)threadIdx.x, sp.n4, 256, sp.n4, sp.ntail, inv, first);
+  else grad_accum_span<true>(acc, g + r.goff + sp.at, (int)threadIdx.x, sp.n4, 256, sp.n4, sp.ntail, inv, first);
 }
 
 // ------------------------------------------------------------------ synthetic token batches
@@ -199,82 +234,148 @@ __device__ __forceinline__ float adamw_new_p(float p, float mh, float vh, float 
   return __builtin_fmaf(-lr, __builtin_fmaf(mh, r, wd * p), p);
 }
 
-template <bool G_BF16>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(16))) void adamw_kernel(
-    float* __restrict__ p, const void* __restrict__ gv, float* __restrict__ m, float* __restrict__ v,
-    bf16* __restrict__ shadow, int64_t n, float lr, float b1, float b2, float eps, float wd, float bc1,
-    float bc2, float gscale, const float* __restrict__ gscale_dev, const float* __restrict__ hyper_dev) {
+struct AdamwScalars {
+  float lr, b1, b2, eps, wd, ibc1, ibc2, gscale;
+};
+__device__ __forceinline__ AdamwScalars adamw_scalars(float lr, float b1, float b2, float eps, float wd, float bc1, float bc2, float gscale,
+                                                      const float* __restrict__ gscale_dev, const float* __restrict__ hyper_dev) {
   if (gscale_dev) gscale *= *gscale_dev;
   if (hyper_dev) {  // step-dependent scalars from device memory (wave-uniform scalar loads)
     lr = hyper_dev[0];
     bc1 = hyper_dev[1];
     bc2 = hyper_dev[2];
   }
-  const int64_t n4 = n / 4;
-  const float ibc1 = 1.f / bc1, ibc2 = 1.f / bc2, omb1 = 1.f - b1, omb2 = 1.f - b2;
-  // Every element is touched exactly once: streaming (non-temporal) accesses keep the 28 B/param
-  // out of the way of the L2.  The kernel is held to 32 registers (amdgpu_num_vgpr counts pairs
-  // of the unified file on this target) so that one of its waves fits on a SIMD beside two
-  // 240-register GEMM waves when it runs on a second stream, and it is launched as a small
-  // grid-stride grid (two workgroups per CU): the whole grid then sweeps five arrays as
-  // contiguous 2 MB fronts, which measured 5.6 TB/s against 4.7 TB/s for one workgroup per 8 KB.
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += stride) {
-    f32x4 pv = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p) + i);
-    f32x4 mv = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(m) + i);
-    f32x4 vv = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(v) + i);
-    float g[4];
-    if (G_BF16) {
-      Pack4 gp;
-      gp.u = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(gv) + i);
+  // (results of vector instructions that are the same in every lane: back to scalar registers)
+  auto uniform = [](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); };
+  return {lr, b1, b2, eps, wd, uniform(1.f / bc1), uniform(1.f / bc2), uniform(gscale)};
+}
+
+// The vector of 4 elements `lane` vectors behind the (wave-uniform) pointers.  Every element is touched exactly once: streaming
+// (non-temporal) accesses keep the 28 B/param out of the way of the L2.  One 32-bit offset register addresses all five arrays and
+// the four loads are requested together: with a 64-bit pointer register pair per array they did not fit the 32 registers of
+// the kernels below and waited for each other.
+template <bool G_BF16>
+__device__ __forceinline__ void adamw_vec(float* __restrict__ p, const void* __restrict__ gv, float* __restrict__ m, float* __restrict__ v,
+                                          bf16* __restrict__ shadow, uint32_t lane, const AdamwScalars& c) {
+  const float lr = c.lr, b1 = c.b1, b2 = c.b2, eps = c.eps, wd = c.wd, ibc1 = c.ibc1, ibc2 = c.ibc2, gscale = c.gscale;
+  const float omb1 = 1.f - b1, omb2 = 1.f - b2;
+  // opaque scalar bases and lane: a loop's pointer arithmetic stays in scalar registers
+  uint64_t pa = (uint64_t)p, ga = (uint64_t)gv, ma = (uint64_t)m, va = (uint64_t)v, sa = (uint64_t)shadow;
+  asm volatile("" : "+v"(lane), "+s"(pa), "+s"(ga), "+s"(ma), "+s"(va), "+s"(sa));
+  const uint32_t o16 = lane * 16, o8 = lane * 8;
+#define GLOBAL(T, base, bytes) ((__attribute__((address_space(1))) T*)((__attribute__((address_space(1))) char*)(base) + (bytes)))
+  f32x4 gf;
+  Pack4 gp;
+  if (G_BF16) gp.u = __builtin_nontemporal_load(GLOBAL(u32x2, ga, o8));
+  else gf = __builtin_nontemporal_load(GLOBAL(f32x4, ga, o16));
+  f32x4 mv = __builtin_nontemporal_load(GLOBAL(f32x4, ma, o16));
+  f32x4 vv = __builtin_nontemporal_load(GLOBAL(f32x4, va, o16));
+  f32x4 pv = __builtin_nontemporal_load(GLOBAL(f32x4, pa, o16));
+  __builtin_amdgcn_sched_barrier(0);
+  Pack4 sh;
 #pragma unroll
-      for (int e = 0; e < 4; e++) g[e] = bf2f(gp.e[e]);
-    } else {
-      f32x4 gf = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(gv) + i);
-#pragma unroll
-      for (int e = 0; e < 4; e++) g[e] = gf[e];
-    }
-    Pack4 sh;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float ge = g[e] * gscale;
-      mv[e] = b1 * mv[e] + omb1 * ge;
-      vv[e] = b2 * vv[e] + omb2 * ge * ge;
-      pv[e] = adamw_new_p(pv[e], mv[e] * ibc1, vv[e] * ibc2, lr, eps, wd);
-      sh.e[e] = f2bf(pv[e]);
-    }
-    __builtin_nontemporal_store(pv, reinterpret_cast<f32x4*>(p) + i);
-    __builtin_nontemporal_store(mv, reinterpret_cast<f32x4*>(m) + i);
-    __builtin_nontemporal_store(vv, reinterpret_cast<f32x4*>(v) + i);
-    if (shadow) __builtin_nontemporal_store(sh.u, reinterpret_cast<u32x2*>(shadow) + i);
+  for (int e = 0; e < 4; e++) {
+    const float ge = (G_BF16 ? bf2f(gp.e[e]) : gf[e]) * gscale;
+    mv[e] = b1 * mv[e] + omb1 * ge;
+    vv[e] = b2 * vv[e] + omb2 * ge * ge;
+    pv[e] = adamw_new_p(pv[e], mv[e] * ibc1, vv[e] * ibc2, lr, eps, wd);
+    sh.e[e] = f2bf(pv[e]);
   }
+  __builtin_nontemporal_store(pv, GLOBAL(f32x4, pa, o16));
+  __builtin_nontemporal_store(mv, GLOBAL(f32x4, ma, o16));
+  __builtin_nontemporal_store(vv, GLOBAL(f32x4, va, o16));
+  if (sa) __builtin_nontemporal_store(sh.u, GLOBAL(u32x2, sa, o8));
+#undef GLOBAL
+}
+// element j (of the last n % 4)
+template <bool G_BF16, typename Int>
+__device__ __forceinline__ void adamw_one(float* __restrict__ p, const void* __restrict__ gv, float* __restrict__ m, float* __restrict__ v,
+                                          bf16* __restrict__ shadow, Int j, const AdamwScalars& c) {
+  const float lr = c.lr, b1 = c.b1, b2 = c.b2, eps = c.eps, wd = c.wd, ibc1 = c.ibc1, ibc2 = c.ibc2, gscale = c.gscale;
+  const float omb1 = 1.f - b1, omb2 = 1.f - b2;
+  const float ge = (G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[j]) : reinterpret_cast<const float*>(gv)[j]) * gscale;
+  // the same operations in the same order as the vector body: where a range is cut does not
+  // change any element's result
+  const float mm = b1 * m[j] + omb1 * ge;
+  const float vv = b2 * v[j] + omb2 * ge * ge;
+  const float pp = adamw_new_p(p[j], mm * ibc1, vv * ibc2, lr, eps, wd);
+  m[j] = mm;
+  v[j] = vv;
+  p[j] = pp;
+  if (shadow) shadow[j] = f2bf(pp);
+}
+
+// The kernel is held to 32 registers (amdgpu_num_vgpr counts pairs
+// of the unified file on this target) so that one of its waves fits on a SIMD beside two
+// 240-register GEMM waves when it runs on a second stream, and it is launched as a small
+// grid-stride grid (two workgroups per CU): the whole grid then sweeps five arrays as
+// contiguous 2 MB fronts, which measured 5.6 TB/s against 4.7 TB/s for one workgroup per 8 KB.
+template <bool G_BF16>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(16))) void adamw_kernel(
+    float* __restrict__ p, const void* __restrict__ gv, float* __restrict__ m, float* __restrict__ v,
+    bf16* __restrict__ shadow, int64_t n, float lr, float b1, float b2, float eps, float wd, float bc1,
+    float bc2, float gscale, const float* __restrict__ gscale_dev, const float* __restrict__ hyper_dev) {
+  const AdamwScalars c = adamw_scalars(lr, b1, b2, eps, wd, bc1, bc2, gscale, gscale_dev, hyper_dev);
+  const int64_t n4 = n / 4, stride = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256; i < n4; i += stride)
+    if (threadIdx.x < (uint32_t)min(n4 - i, (int64_t)256))
+      adamw_vec<G_BF16>(p + i * 4, reinterpret_cast<const char*>(gv) + i * (G_BF16 ? 8 : 16), m + i * 4, v + i * 4,
+                        shadow ? shadow + i * 4 : nullptr, threadIdx.x, c);
   // tail (n % 4) handled by the first threads of block 0
-  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
-    const int64_t i = n4 * 4 + threadIdx.x;
-    const float ge = (G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[i]) : reinterpret_cast<const float*>(gv)[i]) * gscale;
-    // the same operations in the same order as the vector body: where a range is cut does not
-    // change any element's result
-    const float mm = b1 * m[i] + omb1 * ge;
-    const float vv = b2 * v[i] + omb2 * ge * ge;
-    const float pp = adamw_new_p(p[i], mm * ibc1, vv * ibc2, lr, eps, wd);
-    m[i] = mm;
-    v[i] = vv;
-    p[i] = pp;
-    if (shadow) shadow[i] = f2bf(pp);
+  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) adamw_one<G_BF16>(p, gv, m, v, shadow, n4 * 4 + threadIdx.x, c);
+}
+// (also beside GEMM waves, hence the same 32 registers)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(16))) void adamw_ranges_kernel(
+    FlatRanges t, float* __restrict__ p, const bf16* __restrict__ g, const float* __restrict__ gf, float* __restrict__ m, float* __restrict__ v,
+    bf16* __restrict__ shadow, float lr, float b1, float b2, float eps, float wd, float bc1, float bc2,
+    const float* __restrict__ gscale_dev, const float* __restrict__ hyper_dev) {
+  const FlatRange r = t.r[find_range(t)];
+  const RangeSpan sp(r);
+  const AdamwScalars c = adamw_scalars(lr, b1, b2, eps, r.decay ? wd : 0.f, bc1, bc2, 1.f, gscale_dev, hyper_dev);
+  const int64_t o = r.off + sp.at, go = r.goff + sp.at;
+  const int i = threadIdx.x, j = sp.n4 * 4 + i;
+  const void* gr = r.g_f32 ? (const void*)(gf + go) : g + go;
+  p += o, m += o, v += o, shadow += o;
+  if (r.g_f32) {
+    if (i < sp.n4) adamw_vec<false>(p, gr, m, v, shadow, (uint32_t)i, c);
+    if (i < sp.ntail) adamw_one<false>(p, gr, m, v, shadow, j, c);
+  } else {
+    if (i < sp.n4) adamw_vec<true>(p, gr, m, v, shadow, (uint32_t)i, c);
+    if (i < sp.ntail) adamw_one<true>(p, gr, m, v, shadow, j, c);
   }
 }
 
 // sum of squares of a gradient leaf, accumulated (fp32 atomics) into *out
+// (four or eight elements per load where the alignment allows it, two loads in flight: 155 M fp32 188 -> 157 us)
 template <bool G_BF16>
-__global__ __launch_bounds__(256) void sumsq_kernel(const void* __restrict__ gv, int64_t n,
-                                                    float* __restrict__ out) {
+__global__ __launch_bounds__(256) void sumsq_kernel(const void* __restrict__ gv, int64_t n, int vec, float* __restrict__ out) {
+  constexpr int VEC = G_BF16 ? 8 : 4;
   __shared__ float red[4];
-  float s = 0.f;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const float g = G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[i]) : reinterpret_cast<const float*>(gv)[i];
-    s += g * g;
+  float s0 = 0.f, s1 = 0.f;
+  auto load = [&](int64_t i) { return reinterpret_cast<const u32x4*>(gv)[i]; };
+  auto add = [&](const u32x4& q) {
+    Pack8 b;
+    b.u = q;
+    const f32x4 f = (const f32x4&)q;
+#pragma unroll
+    for (int e = 0; e < VEC; e++) {
+      const float g = G_BF16 ? bf2f(b.e[e]) : f[e & 3];
+      (e & 1 ? s1 : s0) += g * g;
+    }
+  };
+  const int64_t nv = vec ? n / VEC : 0, step = (int64_t)gridDim.x * 256;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  for (; i + step < nv; i += 2 * step) {
+    const u32x4 a = load(i), b = load(i + step);
+    add(a);
+    add(b);
   }
-  s = block_sum<4>(s, red);
+  if (i < nv) add(load(i));
+  for (int64_t j = nv * VEC + (int64_t)blockIdx.x * 256 + threadIdx.x; j < n; j += step) {
+    const float g = G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[j]) : reinterpret_cast<const float*>(gv)[j];
+    s0 += g * g;
+  }
+  const float s = block_sum<4>(s0 + s1, red);
   if (threadIdx.x == 0) atomicAdd(out, s);
 }
 
@@ -385,6 +486,22 @@ extern "C" int32_t olmax_grad_accumulate(hipStream_t stream, float* acc, const v
   return OLMAX_OK;
 }
 
+static bool ranges_aligned(const FlatRanges& t) {
+  for (int i = 0; i < t.count; i++)
+    if (t.r[i].off % 4 || t.r[i].goff % 4) return false;
+  return true;
+}
+
+int olmax_grad_accumulate_ranges(hipStream_t stream, const FlatRanges& t, float* acc, const bf16* g, const float* gf, int mini_step) {
+  if (t.blocks == 0) return OLMAX_OK;
+  OLMAX_CHECK(aligned16(acc) && aligned16(gf) && (((uintptr_t)g) & 7) == 0 && ranges_aligned(t), OLMAX_ERR_ALIGN,
+              "olmax_grad_accumulate: acc / fp32 g must be 16-byte aligned, bf16 g 8-byte aligned");
+  hipLaunchKernelGGL(grad_accum_ranges_kernel, dim3((unsigned)t.blocks), dim3(256), 0, stream, t, acc, g, gf,
+                     1.f / (float)(mini_step + 1), (int)(mini_step == 0));
+  OLMAX_LAUNCH_CHECK();
+  return OLMAX_OK;
+}
+
 extern "C" int32_t olmax_sequential_tokens(hipStream_t stream, const int32_t* start_offsets, int32_t* inputs,
                                            int32_t* targets, int32_t B, int32_t S, int32_t V) {
   if (B == 0 || S == 0) return OLMAX_OK;
@@ -450,6 +567,22 @@ int olmax_adamw_grid(hipStream_t stream, float* p, const void* g, float* m, floa
   return OLMAX_OK;
 }
 
+int olmax_adamw_ranges(hipStream_t stream, const FlatRanges& t, float* p, const bf16* g, const float* gf, float* m, float* v, bf16* shadow,
+                       float lr, float b1, float b2, float eps, float wd, int64_t step, const float* grad_scale_dev,
+                       const float* hyper_dev) {
+  if (t.blocks == 0) return OLMAX_OK;
+  OLMAX_CHECK(step >= 1, OLMAX_ERR_ARG, "olmax_adamw: step must be >= 1 (1-based)");
+  OLMAX_CHECK(aligned16(p) && aligned16(m) && aligned16(v) && aligned16(gf) && (((uintptr_t)g) & 7) == 0 && (((uintptr_t)shadow) & 7) == 0 &&
+                  ranges_aligned(t),
+              OLMAX_ERR_ALIGN, "olmax_adamw: buffers must be 16-byte aligned (bf16 buffers 8-byte)");
+  const float bc1 = (float)(1.0 - pow((double)b1, (double)step));
+  const float bc2 = (float)(1.0 - pow((double)b2, (double)step));
+  hipLaunchKernelGGL(adamw_ranges_kernel, dim3((unsigned)t.blocks), dim3(256), 0, stream, t, p, g, gf, m, v, shadow, lr, b1, b2, eps, wd,
+                     bc1, bc2, grad_scale_dev, hyper_dev);
+  OLMAX_LAUNCH_CHECK();
+  return OLMAX_OK;
+}
+
 extern "C" int32_t olmax_adamw(hipStream_t stream, float* p, const void* g, float* m, float* v,
                                void* shadow_bf16, int64_t n, int32_t grad_is_bf16, float lr, float b1,
                                float b2, float eps, float wd, int64_t step, float grad_scale) {
@@ -460,9 +593,10 @@ extern "C" int32_t olmax_adamw(hipStream_t stream, float* p, const void* g, floa
 extern "C" int32_t olmax_sumsq(hipStream_t stream, const void* g, int64_t n, int32_t is_bf16, float* out) {
   if (n == 0) return OLMAX_OK;
   OLMAX_CHECK(g && out && n >= 0, OLMAX_ERR_ARG, "olmax_sumsq: bad argument");
-  const int grid = grid_1d(n, 2048);
-  if (is_bf16) hipLaunchKernelGGL(sumsq_kernel<true>, dim3(grid), dim3(256), 0, stream, g, n, out);
-  else hipLaunchKernelGGL(sumsq_kernel<false>, dim3(grid), dim3(256), 0, stream, g, n, out);
+  const int vec = aligned16(g);
+  const int grid = grid_1d(vec ? (n + 3) / 4 : n, 2048);
+  if (is_bf16) hipLaunchKernelGGL(sumsq_kernel<true>, dim3(grid), dim3(256), 0, stream, g, n, vec, out);
+  else hipLaunchKernelGGL(sumsq_kernel<false>, dim3(grid), dim3(256), 0, stream, g, n, vec, out);
   OLMAX_LAUNCH_CHECK();
   return OLMAX_OK;
 }

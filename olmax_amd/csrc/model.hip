@@ -542,34 +542,35 @@ int model_run(hipStream_t s, const olmax_model_config* c, const int32_t* windows
 }
 
 // AdamW over the leaves [begin, end) of a layout; runs of adjacent bf16-gradient leaves with
-// the same decay become single launches.  leaf_decay (host, one entry per leaf of the layout;
+// the same decay become single launches, all short runs and vectors one together.  leaf_decay (host, one entry per leaf of the layout;
 // NULL: every leaf decays) is the weight-decay mask of AdamWConfig.build.
 int adamw_leaves(hipStream_t s, const olmax_leaf* leaves, int begin, int end, float* master, float* mom, float* var,
                  bf16* shadow, const bf16* G, const float* grad_f32, int64_t step, float lr, float b1, float b2,
                  float eps, float wd, const int32_t* leaf_decay, const float* dscale, int grid_cap = 512,
                  const float* hyper_dev = nullptr) {
   auto decays = [&](int i) { return !leaf_decay || leaf_decay[i] != 0; };
+  FlatRanges small;
+  auto flush = [&]() -> int {
+    const int rc = olmax_adamw_ranges(s, small, master, G, grad_f32, mom, var, shadow, lr, b1, b2, eps, wd, step, dscale, hyper_dev);
+    small = FlatRanges();
+    return rc;
+  };
   int i = begin;
   while (i < end) {
     const olmax_leaf& lf = leaves[i];
-    const float lwd = decays(i) ? wd : 0.f;
-    if (lf.grad_f32) {
-      RC(olmax_adamw_grid(s, master + lf.offset, grad_f32 + lf.grad_f32_offset, mom + lf.offset, var + lf.offset,
-                          shadow + lf.offset, lf.numel, 0, lr, b1, b2, eps, lwd, step, 1.f, dscale, grid_cap, hyper_dev));
-      i++;
+    const bool f32 = lf.grad_f32, decay = decays(i);
+    int64_t n = lf.numel;
+    for (i++; !f32 && i < end && !leaves[i].grad_f32 && leaves[i].offset == lf.offset + n && decays(i) == decay; i++) n += leaves[i].numel;
+    const int64_t goff = f32 ? lf.grad_f32_offset : lf.offset;
+    if (n <= FlatRanges::MAX_N) {
+      if (small.count == FlatRanges::MAX) RC(flush());
+      small.add(lf.offset, goff, n, f32, decay);
     } else {
-      int64_t n = lf.numel;
-      int j = i + 1;
-      while (j < end && !leaves[j].grad_f32 && leaves[j].offset == lf.offset + n && decays(j) == decays(i)) {
-        n += leaves[j].numel;
-        j++;
-      }
-      RC(olmax_adamw_grid(s, master + lf.offset, G + lf.offset, mom + lf.offset, var + lf.offset, shadow + lf.offset, n, 1,
-                          lr, b1, b2, eps, lwd, step, 1.f, dscale, grid_cap, hyper_dev));
-      i = j;
+      RC(olmax_adamw_grid(s, master + lf.offset, f32 ? (const void*)(grad_f32 + goff) : G + goff, mom + lf.offset, var + lf.offset,
+                          shadow + lf.offset, n, !f32, lr, b1, b2, eps, decay ? wd : 0.f, step, 1.f, dscale, grid_cap, hyper_dev));
     }
   }
-  return OLMAX_OK;
+  return flush();
 }
 
 // state of one overlapped train step: AdamW of a leaf group is launched on `opt` as soon as
@@ -826,10 +827,19 @@ extern "C" int32_t olmax_model_adamw(hipStream_t s, const olmax_model_config* c,
   if (max_grad_norm > 0.f) {
     // norm_scratch[0] accumulates sum(g^2), then becomes the clip factor read by the AdamW kernels
     rc = olmax_fill_zero(s, norm_scratch, 8);
-    for (int i = 0; i < nleaf && !rc; i++) {
-      const olmax_leaf& lf = leaves[i];
-      rc = lf.grad_f32 ? olmax_sumsq(s, grad_f32 + lf.grad_f32_offset, lf.numel, 0, norm_scratch)
-                       : olmax_sumsq(s, G + lf.offset, lf.numel, 1, norm_scratch);
+    // runs of leaves adjacent in the bf16 gradients, then in the fp32 ones
+    for (int f32 = 0; f32 < 2; f32++) {
+      auto at = [&](int i) { return f32 ? leaves[i].grad_f32_offset : leaves[i].offset; };
+      int64_t start = 0, n = 0;
+      for (int i = 0; i <= nleaf && !rc; i++) {
+        if (i < nleaf && (leaves[i].grad_f32 != 0) != (f32 != 0)) continue;
+        if (i < nleaf && at(i) == start + n) {
+          n += leaves[i].numel;
+          continue;
+        }
+        if (n) rc = olmax_sumsq(s, f32 ? (const void*)(grad_f32 + start) : G + start, n, !f32, norm_scratch);
+        if (i < nleaf) start = at(i), n = leaves[i].numel;
+      }
     }
     if (!rc) {
       hipLaunchKernelGGL(clip_scale_kernel, dim3(1), dim3(1), 0, s, norm_scratch, max_grad_norm, norm_scratch);
@@ -853,20 +863,26 @@ extern "C" int32_t olmax_model_grad_accumulate(hipStream_t s, const olmax_model_
   olmax_model_layout(c, leaves, nleaf);
   const bf16* G = (const bf16*)grad_bf16;
   int rc = OLMAX_OK;
-  int i = 0;
-  while (i < nleaf && !rc) {
+  FlatRanges small;
+  auto flush = [&]() -> int {
+    const int r = olmax_grad_accumulate_ranges(s, small, acc, G, grad_f32, mini_step);
+    small = FlatRanges();
+    return r;
+  };
+  for (int i = 0; i < nleaf && !rc;) {  // runs of adjacent bf16-gradient leaves, short ones and vectors in one launch
     const olmax_leaf& lf = leaves[i];
-    if (lf.grad_f32) {
-      rc = olmax_grad_accumulate(s, acc + lf.offset, grad_f32 + lf.grad_f32_offset, lf.numel, 0, mini_step);
-      i++;
-    } else {  // runs of adjacent bf16-gradient leaves in one launch
-      int64_t n = lf.numel;
-      int j = i + 1;
-      while (j < nleaf && !leaves[j].grad_f32 && leaves[j].offset == lf.offset + n) n += leaves[j++].numel;
-      rc = olmax_grad_accumulate(s, acc + lf.offset, G + lf.offset, n, 1, mini_step);
-      i = j;
+    const bool f32 = lf.grad_f32;
+    int64_t n = lf.numel;
+    for (i++; !f32 && i < nleaf && !leaves[i].grad_f32 && leaves[i].offset == lf.offset + n; i++) n += leaves[i].numel;
+    const int64_t goff = f32 ? lf.grad_f32_offset : lf.offset;
+    if (n <= FlatRanges::MAX_N) {
+      if (small.count == FlatRanges::MAX) rc = flush();
+      small.add(lf.offset, goff, n, f32, true);
+    } else {
+      rc = olmax_grad_accumulate(s, acc + lf.offset, f32 ? (const void*)(grad_f32 + goff) : G + goff, n, !f32, mini_step);
     }
   }
+  if (!rc) rc = flush();
   delete[] leaves;
   return rc;
 }

@@ -1,0 +1,83 @@
+"""GPU tests of the launches that take many short pieces of the flat parameter buffers at once: AdamW, gradient
+accumulation and the gradient norm over a model's leaves against the same thing leaf by leaf."""
+import dataclasses
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# d_model and hidden decide where a leaf ends inside a workgroup's 1024 elements (or is shorter than that); 24 layers are 49 vectors
+# and 24 runs of matrices, more than one table; width 1032 has runs that are too long for a table
+CASES = [(24, 64, 136), (3, 256, 1024), (2, 1032, 1048), (1, 8, 8)]
+
+
+def _model(layers, d, hidden):
+    from olmax_amd import TransformerRecipe
+    cfg = dataclasses.replace(TransformerRecipe.tiny_llama(), vocab_size=72, d_model=d, hidden_size=hidden, num_layers=layers,
+                              n_heads=2, n_kv_heads=2, head_dim=8)
+    m = cfg.build(batch_size=1, sequence_length=16, seed=1)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    m.grad_bf16.normal_(0.0, 1e-2, generator=g)
+    m.grad_f32.normal_(0.0, 1e-2, generator=g)
+    m.init_optimizer_state()
+    m.m.normal_(0.0, 1e-3, generator=g)
+    m.v.uniform_(1e-6, 1e-4, generator=g)
+    return m
+
+
+def _leaf_grad(m, l):
+    return m.grad_f32[l.grad_f32_offset:l.grad_f32_offset + l.numel] if l.grad_f32 else m.grad_bf16[l.offset:l.offset + l.numel]
+
+
+@pytest.mark.parametrize("layers,d,hidden", CASES)
+@pytest.mark.parametrize("clip", [None, 1e-3])
+def test_adamw_over_all_leaves_equals_adamw_per_leaf(layers, d, hidden, clip):
+    """Bit for bit without clipping (the same operations per element); with it the gradient norm against float64: fp32 sums
+    of positive terms, at most 2^12 in a chain, 2^-24 each."""
+    from olmax_amd import ops
+    print(f"[case] adamw ranges L{layers} d{d} F{hidden} clip {clip}", flush=True)
+    m = _model(layers, d, hidden)
+    p, mm, vv = m.master.clone(), m.m.clone(), m.v.clone()
+    shadow = m.params_bf16.clone()
+    kw = dict(step=3, lr=1e-3, b1=0.9, b2=0.95, eps=1e-8)
+    m.adamw_step(**kw, weight_decay=0.1, no_decay_modules=["*norm*"], max_grad_norm=clip)
+    scale = 1.0
+    if clip:
+        norm = sum(_leaf_grad(m, l).double().square().sum() for l in m.leaves).sqrt().item()
+        assert abs(m.norm_scratch[1].item() - norm) < 2 ** -12 * norm
+        scale = m.norm_scratch[0].item()
+        assert abs(scale - clip / norm) < 2 ** -11 * scale
+    mask = m.weight_decay_mask(["*norm*"])
+    for i, l in enumerate(m.leaves):
+        s = slice(l.offset, l.offset + l.numel)
+        ops.adamw_(p[s], _leaf_grad(m, l), mm[s], vv[s], wd=0.1 if mask[i] else 0.0, shadow=shadow[s], grad_scale=scale, **kw)
+    assert torch.equal(m.master, p) and torch.equal(m.m, mm) and torch.equal(m.v, vv) and torch.equal(m.params_bf16, shadow)
+
+
+@pytest.mark.parametrize("layers,d,hidden", CASES)
+def test_accumulation_over_all_leaves(layers, d, hidden):
+    """The running mean over three micro-batches; acc + (g - acc) / (k + 1) in fp32, three roundings of 2^-24 per step."""
+    print(f"[case] accumulate ranges L{layers} d{d} F{hidden}", flush=True)
+    m = _model(layers, d, hidden)
+    want = torch.zeros(m.num_params, device="cuda", dtype=torch.float64)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    for k in range(3):
+        m.grad_bf16.normal_(0.0, 1.0, generator=g)
+        m.grad_f32.normal_(0.0, 1.0, generator=g)
+        m.accumulate_grads(k)
+        for l in m.leaves:
+            s = slice(l.offset, l.offset + l.numel)
+            want[s] += (_leaf_grad(m, l).double() - want[s]) / (k + 1)
+    assert (m.grad_acc.double() - want).abs().max().item() < 12 * 2 ** -24 * 6
+
+
+@pytest.mark.parametrize("n,shift", [(1, 0), (7, 0), (4099, 0), (4099, 1), (3 << 20, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sum_of_squares(n, shift, dtype):
+    """Vector and element loads; bound as for the norm above."""
+    from olmax_amd import ops
+    print(f"[case] sumsq n{n} shift{shift} {dtype}", flush=True)
+    x = torch.randn(n + shift, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).to(dtype)[shift:]
+    want = x.double().square().sum().item()
+    assert abs(ops.sumsq(x).item() - want) < 2 ** -12 * want
