@@ -388,30 +388,40 @@ __global__ __launch_bounds__(256) void qk_rope_fwd_kernel(
 }
 
 // Backward: dr = rope^T(dy) (rotation by -angle, rounded to bf16), then, if NORM, the RMSNorm
-// backward against the raw projection x; dw[D] accumulated with fp32 atomics.
+// backward against the raw projection x; dw[D] accumulated with fp32 atomics.  All blocks add to the same D addresses, which
+// take one addition after the other, so NORM runs few, large blocks, whose rows meet in registers and LDS first, and a row is
+// fetched while the one before it is worked on.  2048 x 32 heads of 128: 39.6 -> 18.8 us, 4096 x 32: 44 -> 26 (101 MB, 3.9 TB/s); with 128,
+// 512, 1024 blocks 4096 x 32 takes 37, 31, 37.
 template <int D, bool NORM>
-__global__ __launch_bounds__(256) void qk_rope_bwd_kernel(
+__global__ __launch_bounds__(NORM ? 1024 : 256) void qk_rope_bwd_kernel(
     const bf16* __restrict__ dy, bf16* __restrict__ dx, const bf16* __restrict__ x,
     const bf16* __restrict__ w, float* __restrict__ dw, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int64_t tokens, int heads, int seq_len, int64_t lddy,
     int64_t lddx, int64_t ldx, float eps) {
-  __shared__ float sdw[D];
-  if (NORM) {
-    if (threadIdx.x < D) sdw[threadIdx.x] = 0.f;
-    __syncthreads();
-  }
+  constexpr int THREADS = NORM ? 1024 : 256;
   constexpr int LPR = D / 8;  // lanes per row
   const int sub = threadIdx.x & (LPR - 1);
   // a thread always serves the same 8 head-dim columns: its weight-gradient partials stay in
   // registers over the grid-stride loop (few blocks, so few global atomics on the D addresses)
   float dwacc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  const int64_t units = tokens * heads;
-  for (int64_t unit = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR; unit < units; unit += (int64_t)gridDim.x * (256 / LPR)) {
-    const int64_t tok = unit / heads;
-    const int h = (int)(unit % heads);
-    const int pos = (int)(tok % seq_len);
-    Pack8 c;
-    c.u = *reinterpret_cast<const u32x4*>(dy + tok * lddy + h * D + sub * 8);
+  const int64_t units = tokens * heads, step = (int64_t)gridDim.x * (THREADS / LPR);
+  const bool small = units <= 0x7fffffff;  // (a 64-bit division is a hundred instructions)
+  auto token_of = [&](int64_t unit) { return small ? (int64_t)((uint32_t)unit / (uint32_t)heads) : unit / heads; };
+  Pack8 wv, next_dy, next_x;
+  auto fetch = [&](int64_t unit, int64_t tok) {
+    const int h = (int)(unit - tok * heads);
+    next_dy.u = *reinterpret_cast<const u32x4*>(dy + tok * lddy + h * D + sub * 8);
+    if (NORM) next_x.u = *reinterpret_cast<const u32x4*>(x + tok * ldx + h * D + sub * 8);
+  };
+  int64_t unit = (int64_t)blockIdx.x * (THREADS / LPR) + threadIdx.x / LPR, next_tok = 0;
+  if (NORM) wv.u = *reinterpret_cast<const u32x4*>(w + sub * 8);
+  if (unit < units) fetch(unit, next_tok = token_of(unit));
+  for (; unit < units; unit += step) {
+    const int64_t tok = next_tok;
+    const int h = (int)(unit - tok * heads);
+    const int pos = small ? (int)((uint32_t)tok % (uint32_t)seq_len) : (int)(tok % seq_len);
+    const Pack8 c = next_dy, xv = next_x;
+    if (unit + step < units) fetch(unit + step, next_tok = token_of(unit + step));  // under way while this row is worked on
     const int fi = (sub & (LPR / 2 - 1)) * 8;
     const float sign = sub < LPR / 2 ? 1.f : -1.f;
     float g[8];
@@ -425,9 +435,6 @@ __global__ __launch_bounds__(256) void qk_rope_bwd_kernel(
     }
     Pack8 o;
     if (NORM) {
-      Pack8 xv, wv;
-      xv.u = *reinterpret_cast<const u32x4*>(x + tok * ldx + h * D + sub * 8);
-      wv.u = *reinterpret_cast<const u32x4*>(w + sub * 8);
       float ss = 0.f, sxg = 0.f;
       float xf[8], gg[8];
 #pragma unroll
@@ -457,10 +464,13 @@ __global__ __launch_bounds__(256) void qk_rope_bwd_kernel(
     *reinterpret_cast<u32x4*>(dx + tok * lddx + h * D + sub * 8) = o.u;
   }
   if (NORM) {
+    __shared__ __attribute__((aligned(16))) float sdw[THREADS / 64][D];
 #pragma unroll
-    for (int e = 0; e < 8; e++) atomicAdd(&sdw[sub * 8 + e], dwacc[e]);
-    __syncthreads();
-    if (threadIdx.x < D) atomicAdd(&dw[threadIdx.x], sdw[threadIdx.x]);
+    for (int e = 0; e < 8; e++)
+#pragma unroll
+      for (int o = LPR; o < 64; o <<= 1) dwacc[e] += __shfl_xor(dwacc[e], o, 64);
+    if ((threadIdx.x & 63) < LPR) park8(&sdw[threadIdx.x >> 6][sub * 8], dwacc);
+    add_slots<THREADS / 64, THREADS>(&sdw[0][0], dw, D);
   }
 }
 
@@ -692,10 +702,10 @@ extern "C" int32_t olmax_qk_rope_bwd(hipStream_t stream, const void* dy, void* d
   const bf16* dyp = (const bf16*)dy;
   bf16* dxp = (bf16*)dx;
   if ((head_dim == 128 || head_dim == 64) && aligned16(dy) && aligned16(dx) && lddy % 8 == 0 && lddx % 8 == 0 && (!w || (aligned16(w) && aligned16(x) && ldx % 8 == 0))) {
-    const int rows = 2048 / head_dim;  // of a workgroup
-    const unsigned blocks = (unsigned)((tokens * heads + rows - 1) / rows);
-    dim3 grid(w && blocks > 1024 ? 1024 : blocks);
-#define ROPE(D, NORM) hipLaunchKernelGGL((qk_rope_bwd_kernel<D, NORM>), grid, dim3(256), 0, stream, dyp, dxp, (const bf16*)x, (const bf16*)w, dw, cos_t, sin_t, tokens, heads, seq_len, lddy, lddx, ldx, eps)
+    const int threads = w ? 1024 : 256, rows = threads * 8 / head_dim;  // of a workgroup
+    const int64_t blocks = (tokens * heads + rows - 1) / rows;
+    dim3 grid((unsigned)(w && blocks > 256 ? 256 : blocks));
+#define ROPE(D, NORM) hipLaunchKernelGGL((qk_rope_bwd_kernel<D, NORM>), grid, dim3(threads), 0, stream, dyp, dxp, (const bf16*)x, (const bf16*)w, dw, cos_t, sin_t, tokens, heads, seq_len, lddy, lddx, ldx, eps)
     if (head_dim == 128) {
       if (w) ROPE(128, true); else ROPE(128, false);
     } else {
