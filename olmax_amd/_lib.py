@@ -49,9 +49,11 @@ def ptr(t) -> c_void_p:
 
 
 def stream_ptr() -> c_void_p:
+    """Current stream of the current device; the raw handle, without a Stream object around it (0.3 instead of 3 us of
+    an 11 us call)."""
     import torch
 
-    return c_void_p(torch.cuda.current_stream().cuda_stream)
+    return c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 i32, i64, f32, f64, vp = c_int32, c_int64, c_float, c_double, c_void_p
