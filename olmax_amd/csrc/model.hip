@@ -653,9 +653,9 @@ int overlap_launch(OverlapCtx* x, int layer) {
   g_overlapped_launches++;
   if (hipEventRecord(x->ev, x->main) != hipSuccess || hipStreamWaitEvent(x->opt, x->ev, 0) != hipSuccess)
     return olmax_set_error(OLMAX_ERR_LAUNCH, "olmax_model_train_step: event record/wait failed");
-  // One workgroup per CU is the grid that disturbs the GEMMs it runs beside least, but alone it only
-  // reaches 3.3 TB/s against 5.2 TB/s for two per CU: the updates that start when the backward pass
-  // is over (layer 0 and the embedding) have the GPU to themselves and take the fast grid.
+  // Beside the recompute's GEMMs one workgroup per CU (4.3 TB/s) is best: two layers of the 7B step take 44.0, 43.5, 43.2,
+  // 43.1, 44.5, 45.3 ms with 64, 128, 192, 256, 384, 512 workgroups.  The updates that start when the backward pass is over (layer 0
+  // and the embedding) have the GPU to themselves and take two per CU (5.5 TB/s).
   const int grid_cap = (layer == 0 || layer == -2) ? 512 : 256;
   if (layer == -1 && x->head_windows > 0) {
     // final norm now; of the LM head what a window holds, i.e. a layer's worth (the first window,
