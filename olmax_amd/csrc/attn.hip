@@ -932,6 +932,10 @@ bool fast_ok(int D, int S, int max_s, const void* q, const void* k, const void* 
   return (D == 128 || (D == 64 && S <= max_s)) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) && ldq % 8 == 0 &&
          ldk % 8 == 0 && ldv % 8 == 0 && ldo % 8 == 0;
 }
+// A window that reaches past the first key from the last query hides nothing: global.  The kernels add the window to
+// positions, and sums up to 2 S fit; from windows near 2^31 they would wrap, the last query tile of a key would come
+// out before its first, and dK/dV's walk over the tiles would not end.
+int32_t reach(int32_t window, int32_t S) { return window >= S ? -1 : window; }
 constexpr int GENERIC_MAX_S_FWD = 16384, GENERIC_MAX_S_BWD = 8192;  // 64 KB of LDS: one, two floats per key
 
 bool bwd_fast_ok(const void* q, const void* k, const void* v, const void* o, const void* d_o, const void* dq, const void* dk,
@@ -1063,6 +1067,7 @@ extern "C" int32_t olmax_attn_fwd(hipStream_t stream, const void* q, const void*
   OLMAX_CHECK(q && k && v && o && lse, OLMAX_ERR_ARG, "olmax_attn_fwd: null pointer");
   OLMAX_CHECK(B > 0 && S > 0 && H > 0 && KH > 0 && D > 0 && H % KH == 0, OLMAX_ERR_SHAPE, "olmax_attn_fwd: bad shape B=%d S=%d H=%d KH=%d D=%d", B, S, H, KH, D);
   OLMAX_CHECK(ldq >= (int64_t)H * D && ldo >= (int64_t)H * D && ldk >= (int64_t)KH * D && ldv >= (int64_t)KH * D, OLMAX_ERR_SHAPE, "olmax_attn_fwd: row stride smaller than heads*head_dim");
+  window = reach(window, S);
   const float scale = 1.f / sqrtf((float)D);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k, *vp = (const bf16*)v;
   if (fast_ok(D, S, GENERIC_MAX_S_FWD, q, k, v, o, ldq, ldk, ldv, ldo)) {
@@ -1099,6 +1104,7 @@ extern "C" int32_t olmax_attn_bwd(hipStream_t stream, const void* q, const void*
   OLMAX_CHECK(B > 0 && S > 0 && H > 0 && KH > 0 && D > 0 && H % KH == 0, OLMAX_ERR_SHAPE, "olmax_attn_bwd: bad shape");
   OLMAX_CHECK(workspace_bytes >= attn_delta_bytes(B, S, H) && (((uintptr_t)workspace) & 255) == 0, OLMAX_ERR_WORKSPACE, "olmax_attn_bwd: workspace too small or not 256-byte aligned");
   OLMAX_CHECK(ldq >= (int64_t)H * D && ldo >= (int64_t)H * D && lddo >= (int64_t)H * D && lddq >= (int64_t)H * D && ldk >= (int64_t)KH * D && ldv >= (int64_t)KH * D && lddk >= (int64_t)KH * D && lddv >= (int64_t)KH * D, OLMAX_ERR_SHAPE, "olmax_attn_bwd: row stride smaller than heads*head_dim");
+  window = reach(window, S);
   const float scale = 1.f / sqrtf((float)D);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k, *vp = (const bf16*)v, *op = (const bf16*)o, *gop = (const bf16*)d_o;
   float* delta = (float*)workspace;
@@ -1186,6 +1192,7 @@ extern "C" int32_t olmax_attn_bwd_noalloc(hipStream_t stream, const void* q, con
   OLMAX_CHECK(q && k && v && o && lse && d_o && dq && dk && dv, OLMAX_ERR_ARG, "olmax_attn_bwd_noalloc: null pointer");
   OLMAX_CHECK(B > 0 && S > 0 && H > 0 && KH > 0 && D > 0 && H % KH == 0, OLMAX_ERR_SHAPE, "olmax_attn_bwd_noalloc: bad shape");
   OLMAX_CHECK(ldq >= (int64_t)H * D && ldo >= (int64_t)H * D && lddo >= (int64_t)H * D && lddq >= (int64_t)H * D && ldk >= (int64_t)KH * D && ldv >= (int64_t)KH * D && lddk >= (int64_t)KH * D && lddv >= (int64_t)KH * D, OLMAX_ERR_SHAPE, "olmax_attn_bwd_noalloc: row stride smaller than heads*head_dim");
+  window = reach(window, S);
   OLMAX_CHECK((int64_t)B * H * S <= ATTN_SCRATCH_FLOATS, OLMAX_ERR_WORKSPACE,
               "olmax_attn_bwd_noalloc: batch*heads*seq_len = %ld exceeds the built-in scratch of %ld rows; use olmax_attn_bwd with a workspace",
               (long)((int64_t)B * H * S), (long)ATTN_SCRATCH_FLOATS);

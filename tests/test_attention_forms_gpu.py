@@ -70,3 +70,22 @@ def test_key_gradients_split_over_query_groups(S, H, KH, window, softcap):
                                                    (449, 2, 2, None, 0.0)])
 def test_queries_split_over_key_groups(S, H, KH, window, softcap, D):
     check(3, S, H, KH, D, window, softcap, strided=S % 2 == 0)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S,H,KH", [(130, 4, 2), (1, 1, 1)])
+def test_a_window_past_the_first_key_hides_nothing(S, H, KH, D):
+    """From one that just reaches it to the largest integer: the bits of the global mask."""
+    from olmax_amd import ops
+    q, do = rnd(2 * S, H * D, seed=1), rnd(2 * S, H * D, seed=4)
+    k, v = rnd(2 * S, KH * D, seed=2), rnd(2 * S, KH * D, seed=3)
+    kw = dict(B=2, S=S, H=H, KH=KH, D=D)
+
+    def run(window):
+        print(f"[case] attn S{S} H{H} KH{KH} D{D} w{window}", flush=True)
+        o, lse = ops.attn_fwd(q, k, v, window=window, **kw)
+        return (o, lse, *ops.attn_bwd(q, k, v, o, lse, do, window=window, **kw))
+
+    want = run(None)
+    for window in (S - 1, S, S + 1, 2 ** 31 - 65, 2 ** 31 - 1):
+        assert all(torch.equal(a, b) for a, b in zip(run(window), want)), window
