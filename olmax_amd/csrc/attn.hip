@@ -32,6 +32,13 @@ __device__ __forceinline__ float fexp2(float x) { return __builtin_amdgcn_exp2f(
 __device__ __forceinline__ float cap_tanh(float raw, float c1) {
   return __builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(fexp2(raw * c1) + 1.f), 1.f);
 }
+// Its error is an ulp of 1 whatever the result, which the cap multiplies.  At head_dim 128 that drowns in LSE's own error (1e-3 at
+// most: it sums rounded probabilities).  At head_dim 64 LSE is good to 8e-7 and it would be 3e-6 (cap 30) or 5e-6 (cap 50):
+// there the formula is taken as it reads, as the one-wave-per-query kernels take it.
+template <int D>
+__device__ __forceinline__ float cap_tanh_of(float raw, float c1, float scale, float cap) {
+  return D == 64 ? tanhf(raw * scale / cap) : cap_tanh(raw, c1);
+}
 
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LN2 = 0.6931471805599453f;
@@ -261,6 +268,11 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
   };
   const float sc2 = scale * LOG2E;
   const float cap_c1 = CAP ? 2.f * sc2 / cap : 0.f, cap_l2 = cap * LOG2E;  // soft-cap: see cap_tanh
+  // Scores and their maximum are held in log2 units; at head_dim 64 as the products give them (CAP: capped), so that
+  // no constant's rounding gets into LSE through the maximum (log2 units: a sixth more LSE error)
+  constexpr bool LOG2_UNITS = D != 64;
+  const float to_log2 = CAP ? LOG2E : sc2, to_ln = CAP ? 1.f : scale;  // of a difference, of a score (!LOG2_UNITS)
+  auto exp_of = [&](float x, float ref) { return LOG2_UNITS ? fexp2(x - ref) : fexp2((x - ref) * to_log2); };
   FragAddr<D> fa;
   fa.init(lane);
 
@@ -287,12 +299,11 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
 #pragma unroll
         for (int jt = 0; jt < 2; jt++)
           st[jt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sk, jt * 32, s), qf[s], st[jt], 0, 0, 0);
-      // scores in log2 units
       if (CAP) {
 #pragma unroll
         for (int jt = 0; jt < 2; jt++)
 #pragma unroll
-          for (int r = 0; r < 16; r++) st[jt][r] = cap_l2 * cap_tanh(st[jt][r], cap_c1);
+          for (int r = 0; r < 16; r++) st[jt][r] = (LOG2_UNITS ? cap_l2 : cap) * cap_tanh_of<D>(st[jt][r], cap_c1, scale, cap);
       }
       const bool need_mask = (j0 + 63 > iw0) || (window >= 0 && j0 < iw0 + 31 - window);
       if (need_mask) {
@@ -310,16 +321,16 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
       for (int jt = 0; jt < 2; jt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) mt = fmaxf(mt, st[jt][r]);
-      if (!CAP) mt *= sc2;  // sc2 > 0: the max commutes with the scaling
+      if (!CAP && LOG2_UNITS) mt *= sc2;  // sc2 > 0: the max commutes with the scaling
       mt = half_swap_max(mt);
       // Lazy rescaling: the running reference m only moves when some row's maximum grew by more
       // than 2^8; until then exp2(s - m) <= 256 stays well inside fp32/bf16 range and the
       // 64-register rescale of O is skipped (wave-uniform decision).
-      const bool grow = mt > m + 8.f;
+      const bool grow = LOG2_UNITS ? mt > m + 8.f : (mt - m) * to_log2 > 8.f;
       if (__builtin_amdgcn_ballot_w64(grow) != 0) {
         const float m_new = fmaxf(m, mt);
         const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-        const float alpha = fexp2(m - m_use);  // m = -inf -> 0
+        const float alpha = exp_of(m, m_use);  // m = -inf -> 0
         lsum *= alpha;
         m = m_new;
 #pragma unroll
@@ -332,7 +343,7 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
       for (int jt = 0; jt < 2; jt++)
 #pragma unroll
         for (int r = 0; r < 16; r++)
-          st[jt][r] = CAP ? fexp2(st[jt][r] - m_use) : fexp2(__builtin_fmaf(st[jt][r], sc2, -m_use));
+          st[jt][r] = CAP || !LOG2_UNITS ? exp_of(st[jt][r], m_use) : fexp2(__builtin_fmaf(st[jt][r], sc2, -m_use));
       bf16x8 pb[4];
 #pragma unroll
       for (int u = 0; u < 4; u++) pb[u] = pack_bf16x8(st[u >> 1], (u & 1) * 8);
@@ -400,9 +411,9 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
 #pragma unroll
     for (int g = 0; g < KS; g++) {
       const f32x2 st = stats[g * 32];
-      ltot += st[1] * fexp2(st[0] - m_use);
+      ltot += st[1] * exp_of(st[0], m_use);
     }
-    const float alpha = fexp2(m_own - m_use), inv = ltot > 0.f ? 1.f / ltot : 0.f;
+    const float alpha = exp_of(m_own, m_use), inv = ltot > 0.f ? 1.f / ltot : 0.f;
 #pragma unroll
     for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
@@ -411,7 +422,7 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
       if (qi < S) store4(u >> 2, u & 3, v, inv);
     });
   }
-  if (qi < S && lhi == 0 && ks == 0) LSE[((int64_t)b * H + h) * S + qi] = (m + log2f(ltot)) * LN2;
+  if (qi < S && lhi == 0 && ks == 0) LSE[((int64_t)b * H + h) * S + qi] = LOG2_UNITS ? (m + log2f(ltot)) * LN2 : m * to_ln + __logf(ltot);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -523,7 +534,7 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_bwd_dq_kernel(
         for (int r = 0; r < 16; r++) {
           float s = sj[r], chain = 1.f, p;
           if (CAP) {
-            const float th = cap_tanh(s, cap_c1);
+            const float th = cap_tanh_of<D>(s, cap_c1, scale, cap);
             p = fexp2(__builtin_fmaf(th, cap_l2, -lse2));
             chain = 1.f - th * th;
           } else {
@@ -747,7 +758,7 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
           const int i = ib + il + e;
           float s = sa[r], chain = 1.f, p;
           if (CAP) {
-            const float th = cap_tanh(s, cap_c1);
+            const float th = cap_tanh_of<D>(s, cap_c1, scale, cap);
             p = fexp2(__builtin_fmaf(th, cap_l2, -l4[e]));
             chain = 1.f - th * th;
           } else {

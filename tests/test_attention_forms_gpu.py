@@ -57,6 +57,25 @@ def test_head_dim_64(S, H, KH, window, softcap):
     check(2, S, H, KH, 64, window, softcap, strided=S % 2 == 1)
 
 
+@pytest.mark.parametrize("S,H,KH,window,softcap", [(512, 4, 4, None, 0.0), (512, 4, 4, None, 30.0), (512, 4, 2, 128, 50.0), (300, 64, 64, None, 50.0)])
+def test_head_dim_64_normaliser_is_exact_to_fp32(S, H, KH, window, softcap):
+    """LSE against float64, with few workgroups and with enough for the unsplit form: values of 4 to 8 and two or three
+    fp32 roundings of that size (2^-22 each) between the score, the sum's logarithm and their sum: 2^-20 and half of it again."""
+    from olmax_amd import ops
+    print(f"[case] lse S{S} H{H} KH{KH} w{window} cap{softcap}", flush=True)
+    q, k, v = rnd(2 * S, H * 64, seed=1), rnd(2 * S, KH * 64, seed=2), rnd(2 * S, KH * 64, seed=3)
+    _, lse = ops.attn_fwd(q, k, v, B=2, S=S, H=H, KH=KH, D=64, window=window, softcap=softcap)
+    q4, k4 = q.double().view(2, S, H, 64), k.double().view(2, S, KH, 64)
+    i = torch.arange(S, device="cuda")
+    hidden = (i[None] > i[:, None]) | (i[None] < i[:, None] - (S if window is None else window))
+    for b in range(2):
+        for h in range(H):
+            s = q4[b, :, h] @ k4[b, :, h * KH // H].t() / 8
+            s = softcap * torch.tanh(s / softcap) if softcap else s
+            want = torch.logsumexp(s.masked_fill(hidden, -math.inf), -1)
+            assert (lse[b, h].double() - want).abs().max() < 1.5 * 2 ** -20, (b, h)
+
+
 # iterations (query heads x 32-row tiles) that the four query groups share out unevenly, or that some go without
 @pytest.mark.parametrize("S,H,KH,window,softcap", [(1, 2, 2, None, 0.0), (32, 3, 1, None, 0.0), (33, 8, 2, None, 0.0), (65, 3, 1, 0, 0.0), (97, 5, 1, 31, 0.0),
                                                    (160, 2, 2, None, 30.0), (257, 4, 1, None, 0.0), (450, 3, 3, 64, 0.0)])
