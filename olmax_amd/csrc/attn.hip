@@ -197,6 +197,115 @@ __device__ __forceinline__ void add_partials(unsigned char* smem, const f32x16 (
 }
 
 // ---------------------------------------------------------------------------------------
+// Rows of head_dim 64 that come out infinite or NaN.  The tile products take hidden pairs along as zeros, and zero times an
+// infinity or a NaN in a token that a row does not see (V and K of a later one, Q and dO of an earlier one) is NaN.  The
+// one-wave-per-query kernels, which took all of this head_dim before, look at visible pairs only, so a wave that finds such
+// values among those it has stored (one multiply-add each) does their rows over as those kernels do: lane l has key or query
+// l of 64 for the scores, element l of the row for the sums.  Speed does not matter here.
+// ---------------------------------------------------------------------------------------
+__device__ __forceinline__ float dot64(const bf16* a, const bf16* b) {
+  float s = 0.f;
+#pragma unroll 1
+  for (int c = 0; c < 64; c += 8) {
+    Pack8 x, y;
+    x.u = *reinterpret_cast<const u32x4*>(a + c);
+    y.u = *reinterpret_cast<const u32x4*>(b + c);
+#pragma unroll
+    for (int e = 0; e < 8; e++) s += bf2f(x.e[e]) * bf2f(y.e[e]);
+  }
+  return s;
+}
+// score of a pair and d score / d product
+template <bool CAP>
+__device__ __forceinline__ float score64(const bf16* q, const bf16* k, float scale, float cap, float* chain) {
+  const float s = dot64(q, k) * scale;
+  if (!CAP) return s;
+  const float th = tanhf(s / cap);
+  if (chain) *chain = 1.f - th * th;
+  return cap * th;
+}
+// calls row(r) for the rows r of a wave's 32 in which a lane's sum of zeros is not zero
+template <typename Row>
+__device__ __forceinline__ void redo_rows(float zeros, Row row) {
+  const uint64_t bad = __builtin_amdgcn_ballot_w64(zeros != 0.f);
+  if (bad) dma_wait_all();  // the wave's stores to the same rows, made by other lanes
+  for (uint32_t rows = (uint32_t)bad | (uint32_t)(bad >> 32); rows; rows &= rows - 1) row(__builtin_ctz(rows));
+}
+// output row i of the sequence and head that q, k, v point to; lanes [lo, hi) store
+template <bool CAP>
+__device__ __forceinline__ void redo_fwd(const bf16* q, const bf16* K, int64_t ldk, const bf16* V, int64_t ldv, bf16* o, float* lse, int i,
+                                         int window, float scale, float cap, int lane, int lo, int hi) {
+  const int first = window >= 0 ? max(0, i - window) : 0;
+  float mx = -INFINITY, sm = 0.f, acc = 0.f;
+#pragma unroll 1
+  for (int j = first + lane; j <= i; j += 64) mx = fmaxf(mx, score64<CAP>(q, K + j * ldk, scale, cap, nullptr));
+  mx = wave_max(mx);
+#pragma unroll 1
+  for (int j = first + lane; j <= i; j += 64) sm += __expf(score64<CAP>(q, K + j * ldk, scale, cap, nullptr) - mx);
+  const float l = mx + __logf(wave_sum(sm));
+#pragma unroll 1
+  for (int j0 = first; j0 <= i; j0 += 64) {
+    const int n = min(64, i - j0 + 1);
+    float p = 0.f;
+    if (lane < n) p = bf2f(f2bf(__expf(score64<CAP>(q, K + (j0 + lane) * ldk, scale, cap, nullptr) - l)));
+#pragma unroll 1
+    for (int t = 0; t < n; t++) acc += __shfl(p, t, 64) * bf2f(V[(j0 + t) * ldv + lane]);
+  }
+  if (lane >= lo && lane < hi) o[lane] = f2bf(acc);
+  if (lse && lane == 0) *lse = l;
+}
+template <bool CAP>
+__device__ __forceinline__ void redo_dq(const bf16* q, const bf16* K, int64_t ldk, const bf16* V, int64_t ldv, const bf16* o, const bf16* d_o,
+                                        float lse, bf16* dq, int i, int window, float scale, float cap, int lane, int lo, int hi) {
+  const float delta = wave_sum(bf2f(o[lane]) * bf2f(d_o[lane]));
+  float acc = 0.f;
+#pragma unroll 1
+  for (int j0 = window >= 0 ? max(0, i - window) : 0; j0 <= i; j0 += 64) {
+    const int n = min(64, i - j0 + 1);
+    float ds = 0.f;
+    if (lane < n) {
+      float chain = 1.f;
+      const float p = __expf(score64<CAP>(q, K + (j0 + lane) * ldk, scale, cap, &chain) - lse);
+      ds = bf2f(f2bf(p * (dot64(d_o, V + (j0 + lane) * ldv) - delta) * chain));
+    }
+#pragma unroll 1
+    for (int t = 0; t < n; t++) acc += __shfl(ds, t, 64) * bf2f(K[(j0 + t) * ldk + lane]);
+  }
+  if (lane >= lo && lane < hi) dq[lane] = f2bf(acc * scale);
+}
+// key j; Q, dO, lse, ndelta (minus delta) of the first of its rep query heads
+template <bool CAP>
+__device__ __forceinline__ void redo_dkv(const bf16* Q, int64_t ldq, const bf16* dO, int64_t lddo, const float* lse, const float* ndelta,
+                                         const bf16* k, const bf16* v, bf16* dk, bf16* dv, int j, int S, int rep, int window, float scale,
+                                         float cap, int lane, int lo, int hi) {
+  const int last = window >= 0 ? min(S - 1, j + window) : S - 1;
+  float ak = 0.f, av = 0.f;
+#pragma unroll 1
+  for (int r = 0; r < rep; r++, Q += 64, dO += 64, lse += S, ndelta += S)
+#pragma unroll 1
+    for (int i0 = j; i0 <= last; i0 += 64) {
+      const int n = min(64, last - i0 + 1);
+      float p = 0.f, ds = 0.f;
+      if (lane < n) {
+        const int i = i0 + lane;
+        float chain = 1.f;
+        p = __expf(score64<CAP>(Q + i * ldq, k, scale, cap, &chain) - lse[i]);
+        ds = bf2f(f2bf(p * (dot64(dO + i * lddo, v) + ndelta[i]) * chain));
+        p = bf2f(f2bf(p));
+      }
+#pragma unroll 1
+      for (int t = 0; t < n; t++) {
+        ak += __shfl(ds, t, 64) * bf2f(Q[(i0 + t) * ldq + lane]);
+        av += __shfl(p, t, 64) * bf2f(dO[(i0 + t) * lddo + lane]);
+      }
+    }
+  if (lane >= lo && lane < hi) {
+    dk[lane] = f2bf(ak * scale);
+    dv[lane] = f2bf(av);
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // Forward.  grid = ceil(S/(32 QW))*H*B workgroups (see decode_wg) of QW x KS waves; wave (qw, ks) owns queries
 // i0+32qw .. +31 and every KS-th of their K/V tiles.
 // KS = 1 (QW = 4): two workgroups per CU, no merge; what a grid that fills the GPU takes.
@@ -377,11 +486,16 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
     __syncthreads();
   }
   float ltot = half_swap_sum(lsum);
+  float zeros = 0.f;  // of what is stored: NaN if a value is not finite (see redo_rows)
   auto store4 = [&](int dt, int g, const f32x4& v, float mul) {
     bf16* op = O + ((int64_t)b * S + qic) * ldo + h * D;
     Pack4 pk;
 #pragma unroll
-    for (int e = 0; e < 4; e++) pk.e[e] = f2bf(v[e] * mul);
+    for (int e = 0; e < 4; e++) {
+      const float x = v[e] * mul;
+      if (D == 64) zeros = __builtin_fmaf(x, 0.f, zeros);
+      pk.e[e] = f2bf(x);
+    }
     *reinterpret_cast<u32x2*>(op + dt * 32 + g * 8 + lhi * 4) = pk.u;
   };
   if constexpr (KS == 1) {
@@ -422,7 +536,17 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
       if (qi < S) store4(u >> 2, u & 3, v, inv);
     });
   }
-  if (qi < S && lhi == 0 && ks == 0) LSE[((int64_t)b * H + h) * S + qi] = LOG2_UNITS ? (m + log2f(ltot)) * LN2 : m * to_ln + __logf(ltot);
+  if (qi < S && lhi == 0 && ks == 0) {
+    const float lse = LOG2_UNITS ? (m + log2f(ltot)) * LN2 : m * to_ln + __logf(ltot);
+    if (D == 64) zeros = __builtin_fmaf(lse, 0.f, zeros);
+    LSE[((int64_t)b * H + h) * S + qi] = lse;
+  }
+  if constexpr (D == 64)
+    redo_rows(zeros, [&](int r) {
+      const int64_t at = (int64_t)b * S + iw0 + r;
+      redo_fwd<CAP>(Q + at * ldq + h * D, kbase, ldk, vbase, ldv, O + at * ldo + h * D, ks == 0 ? LSE + ((int64_t)b * H + h) * S + iw0 + r : nullptr,
+                    iw0 + r, window, scale, cap, lane, ks * (D / KS), (ks + 1) * (D / KS));
+    });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -577,11 +701,16 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_bwd_dq_kernel(
     dma_wait_all();
     __syncthreads();
   }
+  float zeros = 0.f;  // see redo_rows
   auto store4 = [&](int dt, int g, const f32x4& v) {
     bf16* op = dQ + ((int64_t)b * S + qic) * lddq + h * D;
     Pack4 pk;
 #pragma unroll
-    for (int e = 0; e < 4; e++) pk.e[e] = f2bf(v[e] * scale);
+    for (int e = 0; e < 4; e++) {
+      const float x = v[e] * scale;
+      if (D == 64) zeros = __builtin_fmaf(x, 0.f, zeros);
+      pk.e[e] = f2bf(x);
+    }
     *reinterpret_cast<u32x2*>(op + dt * 32 + g * 8 + lhi * 4) = pk.u;
   };
   if constexpr (KS == 1) {
@@ -596,6 +725,12 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_bwd_dq_kernel(
       if (qi < S) store4(u >> 2, u & 3, v);
     });
   }
+  if constexpr (D == 64)
+    redo_rows(zeros, [&](int r) {
+      const int64_t at = (int64_t)b * S + iw0 + r;
+      redo_dq<CAP>(Q + at * ldq + h * D, kbase, ldk, vbase, ldv, O + at * ldo + h * D, dO + at * lddo + h * D, LSE[((int64_t)b * H + h) * S + iw0 + r],
+                   dQ + at * lddq + h * D, iw0 + r, window, scale, cap, lane, ks * (D / KS), (ks + 1) * (D / KS));
+    });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -805,10 +940,15 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
   }
   bf16* kp = dK + ((int64_t)b * S + kjc) * lddk + kh * D;
   bf16* vp = dV + ((int64_t)b * S + kjc) * lddv + kh * D;
+  float zeros = 0.f;  // see redo_rows
   auto store4 = [&](bf16* p, int dt, int g, const f32x4& v, float mul) {
     Pack4 pk;
 #pragma unroll
-    for (int e = 0; e < 4; e++) pk.e[e] = f2bf(v[e] * mul);
+    for (int e = 0; e < 4; e++) {
+      const float x = v[e] * mul;
+      if (D == 64) zeros = __builtin_fmaf(x, 0.f, zeros);
+      pk.e[e] = f2bf(x);
+    }
     *reinterpret_cast<u32x2*>(p + dt * 32 + g * 8 + lhi * 4) = pk.u;
   };
   if constexpr (QS == 1) {
@@ -831,6 +971,13 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
       if (kj < S) store4(vp, u >> 2, u & 3, v, 1.f);
     });
   }
+  if constexpr (D == 64)
+    redo_rows(zeros, [&](int r) {
+      const int64_t seq = (int64_t)b * S, at = seq + jw0 + r, row = ((int64_t)b * H + kh * rep) * S;
+      redo_dkv<CAP>(Q + seq * ldq + kh * rep * D, ldq, dO + seq * lddo + kh * rep * D, lddo, LSE + row, DELTA + row, K + at * ldk + kh * D,
+                    V + at * ldv + kh * D, dK + at * lddk + kh * D, dV + at * lddv + kh * D, jw0 + r, S, rep, window, scale, cap, lane,
+                    qs * (D / QS), (qs + 1) * (D / QS));
+    });
 }
 
 // ---------------------------------------------------------------------------------------

@@ -108,3 +108,30 @@ def test_a_window_past_the_first_key_hides_nothing(S, H, KH, D):
     want = run(None)
     for window in (S - 1, S, S + 1, 2 ** 31 - 65, 2 ** 31 - 1):
         assert all(torch.equal(a, b) for a, b in zip(run(window), want)), window
+
+
+@pytest.mark.parametrize("B,S,H,KH,window,softcap", [(2, 200, 2, 1, None, 0.0), (1, 300, 4, 4, 70, 30.0), (4, 300, 48, 48, None, 0.0), (4, 270, 60, 60, 100, 30.0)])
+@pytest.mark.parametrize("value", [math.nan, math.inf, -math.inf])
+def test_head_dim_64_keeps_what_a_row_does_not_see_out_of_it(B, S, H, KH, window, softcap, value):
+    """Infinities and NaN in one token of an operand reach the rows that see the token and no other: as on the kernels that
+    work through visible pairs one by one (which take views that are not 16-byte aligned); few workgroups and enough for the
+    unsplit forms.  Finite values: two roundings of P and dS to bf16, bounds as in check()."""
+    from olmax_amd import ops
+    n, at = B * S, S // 2 + 5
+    x = {"q": rnd(n, H * 64, seed=1), "k": rnd(n, KH * 64, seed=2), "v": rnd(n, KH * 64, seed=3), "do": rnd(n, H * 64, seed=4)}
+    kw = dict(B=B, S=S, H=H, KH=KH, D=64, window=window, softcap=softcap)
+    odd = lambda t: torch.cat([t, t.new_zeros(n, 3)], 1)[:, :t.shape[1]]  # noqa: E731
+    for name in x:
+        print(f"[case] {value} in {name}, B{B} S{S} H{H} KH{KH} w{window} cap{softcap}", flush=True)
+        y = {k: t.clone() for k, t in x.items()}
+        y[name][at, 3] = value  # of the first sequence and head
+        got, want = [], []
+        for form, res in ((lambda t: t, got), (odd, want)):
+            q, k, v, do = (form(y[i]) for i in ("q", "k", "v", "do"))
+            res += ops.attn_fwd(q, k, v, **kw)
+            res += ops.attn_bwd(q, k, v, form(got[0]), got[1], do, **kw)  # (gradients of both from the same forward)
+        for a, b in zip(got, want):
+            a, b = a.double(), b.double()
+            ok = b.isfinite()
+            assert torch.equal(ok, a.isfinite()) and torch.equal(a[~ok].nan_to_num(7.0, 8.0, 9.0), b[~ok].nan_to_num(7.0, 8.0, 9.0))
+            assert (a[ok] - b[ok]).norm() <= 1e-2 * b[ok].norm()
