@@ -18,6 +18,7 @@
 // Backward is split in two deterministic kernels (no atomics): dK/dV with the key tile
 // stationary, dQ with the query tile stationary; each recomputes P from the saved LSE.
 #include "common.h"
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -1228,7 +1229,7 @@ extern "C" int32_t olmax_attn_fwd(hipStream_t stream, const void* q, const void*
   window = reach(window, S);
   const float scale = 1.f / sqrtf((float)D);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k, *vp = (const bf16*)v;
-  if (fast_ok(D, S, GENERIC_MAX_S_FWD, q, k, v, o, ldq, ldk, ldv, ldo)) {
+  if (fast_ok(D, S, GENERIC_MAX_S_FWD, q, k, v, o, ldq, ldk, ldv, ldo) && (D == 128 || o != q)) {
     auto go = D == 128 ? launch_fwd_fast<128> : launch_fwd_fast<64>;
     go(stream, qp, kp, vp, (bf16*)o, lse, B, S, H, KH, ldq, ldk, ldv, ldo, window, softcap);
   } else {
@@ -1266,8 +1267,12 @@ extern "C" int32_t olmax_attn_bwd(hipStream_t stream, const void* q, const void*
   const float scale = 1.f / sqrtf((float)D);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k, *vp = (const bf16*)v, *op = (const bf16*)o, *gop = (const bf16*)d_o;
   float* delta = (float*)workspace;
+  // In place: the one-wave-per-query kernels read a row before they write it and dK/dV leave last; the MFMA kernels read Q
+  // and dO again after dQ is written.  head_dim 64 has always taken such calls, so they stay on the former.
+  const void* const outs[] = {dq, dk, dv};
+  const bool in_place = D != 128 && std::any_of(outs, outs + 3, [&](const void* p) { return p == q || p == k || p == v || p == o || p == d_o; });
   // (a workspace of delta alone is head_dim 128's: any other head_dim may meet an unaligned view)
-  if (bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, S, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv) &&
+  if (!in_place && bwd_fast_ok(q, k, v, o, d_o, dq, dk, dv, S, D, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv) &&
       (D == 128 || workspace_bytes >= attn_delta_bytes(B, S, H) + 2 * attn_acc_bytes(B, S, KH, D))) {
     auto go = D == 128 ? launch_bwd_fast<128> : launch_bwd_fast<64>;
     go(stream, qp, kp, vp, op, lse, gop, (bf16*)dq, (bf16*)dk, (bf16*)dv, delta, B, S, H, KH, ldq, ldk, ldv, ldo, lddo,

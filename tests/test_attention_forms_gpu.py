@@ -135,3 +135,24 @@ def test_head_dim_64_keeps_what_a_row_does_not_see_out_of_it(B, S, H, KH, window
             ok = b.isfinite()
             assert torch.equal(ok, a.isfinite()) and torch.equal(a[~ok].nan_to_num(7.0, 8.0, 9.0), b[~ok].nan_to_num(7.0, 8.0, 9.0))
             assert (a[ok] - b[ok]).norm() <= 1e-2 * b[ok].norm()
+
+
+def test_head_dim_64_gradients_in_place():
+    """q | k | v overwritten by their gradients, and dO by dQ; bound as in check()."""
+    from olmax_amd import ops
+    B, S, H, KH, D = 2, 200, 4, 4, 64
+    print("[case] attn in place", flush=True)
+    qkv, do = rnd(B * S, (H + 2 * KH) * D, seed=1), rnd(B * S, H * D, seed=2)
+    cols = lambda t: (t[:, :H * D], t[:, H * D:(H + KH) * D], t[:, (H + KH) * D:])  # noqa: E731
+    kw = dict(B=B, S=S, H=H, KH=KH, D=D)
+    o, lse = ops.attn_fwd(*cols(qkv), **kw)
+    want = ops.attn_bwd(*cols(qkv), o, lse, do, **kw)
+    into_do, fresh = do.clone(), rnd(B * S, 2 * KH * D, seed=3)
+    over = [t.clone() for t in (qkv, qkv)]
+    ops.attn_bwd(*cols(over[0]), o, lse, do, dq=cols(over[0])[0], dk=cols(over[0])[1], dv=cols(over[0])[2], **kw)
+    ops.attn_bwd(*cols(qkv), o, lse, into_do, dq=into_do, dk=fresh[:, :KH * D], dv=fresh[:, KH * D:], **kw)
+    q = cols(over[1])[0]
+    ops.attn_fwd(*cols(over[1]), out=q, **kw)
+    for got in (cols(over[0]), (into_do, fresh[:, :KH * D], fresh[:, KH * D:])):
+        assert all(rel(a, b) < 1e-2 for a, b in zip(got, want))
+    assert rel(q, o) < 1e-2
