@@ -1064,7 +1064,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
                       GemmScratch scratch) {
   // whole 16-byte chunks everywhere: aligned rows, and a chunk never crosses the end of a row
   const bool direct_ok = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 && (a_padded || (a_kc ? K : M) % 8 == 0) &&
-                         (b_kc ? K : N) % 8 == 0 && (a_kc || !b_kc);
+                         (b_kc ? K : N) % 8 == 0;
   const int force_tile = g_force_tile.load(std::memory_order_relaxed);
   int parts;
   int tile = pick_tile(M, N, K, direct_ok, b_kc || force_tile || !aligned16(scratch.p) ? 0 : scratch.bytes, &parts);
@@ -1126,6 +1126,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   } while (0)
   if (a_kc && b_kc) GO(true, true);
   if (a_kc) GO(true, false);
+  if (b_kc) GO(false, true);
   GO(false, false);
 #undef GO
 }
