@@ -938,7 +938,7 @@ extern "C" void olmax_gemm_profile_begin(void) {
 }
 // Stop recording, wait for the recorded events and aggregate per kernel instantiation.
 // keys/ms/flops/launches: host arrays of `cap` entries; returns the number of distinct keys.
-// key = tile | a_layout<<12 | b_layout<<13 | has_residual<<14 | out_f32<<15 | glu_epilogue<<16 | rope_epilogue<<17,
+// key = tile (64: gemm_small_kernel) | a_layout<<12 | b_layout<<13 | has_residual<<14 | out_f32<<15 | glu_epilogue<<16 | rope_epilogue<<17,
 // with a_layout / b_layout bit SET when the operand is reduction-contiguous.  flops / bytes:
 // algorithmic totals (2MNK; every operand and the result moved once).
 extern "C" int32_t olmax_gemm_profile_end(int32_t* keys, double* ms, double* flops, double* bytes, int64_t* launches,
@@ -1108,9 +1108,24 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
     }
   }
   if (tile == 0) {
+    ProfRec rec{};
+    if (g_prof_on) {
+      (void)hipEventCreate(&rec.e0);
+      (void)hipEventCreate(&rec.e1);
+      (void)hipEventRecord(rec.e0, stream);
+    }
     olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32,
                      // eight waves share a tile while there are not more tiles than CUs, else two workgroups fit a CU
                      (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 256 ? 8 : 4);
+    if (g_prof_on) {
+      (void)hipEventRecord(rec.e1, stream);
+      rec.flops = 2.0 * M * N * K;
+      rec.bytes = 2.0 * ((double)M * K + (double)N * K + (double)M * N * (r ? 2 : 1) * (out_f32 ? 2 : 1));
+      rec.key = 64 | (a_kc << 12) | (b_kc << 13) | ((r != nullptr) << 14) | (out_f32 << 15);
+      rec.M = M; rec.N = N; rec.K = K;
+      std::lock_guard<std::mutex> lk(g_prof_mu);
+      g_prof.push_back(rec);
+    }
     OLMAX_LAUNCH_CHECK();
     return OLMAX_OK;
   }

@@ -40,3 +40,13 @@ def test_large_products_of_every_layout_run_on_large_tiles(M, N, K, al, bl):
     got = recorded(lambda: ops.gemm(a, b, a_layout=al, b_layout=bl))
     assert sum(m * n for _, m, n, _, _ in got) == M * N
     assert all((key & 0xfff) >= 128 and (key >> 12 & 3) == (1 - al) + 2 * (1 - bl) for key, *_ in got), got
+
+
+@pytest.mark.parametrize("al,bl", [(0, 0), (0, 1), (1, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K,out_f32", [(77, 2816, 1024, False), (7, 9, 3, True), (512, 256, 512, False)])
+def test_products_of_the_64_wide_kernel_are_recorded(M, N, K, out_f32, al, bl):
+    from olmax_amd import ops
+    print(f"[case] record M{M} N{N} K{K} a{al} b{bl}", flush=True)
+    a, b = operands(M, N, K, al, bl)
+    assert recorded(lambda: ops.gemm(a, b, a_layout=al, b_layout=bl, out_f32=out_f32)) == [
+        (64 | (1 - al) << 12 | (1 - bl) << 13 | out_f32 << 15, M, N, K, 1)]
