@@ -1071,7 +1071,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   if (parts > 1)
     return (a_kc ? launch_split<true, false> : launch_split<false, false>)(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts,
                                                                           (float*)scratch.p);
-  if (force_tile && tile) {
+  if (force_tile && direct_ok && K >= BK) {  // whatever the rule chose, if the problem has a tile of that size
     if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
     if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;
   }

@@ -50,3 +50,22 @@ def test_products_of_the_64_wide_kernel_are_recorded(M, N, K, out_f32, al, bl):
     a, b = operands(M, N, K, al, bl)
     assert recorded(lambda: ops.gemm(a, b, a_layout=al, b_layout=bl, out_f32=out_f32)) == [
         (64 | (1 - al) << 12 | (1 - bl) << 13 | out_f32 << 15, M, N, K, 1)]
+
+
+@pytest.mark.parametrize("al,bl", [(0, 0), (0, 1), (1, 1), (1, 0)])
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 64), (512, 1024, 1024), (264, 1000, 136)])
+def test_a_forced_tile_takes_what_the_rule_gives_to_the_64_wide_kernel(M, N, K, tile, al, bl):
+    """And the result is the same but for the order of K fp32 additions (2^-24 each) before the rounding to bf16 (2^-9)."""
+    from olmax_amd import _lib, ops
+    print(f"[case] forced {tile} M{M} N{N} K{K} a{al} b{bl}", flush=True)
+    a, b = operands(M, N, K, al, bl)
+    want = ops.gemm(a, b, a_layout=al, b_layout=bl).double()
+    res = []
+    _lib.load().olmax_gemm_set_tile(tile)
+    try:
+        got = recorded(lambda: res.append(ops.gemm(a, b, a_layout=al, b_layout=bl)))
+    finally:
+        _lib.load().olmax_gemm_set_tile(0)
+    assert [key & 0xfff for key, *_ in got] == [tile], got
+    assert (res[0].double() - want).norm() < 2 ** -9 * want.norm()
