@@ -1220,6 +1220,13 @@ extern "C" int32_t olmax_gemm_rope_bf16(hipStream_t stream, const void* X, const
 extern "C" int32_t olmax_glu_fwd(hipStream_t stream, const void* gate, const void* up, void* out, int64_t T, int32_t F,
                                  int64_t ldg, int64_t ldu, int64_t ldo, int32_t act);
 
+extern "C" int32_t olmax_gemm_glu_fused(const void* X, const void* W, const void* act_out, int32_t M, int32_t F, int32_t K,
+                                        int64_t ldx, int64_t ldw, int64_t ldact) {
+  const bool fits = aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && K % BK == 0 && M >= 256 && F % 128 == 0 &&
+                    (int64_t)((M + 255) / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
+  return fits && (M % 256 == 0 || (aligned16(act_out) && ldact % 8 == 0));  // ragged rows leave through the whole-line stores only
+}
+
 // Gated-MLP input projection with the activation fused into the GEMM epilogue:
 // act_out[M, F] = f(X Wgate^T) * (X Wup^T), W = [Wgate; Wup] ([2F, K], row stride ldw); gu_out
 // ([M, 2F], optional) receives gate|up for the backward pass.  Falls back to the plain GEMM
@@ -1232,11 +1239,8 @@ extern "C" int32_t olmax_gemm_glu_bf16(hipStream_t stream, const void* X, const 
   OLMAX_CHECK(act == 0 || act == 1, OLMAX_ERR_ARG, "olmax_gemm_glu_bf16: act must be 0 (silu) or 1 (gelu-tanh)");
   OLMAX_CHECK(ldx >= K && ldw >= K && ldact >= F && (!gu_out || ldgu >= 2 * (int64_t)F), OLMAX_ERR_SHAPE,
               "olmax_gemm_glu_bf16: leading dimension smaller than row length");
-  const bool fits = aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && K % BK == 0 && M >= 256 && F % 128 == 0 &&
-                    (int64_t)((M + 255) / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
-  // ragged rows leave through the whole-line stores only
-  const bool lines = aligned16(act_out) && ldact % 8 == 0 && (!gu_out || (aligned16(gu_out) && ldgu % 8 == 0));
-  if (fits && (M % 256 == 0 || lines)) {
+  const bool gu_lines = M % 256 == 0 || !gu_out || (aligned16(gu_out) && ldgu % 8 == 0);
+  if (gu_lines && olmax_gemm_glu_fused(X, W, act_out, M, F, K, ldx, ldw, ldact)) {
 #define GLU(E, RAG) launch_glu<E, RAG>(stream, (const bf16*)X, (const bf16*)W, (bf16*)gu_out, (bf16*)act_out, M, F, K, ldx, ldw, ldgu, ldact)
     if (act == 0) return M % 256 ? GLU(1, 1) : GLU(1, 0);
     return M % 256 ? GLU(2, 1) : GLU(2, 0);

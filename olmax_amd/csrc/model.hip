@@ -204,9 +204,9 @@ int block_forward(hipStream_t s, const olmax_model_config* c, const olmax_block_
   }
   if (defer_mlp) return OLMAX_OK;
   // gate|up projection with the activation in the GEMM epilogue; gate|up themselves are only
-  // written when a backward pass will read them (a.gu doubles as scratch for odd shapes)
-  const bool fused_shape = m.T >= 256 && m.F % 128 == 0 && m.d % 64 == 0 && ((m.T + 255) / 256) * (m.F / 128) >= 128;
-  RC(olmax_gemm_glu_bf16(s, mlp_in, w->wgu, (save_gu || !fused_shape) ? a.gu : nullptr, a.act, (int)m.T, m.F, m.d, m.d,
+  // written when a backward pass will read them (a.gu doubles as scratch for what the fused kernel does not take)
+  const bool fused = olmax_gemm_glu_fused(mlp_in, w->wgu, a.act, (int)m.T, m.F, m.d, m.d, m.d, m.F);
+  RC(olmax_gemm_glu_bf16(s, mlp_in, w->wgu, (save_gu || !fused) ? a.gu : nullptr, a.act, (int)m.T, m.F, m.d, m.d,
                          m.d, 2 * m.F, m.F, c->act));
   if (lt == 0) {
     if (need_y) RC(lin_fwd(s, a.act, m.F, w->wdown, m.F, m.d, y, m.d, a.h, m.d, m.T));

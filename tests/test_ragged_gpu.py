@@ -108,6 +108,30 @@ def test_gated_projection_on_ragged_rows_of_unaligned_views(which):
     assert rel(got, want) < 2 ** -8
 
 
+@pytest.mark.parametrize("T", [1000, 1024])
+@pytest.mark.parametrize("tile", [0, 128])
+def test_forward_of_a_model_whose_weights_are_not_16_byte_aligned(T, tile):
+    """The gated projection then takes the two-step path and needs gate|up as scratch although no backward pass follows; so
+    it does while a tile size is forced.  The loss differs by fp32 orders before bf16 roundings."""
+    from olmax_amd import TransformerConfig, _lib
+    print(f"[case] unaligned weights T{T} tile{tile}", flush=True)
+    cfg = TransformerConfig(vocab_size=512, d_model=128, hidden_size=4096, num_layers=1, n_heads=1, head_dim=128)
+    model = cfg.build(batch_size=1, sequence_length=T, seed=1)
+    ids, labels = (torch.randint(0, 512, (T,), device="cuda", dtype=torch.int32) for _ in range(2))
+    want = model.forward_loss(ids, labels).item()
+    p = model.params_bf16
+    model.params_bf16 = torch.cat([p.new_zeros(1), p])[1:]
+    assert model.params_bf16.data_ptr() % 16
+    _lib.load().olmax_gemm_set_tile(tile)
+    try:
+        got = [model.forward_loss(ids, labels).item()]
+        model.params_bf16 = p
+        got.append(model.forward_loss(ids, labels).item())
+    finally:
+        _lib.load().olmax_gemm_set_tile(0)
+    assert all(abs(x - want) < 1e-4 * want for x in got)
+
+
 @pytest.mark.parametrize("B,S,heads,N,d", [(3, 1000, 24, 3072, 128), (1, 2049, 20, 6144, 64)])
 def test_fused_rope_projection_on_ragged_rows(B, S, heads, N, d):
     from olmax_amd import ops
