@@ -162,11 +162,9 @@ def gated_mlp_in(x, w_gate_up, act: str = "silu", gate_up_out=None, save_gate_up
     F = w_gate_up.shape[0] // 2
     if out is None:
         out = torch.empty(T, F, device=x.device, dtype=BF16)
-    fits = T >= 256 and F % 128 == 0 and d % 64 == 0 and -(-T // 256) * (F // 128) >= 128
-    # what the fused GEMM of a ragged T asks of its operands; without it the two-step path needs gate|up
-    if T % 256 and any(t.data_ptr() % 16 or t.stride(0) % 8 for t in (x, w_gate_up, out)):
-        fits = False
-    if gate_up_out is None and (save_gate_up or not fits):
+    fits = _L().olmax_gemm_glu_fused(ptr(x), ptr(w_gate_up), ptr(out), i32(T), i32(F), i32(d), i64(x.stride(0)),
+                                     i64(w_gate_up.stride(0)), i64(out.stride(0)))
+    if gate_up_out is None and (save_gate_up or not fits):  # (the two-step path needs them as scratch)
         gate_up_out = torch.empty(T, 2 * F, device=x.device, dtype=BF16)
     check(_L().olmax_gemm_glu_bf16(stream_ptr(), ptr(x), ptr(w_gate_up), ptr(gate_up_out), ptr(out), i32(T), i32(F),
                                    i32(d), i64(x.stride(0)), i64(w_gate_up.stride(0)),

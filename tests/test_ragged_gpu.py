@@ -108,6 +108,24 @@ def test_gated_projection_on_ragged_rows_of_unaligned_views(which):
     assert rel(got, want) < 2 ** -8
 
 
+@pytest.mark.parametrize("T,which,tile", [(2048, "x", 0), (2048, "w", 0), (2048, "out", 0), (2048, "none", 256), (2049, "none", 128)])
+def test_gated_projection_gets_scratch_wherever_the_fused_kernel_does_not_run(T, which, tile):
+    """Unaligned operands at whole tiles, and a forced tile size; the result differs by fp32 orders before bf16 roundings."""
+    from olmax_amd import _lib, ops
+    print(f"[case] gated projection T{T}, unaligned {which}, tile {tile}", flush=True)
+    F, d = 2048, 128
+    shift = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)  # noqa: E731
+    x, w, out = rnd(T, d, seed=1), rnd(2 * F, d, seed=2, scale=d ** -0.5), torch.empty(T, F, device="cuda", dtype=BF)
+    want, _ = ops.gated_mlp_in(x, w)
+    args = {k: shift(t) if k == which else t for k, t in (("x", x), ("w", w), ("out", out))}
+    _lib.load().olmax_gemm_set_tile(tile)
+    try:
+        got, _ = ops.gated_mlp_in(args["x"], args["w"], save_gate_up=False, out=args["out"])
+    finally:
+        _lib.load().olmax_gemm_set_tile(0)
+    assert rel(got, want) < 2 ** -8
+
+
 @pytest.mark.parametrize("T", [1000, 1024])
 @pytest.mark.parametrize("tile", [0, 128])
 def test_forward_of_a_model_whose_weights_are_not_16_byte_aligned(T, tile):
