@@ -537,10 +537,11 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
       if (qi < S) store4(u >> 2, u & 3, v, inv);
     });
   }
-  if (qi < S && lhi == 0 && ks == 0) {
+  // (every wave of the row looks at its LSE: a row whose scores are all -inf sums to zero, not to NaN, until it is done over)
+  if (qi < S && lhi == 0 && (D == 64 || ks == 0)) {
     const float lse = LOG2_UNITS ? (m + log2f(ltot)) * LN2 : m * to_ln + __logf(ltot);
     if (D == 64) zeros = __builtin_fmaf(lse, 0.f, zeros);
-    LSE[((int64_t)b * H + h) * S + qi] = lse;
+    if (ks == 0) LSE[((int64_t)b * H + h) * S + qi] = lse;
   }
   if constexpr (D == 64)
     redo_rows(zeros, [&](int r) {

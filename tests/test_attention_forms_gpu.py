@@ -137,6 +137,26 @@ def test_head_dim_64_keeps_what_a_row_does_not_see_out_of_it(B, S, H, KH, window
             assert (a[ok] - b[ok]).norm() <= 1e-2 * b[ok].norm()
 
 
+@pytest.mark.parametrize("B,S,H,KH,window", [(1, 70, 2, 2, None), (2, 200, 4, 2, 0), (4, 300, 48, 48, None)])
+def test_head_dim_64_row_whose_only_score_is_minus_infinity(B, S, H, KH, window):
+    """Such a softmax is NaN in every column, as on the kernels that work through visible pairs one by one, however many
+    waves share the row; few workgroups and enough for the unsplit form."""
+    from olmax_amd import ops
+    print(f"[case] score of -inf, B{B} S{S} H{H} KH{KH} w{window}", flush=True)
+    n = B * S
+    q, k, v = rnd(n, H * 64, seed=1), rnd(n, KH * 64, seed=2), rnd(n, KH * 64, seed=3)
+    at = 0 if window is None else 37  # a token whose query sees this key only
+    q[at, 3], k[at, 3] = 1.0, -math.inf
+    kw = dict(B=B, S=S, H=H, KH=KH, D=64, window=window, softcap=0.0)
+    odd = lambda t: torch.cat([t, t.new_zeros(n, 3)], 1)[:, :t.shape[1]]  # noqa: E731
+    got, want = ops.attn_fwd(q, k, v, **kw), ops.attn_fwd(odd(q), odd(k), odd(v), **kw)
+    assert want[0][at, :64].isnan().all() and want[1][0, 0, at].isnan()
+    for a, b in zip(got, want):
+        ok = b.isfinite()
+        assert torch.equal(ok, a.isfinite())
+        assert (a[ok].double() - b[ok].double()).norm() <= 1e-2 * b[ok].double().norm()
+
+
 def test_head_dim_64_gradients_in_place():
     """q | k | v overwritten by their gradients, and dO by dQ; bound as in check()."""
     from olmax_amd import ops
