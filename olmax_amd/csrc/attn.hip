@@ -1140,28 +1140,44 @@ void bwd_fast_attributes() {
   });
 }
 
-// Whether the forward and dQ take their split kernels: while the workgroups of 128 queries do not fill the CUs twice
-// over, a wave has a SIMD to itself and its chain of key tiles is what takes the time.  Forward | backward (dK/dV
-// included), us, plain -> split: 3 x 1000 tokens, 8 heads (192 workgroups): 25.2 -> 22.5 | 70 -> 62; 2 x 2000 (256):
-// 44.0 -> 36.5 | 122 -> 104; 1 x 6000 (376): 127 -> 101 | 382 -> 330; 1 x 1500, 32 heads (384): 38.6 -> 33.6 | 163 -> 152.  At
-// 512 workgroups the chain decides: 32 tiles 53.5 -> 49.5 | 181 -> 171, 16 tiles 32.3 -> 34.6 | 109 -> 111, 18 tiles in
-// a window 40.6 -> 50.2 | 148 -> 155.  Beyond, the plain kernels' two workgroups per CU keep the SIMDs busy by themselves.
+// Whether the forward and dQ take their split kernels.  While few workgroups of 128 queries share a CU, a wave has a SIMD to itself and its
+// chain of key tiles is what takes the time; a short chain is over before the split pays for its merge.  Forward | dQ, us a call,
+// plain -> split, at n workgroups:
+// head_dim 128 (split: eight waves per workgroup, one on a CU), n <= 256: 1 tile 6.4 -> 8.1 | 2.4 slower, 4 tiles 12.2 -> 12.7 | 0.4 slower,
+// 8 tiles 17.4 -> 16.7 | 2.2 faster, 64 tiles 80.9 -> 65.5 | 37 faster.  Up to 512 the plain kernel has all of its workgroups on the GPU
+// at once and the split one comes in two rounds: n = 320, 20 tiles 32.8 -> 27.7 | 12 faster, n = 384, 4 tiles 16.4 -> 22.6 | 10 slower,
+// 16 tiles 29.2 -> 29.4 | 1.4 faster, n = 512, 16 tiles 31.2 -> 33.2 | 2.4 slower, 64 tiles 93.5 -> 79.5 | 31 faster.  From n = 513 on the plain
+// kernels' two workgroups per CU keep the SIMDs busy by themselves: n = 640, 20 tiles 38 -> 50 | 15 slower.
+// head_dim 64 (split: 64 queries to a workgroup, twice as many of them), n <= 128: 1 tile 5.0 -> 6.2 | 1.6 slower, 2 tiles 7.2 -> 6.9 | 0.2 faster,
+// 8 tiles 12.3 -> 8.9 | 5.1 faster; n = 192: 3 tiles 7.2 -> 11.3 | 6 slower; n = 256: 8 tiles 1.5 slower | 1.5 slower, 16 tiles 19.0 -> 16.9 | 4.4
+// faster; n = 320, 24 tiles 0.9 faster | 0.4 faster; n = 384, 32 tiles 0.5 slower | 3.9 faster; n = 480, 24 tiles 27.3 -> 36.5 | 9.7 slower.
+template <int D>
 bool q_split(int B, int S, int H, int window) {
   const int64_t n = (int64_t)((S + 127) / 128) * H * B;
   const int tiles = (window >= 0 && window < S - 128 ? window + 128 : S + 63) / 64;
-  return n <= 256 || (n <= 512 && tiles >= 24);
+  if (D == 128) return n <= 512 && tiles >= (n <= 256 ? 6 : 12 + 14 * (n - 256) / 256);
+  return n <= 384 && tiles >= (n <= 128 ? 2 : n <= 256 ? 12 : n / 12);
 }
 // Whether dK/dV takes the split kernel.  One workgroup per key tile and K/V head is little parallel work when the
 // heads are few: 224 workgroups for 2 x 1777 tokens of 8 K/V heads leave the GPU waiting for those of the first key tile,
-// which walk the four query heads of 1777 tokens one 32-row tile at a time with one wave per SIMD.  Backward
-// (dQ included), us, plain -> split: 2 x 1777, 32 heads on 8: 453 -> 244; 1 x 4096: 962 -> 530; 1 x 300: 89 -> 47;
-// 3 x 1000, 8 on 8: 95 -> 71; 1 x 6000, 40 on 8 (376 workgroups): 1954 -> 1419.  From 512 workgroups on it depends on
-// the length of the chain: 32 tiles 111 -> 116, 64 tiles 189 -> 182, 256 tiles 606 -> 520, 628 tiles (640 workgroups)
-// 1647 -> 1541; a filled GPU is better off without the halved reuse of Q and dO (1024: 1213 -> 1279, 2048: 1029 -> 1136).
+// which walk the four query heads of 1777 tokens one 32-row tile at a time with one wave per SIMD.  Backward (dQ included), us, plain -> split,
+// at n workgroups of 128 keys and chains of so many 32-row tiles:
+// head_dim 128, n <= 128: 2 tiles 17.3 -> 18.1, 3 tiles 23.0 -> 21.1, 64 tiles 129 -> 66; n = 192, 4 tiles 30.5 -> 33.5; n = 256, 16 tiles 58.1 -> 51.7;
+// n = 320: 16 tiles 82 -> 84, 160 tiles 323 -> 200; n = 384: 8 tiles 47.4 -> 56.5, 32 tiles 102 -> 95, 48 tiles 149 -> 135;
+// n = 448: 4 tiles 45.8 -> 62.8, 8 tiles 49.6 -> 66.7; n = 512: 32 tiles 106 -> 112, 64 tiles 206 -> 204, 128 tiles 344 -> 309; beyond, the split kernel's
+// halved reuse of Q and dO costs more: n = 640: 128 tiles 408 -> 421, 256 tiles 678 -> 655; n = 768: 256 tiles 741 -> 766.
+// head_dim 64: n <= 128: 2 tiles as many, 3 tiles 16.4 -> 14.4, 4 tiles 19.1 -> 15.2; n = 192: 3 tiles 17 -> 19, 5 tiles 21 -> 20; n = 320: 8 tiles 33.0 -> 33.5,
+// 16 tiles 53 -> 50; n = 448: 4 tiles 28.6 -> 36.8, 32 tiles as many; n = 512: 32 tiles 70.2 -> 71.4, 48 tiles 107 -> 102; n = 544: 128 tiles 241 -> 217; n = 640:
+// 128 tiles 237 -> 235, 256 tiles 434 -> 410; n = 768: 256 tiles 459 -> 477.
+template <int D>
 bool dkv_split(int B, int S, int H, int KH, int window) {
   const int64_t n = (int64_t)((S + 127) / 128) * KH * B;
-  const int64_t chain = (int64_t)(H / KH) * ((window >= 0 && window < S - 128 ? window + 128 : S) / 32);
-  return n < 512 || (n < 1024 && chain >= 64);
+  const int64_t chain = (int64_t)(H / KH) * (((window >= 0 && window < S - 128 ? window + 128 : S) + 31) / 32);
+  if (n > 640) return false;
+  if (n > 512) return chain >= (D == 128 ? 200 : 128);
+  if (n <= 128) return chain >= 3;
+  const int base = D == 128 ? 8 : 4;
+  return chain >= (n <= 256 ? base : base + (D == 128 ? 56 : 36) * (n - 256) / 256);
 }
 
 // The two MFMA kernels of the backward pass; delta: fp32 [B, H, S] scratch, fully
@@ -1174,7 +1190,7 @@ void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const b
                      float softcap) {
   const float scale = 1.f / sqrtf((float)D);
   bwd_fast_attributes();
-  const bool split_q = q_split(B, S, H, window), split_kv = dkv_split(B, S, H, KH, window);
+  const bool split_q = q_split<D>(B, S, H, window), split_kv = dkv_split<D>(B, S, H, KH, window);
   auto go = [&](auto cap) {
     constexpr bool CAP = decltype(cap)::value;
     auto qk = [&](auto kern, int qw, int ks) {
@@ -1205,7 +1221,7 @@ void launch_fwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const b
     (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, true, QW, KS>, ATTR, smem_q(D, QW, KS));
     (void)hipFuncSetAttribute((const void*)attn_fwd_kernel<D, false, QW, KS>, ATTR, smem_q(D, QW, KS));
   });
-  const bool split = q_split(B, S, H, window);
+  const bool split = q_split<D>(B, S, H, window);
   auto go = [&](auto cap) {
     constexpr bool CAP = decltype(cap)::value;
     auto run = [&](auto kern, int qw, int ks) {
