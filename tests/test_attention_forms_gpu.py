@@ -22,9 +22,10 @@ def rel(got, want):
     return ((got - want).norm() / (want.norm() + 1e-300)).item()
 
 
-def check(B, S, H, KH, D, window, softcap, strided=False):
-    """Every output against the float64 oracle.  P and dS are rounded to bf16 (2^-9 each) before the second products
-    and the results once more: 2-norm errors of 0.3 % at most; bounds are three times that."""
+def check(B, S, H, KH, D, window, softcap, strided=False, groups=None):
+    """Every output (of the K/V heads `groups` and their query heads only) against the float64 oracle.  P and dS are rounded to
+    bf16 (2^-9 each) before the second products and the results once more: 2-norm errors of 0.3 % at most; bounds are three
+    times that."""
     from olmax_amd import ops
 
     print(f"[case] attn B{B} S{S} H{H} KH{KH} D{D} w{window} cap{softcap}", flush=True)
@@ -39,16 +40,20 @@ def check(B, S, H, KH, D, window, softcap, strided=False):
     o, lse = ops.attn_fwd(q, k, v, out=guard[1:-1], **kw)
     assert (guard[0] == 7).all() and (guard[-1] == 7).all()
     dq, dk, dv = ops.attn_bwd(q, k, v, o, lse, do, **kw)
-    q4, k4, v4, d4 = (t.cpu().double().reshape(B, S, -1, D) for t in (q, k, v, do))
+    groups = list(range(KH)) if groups is None else groups
+    rep = H // KH
+    heads = [g * rep + r for g in groups for r in range(rep)]
+    cut = lambda t: t.reshape(B, S, -1, D)[:, :, heads if t.shape[1] == H * D else groups].double().cpu()  # noqa: E731
+    q4, k4, v4, d4 = (cut(t) for t in (q, k, v, do))
     wo, wlse = ref.attention_fwd(q4, k4, v4, window=window, softcap=softcap)
-    assert rel(o, wo.reshape(B * S, -1)) < 1e-2
-    assert (lse.cpu().double() - wlse).abs().max() < 2e-3
+    assert rel(cut(o), wo) < 1e-2
+    assert (lse[:, heads].cpu().double() - wlse).abs().max() < 2e-3
     want = ref.attention_bwd(q4, k4, v4, wo, wlse, d4, window=window, softcap=softcap)
-    for name, got, w in zip(("dq", "dk", "dv"), (dq, dk, dv), want):
+    for name, got, w in zip(("dq", "dk", "dv"), (cut(dq), cut(dk), cut(dv)), want):
         if w.norm() < 1e-12 * math.sqrt(w.numel()):  # S = 1: dS is exactly zero, what remains is rounding
             assert got.double().norm() < 1e-2 * math.sqrt(got.numel()), name
         else:
-            assert rel(got, w.reshape(B * S, -1)) < 1e-2, name
+            assert rel(got, w) < 1e-2, name
 
 
 @pytest.mark.parametrize("S", [1, 31, 33, 63, 65, 127, 128, 129, 192, 321])
@@ -89,6 +94,27 @@ def test_key_gradients_split_over_query_groups(S, H, KH, window, softcap):
                                                    (449, 2, 2, None, 0.0)])
 def test_queries_split_over_key_groups(S, H, KH, window, softcap, D):
     check(3, S, H, KH, D, window, softcap, strided=S % 2 == 0)
+
+
+# chains long enough for the split forward and dQ (from 6 key tiles on at head_dim 128, 2 at 64): ragged ends, windows, soft-caps
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,H,KH,window,softcap", [(1, 321, 3, 1, None, 0.0), (2, 385, 2, 2, None, 30.0), (1, 450, 4, 2, 300, 0.0), (2, 641, 2, 1, 257, 50.0), (1, 1100, 2, 2, None, 0.0)])
+def test_long_chains_split_over_key_groups(B, S, H, KH, window, softcap, D):
+    check(B, S, H, KH, D, window, softcap, strided=S % 2 == 1)
+
+
+# more workgroups than either rule splits for (n of 128 queries, keys): the forms without a split, over many tiles
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,H,KH,window,softcap", [
+    (1, 1000, 82, 82, None, 0.0),    # n = 656, 656
+    (3, 1000, 28, 28, None, 50.0),   # 672, 672
+    (1, 1301, 60, 60, 300, 0.0),     # 660, 660: windows that start inside a tile
+    (2, 449, 164, 82, 70, 30.0),     # 1312, 656
+    (1, 1000, 132, 33, None, 0.0),   # 1056 plain, 264 split
+    (4, 129, 90, 90, None, 0.0),     # 720, 720: a last tile of one row
+])
+def test_filled_gpus_take_the_forms_without_a_split(B, S, H, KH, window, softcap, D):
+    check(B, S, H, KH, D, window, softcap, strided=S % 2 == 1, groups=[0, KH // 2, KH - 1])
 
 
 @pytest.mark.parametrize("D", [64, 128])
