@@ -41,6 +41,7 @@ namespace {
 
 constexpr int BK = 64;
 typedef u32x4 __attribute__((aligned(2))) u32x4_u;  // 16 bytes at any element (ragged column edges)
+typedef f32x4 __attribute__((aligned(4))) f32x4_u;
 
 #ifndef GEMM_VGPR_CAP
 #define GEMM_VGPR_CAP
@@ -714,6 +715,15 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
     for (int j = 0; j < TN; j++) {
       const int64_t row = m0 + wm * WM + i * 16 + l16e;
       if (!stores_row(wm * WM + i * 16 + l16e)) continue;
+      if (RAG && OUT_F32 && wn * WN + j * 16 + g16e * 4 >= col_lo) {  // (element by element a 2816 x 3200 x 512 takes 46 us, so 24)
+        const int col = n0 + wn * WN + j * 16 + g16e * 4;
+        f32x4 v = acc[i][j];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (HAS_RES) v[r] += bf2f(R[row * ldr + col + r]);
+        *reinterpret_cast<f32x4_u*>(reinterpret_cast<float*>(Cv) + row * ldc + col) = v;
+        continue;
+      }
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int col = n0 + wn * WN + j * 16 + g16e * 4 + r;

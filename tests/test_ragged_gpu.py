@@ -60,6 +60,25 @@ def test_gemm_ragged(M, N, K, al, bl, pad):
     assert torch.equal(res, (out[:M, :N].float() + r.float()).to(BF))
 
 
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("M,N,K", [(256, 258, 64), (300, 1001, 136), (513, 2050, 128), (257, 3203, 72)])
+def test_fp32_results_with_a_residual_at_ragged_edges(M, N, K, tile):
+    """Column groups that the previous tile's end cuts, at any 4-byte alignment; bound as above, one addition more."""
+    from olmax_amd import _lib, ops
+    print(f"[case] fp32 residual M{M} N{N} K{K} tile{tile}", flush=True)
+    a, b, r = rnd(M, K, seed=1), rnd(N, K, seed=2), rnd(M, N + 3, seed=3)[:, :N]
+    want = a.double() @ b.double().t()
+    wide = torch.full((M + 1, N + 16), 7.0, device="cuda", dtype=torch.float32)
+    _lib.load().olmax_gemm_set_tile(tile)
+    try:
+        for res in (None, r):
+            ops.gemm(a, b, residual=res, out=wide[:M, 5:5 + N])
+            assert rel(wide[:M, 5:5 + N], want if res is None else want + r.double()) < (K + 1) ** 0.5 * 2 ** -24 * 8
+    finally:
+        _lib.load().olmax_gemm_set_tile(0)
+    assert (wide[:, :5] == 7).all() and (wide[:, 5 + N:] == 7).all() and (wide[M] == 7).all()
+
+
 def test_gemm_ragged_keeps_a_poisoned_neighbour_out():
     """What lies behind the operands' last rows and columns (NaN here) never reaches the result."""
     from olmax_amd import ops
