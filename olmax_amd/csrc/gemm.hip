@@ -32,6 +32,7 @@
 // every XCD one contiguous run of tiles; runs walk the tile grid in column groups so that
 // the A row-panels and B column-panels a single L2 sees are re-used.
 #include "common.h"
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -1013,14 +1014,17 @@ static int device_cu_count() {
 }
 
 // Estimated time (us) of each kernel on a problem of kt k-tiles, from measurements at 16 to 8192 rows
-// and 256 to 11008 columns (every layout; within about 15 %).  A k-tile costs a 256 tile 1.05 us with
+// and 256 to 11008 columns (every layout; within about 15 %) on the 256 CUs of this GPU.  A k-tile costs a 256 tile 1.05 us with
 // few tiles in flight and 1.52 us with one on every CU (both bound by operand delivery), a 128 tile
 // 0.57 us alone, 0.83 us with one on every CU and 1.08 us with the two that fit, a 64 tile 0.22 us
-// per round.
-static float cost_128(int64_t n, int kt) {
+// per round.  Up to 32 k-tiles and one 128 tile per CU the operands of a whole product stay near: 0.40 us up to 8 k-tiles, rising to 0.6,
+// sooner where B is [K, N].  us of 128 tiles | 64 tiles: 384 x 2816 x 512 6.8 | 7.6, 512 x 4096 x 1024 10.3 | 11.5 ([K, N]: 10.6 | 11.3), 256 x 5632 x 1024
+// 9.9 | 10.8 (10.7 | 10.8), 2048 x 1024 x 1024 11.6 | 10.8 (12.2 | 11.2), 512 x 2816 x 2048 18.0 | 16.6 (21.6 | 16.6).  Beyond, the rates of
+// whole rounds are taken: 512 x 4096 x 4096 39.8 | 28.7, 1024 x 4096 x 4096 42.9 | 50.3.
+static float cost_128(int64_t n, int kt, bool b_kc) {
   auto part = [&](int64_t r) {
     float f = r <= 64 ? 0.57f : r <= 256 ? 0.57f + 0.26f * (r - 64) / 192.f : 0.83f + 0.25f * (r - 256) / 256.f;
-    if (kt <= 32 && r <= 256) f = 0.6f;
+    if (kt <= 32 && r <= 256) f = kt <= 8 ? 0.4f : std::min(0.6f, 0.4f + (b_kc ? 0.0075f : 0.014f) * (kt - 8));
     return f * kt + 4.f;
   };
   return (n / 512) * (1.08f * kt + 4.f) + (n % 512 ? part(n % 512) : 0.f);
@@ -1038,12 +1042,12 @@ static int pick_parts(int64_t n, int kt, int64_t bytes, float* cost) {
     if (const float c = cost_split(n, kt, s); c < *cost) *cost = c, best = s;
   return best;
 }
-static float cost_256(int64_t n, int kt, int64_t bytes) {
+static float cost_256(int64_t n, int kt, int64_t bytes, bool b_kc) {
   const int64_t r = n % 256;
   // (a last round that fills less than half of the CUs is cut off and runs as 128 tiles or shared reductions)
   float last = r == 0 ? 0.f : (1.05f + 0.47f * r / 256.f) * kt + 6.f;
   if (n > 256 && r > 0 && r < 128) {
-    last = cost_128(4 * r, kt) < last ? cost_128(4 * r, kt) : last;
+    last = std::min(last, cost_128(4 * r, kt, b_kc));
     (void)pick_parts(r, kt, bytes, &last);
   }
   return (n / 256) * (1.52f * kt + 6.f) + last;
@@ -1052,16 +1056,16 @@ static float cost_small(int64_t n, int kt) { return ((n + 255) / 256) * (0.22f *
 
 // Which kernel takes a problem.  0: gemm_small (any size and alignment), else the edge of the
 // direct-to-LDS kernel's tiles; *parts > 1: 256 tiles with that many workgroups to a reduction.
-static int pick_tile(int M, int N, int K, bool direct_ok, int64_t bytes, int* parts) {
+static int pick_tile(int M, int N, int K, bool b_kc, bool direct_ok, int64_t bytes, int* parts) {
   *parts = 1;
   if (!direct_ok || M < 128 || N < 128 || K < BK) return 0;
   const int kt = (K + BK - 1) / BK;
   auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
   float best = cost_small(tiles(64), kt);
   int tile = 0;
-  if (const float c = cost_128(tiles(128), kt); c < best) best = c, tile = 128;
+  if (const float c = cost_128(tiles(128), kt, b_kc); c < best) best = c, tile = 128;
   if (M < 256 || N < 256) return tile;
-  if (const float c = cost_256(tiles(256), kt, bytes); c < best) best = c, tile = 256;
+  if (const float c = cost_256(tiles(256), kt, bytes, b_kc); c < best) best = c, tile = 256;
   *parts = pick_parts(tiles(256), K / BK, bytes, &best);
   return *parts > 1 ? 256 : tile;
 }
@@ -1077,7 +1081,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
                          (b_kc ? K : N) % 8 == 0;
   const int force_tile = g_force_tile.load(std::memory_order_relaxed);
   int parts;
-  int tile = pick_tile(M, N, K, direct_ok, b_kc || force_tile || !aligned16(scratch.p) ? 0 : scratch.bytes, &parts);
+  int tile = pick_tile(M, N, K, b_kc, direct_ok, b_kc || force_tile || !aligned16(scratch.p) ? 0 : scratch.bytes, &parts);
   if (parts > 1)
     return (a_kc ? launch_split<true, false> : launch_split<false, false>)(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts,
                                                                           (float*)scratch.p);
