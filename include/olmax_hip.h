@@ -95,11 +95,12 @@ int32_t olmax_qk_rope_bwd(olmax_stream_t stream, const void* dy, void* dx, const
 
 /* ---- Gated MLP input projection with the activation fused into the GEMM epilogue:
  * GatedMLP.forward, src/olmax/nn/mlp.py:69-73 (gate_proj, up_proj, act(gate) * up in one call).
- * W = [Wgate; Wup] ([2F, K], row stride ldw); act_out [M, F]; gu_out ([M, 2F], optional where
- * olmax_gemm_glu_fused says 1: M >= 256, F % 128 == 0, K % 64 == 0, ceil(M / 256) * (F / 128) >= 128,
- * X and W 16-byte aligned with row strides that are multiples of 8, act_out too unless M % 256 == 0;
- * required as scratch otherwise) receives gate|up for the backward pass.  act: 0 = silu, 1 = tanh-approximated gelu.  Results equal
- * olmax_gemm_bf16 followed by olmax_glu_fwd bit for bit. */
+ * W = [Wgate; Wup] ([2F, K], row stride ldw); act_out [M, F]; gu_out ([M, 2F]) receives gate|up for the
+ * backward pass.  act: 0 = silu, 1 = tanh-approximated gelu.  Results equal
+ * olmax_gemm_bf16 followed by olmax_glu_fwd bit for bit where both run on tiles of the same kernel.
+ * olmax_gemm_glu_fused: 0 where gu_out is required as scratch; otherwise it is optional (M >= 256, F % 128 == 0,
+ * K % 64 == 0, ceil(M / 256) * (F / 128) >= 128, X and W 16-byte aligned with row strides that are multiples of 8, act_out
+ * too unless M % 256 == 0): 1 where the fused kernel is the faster way, 2 where the two steps through a gu_out are. */
 int32_t olmax_gemm_glu_fused(const void* X, const void* W, const void* act_out, int32_t M, int32_t F, int32_t K,
                              int64_t ldx, int64_t ldw, int64_t ldact);
 int32_t olmax_gemm_glu_bf16(olmax_stream_t stream, const void* X, const void* W, void* gu_out, void* act_out,

@@ -1042,15 +1042,18 @@ static int pick_parts(int64_t n, int kt, int64_t bytes, float* cost) {
     if (const float c = cost_split(n, kt, s); c < *cost) *cost = c, best = s;
   return best;
 }
+// n tiles of 256, the last round's at what it costs as a round
+static float cost_rounds(int64_t n, int kt) {
+  const int64_t r = n % 256;
+  return (n / 256) * (1.52f * kt + 6.f) + (r ? (1.05f + 0.47f * r / 256.f) * kt + 6.f : 0.f);
+}
 static float cost_256(int64_t n, int kt, int64_t bytes, bool b_kc) {
   const int64_t r = n % 256;
   // (a last round that fills less than half of the CUs is cut off and runs as 128 tiles or shared reductions)
-  float last = r == 0 ? 0.f : (1.05f + 0.47f * r / 256.f) * kt + 6.f;
-  if (n > 256 && r > 0 && r < 128) {
-    last = std::min(last, cost_128(4 * r, kt, b_kc));
-    (void)pick_parts(r, kt, bytes, &last);
-  }
-  return (n / 256) * (1.52f * kt + 6.f) + last;
+  if (n <= 256 || r == 0 || r >= 128) return cost_rounds(n, kt);
+  float last = std::min(cost_rounds(r, kt), cost_128(4 * r, kt, b_kc));
+  (void)pick_parts(r, kt, bytes, &last);
+  return cost_rounds(n - r, kt) + last;
 }
 static float cost_small(int64_t n, int kt) { return ((n + 255) / 256) * (0.22f * kt + 1.2f) + 2.4f; }
 
@@ -1068,6 +1071,46 @@ static int pick_tile(int M, int N, int K, bool b_kc, bool direct_ok, int64_t byt
   if (const float c = cost_256(tiles(256), kt, bytes, b_kc); c < best) best = c, tile = 256;
   *parts = pick_parts(tiles(256), K / BK, bytes, &best);
   return *parts > 1 ? 256 : tile;
+}
+
+// Wave quantisation: with one 256x256 tile per CU per round, a last round that fills less
+// than half of the CUs (e.g. 1376 tiles = 5.375 rounds on 256 CUs) costs a whole round.
+// Such a problem is cut along M or N into a part whose tile count is a whole number of
+// rounds and a remainder that is dispatched again (and gets smaller tiles).
+struct Cut {
+  int rm = 0, cn = 0;  // largest row-tile / column-tile counts giving whole rounds, 0: none
+};
+static Cut find_cut(int tm, int tn) {
+  Cut c;
+  const int ncu = device_cu_count();
+  const int64_t tiles = (int64_t)tm * tn;
+  const int rem = (int)(tiles % ncu);
+  if (!(tiles > ncu && rem > 0 && rem * 2 < ncu)) return c;
+  for (int x = tm - 1; x > 0; x--) if (((int64_t)x * tn) % ncu == 0) { c.rm = x; break; }
+  for (int x = tn - 1; x > 0; x--) if (((int64_t)x * tm) % ncu == 0) { c.cn = x; break; }
+  return c;
+}
+
+// Whether a fused form, which runs in 256 tiles and is never cut, is worth more than the plain product X [M, K] W [N, K]^T followed by
+// elementwise passes of `passes` us; its epilogue costs `per_round` us more than the plain one's.  On whole tiles it is.  Ragged rows
+// leave up to half of a row of tiles unused, and there the plain product may have the better tiles.  us, fused | two steps, of a gated projection
+// with gate|up kept: 384 x 8192 x 2048 (M, F, K) 46 | 33, 896 x 9216 x 2304 109 | 74, 1300 x 5632 x 2048 98 | 67, 2176 x 8192 x 2048 158 | 136; 1500 x 14336 x 4096
+// 317 | 318, 5000 x 8192 x 2048 281 | 303.  Over 133 measured sizes the time lost against the better of the two, in calls: 6.5 always fused, 0.5
+// with this rule (without gate|up 4.0 and 0.4, backward form 3.0 and 0.4; rotary projection, 70 sizes, 2.1 and 0.03).
+static bool fused_wins(int M, int N, int K, float per_round, float passes) {
+  if (M % 256 == 0) return true;
+  const int kt = K / BK, tm = (M + 255) / 256, tn = N / 256;
+  const int64_t n = (int64_t)tm * tn;
+  auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * (N / t); };
+  const Cut cut = find_cut(tm, tn);
+  float plain = std::min(cost_small(tiles(64), kt), cost_128(tiles(128), kt, true));
+  plain = std::min(plain, cut.rm || cut.cn ? cost_256(n, kt, 0, true) : cost_rounds(n, kt));
+  return cost_rounds(n, kt) + per_round * ((n + 255) / 256) <= plain + passes;
+}
+enum GluForm { GLU_SAVE, GLU_ONLY, GLU_BWD };
+static bool glu_fused_wins(int M, int F, int K, GluForm form) {
+  const float e = (float)M * F;  // the elementwise passes move 6 (backward: 16) bytes an element at 5 TB/s
+  return fused_wins(M, 2 * F, K, form == GLU_SAVE ? 6.5f : form == GLU_ONLY ? 2.5f : 9.f, form == GLU_BWD ? 5.f + e * 3e-6f : 2.5f + e * 1.2e-6f);
 }
 
 // olmax_gemm_bf16 behind its argument checks.  a_padded: rows of A may be read up to the next multiple
@@ -1089,36 +1132,25 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
     if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
     if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;
   }
-  // Wave quantisation: with one 256x256 tile per CU per round, a last round that fills less
-  // than half of the CUs (e.g. 1376 tiles = 5.375 rounds on 256 CUs) costs a whole round.
-  // Such a problem is cut along M or N into a part whose tile count is a whole number of
-  // rounds and a remainder that goes through this function again (and gets smaller tiles).
   if (tile == 256 && !force_tile) {
-    const int ncu = device_cu_count();
-    const int tm = (M + 255) / 256, tn = (N + 255) / 256;
-    const int64_t tiles = (int64_t)tm * tn;
-    const int rem = (int)(tiles % ncu);
-    if (tiles > ncu && rem > 0 && rem * 2 < ncu) {
-      int rm = 0, cn = 0;  // largest row-tile / column-tile counts giving whole rounds
-      for (int x = tm - 1; x > 0; x--) if (((int64_t)x * tn) % ncu == 0) { rm = x; break; }
-      for (int x = tn - 1; x > 0; x--) if (((int64_t)x * tm) % ncu == 0) { cn = x; break; }
+    const Cut cut = find_cut((M + 255) / 256, (N + 255) / 256);
+    if (cut.rm || cut.cn) {
+      const int64_t rows = (int64_t)cut.rm * ((N + 255) / 256), cols = (int64_t)cut.cn * ((M + 255) / 256);
       const size_t esz = out_f32 ? 4 : 2;
-      if (rm > 0 && (int64_t)rm * tn >= (int64_t)cn * tm) {
-        const int m1 = rm * 256;
+      if (rows >= cols) {
+        const int m1 = cut.rm * 256;
         int rc = olmax_gemm_padded(stream, a, b, C, r, m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
         if (rc) return rc;
         const bf16* a2 = a_kc ? a + (int64_t)m1 * lda : a + m1;
         return olmax_gemm_padded(stream, a2, b, (char*)C + (int64_t)m1 * ldc * esz, r ? r + (int64_t)m1 * ldr : nullptr,
                                  M - m1, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
       }
-      if (cn > 0) {
-        const int n1 = cn * 256;
-        int rc = olmax_gemm_padded(stream, a, b, C, r, M, n1, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
-        if (rc) return rc;
-        const bf16* b2 = b_kc ? b + (int64_t)n1 * ldb : b + n1;
-        return olmax_gemm_padded(stream, a, b2, (char*)C + (int64_t)n1 * esz, r ? r + n1 : nullptr, M, N - n1, K, lda,
-                                 ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
-      }
+      const int n1 = cut.cn * 256;
+      int rc = olmax_gemm_padded(stream, a, b, C, r, M, n1, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
+      if (rc) return rc;
+      const bf16* b2 = b_kc ? b + (int64_t)n1 * ldb : b + n1;
+      return olmax_gemm_padded(stream, a, b2, (char*)C + (int64_t)n1 * esz, r ? r + n1 : nullptr, M, N - n1, K, lda,
+                               ldb, ldc, ldr, a_kc, b_kc, out_f32, a_padded, scratch);
     }
   }
   if (tile == 0) {
@@ -1194,7 +1226,7 @@ extern "C" int32_t olmax_gemm_rope_bf16(hipStream_t stream, const void* X, const
   const bool fits = aligned16(X) && aligned16(W) && aligned16(out) && aligned16(cos_t) && aligned16(sin_t) && ldx % 8 == 0 &&
                     ldw % 8 == 0 && ldo % 8 == 0 && K % BK == 0 && M >= 256 && N % 256 == 0 && rope_heads % 2 == 0 &&
                     (int64_t)((M + 255) / 256) * (N / 256) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
-  if (fits) {
+  if (fits && fused_wins(M, N, K, 4.f, 3.f + (float)M * rope_heads * 8.5e-5f)) {  // (the rotation moves 512 bytes a head at 6 TB/s)
     constexpr int SMEM = 2 * (256 + 256) * BK * 2;
     auto whole = gemm_bf16_kernel<256, 256, 128, 64, true, true, false, false, 3>;
     auto ragged = gemm_bf16_kernel<256, 256, 128, 64, true, true, false, false, 3, 1>;
@@ -1238,13 +1270,14 @@ extern "C" int32_t olmax_gemm_glu_fused(const void* X, const void* W, const void
                                         int64_t ldx, int64_t ldw, int64_t ldact) {
   const bool fits = aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && K % BK == 0 && M >= 256 && F % 128 == 0 &&
                     (int64_t)((M + 255) / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed);
-  return fits && (M % 256 == 0 || (aligned16(act_out) && ldact % 8 == 0));  // ragged rows leave through the whole-line stores only
+  if (!fits || (M % 256 && !(aligned16(act_out) && ldact % 8 == 0))) return 0;  // ragged rows leave through the whole-line stores only
+  return glu_fused_wins(M, F, K, GLU_ONLY) ? 1 : 2;
 }
 
 // Gated-MLP input projection with the activation fused into the GEMM epilogue:
 // act_out[M, F] = f(X Wgate^T) * (X Wup^T), W = [Wgate; Wup] ([2F, K], row stride ldw); gu_out
 // ([M, 2F], optional) receives gate|up for the backward pass.  Falls back to the plain GEMM
-// plus olmax_glu_fwd (through a caller-provided gu_out) when the shape does not fit the tile.
+// plus olmax_glu_fwd (through a caller-provided gu_out) when the shape does not fit the tile, or when these are faster.
 extern "C" int32_t olmax_gemm_glu_bf16(hipStream_t stream, const void* X, const void* W, void* gu_out, void* act_out,
                                        int32_t M, int32_t F, int32_t K, int64_t ldx, int64_t ldw, int64_t ldgu,
                                        int64_t ldact, int32_t act) {
@@ -1254,7 +1287,7 @@ extern "C" int32_t olmax_gemm_glu_bf16(hipStream_t stream, const void* X, const 
   OLMAX_CHECK(ldx >= K && ldw >= K && ldact >= F && (!gu_out || ldgu >= 2 * (int64_t)F), OLMAX_ERR_SHAPE,
               "olmax_gemm_glu_bf16: leading dimension smaller than row length");
   const bool gu_lines = M % 256 == 0 || !gu_out || (aligned16(gu_out) && ldgu % 8 == 0);
-  if (gu_lines && olmax_gemm_glu_fused(X, W, act_out, M, F, K, ldx, ldw, ldact)) {
+  if (gu_lines && olmax_gemm_glu_fused(X, W, act_out, M, F, K, ldx, ldw, ldact) && (!gu_out || glu_fused_wins(M, F, K, GLU_SAVE))) {
 #define GLU(E, RAG) launch_glu<E, RAG>(stream, (const bf16*)X, (const bf16*)W, (bf16*)gu_out, (bf16*)act_out, M, F, K, ldx, ldw, ldgu, ldact)
     if (act == 0) return M % 256 ? GLU(1, 1) : GLU(1, 0);
     return M % 256 ? GLU(2, 1) : GLU(2, 0);
@@ -1287,7 +1320,7 @@ extern "C" int32_t olmax_gemm_glu_bwd_bf16(hipStream_t stream, const void* X, co
                     F % 128 == 0 && (int64_t)((M + 255) / 256) * (F / 128) >= 128 && !g_force_tile.load(std::memory_order_relaxed) &&
                     aligned16(act_out) && ldact % 8 == 0 && aligned16(dgu_out) && lddgu % 8 == 0 &&
                     ((((uintptr_t)dact) & 7) == 0) && lddact % 4 == 0 && lddact < (1ll << 31);
-  if (fits) {
+  if (fits && glu_fused_wins(M, F, K, GLU_BWD)) {
 #define GLU(E, RAG)                                                                                                               \
   launch_glu<E, RAG>(stream, (const bf16*)X, (const bf16*)W, (bf16*)dgu_out, (bf16*)act_out, M, F, K, ldx, ldw, lddgu, ldact,     \
                      (const bf16*)dact, lddact)

@@ -204,8 +204,8 @@ int block_forward(hipStream_t s, const olmax_model_config* c, const olmax_block_
   }
   if (defer_mlp) return OLMAX_OK;
   // gate|up projection with the activation in the GEMM epilogue; gate|up themselves are only
-  // written when a backward pass will read them (a.gu doubles as scratch for what the fused kernel does not take)
-  const bool fused = olmax_gemm_glu_fused(mlp_in, w->wgu, a.act, (int)m.T, m.F, m.d, m.d, m.d, m.F);
+  // written when a backward pass will read them (a.gu doubles as scratch where the fused kernel does not run or is the slower way)
+  const bool fused = olmax_gemm_glu_fused(mlp_in, w->wgu, a.act, (int)m.T, m.F, m.d, m.d, m.d, m.F) == 1;
   RC(olmax_gemm_glu_bf16(s, mlp_in, w->wgu, (save_gu || !fused) ? a.gu : nullptr, a.act, (int)m.T, m.F, m.d, m.d,
                          m.d, 2 * m.F, m.F, c->act));
   if (lt == 0) {

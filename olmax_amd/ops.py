@@ -166,9 +166,12 @@ def gated_mlp_in(x, w_gate_up, act: str = "silu", gate_up_out=None, save_gate_up
                                      i64(w_gate_up.stride(0)), i64(out.stride(0)))
     if gate_up_out is None and (save_gate_up or not fits):  # (the two-step path needs them as scratch)
         gate_up_out = torch.empty(T, 2 * F, device=x.device, dtype=BF16)
-    check(_L().olmax_gemm_glu_bf16(stream_ptr(), ptr(x), ptr(w_gate_up), ptr(gate_up_out), ptr(out), i32(T), i32(F),
+    gu = gate_up_out
+    if gu is None and fits == 2:  # not needed, but the two steps are faster
+        gu = torch.empty(T, 2 * F, device=x.device, dtype=BF16)
+    check(_L().olmax_gemm_glu_bf16(stream_ptr(), ptr(x), ptr(w_gate_up), ptr(gu), ptr(out), i32(T), i32(F),
                                    i32(d), i64(x.stride(0)), i64(w_gate_up.stride(0)),
-                                   i64(0 if gate_up_out is None else gate_up_out.stride(0)), i64(out.stride(0)),
+                                   i64(0 if gu is None else gu.stride(0)), i64(out.stride(0)),
                                    i32(_ACT[act])))
     return out, gate_up_out
 

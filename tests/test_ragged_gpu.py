@@ -127,6 +127,35 @@ def test_gated_projection_on_ragged_rows_of_unaligned_views(which):
     assert rel(got, want) < 2 ** -8
 
 
+@pytest.mark.parametrize("T,F,d", [(384, 8192, 512), (300, 8192, 576), (900, 9216, 768)])
+def test_gated_projection_of_few_ragged_rows_takes_two_steps(T, F, d):
+    """Where that is faster; the rows of a whole number of 256 take the fused kernel.  fp32 orders before bf16 roundings."""
+    from olmax_amd import _lib, ops
+    print(f"[case] gated projection in two steps T{T} F{F} d{d}", flush=True)
+    whole = -(-T // 256) * 256
+    x, w, dact = rnd(whole, d, seed=1), rnd(2 * F, d, seed=2, scale=d ** -0.5), rnd(whole, F, seed=3)
+    args = lambda t: (*map(_lib.ptr, (x, w, dact)), *map(_lib.i32, (t, F, d)), *map(_lib.i64, (d, d, F)))  # noqa: E731
+    assert _lib.load().olmax_gemm_glu_fused(*args(T)) == 2 and _lib.load().olmax_gemm_glu_fused(*args(whole)) == 1
+    want, want_gu = ops.gated_mlp_in(x, w)
+    got, got_gu = ops.gated_mlp_in(x[:T], w)
+    only, none = ops.gated_mlp_in(x[:T], w, save_gate_up=False)
+    assert rel(got, want[:T]) < 2 ** -8 and rel(got_gu, want_gu[:T]) < 2 ** -8 and torch.equal(only, got) and none is None
+    want, want_dgu = ops.gated_mlp_in_bwd(x, w, dact)
+    got, got_dgu = ops.gated_mlp_in_bwd(x[:T], w, dact[:T])
+    assert rel(got, want[:T]) < 2 ** -8 and rel(got_dgu, want_dgu[:T]) < 2 ** -8
+
+
+def test_rotary_projection_of_few_ragged_rows_takes_two_steps():
+    from olmax_amd import ops
+    print("[case] rope projection in two steps", flush=True)
+    T, heads, N, d = 640, 64, 12288, 512
+    x, w = rnd(768, d, seed=1), rnd(N, d, seed=2, scale=d ** -0.5)
+    cos, sin = ops.rope_tables(768, 128, 10000.0, "cuda")
+    want = ops.qkv_rope_proj(x, w, cos, sin, rope_heads=heads, seq_len=768)
+    got = ops.qkv_rope_proj(x[:T], w, cos, sin, rope_heads=heads, seq_len=768)
+    assert rel(got, want[:T]) < 2 ** -8
+
+
 @pytest.mark.parametrize("T,which,tile", [(2048, "x", 0), (2048, "w", 0), (2048, "out", 0), (2048, "none", 256), (2049, "none", 128)])
 def test_gated_projection_gets_scratch_wherever_the_fused_kernel_does_not_run(T, which, tile):
     """Unaligned operands at whole tiles, and a forced tile size; the result differs by fp32 orders before bf16 roundings."""
