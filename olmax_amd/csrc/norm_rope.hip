@@ -632,24 +632,26 @@ extern "C" int32_t olmax_rmsnorm_bwd(hipStream_t stream, const void* x, const vo
   const bf16 *xp = (const bf16*)x, *wp = (const bf16*)w, *dyp = (const bf16*)dy, *drp = (const bf16*)dres;
   bf16* dxp = (bf16*)dx;
   // SLOTS rows in flight per block of THREADS; the LDS row of each (64 KB at most) holds its column sums
-#define OLMAX_NORM_BWD(SLOTS, THREADS, ...)                                                                                       \
+#define OLMAX_NORM_BWD(SLOTS, THREADS, CAP, ...)                                                                                     \
   do {                                                                                                                            \
     auto kern = __VA_ARGS__;                                                                                                      \
     static std::once_flag once;                                                                                                   \
     std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 65536); }); \
-    hipLaunchKernelGGL(kern, dim3(grid_for(rows, SLOTS, 256)), dim3(THREADS), dw ? (size_t)SLOTS * d * 4 : 0, stream, xp, wp, dyp, drp, \
+    hipLaunchKernelGGL(kern, dim3(grid_for(rows, SLOTS, CAP)), dim3(THREADS), dw ? (size_t)SLOTS * d * 4 : 0, stream, xp, wp, dyp, drp, \
                        dxp, dw, rows, d, ldx, lddy, lddres, lddx, eps);                                                           \
   } while (0)
   if (vec && d % 8 == 0 && d <= 256) {
-    OLMAX_NORM_BWD(16, 256, rmsnorm_bwd_kernel<16, 2, 256>);
+    OLMAX_NORM_BWD(16, 256, 256, rmsnorm_bwd_kernel<16, 2, 256>);
   } else if (vec && d % 8 == 0 && d <= 1024) {
-    OLMAX_NORM_BWD(16, 1024, rmsnorm_bwd_split_kernel<1, 2, 1024>);
+    // without dw nothing has to meet: small workgroups start sooner (512 x 512: 4.0 -> 3.2 us) and do as well on many rows
+    if (dw) OLMAX_NORM_BWD(16, 1024, 256, rmsnorm_bwd_split_kernel<1, 2, 1024>);
+    else OLMAX_NORM_BWD(4, 256, 1024, rmsnorm_bwd_split_kernel<1, 2, 256>);
   } else if (vec && d % 8 == 0 && d <= 2048) {
-    OLMAX_NORM_BWD(8, 1024, rmsnorm_bwd_split_kernel<2, 2, 1024>);
+    OLMAX_NORM_BWD(8, 1024, 256, rmsnorm_bwd_split_kernel<2, 2, 1024>);
   } else if (vec && d % 8 == 0 && d <= 4096) {
-    OLMAX_NORM_BWD(4, 1024, rmsnorm_bwd_split_kernel<4, 2, 1024>);
+    OLMAX_NORM_BWD(4, 1024, 256, rmsnorm_bwd_split_kernel<4, 2, 1024>);
   } else if (vec && d % 8 == 0 && d <= 8192) {
-    OLMAX_NORM_BWD(2, 1024, rmsnorm_bwd_split_kernel<8, 2, 1024>);
+    OLMAX_NORM_BWD(2, 1024, 256, rmsnorm_bwd_split_kernel<8, 2, 1024>);
   } else {
     hipLaunchKernelGGL(rmsnorm_bwd_generic, dim3(grid_for(rows, 1, 1 << 16)), dim3(256), 0, stream, xp, wp, dyp, drp, dxp, dw, rows, d, ldx, lddy, lddres, lddx, eps);
   }
