@@ -421,7 +421,7 @@ __global__ __launch_bounds__(NORM ? 1024 : 256) void qk_rope_bwd_kernel(
     const int h = (int)(unit - tok * heads);
     const int pos = small ? (int)((uint32_t)tok % (uint32_t)seq_len) : (int)(tok % seq_len);
     const Pack8 c = next_dy, xv = next_x;
-    if (unit + step < units) fetch(unit + step, next_tok = token_of(unit + step));  // under way while this row is worked on
+    if (NORM && unit + step < units) fetch(unit + step, next_tok = token_of(unit + step));  // under way while this row is worked on
     const int fi = (sub & (LPR / 2 - 1)) * 8;
     const float sign = sub < LPR / 2 ? 1.f : -1.f;
     float g[8];
@@ -462,6 +462,7 @@ __global__ __launch_bounds__(NORM ? 1024 : 256) void qk_rope_bwd_kernel(
       for (int e = 0; e < 8; e++) o.e[e] = f2bf(g[e]);
     }
     *reinterpret_cast<u32x4*>(dx + tok * lddx + h * D + sub * 8) = o.u;
+    if (!NORM) break;  // (its grid has a row for every group of lanes)
   }
   if (NORM) {
     __shared__ __attribute__((aligned(16))) float sdw[THREADS / 64][D];
