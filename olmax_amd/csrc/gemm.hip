@@ -927,7 +927,7 @@ int launch_split(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf1
     (void)hipEventRecord(rec.e1, s);
     rec.flops = 2.0 * M * N * K;
     rec.bytes = 2.0 * ((double)M * K + (double)N * K + (double)M * N * (R ? 2 : 1) * (out_f32 ? 2 : 1));
-    rec.key = 256 | (A_KC << 12) | (B_KC << 13) | ((R != nullptr) << 14) | (out_f32 << 15);
+    rec.key = 256 | (A_KC << 12) | (B_KC << 13) | ((R != nullptr) << 14) | (out_f32 << 15) | (1 << 18);
     rec.M = M; rec.N = N; rec.K = K;
     std::lock_guard<std::mutex> lk(g_prof_mu);
     g_prof.push_back(rec);
@@ -949,8 +949,8 @@ extern "C" void olmax_gemm_profile_begin(void) {
 }
 // Stop recording, wait for the recorded events and aggregate per kernel instantiation.
 // keys/ms/flops/launches: host arrays of `cap` entries; returns the number of distinct keys.
-// key = tile (64: gemm_small_kernel) | a_layout<<12 | b_layout<<13 | has_residual<<14 | out_f32<<15 | glu_epilogue<<16 | rope_epilogue<<17,
-// with a_layout / b_layout bit SET when the operand is reduction-contiguous.  flops / bytes:
+// key = tile (64: gemm_small_kernel) | a_layout<<12 | b_layout<<13 | has_residual<<14 | out_f32<<15 | glu_epilogue<<16 | rope_epilogue<<17 |
+// shared_reduction<<18, with a_layout / b_layout bit SET when the operand is reduction-contiguous.  flops / bytes:
 // algorithmic totals (2MNK; every operand and the result moved once).
 extern "C" int32_t olmax_gemm_profile_end(int32_t* keys, double* ms, double* flops, double* bytes, int64_t* launches,
                                           int32_t cap) {
