@@ -310,7 +310,8 @@ __device__ __forceinline__ void adamw_one(float* __restrict__ p, const void* __r
 // 240-register GEMM waves when it runs on a second stream, and it is launched as a small
 // grid-stride grid (two workgroups per CU): the whole grid then sweeps five arrays as
 // contiguous 2 MB fronts, which measured 5.6 TB/s against 4.7 TB/s for one workgroup per 8 KB.  The scalar bases of adamw_vec
-// bring the width-1024 step from 7490 to 7226 us and two layers of the 7B step from 45.0 to 43.1 ms.
+// bring the width-1024 step from 7490 to 7226 us; two layers of the 7B step move by less than boxes differ (everything since the ragged GEMM forms
+// came, together: 44.6 -> 43.3 and 44.7 -> 43.6 ms).
 template <bool G_BF16>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(16))) void adamw_kernel(
     float* __restrict__ p, const void* __restrict__ gv, float* __restrict__ m, float* __restrict__ v,
