@@ -1151,12 +1151,16 @@ void bwd_fast_attributes() {
 // head_dim 64 (split: 64 queries to a workgroup, twice as many of them), n <= 128: 1 tile 5.0 -> 6.2 | 1.6 slower, 2 tiles 7.2 -> 6.9 | 0.2 faster,
 // 8 tiles 12.3 -> 8.9 | 5.1 faster; n = 192: 3 tiles 7.2 -> 11.3 | 6 slower; n = 256: 8 tiles 1.5 slower | 1.5 slower, 16 tiles 19.0 -> 16.9 | 4.4
 // faster; n = 320, 24 tiles 0.9 faster | 0.4 faster; n = 384, 32 tiles 0.5 slower | 3.9 faster; n = 480, 24 tiles 27.3 -> 36.5 | 9.7 slower.
+// A window of half the sequence or less makes the chains equal, and with nothing short to start late a second round costs all of one: n = 312, 18
+// tiles 32.7 -> 43.6 | 5 slower, n = 288, 34 tiles 56 -> 46 | 15 faster, n = 384, 34 tiles 63 -> 73; head_dim 64, n = 192, 18 tiles 23 -> 24, n = 224, 26 tiles 33 -> 28.
+bool even_chains(int S, int window) { return window >= 0 && window <= S / 2; }
 template <int D>
 bool q_split(int B, int S, int H, int window) {
   const int64_t n = (int64_t)((S + 127) / 128) * H * B;
   const int tiles = (window >= 0 && window < S - 128 ? window + 128 : S + 63) / 64;
-  if (D == 128) return n <= 512 && tiles >= (n <= 256 ? 6 : 12 + 14 * (n - 256) / 256);
-  return n <= 384 && tiles >= (n <= 128 ? 2 : n <= 256 ? 12 : n / 12);
+  const bool even = even_chains(S, window);
+  if (D == 128) return n <= 256 ? tiles >= 6 : even ? n <= 300 && tiles >= 26 : n <= 512 && tiles >= 12 + 14 * (n - 256) / 256;
+  return n <= 128 ? tiles >= 2 : n <= 256 ? tiles >= (even ? 26 : 12) : !even && n <= 384 && tiles >= n / 12;
 }
 // Whether dK/dV takes the split kernel.  One workgroup per key tile and K/V head is little parallel work when the
 // heads are few: 224 workgroups for 2 x 1777 tokens of 8 K/V heads leave the GPU waiting for those of the first key tile,
@@ -1169,13 +1173,15 @@ bool q_split(int B, int S, int H, int window) {
 // head_dim 64: n <= 128: 2 tiles as many, 3 tiles 16.4 -> 14.4, 4 tiles 19.1 -> 15.2; n = 192: 3 tiles 17 -> 19, 5 tiles 21 -> 20; n = 320: 8 tiles 33.0 -> 33.5,
 // 16 tiles 53 -> 50; n = 448: 4 tiles 28.6 -> 36.8, 32 tiles as many; n = 512: 32 tiles 70.2 -> 71.4, 48 tiles 107 -> 102; n = 544: 128 tiles 241 -> 217; n = 640:
 // 128 tiles 237 -> 235, 256 tiles 434 -> 410; n = 768: 256 tiles 459 -> 477.
+// Equal chains (see above), head_dim 128: n = 192: 12 tiles 53 -> 54, 20 tiles 71 -> 70, 52 tiles 145 -> 134; n = 384: 36 tiles 130 -> 135, 72 tiles 237 -> 236, 97 tiles 271 -> 260;
+// n = 448: 97 tiles 294 -> 306, 272 tiles 742 -> 755; head_dim 64: n = 288: 20 tiles 57 -> 58, 28 tiles 68 -> 66; n = 384: 36 tiles as many, 68 tiles 138 -> 135; n = 512: 97 tiles 196 -> 197.
 template <int D>
 bool dkv_split(int B, int S, int H, int KH, int window) {
   const int64_t n = (int64_t)((S + 127) / 128) * KH * B;
   const int64_t chain = (int64_t)(H / KH) * (((window >= 0 && window < S - 128 ? window + 128 : S) + 31) / 32);
-  if (n > 640) return false;
-  if (n > 512) return chain >= (D == 128 ? 200 : 128);
   if (n <= 128) return chain >= 3;
+  if (even_chains(S, window)) return n <= 384 && chain >= (D == 128 ? (n <= 256 ? 20 : 60) : n <= 256 ? 4 : 20 + (n - 256) / 4);
+  if (n > 512) return n <= 640 && chain >= (D == 128 ? 200 : 128);
   const int base = D == 128 ? 8 : 4;
   return chain >= (n <= 256 ? base : base + (D == 128 ? 56 : 36) * (n - 256) / 256);
 }
