@@ -7,10 +7,12 @@
 //
 // One block owns one row of logits.  bf16 rows of up to 163840 entries are loaded ONCE into the
 // block's registers (128-bit loads), reduced to max and sum-exp, and written back as
-// d logits = (softmax - onehot) * dloss / n_counted from the registers; longer or fp32 rows take
+// d logits = (softmax - onehot) * dloss / n_counted from the registers; longer ones keep 131072 entries
+// there and read the rest again; soft-capped longer and fp32 rows take
 // the streaming form (online max / sum-exp in pass 1, a second read of the row in pass 2).
 // Optional final-logit soft-cap z = c*tanh(x/c) is applied on the fly in both passes.
 #include "common.h"
+#include <type_traits>
 
 namespace {
 
@@ -69,14 +71,15 @@ template <> struct Io<float> {
   static __device__ __forceinline__ void st1(float* p, float f) { *p = f; }
 };
 
-template <typename T, bool CAP>
-__global__ __launch_bounds__(256) void ce_row_kernel(
+template <typename T, bool CAP, int THREADS>
+__global__ __launch_bounds__(THREADS) void ce_row_kernel(
     const T* __restrict__ logits, T* __restrict__ dlogits, const int32_t* __restrict__ labels,
     float* __restrict__ row_loss, float* __restrict__ lse_out, const int32_t* __restrict__ n_counted,
     int64_t rows, int V, int64_t ld, int64_t ldd, int32_t ignore_index, float cap, float dloss,
     int vec_ok, const float* __restrict__ drow, int mean, int pad) {
   constexpr int VEC = Io<T>::VEC;
-  __shared__ float red[4];
+  constexpr int NW = THREADS / 64;
+  __shared__ float red[NW];
   __shared__ float label_logit;
   const int64_t row = blockIdx.x;
   const T* zr = logits + row * ld;
@@ -98,7 +101,7 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
   // ---- pass 1: online max / sum-exp ----
   float mx = -INFINITY, sm = 0.f;
   const int nvec = vec_ok ? V / VEC : 0;
-  for (int i = threadIdx.x; i < nvec; i += 256) {
+  for (int i = threadIdx.x; i < nvec; i += THREADS) {
     float f[VEC];
     Io<T>::load(zr + i * VEC, f);
     float cm = -INFINITY;
@@ -114,7 +117,7 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
 #pragma unroll
     for (int e = 0; e < VEC; e++) sm += __expf(f[e] - mx);
   }
-  for (int i = nvec * VEC + threadIdx.x; i < V; i += 256) {
+  for (int i = nvec * VEC + threadIdx.x; i < V; i += THREADS) {
     float f = Io<T>::ld1(zr + i);
     if (CAP) f = cap * fast_tanh(f * inv_cap);
     if (f > mx) {
@@ -123,9 +126,9 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
     }
     sm += __expf(f - mx);
   }
-  const float gmx = block_max<4>(mx, red);
+  const float gmx = block_max<NW>(mx, red);
   sm = (mx == -INFINITY) ? 0.f : sm * __expf(mx - gmx);
-  const float gsm = block_sum<4>(sm, red);
+  const float gsm = block_sum<NW>(sm, red);
   const float lse = gmx + __logf(gsm);
   if (threadIdx.x == 0) {
     row_loss[row] = (counted && inrange) ? (lse - label_logit) : 0.f;
@@ -136,7 +139,7 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
   T* dr = dlogits + row * ldd;
   // d(reduced loss) / d(row loss): 1/n for "mean", 1 for "sum", the row's own cotangent for "none"
   const float scale = (counted && inrange) ? dloss * (drow ? drow[row] : 1.f) / (mean ? (float)(*n_counted) : 1.f) : 0.f;
-  for (int i = threadIdx.x; i < nvec; i += 256) {
+  for (int i = threadIdx.x; i < nvec; i += THREADS) {
     float f[VEC];
     Io<T>::load(zr + i * VEC, f);
 #pragma unroll
@@ -153,7 +156,7 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
     }
     Io<T>::store(dr + i * VEC, f);
   }
-  for (int i = nvec * VEC + threadIdx.x; i < V; i += 256) {
+  for (int i = nvec * VEC + threadIdx.x; i < V; i += THREADS) {
     float z = Io<T>::ld1(zr + i), chain = 1.f;
     if (CAP) {
       const float t = fast_tanh(z * inv_cap);
@@ -164,21 +167,30 @@ __global__ __launch_bounds__(256) void ce_row_kernel(
     if (i == label) p -= 1.f;
     Io<T>::st1(dr + i, p * scale * chain);
   }
-  for (int i = V + threadIdx.x; i < V + pad; i += 256) Io<T>::st1(dr + i, 0.f);
+  for (int i = V + threadIdx.x; i < V + pad; i += THREADS) Io<T>::st1(dr + i, 0.f);
 }
 
-// The same row computation for bf16 rows short enough to keep in registers between the two
-// passes (THREADS x MAXV vectors of 8): the logits are read from memory once and the gradient
+// The same row computation for bf16 rows kept in registers between the two passes (THREADS x MAXV
+// vectors of 8): the logits are read from memory once and the gradient
 // written once, 4 B per logit instead of 6.  Max and sum-exp are two plain block reductions (no
 // online rescaling needed when the whole row is at hand).  PAD: V is not a multiple of 8 and the rows
 // have room up to the next one; those logits are left out and their gradient is written as zero.
-template <bool CAP, int THREADS, int MAXV, bool PAD>
-__global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
+// TAIL: a longer row; what the registers do not hold is reduced online and read a second time, right after
+// (4096 x 262144: 1.26 ms all read twice by 4 waves, 1.10 by 16, 1.04 with half of the row held).
+//
+// Bound by memory (8192 x 50304: 1.65 GB in 320 us = 5.1 TB/s) as long as the vector instructions stay below it,
+// about 12 a logit: the maximum is taken of raw values, missing logits are minus infinity instead of a test in each pass,
+// only the one vector that holds the label looks for it, and the gradient's exponential is one fma and exp2.
+template <bool CAP, int THREADS, int MAXV, bool PAD, bool TAIL>
+__global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
     const bf16* __restrict__ logits, bf16* __restrict__ dlogits, const int32_t* __restrict__ labels,
     float* __restrict__ row_loss, float* __restrict__ lse_out, const int32_t* __restrict__ n_counted,
     int V, int64_t ld, int64_t ldd, int32_t ignore_index, float cap, float dloss,
     const float* __restrict__ drow, int mean) {
   constexpr int NW = THREADS / 64;
+  constexpr int HELD = MAXV * THREADS;  // vectors in registers
+  constexpr uint32_t NEG_INF2 = 0xff80ff80u;
+  constexpr float LOG2E = 1.4426950408889634f;
   __shared__ float red[NW];
   __shared__ float label_logit;
   const int64_t row = blockIdx.x;
@@ -198,33 +210,84 @@ __global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
     }
     label_logit = zl;
   }
-  Pack8 c[MAXV];
+  // a vector of the row; logits that do not exist are minus infinity: nothing to the maximum, nothing to the sum
+  auto fetch = [&](int idx) {
+    Pack8 v;
+    v.u = u32x4{NEG_INF2, NEG_INF2, NEG_INF2, NEG_INF2};
+    if (idx < nvec) {
+      v.u = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(zr) + idx);
+      if (PAD && idx == nvec - 1) {
 #pragma unroll
-  for (int i = 0; i < MAXV; i++) {
-    const int idx = i * THREADS + threadIdx.x;
-    if (idx < nvec) c[i].u = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(zr) + idx);
-  }
+        for (int e = 1; e < 8; e++)
+          if (idx * 8 + e >= V) v.u[e >> 1] = e & 1 ? (v.u[e >> 1] & 0xffffu) | (NEG_INF2 & 0xffff0000u) : NEG_INF2;
+      }
+    }
+    return v;
+  };
+  // the soft-cap t = tanh(z / cap) with its factors in one multiply; it takes minus infinity to -cap, so under
+  // it the logits that do not exist are left out by their index (exists)
+  const float cap_k = CAP ? 2.f * LOG2E * inv_cap : 0.f;
+  auto soft = [&](float f) { return 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(f * cap_k) + 1.f); };
   auto value = [&](bf16 x) {
     const float f = bf2f(x);
-    return CAP ? cap * fast_tanh(f * inv_cap) : f;
+    return CAP ? cap * soft(f) : f;
   };
-  float mx = -INFINITY;
+  auto exists = [&](int idx, int e) { return !CAP || !PAD || idx * 8 + e < V; };
+  // exponentials of a vector against ref, added in pairs
+  auto exps = [&](const Pack8& v, int idx, float ref) {
+    float x[8];
 #pragma unroll
-  for (int i = 0; i < MAXV; i++)
-    if (i * THREADS + threadIdx.x < nvec) {
+    for (int e = 0; e < 8; e++) x[e] = exists(idx, e) ? __expf(value(v.e[e]) - ref) : 0.f;
+    return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+  };
+  Pack8 c[MAXV];
 #pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (!PAD || (i * THREADS + (int)threadIdx.x) * 8 + e < V) mx = fmaxf(mx, value(c[i].e[e]));
+  for (int i = 0; i < MAXV; i++) c[i] = fetch(i * THREADS + threadIdx.x);
+  float mx = -INFINITY, tsm = 0.f;
+  if (TAIL) {
+    constexpr int U = 4;
+    for (int i0 = HELD + threadIdx.x; i0 < nvec; i0 += U * THREADS) {
+      Pack8 t[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) t[u] = fetch(i0 + u * THREADS);
+      float cm = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) cm = fmaxf(cm, bf2f(t[u].e[e]));
+      if (CAP) cm = cap * soft(cm);
+      if (cm > mx) {
+        tsm *= __expf(mx - cm);
+        mx = cm;
+      }
+      const float ref = mx == -INFINITY ? 0.f : mx;  // nothing but minus infinity so far: the sum stays 0
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (!CAP || i0 + u * THREADS < nvec) tsm += exps(t[u], i0 + u * THREADS, ref);
     }
+  }
+  const float tmx = mx;
+  float rmx = -INFINITY;  // of the raw logits: the soft-cap rises with them
+  // each pass unpacks a vector when its turn comes: hidden from the compiler, which otherwise keeps all
+  // unpacked logits of a pass for the next and spills
+  auto keep = [](Pack8& v) {
+    asm volatile("" : "+v"(v.u));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int i = 0; i < MAXV; i++) {
+    keep(c[i]);
+#pragma unroll
+    for (int e = 0; e < 8; e++) rmx = fmaxf(rmx, bf2f(c[i].e[e]));
+  }
+  mx = fmaxf(mx, CAP ? cap * soft(rmx) : rmx);
   const float gmx = block_max<NW>(mx, red);
-  float sm = 0.f;
+  float sm = TAIL ? (tmx == -INFINITY ? tsm : tsm * __expf(tmx - gmx)) : 0.f;
 #pragma unroll
-  for (int i = 0; i < MAXV; i++)
-    if (i * THREADS + threadIdx.x < nvec) {
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (!PAD || (i * THREADS + (int)threadIdx.x) * 8 + e < V) sm += __expf(value(c[i].e[e]) - gmx);
-    }
+  for (int i = 0; i < MAXV; i++) {
+    keep(c[i]);
+    if (!CAP || i * THREADS + threadIdx.x < nvec) sm += exps(c[i], i * THREADS + threadIdx.x, gmx);
+  }
   const float gsm = block_sum<NW>(sm, red);
   const float lse = gmx + __logf(gsm);
   if (threadIdx.x == 0) {
@@ -235,25 +298,49 @@ __global__ __launch_bounds__(THREADS) void ce_row_regs_kernel(
   bf16* dr = dlogits + row * ldd;
   // d(reduced loss) / d(row loss): 1/n for "mean", 1 for "sum", the row's own cotangent for "none"
   const float scale = (counted && inrange) ? dloss * (drow ? drow[row] : 1.f) / (mean ? (float)(*n_counted) : 1.f) : 0.f;
-#pragma unroll
-  for (int i = 0; i < MAXV; i++) {
-    const int idx = i * THREADS + threadIdx.x;
-    if (idx < nvec) {
-      Pack8 o;
+  const float lse2 = lse * LOG2E;
+  auto store = [&](int idx, const Pack8& v) {
+    Pack8 o;
+    auto grads = [&](auto has_label) {
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        float z = bf2f(c[i].e[e]), chain = 1.f;
+        float z = bf2f(v.e[e]), chain = 1.f;
         if (CAP) {
-          const float t = fast_tanh(z * inv_cap);
+          const float t = soft(z);
           z = cap * t;
           chain = 1.f - t * t;
         }
-        float p = __expf(z - lse);
-        if (idx * 8 + e == label) p -= 1.f;
-        o.e[e] = f2bf(!PAD || idx * 8 + e < V ? p * scale * chain : 0.f);
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(z, LOG2E, -lse2));
+        if (has_label && idx * 8 + e == label) p -= 1.f;
+        o.e[e] = f2bf(p * scale * chain);
       }
-      *(reinterpret_cast<u32x4*>(dr) + idx) = o.u;
+    };
+    if (idx == label >> 3) grads(std::true_type());
+    else grads(std::false_type());
+    if (PAD && idx == nvec - 1) {
+#pragma unroll
+      for (int e = 1; e < 8; e++)
+        if (idx * 8 + e >= V) o.e[e] = f2bf(0.f);
     }
+    *(reinterpret_cast<u32x4*>(dr) + idx) = o.u;
+  };
+  if (TAIL) {  // what was read last first
+    constexpr int U = 4;
+    for (int i0 = HELD + (nvec - HELD - 1 - (int)threadIdx.x) / (U * THREADS) * (U * THREADS) + (int)threadIdx.x; i0 >= HELD; i0 -= U * THREADS) {
+      Pack8 t[U];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (i0 + u * THREADS < nvec) t[u].u = *(reinterpret_cast<const u32x4*>(zr) + i0 + u * THREADS);
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (i0 + u * THREADS < nvec) store(i0 + u * THREADS, t[u]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MAXV; i++) {
+    const int idx = i * THREADS + threadIdx.x;
+    keep(c[i]);
+    if (idx < nvec) store(idx, c[i]);
   }
 }
 
@@ -297,27 +384,40 @@ static int cross_entropy(hipStream_t stream, const void* logits, void* dlogits, 
   const int vec_ok = aligned16(logits) && (!dlogits || aligned16(dlogits)) && ld % vecw == 0 && (!dlogits || ldd % vecw == 0);
   const bool cap = softcap > 0.f;
   dim3 grid((unsigned)T);
-#define CE_GO(TY, CAPV)                                                                          \
-  hipLaunchKernelGGL((ce_row_kernel<TY, CAPV>), grid, dim3(256), 0, stream, (const TY*)logits,   \
+#define CE_GO(TY, CAPV, TH)                                                                      \
+  hipLaunchKernelGGL((ce_row_kernel<TY, CAPV, TH>), grid, dim3(TH), 0, stream, (const TY*)logits, \
                      (TY*)dlogits, labels, row_loss, lse_out, n_counted, T, V, ld, ldd,          \
                      ignore_index, softcap, dloss, vec_ok, dloss_rows, mean, padded ? (8 - V % 8) % 8 : 0)
-#define CE_REGS_P(CAPV, TH, MV, PADV)                                                                          \
-  hipLaunchKernelGGL((ce_row_regs_kernel<CAPV, TH, MV, PADV>), grid, dim3(TH), 0, stream, (const bf16*)logits, \
+#define CE_REGS_P(CAPV, TH, MV, PADV, TAILV)                                                                          \
+  hipLaunchKernelGGL((ce_row_regs_kernel<CAPV, TH, MV, PADV, TAILV>), grid, dim3(TH), 0, stream, (const bf16*)logits, \
                      (bf16*)dlogits, labels, row_loss, lse_out, n_counted, V, ld, ldd, ignore_index, softcap, dloss, dloss_rows, mean)
-#define CE_REGS(CAPV, TH, MV)                                                                                  \
-  do { if (V % 8) CE_REGS_P(CAPV, TH, MV, true); else CE_REGS_P(CAPV, TH, MV, false); } while (0)
+#define CE_REGS_T(CAPV, TH, MV, TAILV)                                                                         \
+  do { if (V % 8) CE_REGS_P(CAPV, TH, MV, true, TAILV); else CE_REGS_P(CAPV, TH, MV, false, TAILV); } while (0)
+#define CE_REGS(TH, MV) do { if (cap) CE_REGS_T(true, TH, MV, false); else CE_REGS_T(false, TH, MV, false); } while (0)
   const bool regs_ok = !logits_f32 && vec_ok && (V % 8 == 0 || padded);
   if (logits_f32) {
-    if (cap) CE_GO(float, true); else CE_GO(float, false);
-  } else if (regs_ok && V <= 512 * 8 * 26) {  // up to 106496 logits: 8 waves holding 26 vectors each
-    if (cap) CE_REGS(true, 512, 26); else CE_REGS(false, 512, 26);
-  } else if (regs_ok && V <= 1024 * 8 * 20) {  // up to 163840 logits: 16 waves holding 20 vectors each (128 registers per lane)
-    if (cap) CE_REGS(true, 1024, 20); else CE_REGS(false, 1024, 20);
+    if (cap) CE_GO(float, true, 256); else CE_GO(float, false, 256);
+  } else if (regs_ok && V <= 1024 * 8 * 20) {
+    // The fewest threads that hold the row, so that as many rows as possible are on a CU in different phases: us with the
+    // workgroup below | the one of 512 threads x 26 vectors (1024 x 20) that held all rows: 2048 x 4096 20 | 46, 1500 x 16384 27 | 51, 8192 x 50304 320 | 425,
+    // 8192 x 100352 680 | 740, 4096 x 128256 424 | 493 (the last two only from the arithmetic)
+    if (V <= 256 * 8 * 2) CE_REGS(256, 2);
+    else if (V <= 256 * 8 * 8) CE_REGS(256, 8);
+    else if (V <= 256 * 8 * 25) CE_REGS(256, 25);
+    else if (V <= 512 * 8 * 25) CE_REGS(512, 25);
+    else CE_REGS(1024, 20);
+  } else if (regs_ok && !cap) {
+    CE_REGS_T(false, 1024, 16, true);
+  } else if (V > 1024 * 8 * 20) {
+    // rows of half a megabyte: a whole GPU of 16-wave workgroups has 134 to 268 MB of them in flight, which the memory-side
+    // cache still holds for the second pass (8192 x 256000, soft-cap: 2.55 ms with 4 waves, 2.34 with 16)
+    if (cap) CE_GO(bf16, true, 1024); else CE_GO(bf16, false, 1024);
   } else {
-    if (cap) CE_GO(bf16, true); else CE_GO(bf16, false);
+    if (cap) CE_GO(bf16, true, 256); else CE_GO(bf16, false, 256);
   }
 #undef CE_GO
 #undef CE_REGS
+#undef CE_REGS_T
 #undef CE_REGS_P
   if (reduction != 2) hipLaunchKernelGGL(ce_finalize_kernel, dim3(1), dim3(1024), 0, stream, row_loss, T, n_counted, loss, mean);
   OLMAX_LAUNCH_CHECK();

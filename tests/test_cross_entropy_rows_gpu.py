@@ -1,0 +1,51 @@
+"""GPU parity tests of the cross entropy at the row lengths where its kernels change, at the ends of their vectors."""
+import pytest
+import torch
+
+from oracle import ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("V", [8, 4096, 4104, 16384, 16392, 51200, 51208, 102400, 102408, 163840, 163848, 163840 + 8 * 4096 + 8])
+@pytest.mark.parametrize("cap", [0.0, 20.0])
+def test_row_lengths(V, cap):
+    """Gradients are rounded to bf16 once: 2^-9 of the value, and fp32 exponentials of |z - lse| < 40 in front of it: 40 * 2^-23.
+    Rows with whole vectors of minus infinity (a masked vocabulary) and with the label at either end are among them."""
+    from olmax_amd import ops
+    print(f"[case] ce rows V{V} cap{cap}", flush=True)
+    g = torch.Generator().manual_seed(V)
+    z = (torch.randn(6, V, generator=g) * 3).to(torch.bfloat16)
+    if V > 64:
+        z[3, : V // 2 // 8 * 8] = float("-inf")
+        z[4, V // 2 // 8 * 8:] = float("-inf")
+    labels = torch.tensor([0, V - 1, V // 2, V - 1, 0, -100], dtype=torch.int32)
+    want = ref.cross_entropy_bwd(z.double(), labels.long(), softcap=cap)
+    loss, lse = ref.cross_entropy_fwd(z.double(), labels.long(), softcap=cap)[:2]
+    for inplace in (False, True):
+        got = ops.cross_entropy(z.cuda(), labels.cuda(), softcap=cap, inplace=inplace)
+        assert abs(got[0].item() - loss.item()) < 1e-5 * abs(loss.item())
+        assert ((got[2].cpu().double() - lse)[:5].abs() < 1e-6 * lse[:5].abs() + 1e-6).all()
+        # near the label and under the soft-cap 1 - p and 1 - t^2 cancel: 2^-22 of the row's scale 1/5
+        err = (got[1].cpu().double() - want).abs() - (2 ** -8 * want.abs() + 2 ** -22 / 5)
+        assert err.max().item() <= 0, (err.argmax().item() // V, err.argmax().item() % V)
+
+
+@pytest.mark.parametrize("V", [4091, 16379, 51199, 102397, 163835, 163843])
+@pytest.mark.parametrize("cap", [0.0, 20.0])
+def test_padded_rows(V, cap):
+    """The LM head's own logits, rows padded to whole vectors.  A row of one token's dW is its dlogits times h: relative error of two
+    bf16 roundings, 2^-8, on top of the logits' own, 2^-9 of |z| < 8 in the exponent."""
+    from olmax_amd import ops
+    print(f"[case] ce padded V{V} cap{cap}", flush=True)
+    g = torch.Generator().manual_seed(V)
+    h = torch.randn(2, 64, generator=g).to(torch.bfloat16)
+    W = (torch.randn(V, 64, generator=g) * 0.1).to(torch.bfloat16)
+    labels = torch.tensor([V - 1, V - 2], dtype=torch.int32)
+    loss, dh, dW = ops.lmhead_ce(h.cuda(), W.cuda(), labels.cuda(), softcap=cap, dw_f32=True)
+    z = (h.double() @ W.double().t()).to(torch.bfloat16).double()
+    assert abs(loss.item() - ref.cross_entropy_fwd(z, labels.long(), softcap=cap)[0].item()) < 1e-4
+    d = ref.cross_entropy_bwd(z, labels.long(), softcap=cap)
+    for got, want in ((dW, d.t() @ h.double()), (dh, d @ W.double())):
+        assert ((got.cpu().double() - want).norm() / want.norm()).item() < 2 ** -8
+    assert ((dW.cpu().double() - d.t() @ h.double())[-8:].norm() / (d.t() @ h.double())[-8:].norm()).item() < 2 ** -7
