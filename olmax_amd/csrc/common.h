@@ -159,9 +159,12 @@ int olmax_adamw_grid(hipStream_t stream, float* p, const void* g, float* m, floa
                      int32_t grad_is_bf16, float lr, float b1, float b2, float eps, float wd, int64_t step,
                      float grad_scale, const float* grad_scale_dev, int grid_cap, const float* hyper_dev = nullptr);
 
-// gemm_small.hip: any M, N, K and alignment; `groups` (4 or 8) waves share a 64 x 64 tile's reduction
+// gemm_small.hip: any M, N, K and alignment; `groups` (4 or 8) waves share a tile's reduction; tiles of 64 x 64 or 32 x 32
 void olmax_gemm_small(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N, int K, int64_t lda,
-                      int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, int groups);
+                      int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, int tile, int groups);
+// dX [T, in] = dY [T, out] W [out, in] (+ R) and dW [out, in] = dY^T X [T, in] in one launch; false: not these sizes, nothing was launched
+bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, void* dw, int T, int in,
+                           int out, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw, bool dw_f32);
 // memory a GEMM may use for partial results until it is done; what it holds before and after does not matter
 struct GemmScratch {
   void* p = nullptr;
@@ -171,6 +174,9 @@ struct GemmScratch {
 int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C, const bf16* r, int M, int N, int K,
                       int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded,
                       GemmScratch scratch = GemmScratch());
+// gemm.hip: both gradients of Y = X W^T (dY [T, out], W [out, in]), dX (+ R) first: one launch where neither fills the GPU
+int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, void* dw, int T, int in, int out,
+                     int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw, bool dw_f32, bool dy_padded, GemmScratch scratch);
 // lmhead_ce.hip: olmax_lmhead_ce, its two gradient products with scratch memory
 int olmax_lmhead_ce_scratch(hipStream_t stream, const void* h, const void* W, const int32_t* labels, float* loss, void* dh, void* dW,
                             void* workspace, int64_t workspace_bytes, int64_t T, int32_t d, int32_t V, int32_t ignore_index,

@@ -950,7 +950,7 @@ extern "C" void olmax_gemm_profile_begin(void) {
 // Stop recording, wait for the recorded events and aggregate per kernel instantiation.
 // keys/ms/flops/launches: host arrays of `cap` entries; returns the number of distinct keys.
 // key = tile (64: gemm_small_kernel) | a_layout<<12 | b_layout<<13 | has_residual<<14 | out_f32<<15 | glu_epilogue<<16 | rope_epilogue<<17 |
-// shared_reduction<<18, with a_layout / b_layout bit SET when the operand is reduction-contiguous.  flops / bytes:
+// shared_reduction<<18 | both_gradients<<19 (M, N, K: T, in, out), with a_layout / b_layout bit SET when the operand is reduction-contiguous.  flops / bytes:
 // algorithmic totals (2MNK; every operand and the result moved once).
 extern "C" int32_t olmax_gemm_profile_end(int32_t* keys, double* ms, double* flops, double* bytes, int64_t* launches,
                                           int32_t cap) {
@@ -1055,16 +1055,23 @@ static float cost_256(int64_t n, int kt, int64_t bytes, bool b_kc) {
   (void)pick_parts(r, kt, bytes, &last);
   return cost_rounds(n - r, kt) + last;
 }
-static float cost_small(int64_t n, int kt) { return ((n + 255) / 256) * (0.22f * kt + 1.2f) + 2.4f; }
+static float cost_64(int64_t n, int kt) { return ((n + 255) / 256) * (0.22f * kt + 1.2f) + 2.4f; }
+// 32 tiles: 0.165 us per k-tile while each has a CU, 0.235 (0.30 where A is [K, M], whose lines are then 64 bytes) with two on every CU
+static float cost_32(int64_t n, int kt, bool a_kc) {
+  const float two = a_kc ? 0.235f : 0.30f;
+  return 3.6f + kt * (n <= 256 ? 0.165f : n <= 512 ? 0.165f + (two - 0.165f) * (n - 256) / 256.f : two * n / 512.f);
+}
+static int64_t tiles_of(int M, int N, int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); }
+static float cost_small(int M, int N, int kt, bool a_kc) { return std::min(cost_64(tiles_of(M, N, 64), kt), cost_32(tiles_of(M, N, 32), kt, a_kc)); }
 
 // Which kernel takes a problem.  0: gemm_small (any size and alignment), else the edge of the
 // direct-to-LDS kernel's tiles; *parts > 1: 256 tiles with that many workgroups to a reduction.
-static int pick_tile(int M, int N, int K, bool b_kc, bool direct_ok, int64_t bytes, int* parts) {
+static int pick_tile(int M, int N, int K, bool a_kc, bool b_kc, bool direct_ok, int64_t bytes, int* parts) {
   *parts = 1;
   if (!direct_ok || M < 128 || N < 128 || K < BK) return 0;
   const int kt = (K + BK - 1) / BK;
-  auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
-  float best = cost_small(tiles(64), kt);
+  auto tiles = [&](int t) { return tiles_of(M, N, t); };
+  float best = cost_small(M, N, kt, a_kc);
   int tile = 0;
   if (const float c = cost_128(tiles(128), kt, b_kc); c < best) best = c, tile = 128;
   if (M < 256 || N < 256) return tile;
@@ -1103,7 +1110,7 @@ static bool fused_wins(int M, int N, int K, float per_round, float passes) {
   const int64_t n = (int64_t)tm * tn;
   auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * (N / t); };
   const Cut cut = find_cut(tm, tn);
-  float plain = std::min(cost_small(tiles(64), kt), cost_128(tiles(128), kt, true));
+  float plain = std::min(cost_64(tiles(64), kt), cost_128(tiles(128), kt, true));
   plain = std::min(plain, cut.rm || cut.cn ? cost_256(n, kt, 0, true) : cost_rounds(n, kt));
   return cost_rounds(n, kt) + per_round * ((n + 255) / 256) <= plain + passes;
 }
@@ -1124,7 +1131,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
                          (b_kc ? K : N) % 8 == 0;
   const int force_tile = g_force_tile.load(std::memory_order_relaxed);
   int parts;
-  int tile = pick_tile(M, N, K, b_kc, direct_ok, b_kc || force_tile || !aligned16(scratch.p) ? 0 : scratch.bytes, &parts);
+  int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, b_kc || force_tile || !aligned16(scratch.p) ? 0 : scratch.bytes, &parts);
   if (parts > 1)
     return (a_kc ? launch_split<true, false> : launch_split<false, false>)(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts,
                                                                           (float*)scratch.p);
@@ -1160,9 +1167,13 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
       (void)hipEventCreate(&rec.e1);
       (void)hipEventRecord(rec.e0, stream);
     }
-    olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32,
-                     // eight waves share a tile while there are not more tiles than CUs, else two workgroups fit a CU
-                     (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 256 ? 8 : 4);
+    const int64_t n64 = tiles_of(M, N, 64), n32 = tiles_of(M, N, 32);
+    const int kt = (K + BK - 1) / BK;
+    // (the 0.6 us: one round of 64 tiles, measured at 4 to 128 k-tiles; pick_tile's boundaries were measured without)
+    const int edge = !force_tile && cost_32(n32, kt, a_kc) < cost_64(n64, kt) + 0.6f ? 32 : 64;
+    // eight waves share a tile while there are not more tiles than CUs, else two workgroups fit a CU; a 32 tile needs them from 16 k-tiles on
+    const int groups = edge == 64 ? (n64 <= 256 ? 8 : 4) : (n32 <= 256 && kt >= 16 ? 8 : 4);
+    olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, edge, groups);
     if (g_prof_on) {
       (void)hipEventRecord(rec.e1, stream);
       rec.flops = 2.0 * M * N * K;
@@ -1190,6 +1201,62 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   if (b_kc) GO(false, true);
   GO(false, false);
 #undef GO
+}
+
+// us of the two products of olmax_gemm_grads as one launch of 4-wave workgroups, two of which fit a CU: what their k-tiles take with every
+// CU busy, or the longer of the two chains.  Measured over T 64 to 8192 and widths 256 to 5632: two launches 14 to 64, within 25 %.
+static float cost_pair(int T, int in, int out) {
+  auto part = [&](int M, int N, int K, float* chain) {
+    const int kt = (K + BK - 1) / BK;
+    const int64_t n32 = tiles_of(M, N, 32), n = n32 <= 256 ? n32 : tiles_of(M, N, 64);
+    *chain = std::max(*chain, n32 <= 256 ? 3.6f + 0.165f * kt : 4.2f + 0.22f * kt);
+    return n * ((n32 <= 256 ? 0.00046f : 0.00086f) * kt + 0.0047f);
+  };
+  float chain = 0.f;
+  const float work = part(T, in, out, &chain) + part(out, in, T, &chain) + 3.5f;
+  return std::max(work, chain);
+}
+
+int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, void* dw, int T, int in, int out,
+                     int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw, bool dw_f32, bool dy_padded, GemmScratch scratch) {
+  // what the better kernels take one after the other, as pick_tile sees them
+  auto alone = [&](int M, int N, int K, bool a_kc) {
+    const int kt = (K + BK - 1) / BK;
+    float c = cost_small(M, N, kt, a_kc);
+    if (M >= 128 && N >= 128) c = std::min(c, cost_128(tiles_of(M, N, 128), kt, false));
+    if (M >= 256 && N >= 256) {
+      c = std::min(c, cost_256(tiles_of(M, N, 256), kt, scratch.bytes, false));
+      (void)pick_parts(tiles_of(M, N, 256), K / BK, scratch.bytes, &c);
+    }
+    return c;
+  };
+  if (!g_force_tile.load(std::memory_order_relaxed) && cost_pair(T, in, out) < 0.9f * (alone(T, in, out, true) + alone(out, in, T, false))) {
+    ProfRec rec{};
+    if (g_prof_on) {
+      (void)hipEventCreate(&rec.e0);
+      (void)hipEventCreate(&rec.e1);
+      (void)hipEventRecord(rec.e0, s);
+    }
+    const bool done = olmax_gemm_small_pair(s, dy, w, x, dx, r, dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw, dw_f32);
+    if (g_prof_on) {
+      (void)hipEventRecord(rec.e1, s);
+      rec.flops = 4.0 * T * in * out;
+      rec.bytes = 2.0 * ((double)T * out + 2.0 * T * in + (r ? 1.0 * T * in : 0.0) + (dw_f32 ? 3.0 : 2.0) * in * out);
+      rec.key = 64 | (1 << 19);
+      rec.M = T; rec.N = in; rec.K = out;
+      std::lock_guard<std::mutex> lk(g_prof_mu);
+      if (done) {
+        g_prof.push_back(rec);
+      } else {
+        (void)hipEventDestroy(rec.e0);
+        (void)hipEventDestroy(rec.e1);
+      }
+    }
+    OLMAX_LAUNCH_CHECK();
+    if (done) return OLMAX_OK;
+  }
+  const int rc = olmax_gemm_padded(s, dy, w, dx, r, T, in, out, lddy, ldw, lddx, ldr, true, false, false, dy_padded, scratch);
+  return rc ? rc : olmax_gemm_padded(s, dy, x, dw, nullptr, out, in, T, lddy, ldx, lddw, 0, false, false, dw_f32, dy_padded, scratch);
 }
 
 extern "C" int32_t olmax_gemm_bf16(hipStream_t stream, const void* A, const void* B, void* C,

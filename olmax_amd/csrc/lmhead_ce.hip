@@ -475,6 +475,8 @@ int olmax_lmhead_ce_scratch(hipStream_t stream, const void* h, const void* W, co
   rc = cross_entropy(stream, logits, need_grad ? logits : nullptr, labels, loss, nullptr, nullptr, ce_ws,
                      olmax_cross_entropy_workspace_bytes(T), T, V, ldl, ldl, 0, ignore_index, softcap, 1.f, 0, true);
   if (rc) return rc;
+  if (dh && dW)
+    return olmax_gemm_grads(stream, logits, wp, hp, (bf16*)dh, nullptr, dW, (int)T, d, V, ldl, d, d, d, 0, d, dw_f32 != 0, true, scratch);
   if (dh) {
     rc = olmax_gemm_padded(stream, logits, wp, dh, nullptr, (int)T, d, V, ldl, d, d, 0, true, false, false, true, scratch);
     if (rc) return rc;

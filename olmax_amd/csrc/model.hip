@@ -133,6 +133,12 @@ int lin_dw(hipStream_t s, const bf16* dy, int64_t lddy, const bf16* x, int64_t l
   return olmax_gemm_padded(s, dy, x, dW, nullptr, out, in, (int)T, lddy, ldx, in, 0, false, false, false, false, ws);
 }
 
+// both: dx = dy W (+ res), dW = dy^T x
+int lin_grads(hipStream_t s, const bf16* dy, int64_t lddy, const void* W, const bf16* x, int64_t ldx, int in, int out, bf16* dx, int64_t lddx,
+              const bf16* res, int64_t ldres, void* dW, int64_t T, GemmScratch ws) {
+  return olmax_gemm_grads(s, dy, (const bf16*)W, x, dx, res, dW, (int)T, in, out, lddy, in, ldx, lddx, ldres, in, false, false, ws);
+}
+
 // need_y == false (recompute before the backward): the block output itself is not an input of
 // the backward pass, so the GEMM / norm that only produces it is skipped.
 // Points inside a block's backward pass at which the overlapped train step may start queued
@@ -226,8 +232,7 @@ int attn_backward(hipStream_t s, const olmax_model_config* c, const olmax_block_
                   const Acts& a, const Tmp& t) {
   const Dims m = dims_of(c);
   const float eps = c->eps;
-  RC(lin_dx(s, d_attn_out, m.d, w->wo, m.HD, m.d, t.d_o, m.HD, nullptr, 0, m.T, t.in_attn()));
-  RC(lin_dw(s, d_attn_out, m.d, a.o, m.HD, m.HD, m.d, g->wo, m.T, t.in_attn()));
+  RC(lin_grads(s, d_attn_out, m.d, w->wo, a.o, m.HD, m.HD, m.d, t.d_o, m.HD, nullptr, 0, g->wo, m.T, t.in_attn()));
   const bf16* vp = a.qkv + m.HD + m.KD;
   RC(hook_point(POINT_ATTN_BWD));
   if (c->qk_norm) {
@@ -253,8 +258,7 @@ int attn_backward(hipStream_t s, const olmax_model_config* c, const olmax_block_
     RC(olmax_qk_rope_bwd(s, t.dqkv, t.dqkv, nullptr, nullptr, nullptr, cos_t, sin_t, m.T, m.H + m.K, m.D, m.S, m.QKV,
                          m.QKV, 0, eps));
   }
-  RC(lin_dx(s, t.dqkv, m.QKV, w->wqkv, m.d, m.QKV, dxin, m.d, res_for_dx, m.d, m.T, t.in_attn()));
-  RC(lin_dw(s, t.dqkv, m.QKV, attn_in, m.d, m.d, m.QKV, g->wqkv, m.T, t.in_attn()));
+  RC(lin_grads(s, t.dqkv, m.QKV, w->wqkv, attn_in, m.d, m.d, m.QKV, dxin, m.d, res_for_dx, m.d, g->wqkv, m.T, t.in_attn()));
   return OLMAX_OK;
 }
 
@@ -268,15 +272,14 @@ int mlp_backward(hipStream_t s, const olmax_model_config* c, const olmax_block_w
   const Dims m = dims_of(c);
   if (deferred) {
     RC(olmax_gemm_glu_bwd_bf16(s, mlp_in, w->wgu, t.dact, a.act, t.dgu, (int)m.T, m.F, m.d, m.d, m.d, m.F, m.F, 2 * m.F, c->act));
+    RC(lin_dw(s, d_mlp_out, m.d, a.act, m.F, m.F, m.d, g->wdown, m.T, t.in_mlp()));
   } else {
-    RC(lin_dx(s, d_mlp_out, m.d, w->wdown, m.F, m.d, t.dact, m.F, nullptr, 0, m.T, t.in_mlp()));
+    RC(lin_grads(s, d_mlp_out, m.d, w->wdown, a.act, m.F, m.F, m.d, t.dact, m.F, nullptr, 0, g->wdown, m.T, t.in_mlp()));
   }
-  RC(lin_dw(s, d_mlp_out, m.d, a.act, m.F, m.F, m.d, g->wdown, m.T, t.in_mlp()));
   if (!deferred)
     RC(olmax_glu_bwd(s, a.gu, a.gu + m.F, t.dact, t.dgu, t.dgu + m.F, m.T, m.F, 2 * m.F, 2 * m.F, m.F, 2 * m.F, 2 * m.F,
                      c->act));
-  RC(lin_dx(s, t.dgu, 2 * m.F, w->wgu, m.d, 2 * m.F, dxin, m.d, res_for_dx, m.d, m.T, t.in_mlp()));
-  RC(lin_dw(s, t.dgu, 2 * m.F, mlp_in, m.d, m.d, 2 * m.F, g->wgu, m.T, t.in_mlp()));
+  RC(lin_grads(s, t.dgu, 2 * m.F, w->wgu, mlp_in, m.d, m.d, 2 * m.F, dxin, m.d, res_for_dx, m.d, g->wgu, m.T, t.in_mlp()));
   return OLMAX_OK;
 }
 

@@ -1,0 +1,48 @@
+"""GPU parity tests of products in 32 x 32 tiles, and of two gradients in one launch, at the edges of tiles, chunks and k-tiles."""
+import pytest
+import torch
+
+from oracle import ref
+from test_gemm_choice_gpu import operands, recorded, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("al,bl", [(0, 0), (0, 1), (1, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 33, 63), (32, 32, 64), (33, 40, 65), (40, 96, 1024), (100, 256, 1032), (256, 256, 2048),
+                                   (77, 1024, 2816), (520, 264, 1000), (16, 4096, 4096)])
+def test_tiles_of_32(M, N, K, al, bl):
+    """Against float64: K fp32 additions (2^-24 each) and one rounding to bf16, 2^-9 of the value."""
+    from olmax_amd import ops
+    print(f"[case] tiles of 32 M{M} N{N} K{K} a{al} b{bl}", flush=True)
+    a, b = operands(M, N, K, al, bl)
+    r = rnd(M, N, seed=3)
+    want = (a if al == 0 else a.t()).double() @ (b.t() if bl == 0 else b).double()
+    scale = 2 ** -22 * K ** 0.5 * 6  # of the sum's terms, N(0, 1) products
+    for res in (None, r):
+        got = ops.gemm(a, b, a_layout=al, b_layout=bl, residual=res).double()
+        full = want if res is None else want + res.double()
+        # with a residual the product is rounded first, then the sum
+        assert ((got - full).abs() <= 2 ** -8 * (want.abs() + full.abs()) + scale).all()
+    assert ((ops.gemm(a, b, a_layout=al, b_layout=bl, out_f32=True).double() - want).abs() <= scale).all()
+
+
+@pytest.mark.parametrize("T,d,V,pair", [(2048, 256, 4096, True), (64, 1024, 512, True), (100, 264, 520, True), (1001, 64, 2056, True),
+                                        (2048, 1024, 256, True), (65, 40, 72, True), (300, 256, 1003, False), (63, 256, 512, False)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_both_gradients_in_one_launch(T, d, V, pair, f32):
+    """dh and dW of the LM head.  The oracle takes the logits as this library rounds them; dlogits and the results are rounded to
+    bf16, 2^-9 each, and a handful of logits round the other way: 8e-3 of a row's or column's norm, as two of each."""
+    from olmax_amd import ops
+    print(f"[case] pair T{T} d{d} V{V} f32{f32}", flush=True)
+    h, W = rnd(T, d, seed=1), rnd(V, d, seed=2, scale=0.1)
+    labels = torch.arange(T, device="cuda", dtype=torch.int32) * 7 % V
+    out = []
+    got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels, dw_f32=f32)))
+    assert any(key >> 19 & 1 for key, *_ in got) == pair, got
+    z = (h.double() @ W.double().t()).to(torch.bfloat16).double().cpu()
+    dz = ref.cross_entropy_bwd(z, labels.cpu().long()).cuda()
+    for g, w in ((out[1], dz @ W.double()), (out[2], dz.t() @ h.double())):
+        for dim in (0, 1):
+            e = (g.double() - w).norm(dim=dim) / (w.norm(dim=dim) + 1e-3 * w.norm())
+            assert e.max().item() < 8e-3, (dim, e.argmax().item(), e.max().item())
