@@ -90,12 +90,14 @@ std::mutex g_prof_mu;
 // the loop, which then sees whole k-tiles only: it is fetched with per-lane addresses, and the wave
 // that fetched a chunk past the end overwrites it with zeros in LDS once its own fetches have landed,
 // before the barrier that publishes the stage.  Wants M >= BM, N >= BN, K >= 64 and 16-byte chunks that do not cross the end of a row (see olmax_gemm_padded).
-template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI = 0, int RAG = 0>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm_bf16_kernel(
+//
+// The tile that workgroup `pid` of `nwg` takes; the residual of a HAS_RES form may be null.
+template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI, int RAG>
+__device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
     const bf16* __restrict__ R, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     int64_t ldr, int tiles_m, int tiles_n, int c_vec, const float* __restrict__ cos_t,
-    const float* __restrict__ sin_t, int seq_len, int rope_cols, int order) {
+    const float* __restrict__ sin_t, int seq_len, int rope_cols, int order, int pid, const int nwg, unsigned char* smem) {
   constexpr int GLU = (EPI == 1 || EPI == 2) ? EPI : (EPI == 4 ? 1 : (EPI == 5 ? 2 : 0));
   constexpr bool GLU_BWD = EPI == 4 || EPI == 5;
   constexpr bool ROPE = EPI == 3;
@@ -111,15 +113,13 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
   constexpr int NINS = A_INS + B_INS;
   constexpr int STAGE = A_BYTES + B_BYTES;
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [A stage 0 | A stage 1 | B stage 0 | B stage 1]
+  // LDS: [A stage 0 | A stage 1 | B stage 0 | B stage 1]
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
   // ---- XCD-aware tile assignment ----
-  const int nwg = gridDim.x;
-  int pid = blockIdx.x;
   int tile_m, tile_n;
   if (order > 0) {
     // Windows of 8 x 4 tiles (what the 32 CUs of an XCD hold at a time: 12 operand panels for
@@ -681,7 +681,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
       }
       return;
     }
-    if (HAS_RES) {
+    if (HAS_RES && R) {
       Pack8 rr[WM / 8];
 #pragma unroll
       for (int t = 0; t < WM / 8; t++) {  // all residual lines requested before the first is needed
@@ -721,7 +721,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
         f32x4 v = acc[i][j];
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          if (HAS_RES) v[r] += bf2f(R[row * ldr + col + r]);
+          if (HAS_RES && R) v[r] += bf2f(R[row * ldr + col + r]);
         *reinterpret_cast<f32x4_u*>(reinterpret_cast<float*>(Cv) + row * ldc + col) = v;
         continue;
       }
@@ -730,13 +730,52 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
         const int col = n0 + wn * WN + j * 16 + g16e * 4 + r;
         if (RAG && col < n0 + col_lo) continue;
         float v = acc[i][j][r];
-        if (HAS_RES) v = (OUT_F32 ? v : bf2f(f2bf(v))) + bf2f(R[row * ldr + col]);  // bf16 output: round, add, round
+        if (HAS_RES && R) v = (OUT_F32 ? v : bf2f(f2bf(v))) + bf2f(R[row * ldr + col]);  // bf16 output: round, add, round
         if (OUT_F32)
           reinterpret_cast<float*>(Cv)[row * ldc + col] = v;
         else
           reinterpret_cast<bf16*>(Cv)[row * ldc + col] = f2bf(v);
       }
     }
+}
+
+template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI = 0, int RAG = 0>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm_bf16_kernel(
+    const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
+    const bf16* __restrict__ R, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+    int64_t ldr, int tiles_m, int tiles_n, int c_vec, const float* __restrict__ cos_t,
+    const float* __restrict__ sin_t, int seq_len, int rope_cols, int order) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  gemm_tile<BM, BN, WM, WN, A_KC, B_KC, HAS_RES, OUT_F32, EPI, RAG>(A, B, Cv, R, M, N, K, lda, ldb, ldc, ldr, tiles_m, tiles_n, c_vec, cos_t,
+                                                                    sin_t, seq_len, rope_cols, order, blockIdx.x, gridDim.x, smem);
+}
+
+// dX = dY W (+ R) and dW = dY^T X in one launch of T x T tiles: the second starts on the CUs that the first's last round of tiles
+// leaves idle.  Workgroups [0, n_first) are the product with the longer reduction (and padding up to a whole number of XCDs).
+// us, two calls -> one, T x in x out: tiles of 128: 3000 x 1024 x 3072 76 -> 54, 3000 x 2816 x 1024 63 -> 41, 1024 x 4096 x 4096 79 -> 71;
+// tiles of 256: 2048 x 11008 x 4096 343 -> 306, 1500 x 14336 x 4096 368 -> 316, 8192 x 11008 x 4096 1141 -> 1091.
+// 240 registers (the cap counts pairs): as in the single kernels a wave of the overlapped update fits beside two of these.
+struct PairSide {
+  const bf16 *A, *B, *R;
+  bf16* C;
+  int M, N, K;
+  int64_t lda, ldb, ldc, ldr;
+  int tiles_m, tiles_n, order, nwg;
+};
+template <int T, int W, int RAGX, int RAGW>
+__global__ __launch_bounds__((T / W) * (T / 64) * 64) __attribute__((amdgpu_num_vgpr(120))) void gemm_pair_kernel(const PairSide x, const PairSide w, int x_first, int n_first) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const bool second = (int)blockIdx.x >= n_first;
+  const int pid = second ? blockIdx.x - n_first : blockIdx.x;
+  if (second != (x_first != 0)) {
+    if (pid >= x.nwg) return;
+    gemm_tile<T, T, W, 64, true, false, true, false, 0, RAGX>(x.A, x.B, x.C, x.R, x.M, x.N, x.K, x.lda, x.ldb, x.ldc, x.ldr, x.tiles_m, x.tiles_n, 1,
+                                                              nullptr, nullptr, 1, 0, x.order, pid, x.nwg, smem);
+  } else {
+    if (pid >= w.nwg) return;
+    gemm_tile<T, T, W, 64, false, false, false, false, 0, RAGW>(w.A, w.B, w.C, nullptr, w.M, w.N, w.K, w.lda, w.ldb, w.ldc, 0, w.tiles_m, w.tiles_n, 1,
+                                                                nullptr, nullptr, 1, 0, w.order, pid, w.nwg, smem);
+  }
 }
 
 std::atomic<int> g_order{0};  // diagnostic override of the tile order, process-wide: 0 automatic, -1 run order, > 0 that many strips
@@ -747,12 +786,14 @@ std::atomic<int> g_order{0};  // diagnostic override of the tile order, process-
 //     a weight matrix beyond the cache (the LM head) wants every row in flight instead;
 //   input gradients (dX = dY W): 2 strips, -2 % at K = 4096, -3.5 % on the LM head, else neutral;
 //   weight gradients (dW = dY^T X): 4 strips, -3 % to -5 % on every shape.
-// Grids that would need padded windows keep the run order (the padding costs more than it gains).
+// Grids that would need padded windows keep the run order (the padding costs more than it gains), and so do those whose windows the
+// XCDs cannot share evenly (4 windows keep half of the GPU from the operands: 2048 x 4096 x 4096 108 us, run order 100, 6144 x 4096 x 2048
+// as a weight gradient 108, 100; a second product in the same launch waits for the XCDs that have too many).
 int tile_order(int tm, int tn, bool a_kc, bool b_kc, int N, int K) {
   const int o = g_order.load(std::memory_order_relaxed);
   if (o < 0) return 0;
   if (o > 0) return o;
-  if (tm % 8 || tn % 4) return 0;
+  if (tm % 8 || tn % 4 || tm / 8 * (tn / 4) % 8) return 0;
   const int strips = tm / 8;
   if (a_kc && b_kc) return (int64_t)N * K * 2 <= (128ll << 20) ? 1 : (strips < 8 ? strips : 8);
   if (a_kc) return strips < 2 ? strips : 2;
@@ -829,6 +870,22 @@ int launch_glu(hipStream_t s, const bf16* A, const bf16* B, bf16* gu, bf16* act,
   }
   OLMAX_LAUNCH_CHECK();
   return OLMAX_OK;
+}
+
+template <int T, int W, int RAGX, int RAGW>
+void launch_pair(hipStream_t s, PairSide x, PairSide w) {
+  auto kern = gemm_pair_kernel<T, W, RAGX, RAGW>;
+  constexpr int SMEM = 4 * T * BK * 2;
+  static std::once_flag attr_once;  // per instantiation
+  std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM); });
+  for (auto p : {&x, &w}) {
+    p->tiles_m = (p->M + T - 1) / T;
+    p->tiles_n = (p->N + T - 1) / T;
+    p->order = tile_order(p->tiles_m, p->tiles_n, p == &x, false, p->N, p->K);
+    p->nwg = (int)order_grid(p->order, p->tiles_m, p->tiles_n);
+  }
+  const int x_first = x.K > w.K, n_first = ((x_first ? x.nwg : w.nwg) + 7) & ~7;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_first + (x_first ? w.nwg : x.nwg))), dim3((T / W) * (T / 64) * 64), SMEM, s, x, w, x_first, n_first);
 }
 
 template <bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32>
@@ -1203,9 +1260,15 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
 #undef GO
 }
 
-// us of the two products of olmax_gemm_grads as one launch of 4-wave workgroups, two of which fit a CU: what their k-tiles take with every
-// CU busy, or the longer of the two chains.  Measured over T 64 to 8192 and widths 256 to 5632: two launches 14 to 64, within 25 %.
-static float cost_pair(int T, int in, int out) {
+// The two products of olmax_gemm_grads as one launch: what it costs in each kernel that can run it.  Measured, with the two calls, on 312
+// sizes (T 130 to 8192, widths 256 to 28672): the least of these estimates and of the calls' takes 11 % less than the calls, the best 13 %;
+// what it loses where the calls were better is 4 % at most.
+struct Work {
+  int64_t n;  // tiles
+  int kt;
+};
+// 64 and 32 tiles in 4-wave workgroups, two of which fit a CU: their k-tiles with every CU busy, or the longer of the two chains
+static float pair_small(int T, int in, int out) {
   auto part = [&](int M, int N, int K, float* chain) {
     const int kt = (K + BK - 1) / BK;
     const int64_t n32 = tiles_of(M, N, 32), n = n32 <= 256 ? n32 : tiles_of(M, N, 64);
@@ -1214,35 +1277,87 @@ static float cost_pair(int T, int in, int out) {
   };
   float chain = 0.f;
   const float work = part(T, in, out, &chain) + part(out, in, T, &chain) + 3.5f;
-  return std::max(work, chain);
+  return std::max(work, chain) / 0.9f;
+}
+// 128 tiles, 512 at a time: 1 us per k-tile of each, 17 % more where they end unevenly; or the long chains, beside the others and then alone
+static float pair_128(Work l, Work s) {
+  const int64_t n = l.n + s.n;
+  const float work = (float)(l.n * l.kt + s.n * s.kt) / 512 * (n < 800 ? 1.17f : 1.f) + 4.f * n / 512 + 2.f;
+  const float both = std::min((float)l.kt, s.n * (s.kt + 4.f) / std::max<int64_t>(1, 512 - l.n));
+  const float alone = l.n <= 128 ? 0.62f : l.n <= 256 ? 0.62f + 0.25f * (l.n - 128) / 128 : 0.87f;
+  return std::max(work, 1.08f * both + alone * (l.kt - both) + 4.f) / 0.96f;
+}
+// 256 tiles, one on a CU: the long ones in rounds, the short ones on the CUs that the last of these leaves, then on all
+static float pair_256(Work l, Work s) {
+  const int64_t n = l.n + s.n, r = l.n % 256;
+  const float f = n >= 256 ? 1.52f : 1.05f + 0.47f * n / 256, a = f * l.kt + 6.f, b = f * s.kt + 6.f;
+  const float t0 = (l.n / 256) * a, t1 = r ? t0 + a : t0;  // the first and the last CU is free for short ones
+  auto early = [&](float t) { return t <= t0 ? 0 : (int64_t)((t - t0) / b + 1e-3f); };  // short ones that a CU has ended by t
+  auto late = [&](float t) { return t <= t1 ? 0 : (int64_t)((t - t1) / b + 1e-3f); };
+  auto done = [&](float t) { return (256 - r) * early(t) + r * late(t); };
+  float t = t1;
+  while (done(t) < s.n) t = std::min(t0 + (early(t) + 1) * b, t1 + (late(t) + 1) * b);
+  if (n >= 256) {  // the last ones have less company
+    const float busy = std::min(1.f, (s.n - done(t - b) + (r && t - b < t1 ? r : 0)) / 256.f);
+    t = std::max(t1, t - b + (1.05f + 0.47f * busy) * s.kt + 6.f);
+  }
+  return t / 0.97f;
 }
 
 int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, void* dw, int T, int in, int out,
                      int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw, bool dw_f32, bool dy_padded, GemmScratch scratch) {
   // what the better kernels take one after the other, as pick_tile sees them
+  const int64_t bytes = aligned16(scratch.p) ? scratch.bytes : 0;
   auto alone = [&](int M, int N, int K, bool a_kc) {
     const int kt = (K + BK - 1) / BK;
     float c = cost_small(M, N, kt, a_kc);
     if (M >= 128 && N >= 128) c = std::min(c, cost_128(tiles_of(M, N, 128), kt, false));
     if (M >= 256 && N >= 256) {
-      c = std::min(c, cost_256(tiles_of(M, N, 256), kt, scratch.bytes, false));
-      (void)pick_parts(tiles_of(M, N, 256), K / BK, scratch.bytes, &c);
+      c = std::min(c, cost_256(tiles_of(M, N, 256), kt, bytes, false));
+      (void)pick_parts(tiles_of(M, N, 256), K / BK, bytes, &c);
     }
     return c;
   };
-  if (!g_force_tile.load(std::memory_order_relaxed) && cost_pair(T, in, out) < 0.9f * (alone(T, in, out, true) + alone(out, in, T, false))) {
+  float best = alone(T, in, out, true) + alone(out, in, T, false);
+  int tile = 0;  // of the one launch, 0: two calls
+  if (const float c = pair_small(T, in, out); c < best && out % 8 == 0 && in % 8 == 0 && T >= 64) best = c, tile = 64;
+  // whole chunks and vector stores, whole k-tiles in the first product
+  const bool direct = !dw_f32 && out % BK == 0 && in % 8 == 0 && lddy % 8 == 0 && ldw % 8 == 0 && ldx % 8 == 0 && lddx % 8 == 0 && lddw % 8 == 0 &&
+                      (!r || (ldr % 8 == 0 && aligned16(r))) && aligned16(dy) && aligned16(w) && aligned16(x) && aligned16(dx) && aligned16(dw);
+  for (int t = 128; t <= 256; t *= 2) {
+    if (!direct || T < t || in < t || out < t) continue;
+    const Work wx = {tiles_of(T, in, t), out / BK}, ww = {tiles_of(out, in, t), (T + BK - 1) / BK};
+    const Work &l = wx.kt > ww.kt ? wx : ww, &sh = wx.kt > ww.kt ? ww : wx;
+    if (const float c = t == 128 ? pair_128(l, sh) : pair_256(l, sh); c < best) best = c, tile = t;
+  }
+  if (tile && !g_force_tile.load(std::memory_order_relaxed)) {
     ProfRec rec{};
     if (g_prof_on) {
       (void)hipEventCreate(&rec.e0);
       (void)hipEventCreate(&rec.e1);
       (void)hipEventRecord(rec.e0, s);
     }
-    const bool done = olmax_gemm_small_pair(s, dy, w, x, dx, r, dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw, dw_f32);
+    bool done = true;
+    if (tile == 64) {
+      done = olmax_gemm_small_pair(s, dy, w, x, dx, r, dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw, dw_f32);
+    } else {
+      const PairSide px = {dy, w, r, dx, T, in, out, lddy, ldw, lddx, ldr}, pw = {dy, x, nullptr, (bf16*)dw, out, in, T, lddy, ldx, lddw, 0};
+      const bool rx = T % tile || in % tile;
+      const int rw = T % BK ? 2 : out % tile || in % tile;
+#define PAIR(E, W)                                                                                                              \
+  do {                                                                                                                          \
+    if (rx) rw == 2 ? launch_pair<E, W, 1, 2>(s, px, pw) : rw ? launch_pair<E, W, 1, 1>(s, px, pw) : launch_pair<E, W, 1, 0>(s, px, pw); \
+    else rw == 2 ? launch_pair<E, W, 0, 2>(s, px, pw) : rw ? launch_pair<E, W, 0, 1>(s, px, pw) : launch_pair<E, W, 0, 0>(s, px, pw);    \
+  } while (0)
+      if (tile == 128) PAIR(128, 64);
+      else PAIR(256, 128);
+#undef PAIR
+    }
     if (g_prof_on) {
       (void)hipEventRecord(rec.e1, s);
       rec.flops = 4.0 * T * in * out;
       rec.bytes = 2.0 * ((double)T * out + 2.0 * T * in + (r ? 1.0 * T * in : 0.0) + (dw_f32 ? 3.0 : 2.0) * in * out);
-      rec.key = 64 | (1 << 19);
+      rec.key = tile | (1 << 19);
       rec.M = T; rec.N = in; rec.K = out;
       std::lock_guard<std::mutex> lk(g_prof_mu);
       if (done) {

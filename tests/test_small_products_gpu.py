@@ -1,4 +1,5 @@
-"""GPU parity tests of products in 32 x 32 tiles, and of two gradients in one launch, at the edges of tiles, chunks and k-tiles."""
+"""GPU parity tests of products in 32 x 32 tiles, and of two gradients in one launch (every size of tile), at the edges of tiles, chunks
+and k-tiles."""
 import pytest
 import torch
 
@@ -40,9 +41,62 @@ def test_both_gradients_in_one_launch(T, d, V, pair, f32):
     out = []
     got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels, dw_f32=f32)))
     assert any(key >> 19 & 1 for key, *_ in got) == pair, got
+    check_gradients(h, W, labels, *out[1:])
+
+
+def check_gradients(h, W, labels, dh, dW):
     z = (h.double() @ W.double().t()).to(torch.bfloat16).double().cpu()
     dz = ref.cross_entropy_bwd(z, labels.cpu().long()).cuda()
-    for g, w in ((out[1], dz @ W.double()), (out[2], dz.t() @ h.double())):
+    for g, w in ((dh, dz @ W.double()), (dW, dz.t() @ h.double())):
         for dim in (0, 1):
             e = (g.double() - w).norm(dim=dim) / (w.norm(dim=dim) + 1e-3 * w.norm())
             assert e.max().item() < 8e-3, (dim, e.argmax().item(), e.max().item())
+
+
+@pytest.mark.parametrize("T,d,V,tile", [
+    (4096, 1024, 3072, 128), (4096, 1032, 3072, 128),  # whole tiles; ragged columns in both products
+    (3000, 1024, 3072, 128), (3000, 1024, 2880, 128),  # ragged rows and a partial k-tile of dW; dW ragged too
+    (4160, 1024, 3072, 128), (4096, 1024, 2880, 128),  # ragged rows, whole k-tiles; only dW ragged
+    (2048, 11008, 4096, 256), (2048, 11000, 4096, 256), (2000, 11008, 4096, 256), (2000, 11008, 3904, 256), (1984, 11008, 4096, 256),
+    (2048, 11008, 3904, 256),
+])
+def test_both_gradients_in_one_launch_of_large_tiles(T, d, V, tile):
+    """As above; the launch is in tiles of the expected size."""
+    from olmax_amd import ops
+    print(f"[case] pair T{T} d{d} V{V} tile{tile}", flush=True)
+    h, W = rnd(T, d, seed=1), rnd(V, d, seed=2, scale=0.02)
+    labels = torch.arange(T, device="cuda", dtype=torch.int32) * 7 % V
+    out = []
+    got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels)))
+    assert (tile | 1 << 19, T, d, V, 1) in got, got
+    check_gradients(h, W, labels, *out[1:])
+
+
+@pytest.mark.parametrize("seq", [1500, 2048])
+def test_a_residual_joins_the_first_product(seq):
+    """Post-norm blocks add the residual's gradient in dX.  Against the two calls, which a forced tile brings back: the products are
+    rounded to bf16 (2^-9 each) and four of them follow one another."""
+    from olmax_amd import TransformerRecipe, _lib
+    from olmax_amd.layer import TransformerBlock
+    import dataclasses
+    cfg = dataclasses.replace(TransformerRecipe.olmo2_7B(), num_layers=1)
+    block = TransformerBlock(cfg, batch_size=1, sequence_length=seq)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for w in (block.wqkv, block.wo, block.wgu, block.wdown):
+        w.normal_(0.0, 0.02, generator=g)
+    x, dy = rnd(seq, cfg.d_model, seed=2), rnd(seq, cfg.d_model, seed=3)
+    block.forward(x)
+    res, dx = {}, []
+    got = recorded(lambda: dx.append(block.backward(dy)))
+    assert any(key >> 19 & 1 for key, *_ in got), got
+    res[0] = [dx[0].clone()] + [v.clone() for v in block.grads.values()]
+    for v in block.grads.values():
+        v.zero_()
+    _lib.load().olmax_gemm_set_tile(256)
+    try:
+        got = recorded(lambda: dx.append(block.backward(dy)))
+    finally:
+        _lib.load().olmax_gemm_set_tile(0)
+    assert not any(key >> 19 & 1 for key, *_ in got), got
+    for a, b in zip(res[0], [dx[1]] + list(block.grads.values())):
+        assert ((a.double() - b.double()).norm() / b.double().norm()).item() < 2 ** -7
