@@ -787,13 +787,15 @@ std::atomic<int> g_order{0};  // diagnostic override of the tile order, process-
 //   input gradients (dX = dY W): 2 strips, -2 % at K = 4096, -3.5 % on the LM head, else neutral;
 //   weight gradients (dW = dY^T X): 4 strips, -3 % to -5 % on every shape.
 // Grids that would need padded windows keep the run order (the padding costs more than it gains), and so do those whose windows the
-// XCDs cannot share evenly (4 windows keep half of the GPU from the operands: 2048 x 4096 x 4096 108 us, run order 100, 6144 x 4096 x 2048
-// as a weight gradient 108, 100; a second product in the same launch waits for the XCDs that have too many).
+// XCDs cannot share evenly, up to three rounds of them (4 windows keep half of the GPU from the operands: 2048 x 4096 x 4096 108 us, run
+// order 100, 6144 x 4096 x 2048 as a weight gradient 108, 100; a second product in the same launch waits for the XCDs that have too many;
+// 196 windows, 100352 x 4096 x 8192 as a weight gradient: 4902 us, run order 5266).
 int tile_order(int tm, int tn, bool a_kc, bool b_kc, int N, int K) {
   const int o = g_order.load(std::memory_order_relaxed);
   if (o < 0) return 0;
   if (o > 0) return o;
-  if (tm % 8 || tn % 4 || tm / 8 * (tn / 4) % 8) return 0;
+  const int windows = tm / 8 * (tn / 4);
+  if (tm % 8 || tn % 4 || (windows < 24 && windows % 8)) return 0;
   const int strips = tm / 8;
   if (a_kc && b_kc) return (int64_t)N * K * 2 <= (128ll << 20) ? 1 : (strips < 8 ? strips : 8);
   if (a_kc) return strips < 2 ? strips : 2;
