@@ -57,3 +57,34 @@ def stream_ptr() -> c_void_p:
 
 
 i32, i64, f32, f64, vp = c_int32, c_int64, c_float, c_double, c_void_p
+
+# Argument types of the entry points that a program calls once per layer and pass: P pointer, I int32, L int64, F float.
+_SIGNATURES = {
+    "olmax_gemm_bf16": "PPPPPIIILLLLIII",
+    "olmax_rmsnorm_fwd": "PPPPLILLF",
+    "olmax_rmsnorm_bwd": "PPPPPPPLILLLLF",
+    "olmax_fill_zero": "PPL",
+    "olmax_attn_fwd": "PPPPPPIIIIILLLLIF",
+    "olmax_attn_bwd": "PPPPPPPPPPPLIIIIILLLLLLLLIF",
+}
+_typed = {}
+
+
+def typed(name: str):
+    """Entry point `name` with its argument types set, on a handle of its own: it takes plain integers, floats and None, which ctypes
+    converts in C (0.1 us an argument less than an object around each)."""
+    f = _typed.get(name)
+    if f is None:
+        load()
+        f = getattr(ctypes.CDLL(str(_LIB_PATH)), name)
+        f.argtypes = [{"P": vp, "I": i32, "L": i64, "F": f32}[c] for c in _SIGNATURES[name]]
+        f.restype = i32
+        _typed[name] = f
+    return f
+
+
+def raw_stream() -> int:
+    """Current stream of the current device, as an integer."""
+    import torch
+
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())

@@ -13,7 +13,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._lib import check, f32, i32, i64, ptr, stream_ptr
+from ._lib import check, f32, i32, i64, ptr, raw_stream, stream_ptr, typed
 
 BF16 = torch.bfloat16
 
@@ -42,20 +42,24 @@ def gemm(a: torch.Tensor, b: torch.Tensor, *, a_layout: int = 0, b_layout: int =
     _need_gpu(a, b, residual, out)
     a, b = _rows2d(a), _rows2d(b)
     assert a.dtype == BF16 and b.dtype == BF16
-    M, K = (a.shape if a_layout == 0 else (a.shape[1], a.shape[0]))
-    N, Kb = (b.shape if b_layout == 0 else (b.shape[1], b.shape[0]))
+    M, K = a.shape
+    N, Kb = b.shape
+    if a_layout != 0:
+        M, K = K, M
+    if b_layout != 0:
+        N, Kb = Kb, N
     assert K == Kb, f"reduction dims differ: {K} vs {Kb}"
     if out is None:
-        out = torch.empty(M, N, device=a.device, dtype=torch.float32 if out_f32 else BF16)
-    assert out.shape == (M, N) and out.stride(1) == 1
-    ldr = 0
+        out = a.new_empty((M, N), dtype=torch.float32) if out_f32 else a.new_empty((M, N))
+    else:
+        assert out.shape == (M, N) and out.stride(1) == 1
+    ldr, r = 0, None
     if residual is not None:
         residual = _rows2d(residual)
         assert residual.shape == (M, N) and residual.dtype == BF16
-        ldr = residual.stride(0)
-    check(_L().olmax_gemm_bf16(stream_ptr(), ptr(a), ptr(b), ptr(out), ptr(residual), i32(M), i32(N), i32(K),
-                               i64(a.stride(0)), i64(b.stride(0)), i64(out.stride(0)), i64(ldr),
-                               i32(a_layout), i32(b_layout), i32(1 if out.dtype == torch.float32 else 0)))
+        ldr, r = residual.stride(0), residual.data_ptr()
+    check(typed("olmax_gemm_bf16")(raw_stream(), a.data_ptr(), b.data_ptr(), out.data_ptr(), r, M, N, K, a.stride(0), b.stride(0),
+                                   out.stride(0), ldr, a_layout, b_layout, 1 if out.dtype == torch.float32 else 0))
     return out
 
 
@@ -78,10 +82,11 @@ def linear_bwd_weight(dy, x, out=None, out_f32=False):
 def rms_norm_fwd(x, w, eps: float, out=None):
     _need_gpu(x, w)
     x = _rows2d(x)
+    T, d = x.shape
     if out is None:
-        out = torch.empty(x.shape, device=x.device, dtype=BF16)
-    check(_L().olmax_rmsnorm_fwd(stream_ptr(), ptr(x), ptr(w), ptr(out), i64(x.shape[0]), i32(x.shape[1]),
-                                 i64(x.stride(0)), i64(out.stride(0)), f32(eps)))
+        out = x.new_empty((T, d), dtype=BF16)
+    check(typed("olmax_rmsnorm_fwd")(raw_stream(), x.data_ptr(), None if w is None else w.data_ptr(), out.data_ptr(), T, d, x.stride(0),
+                                     out.stride(0), eps))
     return out
 
 
@@ -89,13 +94,16 @@ def rms_norm_bwd(x, w, dy, eps: float, dres=None, dw: Optional[torch.Tensor] = N
     """Returns (dx [+ dres], dw fp32).  `dw` (fp32 [d]) is accumulated into when given."""
     _need_gpu(x, w, dy)
     x, dy = _rows2d(x), _rows2d(dy)
+    T, d = x.shape
     if out is None:
-        out = torch.empty(x.shape, device=x.device, dtype=BF16)
+        out = x.new_empty((T, d), dtype=BF16)
+    stream = raw_stream()
     if dw is None and w is not None:
-        dw = torch.zeros(x.shape[1], device=x.device, dtype=torch.float32)
-    check(_L().olmax_rmsnorm_bwd(stream_ptr(), ptr(x), ptr(w), ptr(dy), ptr(dres), ptr(out), ptr(dw),
-                                 i64(x.shape[0]), i32(x.shape[1]), i64(x.stride(0)), i64(dy.stride(0)),
-                                 i64(0 if dres is None else dres.stride(0)), i64(out.stride(0)), f32(eps)))
+        dw = x.new_empty((d,), dtype=torch.float32)
+        check(typed("olmax_fill_zero")(stream, dw.data_ptr(), 4 * d))
+    check(typed("olmax_rmsnorm_bwd")(stream, x.data_ptr(), None if w is None else w.data_ptr(), dy.data_ptr(),
+                                     None if dres is None else dres.data_ptr(), out.data_ptr(), None if dw is None else dw.data_ptr(), T, d,
+                                     x.stride(0), dy.stride(0), 0 if dres is None else dres.stride(0), out.stride(0), eps))
     return out, dw
 
 
@@ -231,9 +239,8 @@ def attn_fwd(q, k, v, *, B: int, S: int, H: int, KH: int, D: int, window: Option
     if out is None:
         out = torch.empty(B * S, H * D, device=q.device, dtype=BF16)
     lse = torch.empty(B, H, S, device=q.device, dtype=torch.float32)
-    check(_L().olmax_attn_fwd(stream_ptr(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(lse), i32(B), i32(S), i32(H),
-                              i32(KH), i32(D), i64(q.stride(0)), i64(k.stride(0)), i64(v.stride(0)),
-                              i64(out.stride(0)), i32(-1 if window is None else window), f32(softcap)))
+    check(typed("olmax_attn_fwd")(raw_stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), B, S, H, KH, D,
+                                  q.stride(0), k.stride(0), v.stride(0), out.stride(0), -1 if window is None else window, softcap))
     return out, lse
 
 
@@ -250,11 +257,10 @@ def attn_bwd(q, k, v, o, lse, do, *, B: int, S: int, H: int, KH: int, D: int, wi
         dk = torch.empty(B * S, KH * D, device=q.device, dtype=BF16)
     if dv is None:
         dv = torch.empty(B * S, KH * D, device=q.device, dtype=BF16)
-    check(L.olmax_attn_bwd(stream_ptr(), ptr(q), ptr(k), ptr(v), ptr(o), ptr(lse), ptr(do), ptr(dq), ptr(dk), ptr(dv),
-                           ptr(ws), i64(nbytes), i32(B), i32(S), i32(H), i32(KH), i32(D), i64(q.stride(0)),
-                           i64(k.stride(0)), i64(v.stride(0)), i64(o.stride(0)), i64(do.stride(0)),
-                           i64(dq.stride(0)), i64(dk.stride(0)), i64(dv.stride(0)),
-                           i32(-1 if window is None else window), f32(softcap)))
+    check(typed("olmax_attn_bwd")(raw_stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), do.data_ptr(),
+                                  dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), nbytes, B, S, H, KH, D, q.stride(0), k.stride(0),
+                                  v.stride(0), o.stride(0), do.stride(0), dq.stride(0), dk.stride(0), dv.stride(0),
+                                  -1 if window is None else window, softcap))
     return dq, dk, dv
 
 
