@@ -159,6 +159,16 @@ int olmax_adamw_grid(hipStream_t stream, float* p, const void* g, float* m, floa
                      int32_t grad_is_bf16, float lr, float b1, float b2, float eps, float wd, int64_t step,
                      float grad_scale, const float* grad_scale_dev, int grid_cap, const float* hyper_dev = nullptr);
 
+// elementwise.hip: first_use[row] = first token that names an embedding row (INT32_MAX: none); the update of the rows without one, elements
+// [at, at + n) of the [V, d] table (multiples of 4, d >= 1024; g null: zero gradients), and of the rows with one.
+int olmax_first_use(hipStream_t stream, const int32_t* ids, int32_t* first_use, int64_t T, int V);
+int olmax_adamw_unused_rows(hipStream_t stream, float* p, const float* g, float* m, float* v, bf16* shadow, const int32_t* first_use, int64_t at,
+                            int64_t n, int d, float lr, float b1, float b2, float eps, float wd, int64_t step, int grid_cap,
+                            const float* hyper_dev);
+int olmax_adamw_used_rows(hipStream_t stream, float* p, const float* g, float* m, float* v, bf16* shadow, const int32_t* ids,
+                          const int32_t* first_use, int64_t T, int V, int d, float lr, float b1, float b2, float eps, float wd, int64_t step,
+                          const float* hyper_dev);
+
 // gemm_small.hip: any M, N, K and alignment; `groups` (4 or 8) waves share a tile's reduction; tiles of 64 x 64 or 32 x 32
 void olmax_gemm_small(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N, int K, int64_t lda,
                       int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, int tile, int groups);

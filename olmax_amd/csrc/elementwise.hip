@@ -254,7 +254,8 @@ __device__ __forceinline__ AdamwScalars adamw_scalars(float lr, float b1, float 
 // (non-temporal) accesses keep the 28 B/param out of the way of the L2.  One 32-bit offset register addresses all five arrays and
 // the four loads are requested together: with a 64-bit pointer register pair per array they did not fit the 32 registers of
 // the kernels below and waited for each other.
-template <bool G_BF16>
+// HAS_G false: the gradient is zero and not read.
+template <bool G_BF16, bool HAS_G = true>
 __device__ __forceinline__ void adamw_vec(float* __restrict__ p, const void* __restrict__ gv, float* __restrict__ m, float* __restrict__ v,
                                           bf16* __restrict__ shadow, uint32_t lane, const AdamwScalars& c) {
   const float lr = c.lr, b1 = c.b1, b2 = c.b2, eps = c.eps, wd = c.wd, ibc1 = c.ibc1, ibc2 = c.ibc2, gscale = c.gscale;
@@ -266,7 +267,8 @@ __device__ __forceinline__ void adamw_vec(float* __restrict__ p, const void* __r
 #define GLOBAL(T, base, bytes) ((__attribute__((address_space(1))) T*)((__attribute__((address_space(1))) char*)(base) + (bytes)))
   f32x4 gf;
   Pack4 gp;
-  if (G_BF16) gp.u = __builtin_nontemporal_load(GLOBAL(u32x2, ga, o8));
+  if (!HAS_G) gf = f32x4{0.f, 0.f, 0.f, 0.f};
+  else if (G_BF16) gp.u = __builtin_nontemporal_load(GLOBAL(u32x2, ga, o8));
   else gf = __builtin_nontemporal_load(GLOBAL(f32x4, ga, o16));
   f32x4 mv = __builtin_nontemporal_load(GLOBAL(f32x4, ma, o16));
   f32x4 vv = __builtin_nontemporal_load(GLOBAL(f32x4, va, o16));
@@ -344,6 +346,50 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(16))) void adam
   } else {
     if (i < sp.n4) adamw_vec<true>(p, gr, m, v, shadow, (uint32_t)i, c);
     if (i < sp.ntail) adamw_one<true>(p, gr, m, v, shadow, j, c);
+  }
+}
+
+// An embedding's update in two parts, so that the larger one need not wait for the scatter-add at the end of the backward pass: rows that no
+// token of the batch names (their gradient is zero, or under a tied head final with the head's weight gradient), and the
+// others.  first_use[row]: the first token that names it, INT32_MAX if none does.  (gscale, 1 here, is an argument as in adamw_kernel: as a
+// constant the multiplication goes, other products become fused ones, and an element depends on the kernel by an ulp.)
+__global__ __launch_bounds__(256) void first_use_kernel(const int32_t* __restrict__ ids, int32_t* __restrict__ first_use, int64_t T, int V) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t < T) atomicMin(&first_use[wrap_clamp_id(ids[t], V)], (int32_t)t);
+}
+// n elements from element `off` of row `row` on (both multiples of 4, rows of d >= 1024: a workgroup's 1024 elements lie in two
+// rows at most, whose flags are scalar loads).  Registers and grid as adamw_kernel.
+template <bool HAS_G>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(16))) void adamw_unused_rows_kernel(
+    float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v, bf16* __restrict__ shadow, int64_t n,
+    const int32_t* __restrict__ first_use, int row, int off, int d, float lr, float b1, float b2, float eps, float wd, float bc1, float bc2,
+    float gscale, const float* __restrict__ hyper_dev) {
+  const AdamwScalars c = adamw_scalars(lr, b1, b2, eps, wd, bc1, bc2, gscale, nullptr, hyper_dev);
+  const int64_t n4 = n / 4, stride = (int64_t)gridDim.x * 256;
+  const int step_rows = (int)(stride * 4 / d), step_off = (int)(stride * 4 % d);
+  const int64_t at = (int64_t)off + (int64_t)blockIdx.x * 1024;
+  row += (int)(at / d);
+  off = (int)(at % d);
+  for (int64_t i = (int64_t)blockIdx.x * 256; i < n4; i += stride) {
+    const bool here = first_use[row] == INT32_MAX, next = off + 1024 > d && i + (d - off) / 4 < n4 && first_use[row + 1] == INT32_MAX;
+    if ((off + (int)threadIdx.x * 4 < d ? here : next) && threadIdx.x < (uint32_t)min(n4 - i, (int64_t)256))
+      adamw_vec<false, HAS_G>(p + i * 4, g + i * 4, m + i * 4, v + i * 4, shadow + i * 4, threadIdx.x, c);
+    row += step_rows;
+    off += step_off;
+    if (off >= d) off -= d, row++;
+  }
+}
+__global__ __launch_bounds__(256) void adamw_used_rows_kernel(
+    float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v, bf16* __restrict__ shadow,
+    const int32_t* __restrict__ ids, const int32_t* __restrict__ first_use, int64_t T, int V, int d, float lr, float b1, float b2, float eps,
+    float wd, float bc1, float bc2, float gscale, const float* __restrict__ hyper_dev) {
+  const AdamwScalars c = adamw_scalars(lr, b1, b2, eps, wd, bc1, bc2, gscale, nullptr, hyper_dev);
+  for (int64_t t = blockIdx.x; t < T; t += gridDim.x) {
+    const int row = wrap_clamp_id(ids[t], V);
+    if (first_use[row] != t) continue;
+    const int64_t o = (int64_t)row * d;
+    for (int j = 0; j < d; j += 1024)
+      if (j + (int)threadIdx.x * 4 < d) adamw_vec<false>(p + o + j, g + o + j, m + o + j, v + o + j, shadow + o + j, threadIdx.x, c);
   }
 }
 
@@ -549,6 +595,35 @@ extern "C" int32_t olmax_adamw_dev(hipStream_t stream, float* p, const void* g, 
 
 // Library-internal form with the grid size exposed: the overlapped train step runs it with one
 // workgroup per CU on its second stream, which disturbs the GEMMs it shares the GPU with least.
+int olmax_first_use(hipStream_t stream, const int32_t* ids, int32_t* first_use, int64_t T, int V) {
+  hipLaunchKernelGGL(fill_u32_kernel, dim3(grid_1d(V)), dim3(256), 0, stream, (uint32_t*)first_use, 0x7fffffffu, (int64_t)V);
+  hipLaunchKernelGGL(first_use_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, stream, ids, first_use, T, V);
+  OLMAX_LAUNCH_CHECK();
+  return OLMAX_OK;
+}
+
+int olmax_adamw_unused_rows(hipStream_t stream, float* p, const float* g, float* m, float* v, bf16* shadow, const int32_t* first_use, int64_t at,
+                            int64_t n, int d, float lr, float b1, float b2, float eps, float wd, int64_t step, int grid_cap,
+                            const float* hyper_dev) {
+  if (n == 0) return OLMAX_OK;
+  const float bc1 = (float)(1.0 - pow((double)b1, (double)step)), bc2 = (float)(1.0 - pow((double)b2, (double)step));
+  auto kern = g ? adamw_unused_rows_kernel<true> : adamw_unused_rows_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3(grid_1d(n / 4, grid_cap)), dim3(256), 0, stream, p + at, g ? g + at : nullptr, m + at, v + at, shadow + at, n,
+                     first_use, (int)(at / d), (int)(at % d), d, lr, b1, b2, eps, wd, bc1, bc2, 1.f, hyper_dev);
+  OLMAX_LAUNCH_CHECK();
+  return OLMAX_OK;
+}
+
+int olmax_adamw_used_rows(hipStream_t stream, float* p, const float* g, float* m, float* v, bf16* shadow, const int32_t* ids,
+                          const int32_t* first_use, int64_t T, int V, int d, float lr, float b1, float b2, float eps, float wd, int64_t step,
+                          const float* hyper_dev) {
+  const float bc1 = (float)(1.0 - pow((double)b1, (double)step)), bc2 = (float)(1.0 - pow((double)b2, (double)step));
+  hipLaunchKernelGGL(adamw_used_rows_kernel, dim3((unsigned)(T < 2048 ? T : 2048)), dim3(256), 0, stream, p, g, m, v, shadow, ids, first_use, T, V, d,
+                     lr, b1, b2, eps, wd, bc1, bc2, 1.f, hyper_dev);
+  OLMAX_LAUNCH_CHECK();
+  return OLMAX_OK;
+}
+
 int olmax_adamw_grid(hipStream_t stream, float* p, const void* g, float* m, float* v, void* shadow_bf16, int64_t n,
                      int32_t grad_is_bf16, float lr, float b1, float b2, float eps, float wd, int64_t step,
                      float grad_scale, const float* grad_scale_dev, int grid_cap, const float* hyper_dev) {

@@ -10,6 +10,7 @@
 // eqx.filter_value_and_grad, is written out by hand here.
 #include "common.h"
 #include "olmax_hip.h"
+#include <algorithm>
 
 namespace {
 
@@ -381,6 +382,7 @@ struct ModelWs {
   bf16 *da, *db;  // [T, d] gradient ping-pong
   void* head_ws;
   int64_t head_ws_bytes;
+  int32_t* first_use;  // [vocab], see EARLY_EMBEDDING
   Tmp tmp;
   char* acts_base;
   int64_t acts_stride;
@@ -394,6 +396,7 @@ ModelWs carve_model(const olmax_model_config* c, Arena& a, bool need_bwd) {
   w.db = a.take<bf16>(m.T * m.d);
   w.head_ws_bytes = olmax_lmhead_ce_workspace_bytes(m.T, c->vocab);
   w.head_ws = a.take<char>(w.head_ws_bytes);
+  w.first_use = a.take<int32_t>(c->vocab);
   if (need_bwd) w.tmp = carve_tmp(c, a);
   Arena probe(nullptr);
   carve_acts(c, probe);
@@ -607,7 +610,16 @@ struct OverlapCtx {
   int64_t head_done = 0;    // elements of it already updated
   int head_windows = 0;     // windows still to come
   int64_t layer_numel = 0;  // parameters of one layer (the size of a window's own update)
+  // A large embedding's rows that no token of the batch names are final with the head's gradients: their update is spread over the
+  // windows too, and only the rows of the batch wait for the end of the backward pass.
+  const int32_t *first_use = nullptr, *ids = nullptr;  // null: the embedding is updated whole at the end
+  int64_t T = 0, embed_numel = 0, embed_done = 0;
+  int vocab = 0, d = 0, layers = 0;
+  float embed_wd = 0.f;
+  bool tied = false;
 };
+// From this many parameters on the embedding's update takes the two parts: 0.4 ms or more at the end of a step.
+constexpr int64_t EARLY_EMBEDDING = 64 << 20;
 // AdamW launches the last olmax_model_train_step of this host thread put on its optimizer stream
 // (0: the step took the sequential branch); read back by tests through
 // olmax_model_last_step_overlapped_launches
@@ -640,6 +652,15 @@ int overlap_head_chunk(OverlapCtx* x, int64_t n, int grid_cap) {
                           lwd, x->step, 1.f, nullptr, grid_cap, x->hyper_dev);
 }
 
+// up to n more elements of the embedding's unnamed rows
+int overlap_embed_chunk(OverlapCtx* x, int64_t n, int grid_cap) {
+  n = std::min((n + 3) / 4 * 4, x->embed_numel - x->embed_done);
+  const int64_t at = x->embed_done;
+  x->embed_done += n;
+  return olmax_adamw_unused_rows(x->opt, x->master, x->tied ? x->grad_f32 : nullptr, x->mom, x->var, x->shadow, x->first_use, at, n, x->d, x->lr,
+                                 x->b1, x->b2, x->eps, x->embed_wd, x->step, grid_cap, x->hyper_dev);
+}
+
 int overlap_launch(OverlapCtx* x, int layer) {
   int begin = -1, end = -1;
   for (int i = 0; i < x->nleaf; i++) {
@@ -660,6 +681,11 @@ int overlap_launch(OverlapCtx* x, int layer) {
   // 43.1, 44.5, 45.3 ms with 64, 128, 192, 256, 384, 512 workgroups.  The updates that start when the backward pass is over (layer 0
   // and the embedding) have the GPU to themselves and take two per CU (5.5 TB/s).
   const int grid_cap = (layer == 0 || layer == -2) ? 512 : 256;
+  if (layer == -2 && x->first_use) {
+    RC(overlap_embed_chunk(x, x->embed_numel, grid_cap));  // (nothing left unless the model has no layers)
+    return olmax_adamw_used_rows(x->opt, x->master, x->grad_f32, x->mom, x->var, x->shadow, x->ids, x->first_use, x->T, x->vocab, x->d, x->lr, x->b1,
+                                 x->b2, x->eps, x->embed_wd, x->step, x->hyper_dev);
+  }
   if (layer == -1 && x->head_windows > 0) {
     // final norm now; of the LM head what a window holds, i.e. a layer's worth (the first window,
     // the top layer's recompute, has no layer update beside it); the rest follows in even shares
@@ -672,9 +698,12 @@ int overlap_launch(OverlapCtx* x, int layer) {
                         x->b2, x->eps, x->wd, x->leaf_decay, nullptr, grid_cap, x->hyper_dev));
       }
     }
-    if (x->head_leaf < 0) return OLMAX_OK;
-    x->head_windows--;
-    return overlap_head_chunk(x, (x->layer_numel + 3) / 4 * 4, grid_cap);
+    if (x->head_leaf >= 0) {
+      x->head_windows--;
+      RC(overlap_head_chunk(x, (x->layer_numel + 3) / 4 * 4, grid_cap));
+    }
+    // (of a tied model at least a layer's worth, for the same reason as the head's)
+    return x->first_use ? overlap_embed_chunk(x, std::max(x->tied ? x->layer_numel : 0, x->embed_numel / x->layers), grid_cap) : OLMAX_OK;
   }
   RC(adamw_leaves(x->opt, x->leaves, begin, end, x->master, x->mom, x->var, x->shadow, x->G, x->grad_f32, x->step, x->lr,
                   x->b1, x->b2, x->eps, x->wd, x->leaf_decay, nullptr, grid_cap, x->hyper_dev));
@@ -687,6 +716,7 @@ int overlap_launch(OverlapCtx* x, int layer) {
       x->head_windows--;
     }
   }
+  if (x->first_use && layer > 0) return overlap_embed_chunk(x, (x->embed_numel - x->embed_done + layer - 1) / layer, grid_cap);
   return OLMAX_OK;
 }
 
@@ -978,6 +1008,25 @@ extern "C" int32_t olmax_model_train_step(hipStream_t stream, hipStream_t opt_st
   int rc = OLMAX_OK;
   if (hipEventRecord(ev, stream) != hipSuccess || hipStreamWaitEvent(opt_stream, ev, 0) != hipSuccess)
     rc = olmax_set_error(OLMAX_ERR_LAUNCH, "olmax_model_train_step: event record/wait failed");
+  const Dims m = dims_of(c);
+  if (!rc && (int64_t)c->vocab * m.d >= EARLY_EMBEDDING && m.d >= 1024 && m.T < c->vocab && c->n_layers > 0 && ids && workspace &&
+      (((uintptr_t)workspace) & 255) == 0 && workspace_bytes >= olmax_model_workspace_bytes(c) && aligned16(master) && aligned16(mom) &&
+      aligned16(var) && aligned16(grad_f32) && aligned16(params_bf16)) {
+    Arena arena(workspace);
+    int32_t* first_use = carve_model(c, arena, true).first_use;
+    rc = olmax_first_use(stream, ids, first_use, m.T, c->vocab);
+    x.first_use = first_use;
+    x.ids = ids;
+    x.T = m.T;
+    x.vocab = c->vocab;
+    x.d = m.d;
+    x.layers = c->n_layers;
+    x.tied = c->tied;
+    x.embed_numel = (int64_t)c->vocab * m.d;
+    x.embed_wd = wd;
+    for (int i = 0; i < nleaf; i++)
+      if (leaves[i].kind == OLMAX_LEAF_EMBEDDING && leaf_decay && !leaf_decay[i]) x.embed_wd = 0.f;
+  }
   GradReady ready;
   ready.fn = overlap_ready;
   ready.ctx = &x;
