@@ -1190,10 +1190,12 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
                          (b_kc ? K : N) % 8 == 0;
   const int force_tile = g_force_tile.load(std::memory_order_relaxed);
   int parts;
-  int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, b_kc || force_tile || !aligned16(scratch.p) ? 0 : scratch.bytes, &parts);
-  if (parts > 1)
-    return (a_kc ? launch_split<true, false> : launch_split<false, false>)(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts,
-                                                                          (float*)scratch.p);
+  if ((b_kc && !a_kc) || force_tile || !aligned16(scratch.p)) scratch = GemmScratch();  // (no caller has that layout)
+  int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, scratch.bytes, &parts);
+  if (parts > 1) {
+    auto go = !a_kc ? launch_split<false, false> : b_kc ? launch_split<true, true> : launch_split<true, false>;
+    return go(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts, (float*)scratch.p);
+  }
   if (force_tile && direct_ok && K >= BK) {  // whatever the rule chose, if the problem has a tile of that size
     if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
     if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;

@@ -120,8 +120,8 @@ Tmp carve_tmp(const olmax_model_config* c, Arena& a) {
 
 // y[T,out] = x[T,in] W[out,in]^T (+ res)
 int lin_fwd(hipStream_t s, const bf16* x, int64_t ldx, const void* W, int in, int out, bf16* y, int64_t ldy,
-            const bf16* res, int64_t ldres, int64_t T) {
-  return olmax_gemm_bf16(s, x, W, y, res, (int)T, out, in, ldx, in, ldy, ldres, 0, 0, 0);
+            const bf16* res, int64_t ldres, int64_t T, GemmScratch ws = GemmScratch()) {
+  return olmax_gemm_padded(s, x, (const bf16*)W, y, res, (int)T, out, in, ldx, in, ldy, ldres, true, true, false, false, ws);
 }
 // dx[T,in] = dy[T,out] W[out,in] (+ res)
 int lin_dx(hipStream_t s, const bf16* dy, int64_t lddy, const void* W, int in, int out, bf16* dx, int64_t lddx,
@@ -140,6 +140,7 @@ int lin_grads(hipStream_t s, const bf16* dy, int64_t lddy, const void* W, const 
   return olmax_gemm_grads(s, dy, (const bf16*)W, x, dx, res, dW, (int)T, in, out, lddy, in, ldx, lddx, ldres, in, false, false, ws);
 }
 
+// ws: for partial results of the products (none of the buffers of `a`).
 // need_y == false (recompute before the backward): the block output itself is not an input of
 // the backward pass, so the GEMM / norm that only produces it is skipped.
 // Points inside a block's backward pass at which the overlapped train step may start queued
@@ -157,7 +158,7 @@ inline int hook_point(int point) { return g_hook.fn ? g_hook.fn(g_hook.ctx, poin
 // (olmax_gemm_glu_bwd_bf16), so gate | up are never written.
 int block_forward(hipStream_t s, const olmax_model_config* c, const olmax_block_weights* w, int window,
                   const float* cos_t, const float* sin_t, const bf16* x, bf16* y, const Acts& a,
-                  bool need_y = true, bool save_gu = true, bool defer_mlp = false) {
+                  GemmScratch ws, bool need_y = true, bool save_gu = true, bool defer_mlp = false) {
   const Dims m = dims_of(c);
   const int lt = c->layer_type;
   const float eps = c->eps;
@@ -199,9 +200,9 @@ int block_forward(hipStream_t s, const olmax_model_config* c, const olmax_block_
   RC(olmax_attn_fwd(s, qp, kp, a.qkv + m.HD + m.KD, a.o, a.lse, m.B, m.S, m.H, m.K, m.D, ldqk, ldqk, m.QKV, m.HD,
                     window, c->attn_softcap));
   if (lt == 0) {
-    RC(lin_fwd(s, a.o, m.HD, w->wo, m.HD, m.d, a.h, m.d, x, m.d, m.T));
+    RC(lin_fwd(s, a.o, m.HD, w->wo, m.HD, m.d, a.h, m.d, x, m.d, m.T, ws));
   } else {
-    RC(lin_fwd(s, a.o, m.HD, w->wo, m.HD, m.d, a.a_out, m.d, nullptr, 0, m.T));
+    RC(lin_fwd(s, a.o, m.HD, w->wo, m.HD, m.d, a.a_out, m.d, nullptr, 0, m.T, ws));
     RC(olmax_rmsnorm_fwd_res(s, a.a_out, w->attn_norm, x, a.h, m.T, m.d, m.d, m.d, m.d, eps));
   }
   const bf16* mlp_in = a.h;
@@ -216,9 +217,9 @@ int block_forward(hipStream_t s, const olmax_model_config* c, const olmax_block_
   RC(olmax_gemm_glu_bf16(s, mlp_in, w->wgu, (save_gu || !fused) ? a.gu : nullptr, a.act, (int)m.T, m.F, m.d, m.d,
                          m.d, 2 * m.F, m.F, c->act));
   if (lt == 0) {
-    if (need_y) RC(lin_fwd(s, a.act, m.F, w->wdown, m.F, m.d, y, m.d, a.h, m.d, m.T));
+    if (need_y) RC(lin_fwd(s, a.act, m.F, w->wdown, m.F, m.d, y, m.d, a.h, m.d, m.T, ws));
   } else {
-    RC(lin_fwd(s, a.act, m.F, w->wdown, m.F, m.d, a.m_out, m.d, nullptr, 0, m.T));
+    RC(lin_fwd(s, a.act, m.F, w->wdown, m.F, m.d, a.m_out, m.d, nullptr, 0, m.T, ws));
     if (need_y) RC(olmax_rmsnorm_fwd_res(s, a.m_out, w->mlp_norm, a.h, y, m.T, m.d, m.d, m.d, m.d, eps));
   }
   return OLMAX_OK;
@@ -481,7 +482,7 @@ int model_run(hipStream_t s, const olmax_model_config* c, const int32_t* windows
     Arena aa(w.acts_base + (keep ? (int64_t)l * w.acts_stride : 0));
     Acts acts = carve_acts(c, aa);
     RC(block_forward(s, c, &bw, windows[l], cos_tables[l], sin_tables[l], w.xs + (int64_t)l * Td,
-                     w.xs + (int64_t)(l + 1) * Td, acts, true, keep));
+                     w.xs + (int64_t)(l + 1) * Td, acts, w.tmp.in_mlp(), true, keep));
   }
   Range rg_head("olmax.lm_head_and_loss", 0);
   const bf16* xl = w.xs + (int64_t)nl * Td;
@@ -534,7 +535,7 @@ int model_run(hipStream_t s, const olmax_model_config* c, const int32_t* windows
     }
     if (!keep) {
       // full-block recompute of everything the backward reads
-      RC(block_forward(s, c, &bw, windows[l], cos_tables[l], sin_tables[l], xin, dnext, acts, false, true, defer));
+      RC(block_forward(s, c, &bw, windows[l], cos_tables[l], sin_tables[l], xin, dnext, acts, w.tmp.in_mlp(), false, true, defer));
     }
     RC(block_backward(s, c, &bw, &bg, windows[l], cos_tables[l], sin_tables[l], xin, dcur, dnext, acts, w.tmp, defer));
     RC(ready(l));
@@ -778,11 +779,17 @@ extern "C" int32_t olmax_model_layout(const olmax_model_config* c, olmax_leaf* o
   return n;
 }
 
-extern "C" int64_t olmax_block_acts_bytes(const olmax_model_config* c) {
-  if (check_cfg(c)) return -1;
+// What a block keeps for its backward pass, and room behind it for the parts of its forward products' reductions: eight for every tile of the
+// output, up to one for each CU (the whole-model step has the attention part's backward buffers for it).
+static int64_t acts_bytes_of(const olmax_model_config* c) {
   Arena a(nullptr);
   carve_acts(c, a);
   return a.off;
+}
+extern "C" int64_t olmax_block_acts_bytes(const olmax_model_config* c) {
+  if (check_cfg(c)) return -1;
+  const Dims m = dims_of(c);
+  return acts_bytes_of(c) + (std::min<int64_t>(256, (m.T + 255) / 256 * ((m.d + 255) / 256) * 8) << 18);
 }
 extern "C" int64_t olmax_block_tmp_bytes(const olmax_model_config* c) {
   if (check_cfg(c)) return -1;
@@ -802,11 +809,11 @@ extern "C" int32_t olmax_block_fwd(hipStream_t s, const olmax_model_config* c, c
                                    void* acts, int64_t acts_bytes) {
   RC(check_cfg(c));
   OLMAX_CHECK(w && cos_t && sin_t && x && y && acts, OLMAX_ERR_ARG, "olmax_block_fwd: null pointer");
-  OLMAX_CHECK(acts_bytes >= olmax_block_acts_bytes(c) && (((uintptr_t)acts) & 255) == 0, OLMAX_ERR_WORKSPACE,
+  OLMAX_CHECK(acts_bytes >= acts_bytes_of(c) && (((uintptr_t)acts) & 255) == 0, OLMAX_ERR_WORKSPACE,
               "olmax_block_fwd: activation buffer too small or not 256-byte aligned");
   Arena a(acts);
   Acts ac = carve_acts(c, a);
-  return block_forward(s, c, w, window, cos_t, sin_t, (const bf16*)x, (bf16*)y, ac);
+  return block_forward(s, c, w, window, cos_t, sin_t, (const bf16*)x, (bf16*)y, ac, GemmScratch{a.base + a.off, acts_bytes - a.off});
 }
 
 extern "C" int32_t olmax_block_bwd(hipStream_t s, const olmax_model_config* c, const olmax_block_weights* w,
@@ -815,7 +822,7 @@ extern "C" int32_t olmax_block_bwd(hipStream_t s, const olmax_model_config* c, c
                                    int64_t tmp_bytes) {
   RC(check_cfg(c));
   OLMAX_CHECK(w && g && cos_t && sin_t && x && dy && dx && acts && tmp, OLMAX_ERR_ARG, "olmax_block_bwd: null pointer");
-  OLMAX_CHECK(acts_bytes >= olmax_block_acts_bytes(c) && tmp_bytes >= olmax_block_tmp_bytes(c) &&
+  OLMAX_CHECK(acts_bytes >= acts_bytes_of(c) && tmp_bytes >= olmax_block_tmp_bytes(c) &&
                   (((uintptr_t)acts) & 255) == 0 && (((uintptr_t)tmp) & 255) == 0,
               OLMAX_ERR_WORKSPACE, "olmax_block_bwd: workspace too small or not 256-byte aligned");
   Arena a(acts);
