@@ -1232,8 +1232,9 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
     const int kt = (K + BK - 1) / BK;
     // (the 0.6 us: one round of 64 tiles, measured at 4 to 128 k-tiles; pick_tile's boundaries were measured without)
     const int edge = !force_tile && cost_32(n32, kt, a_kc) < cost_64(n64, kt) + 0.6f ? 32 : 64;
-    // eight waves share a tile while there are not more tiles than CUs, else two workgroups fit a CU; a 32 tile needs them from 16 k-tiles on
-    const int groups = edge == 64 ? (n64 <= 256 ? 8 : 4) : (n32 <= 256 && kt >= 16 ? 8 : 4);
+    // eight waves share a tile while there are not more 64 tiles than CUs, else two workgroups fit a CU.  (A 32 tile does as well with four, 300 x 1024 x 2816
+    // 11.0 us against 11.6, but a chain of fp32 additions twice as long is 7 to 29 % further from the exact sum; up to four k-tiles there is none.)
+    const int groups = n64 <= 256 && (edge == 64 || kt > 4) ? 8 : 4;
     olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, edge, groups);
     if (g_prof_on) {
       (void)hipEventRecord(rec.e1, stream);
@@ -1324,7 +1325,8 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
   };
   float best = alone(T, in, out, true) + alone(out, in, T, false);
   int tile = 0;  // of the one launch, 0: two calls
-  if (const float c = pair_small(T, in, out); c < best && out % 8 == 0 && in % 8 == 0 && T >= 64) best = c, tile = 64;
+  // (bf16 gradients: the four waves' longer chains of fp32 additions are 1e-8 of the sum, and would show in an fp32 one)
+  if (const float c = pair_small(T, in, out); c < best && !dw_f32 && out % 8 == 0 && in % 8 == 0 && T >= 64) best = c, tile = 64;
   // whole chunks and vector stores, whole k-tiles in the first product
   const bool direct = !dw_f32 && out % BK == 0 && in % 8 == 0 && lddy % 8 == 0 && ldw % 8 == 0 && ldx % 8 == 0 && lddx % 8 == 0 && lddw % 8 == 0 &&
                       (!r || (ldr % 8 == 0 && aligned16(r))) && aligned16(dy) && aligned16(w) && aligned16(x) && aligned16(dx) && aligned16(dw);
@@ -1343,7 +1345,7 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
     }
     bool done = true;
     if (tile == 64) {
-      done = olmax_gemm_small_pair(s, dy, w, x, dx, r, dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw, dw_f32);
+      done = olmax_gemm_small_pair(s, dy, w, x, dx, r, (bf16*)dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw);
     } else {
       const PairSide px = {dy, w, r, dx, T, in, out, lddy, ldw, lddx, ldr}, pw = {dy, x, nullptr, (bf16*)dw, out, in, T, lddy, ldx, lddw, 0};
       const bool rx = T % tile || in % tile;

@@ -13,7 +13,7 @@
 // 128 x 128 tiles, 32 us here; 300 x 1024 x 2816: 31 -> 12.7 us; the bounds-checked scalar kernel it
 // also replaces ran at 5-20 TFLOP/s (77 x 2816 x 1024: 47 -> 7 us).
 // Where not even 64 x 64 tiles find a CU each, 32 x 32 ones do: half the bytes per k-tile and wave, four times the CUs.
-// us, 64 -> 32: 256 x 256 x 2048 11.5 -> 8.8, 16 x 4096 x 4096 17.9 -> 11.3, 512 x 256 x 768 7.2 -> 4.8.  (Two or four k-tiles in
+// us, 64 -> 32: 256 x 256 x 2048 11.5 -> 8.8, 16 x 4096 x 4096 17.9 -> 11.3, 512 x 256 x 768 7.2 -> 5.1.  (Two or four k-tiles in
 // flight per wave instead of one: no change with either tile, so it is not the latency of one load that is waited for.)
 // Operands travel as 8 rows of 128 B per instruction into registers (the next k-tile's while this one is
 // multiplied), are parked in the wave's own LDS slabs and read back as MFMA fragments (k-contiguous:
@@ -368,12 +368,12 @@ void olmax_gemm_small(hipStream_t s, const bf16* A, const bf16* B, void* C, cons
   }
 }
 
-bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, void* dw, int T, int in,
-                           int out, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw, bool dw_f32) {
+bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, bf16* dw, int T, int in,
+                           int out, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw) {
   // whole chunks, 32-bit line offsets and at least a tile of rows: the one mode that is built
   if (out % 8 || in % 8 || T < 64 || lddy >= (1 << 25) || ldw >= (1 << 25) || ldx >= (1 << 25)) return false;
   const Problem px = {dy, w, dx, r, T, in, out, lddy, ldw, lddx, ldr, 0};
-  const Problem pw = {dy, x, dw, nullptr, out, in, T, lddy, ldx, lddw, 0, dw_f32};
+  const Problem pw = {dy, x, dw, nullptr, out, in, T, lddy, ldx, lddw, 0, 0};
   // tiles of 32 while they find a CU each
   auto go = tiles<32>(px) <= 256 ? (tiles<32>(pw) <= 256 ? launch_pair<32, 32> : launch_pair<32, 64>)
                                  : (tiles<32>(pw) <= 256 ? launch_pair<64, 32> : launch_pair<64, 64>);

@@ -40,7 +40,7 @@ def test_both_gradients_in_one_launch(T, d, V, pair, f32):
     labels = torch.arange(T, device="cuda", dtype=torch.int32) * 7 % V
     out = []
     got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels, dw_f32=f32)))
-    assert any(key >> 19 & 1 for key, *_ in got) == pair, got
+    assert any(key >> 19 & 1 for key, *_ in got) == (pair and not f32), got  # (fp32 results keep the kernels with the shorter chains)
     check_gradients(h, W, labels, *out[1:])
 
 
