@@ -321,7 +321,7 @@ def main():
         k = keys[i]
         name = "gemm_%s_kernel<tile%d,%s,%s%s%s%s>" % ("small" if k & 0xfff == 64 else "bf16", k & 0xfff, "A_KC" if k >> 12 & 1 else "A_MC", "B_KC" if k >> 13 & 1 else "B_NC",
                                                             ",res" if k >> 14 & 1 else "", ",f32out" if k >> 15 & 1 else "",
-                                                            ",glu" if k >> 16 & 1 else ",rope" if k >> 17 & 1 else ",shared" if k >> 18 & 1 else "")
+                                                            ",glu" if k >> 16 & 1 else ",rope" if k >> 17 & 1 else ",shared" if k >> 18 & 1 else ",both gradients" if k >> 19 & 1 else "")
         per.append({"kernel": name, "key": k, "launches": ln[i], "total_ms": ms[i], "avg_ms": ms[i] / ln[i],
                     "tflops": fl[i] / ms[i] / 1e9, "algorithmic_bytes_per_launch": by[i] / ln[i]})
     per.sort(key=lambda r: -r["total_ms"])
