@@ -369,6 +369,8 @@ typedef struct {
   void *wqkv, *wo, *wgu, *wdown;                /* bf16, overwritten */
   float *attn_norm, *mlp_norm, *attn_in_norm, *mlp_in_norm, *q_norm, *k_norm; /* fp32, accumulated */
 } olmax_block_grads;
+/* What a block keeps for its backward pass and room behind it for partial results of its forward products (64 MB at most); a buffer
+ * without that room is taken too, and the products then run without it. */
 int64_t olmax_block_acts_bytes(const olmax_model_config* cfg);
 int64_t olmax_block_tmp_bytes(const olmax_model_config* cfg);
 int32_t olmax_block_fwd(olmax_stream_t stream, const olmax_model_config* cfg, const olmax_block_weights* w,
