@@ -180,7 +180,9 @@ __global__ __launch_bounds__(THREADS) void ce_row_kernel(
 //
 // Bound by memory (8192 x 50304: 1.65 GB in 320 us = 5.1 TB/s) as long as the vector instructions stay below it,
 // about 12 a logit: the maximum is taken of raw values, missing logits are minus infinity instead of a test in each pass,
-// only the one vector that holds the label looks for it, and the gradient's exponential is one fma and exp2.
+// only the one vector that holds the label looks for it, and the gradient's exponential is one fma and exp2.  The fma's
+// constant lse * log2(e) is rounded: half an ulp of it is a factor of exp(1.1e-5) at 256, exp(0.04) at 1e6, and infinite at the type's lowest
+// value.  From 256 on (and for the label's vector) lse is subtracted first, which is exact where it matters.
 template <bool CAP, int THREADS, int MAXV, bool PAD, bool TAIL>
 __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
     const bf16* __restrict__ logits, bf16* __restrict__ dlogits, const int32_t* __restrict__ labels,
@@ -299,9 +301,10 @@ __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
   // d(reduced loss) / d(row loss): 1/n for "mean", 1 for "sum", the row's own cotangent for "none"
   const float scale = (counted && inrange) ? dloss * (drow ? drow[row] : 1.f) / (mean ? (float)(*n_counted) : 1.f) : 0.f;
   const float lse2 = lse * LOG2E;
+  const bool far = !(fabsf(lse) < 256.f);
   auto store = [&](int idx, const Pack8& v) {
     Pack8 o;
-    auto grads = [&](auto has_label) {
+    auto grads = [&](auto general) {
 #pragma unroll
       for (int e = 0; e < 8; e++) {
         float z = bf2f(v.e[e]), chain = 1.f;
@@ -310,12 +313,12 @@ __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
           z = cap * t;
           chain = 1.f - t * t;
         }
-        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(z, LOG2E, -lse2));
-        if (has_label && idx * 8 + e == label) p -= 1.f;
+        float p = general ? __expf(z - lse) : __builtin_amdgcn_exp2f(__builtin_fmaf(z, LOG2E, -lse2));
+        if (general && idx * 8 + e == label) p -= 1.f;
         o.e[e] = f2bf(p * scale * chain);
       }
     };
-    if (idx == label >> 3) grads(std::true_type());
+    if (far || idx == label >> 3) grads(std::true_type());
     else grads(std::false_type());
     if (PAD && idx == nvec - 1) {
 #pragma unroll

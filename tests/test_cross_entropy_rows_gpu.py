@@ -49,3 +49,27 @@ def test_padded_rows(V, cap):
     for got, want in ((dW, d.t() @ h.double()), (dh, d @ W.double())):
         assert ((got.cpu().double() - want).norm() / want.norm()).item() < 2 ** -8
     assert ((dW.cpu().double() - d.t() @ h.double())[-8:].norm() / (d.t() @ h.double())[-8:].norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("V", [4096, 51200, 163840, 163848 + 8 * 4096])
+def test_rows_far_from_zero(V):
+    """Logits whose sum of exponentials lies where half an ulp of lse * log2(e) is not small: rows about 1000 and 1e6, a row of the
+    type's lowest value (its lse rounds to the logit: exp(0) each), and one logit above such a mask.  The bound is lse's own
+    rounding, 2^-24 of it, and a bf16 store."""
+    from olmax_amd import ops
+    print(f"[case] ce far V{V}", flush=True)
+    low = torch.finfo(torch.bfloat16).min
+    z = torch.full((4, V), low)
+    z[0] = torch.randint(0, 4, (V,), generator=torch.Generator().manual_seed(V)) * 4.0 + 1000
+    z[1] = -1e6
+    z[3, 9] = 2.0
+    z = z.to(torch.bfloat16)
+    labels = torch.tensor([1, 2, 3, 9], dtype=torch.int32)
+    loss, dz, lse = ops.cross_entropy(z.cuda(), labels.cuda())
+    zd = z.double()
+    p = (zd - lse.cpu().double()[:, None]).exp()  # against the lse that the row has in fp32
+    assert torch.isfinite(dz).all()
+    want = p / 4
+    want[torch.arange(4), labels.long()] -= 0.25
+    err = (dz.cpu().double() - want).abs() - (2 ** -8 * want.abs() + 2 ** -22 / 4)
+    assert err.max().item() <= 0, (err.argmax().item() // V, err.argmax().item() % V)
