@@ -1115,10 +1115,13 @@ static float cost_256(int64_t n, int kt, int64_t bytes, bool b_kc) {
   return cost_rounds(n - r, kt) + last;
 }
 static float cost_64(int64_t n, int kt) { return ((n + 255) / 256) * (0.22f * kt + 1.2f) + 2.4f; }
-// 32 tiles: 0.165 us per k-tile while each has a CU, 0.235 (0.30 where A is [K, M], whose lines are then 64 bytes) with two on every CU
+// 32 tiles: 0.165 us per k-tile while each has a CU, 0.235 (0.30 where A is [K, M], whose lines are then 64 bytes) with two on every CU; from 1024 on
+// 0.8 us for each further 512, so that larger tiles take many short ones (us in 32 tiles, and so: 8191 x 4099 x 64 54, 24; 2048 x
+// 1024 x 16 6.7, 5.6; but 1024 x 1024 x 16 4.4, 4.9).
 static float cost_32(int64_t n, int kt, bool a_kc) {
   const float two = a_kc ? 0.235f : 0.30f;
-  return 3.6f + kt * (n <= 256 ? 0.165f : n <= 512 ? 0.165f + (two - 0.165f) * (n - 256) / 256.f : two * n / 512.f);
+  if (n <= 512) return 3.6f + kt * (n <= 256 ? 0.165f : 0.165f + (two - 0.165f) * (n - 256) / 256.f);
+  return 3.6f + two * kt * n / 512.f + (n > 1024 ? 0.8f * (n - 1024) / 512.f : 0.f);
 }
 static int64_t tiles_of(int M, int N, int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); }
 static float cost_small(int M, int N, int kt, bool a_kc) { return std::min(cost_64(tiles_of(M, N, 64), kt), cost_32(tiles_of(M, N, 32), kt, a_kc)); }

@@ -28,6 +28,19 @@ def test_tiles_of_32(M, N, K, al, bl):
     assert ((ops.gemm(a, b, a_layout=al, b_layout=bl, out_f32=True).double() - want).abs() <= scale).all()
 
 
+@pytest.mark.parametrize("M,N,bl", [(3000, 8200, 0), (4096, 4096, 1)])
+def test_one_k_tile_of_many_outputs(M, N, bl):
+    """A single k-tile over many outputs goes to 128 or 256 tiles: thousands of 32 x 32 ones take twice as long.  Bounds as above."""
+    from olmax_amd import ops
+    print(f"[case] one k-tile M{M} N{N} b{bl}", flush=True)
+    a, b = operands(M, N, 64, 0, bl)
+    out = []
+    got = recorded(lambda: out.append(ops.gemm(a, b, b_layout=bl)))
+    assert all(key & 0xfff != 64 for key, *_ in got) and got, got
+    want = a.double() @ (b.t() if bl == 0 else b).double()
+    assert ((out[0].double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -22 * 48).all()
+
+
 @pytest.mark.parametrize("T,d,V,pair", [(2048, 256, 4096, True), (64, 1024, 512, True), (100, 264, 520, True), (1001, 64, 2056, True),
                                         (2048, 1024, 256, True), (65, 40, 72, True), (300, 256, 1003, False), (63, 256, 512, False)])
 @pytest.mark.parametrize("f32", [False, True])
