@@ -73,3 +73,33 @@ def test_rows_far_from_zero(V):
     want[torch.arange(4), labels.long()] -= 0.25
     err = (dz.cpu().double() - want).abs() - (2 ** -8 * want.abs() + 2 ** -22 / 4)
     assert err.max().item() <= 0, (err.argmax().item() // V, err.argmax().item() % V)
+
+
+@pytest.mark.parametrize("V", [16392, 51200, 51208, 102400, 51199, 102397])
+@pytest.mark.parametrize("cap", [0.0, 20.0])
+@pytest.mark.parametrize("T", [256, 257])
+def test_number_of_rows(V, cap, T):
+    """Up to 256 rows take more threads each.  Bounds as above, the padded ones in the norm of dW and dh."""
+    from olmax_amd import ops
+    print(f"[case] ce T{T} V{V} cap{cap}", flush=True)
+    g = torch.Generator().manual_seed(V)
+    labels = torch.arange(T, dtype=torch.int32) * 977 % V
+    labels[-1] = V - 1
+    if V % 8 == 0:
+        few = (torch.randn(4, V, generator=g) * 3).to(torch.bfloat16).cuda()
+        z = few.repeat((T + 3) // 4, 1)[:T]
+        loss, d, lse = ops.cross_entropy(z, labels.cuda(), softcap=cap)
+        rows = [0, 1, 255, T - 1]
+        zr = z[rows].cpu()
+        want = ref.cross_entropy_bwd(zr.double(), labels[rows].long(), softcap=cap) * (4 / T)
+        err = (d[rows].cpu().double() - want).abs() - (2 ** -8 * want.abs() + 2 ** -22 / T)
+        assert err.max().item() <= 0
+        assert (lse.view(-1)[4:] == lse[:-4]).all()
+        return
+    h = torch.randn(T, 64, generator=g).to(torch.bfloat16).cuda()
+    W = (torch.randn(V, 64, generator=g) * 0.1).to(torch.bfloat16).cuda()
+    loss, dh, dW = ops.lmhead_ce(h, W, labels.cuda(), softcap=cap, dw_f32=True)
+    z = (h.double() @ W.double().t()).to(torch.bfloat16).double().cpu()
+    d = ref.cross_entropy_bwd(z, labels.long(), softcap=cap).cuda()
+    for got, want in ((dW, d.t() @ h.double()), (dh, d @ W.double())):
+        assert ((got.double() - want).norm() / want.norm()).item() < 2 ** -7
