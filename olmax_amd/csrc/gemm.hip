@@ -1339,6 +1339,10 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
     const Work &l = wx.kt > ww.kt ? wx : ww, &sh = wx.kt > ww.kt ? ww : wx;
     if (const float c = t == 128 ? pair_128(l, sh) : pair_256(l, sh); c < best) best = c, tile = t;
   }
+  // dW may take the place of W or of the residual, which the first product alone reads: not beside it
+  auto meet = [](const void* p, int64_t n, const void* q, int64_t m) { return p && q && (uintptr_t)p < (uintptr_t)q + m && (uintptr_t)q < (uintptr_t)p + n; };
+  const int64_t dw_bytes = ((out - 1) * lddw + in) * (dw_f32 ? 4 : 2);
+  if (meet(dw, dw_bytes, w, ((out - 1) * ldw + in) * 2) || meet(dw, dw_bytes, r, ((T - 1) * ldr + in) * 2)) tile = 0;
   if (tile && !g_force_tile.load(std::memory_order_relaxed)) {
     ProfRec rec{};
     if (g_prof_on) {

@@ -113,3 +113,19 @@ def test_a_residual_joins_the_first_product(seq):
     assert not any(key >> 19 & 1 for key, *_ in got), got
     for a, b in zip(res[0], [dx[1]] + list(block.grads.values())):
         assert ((a.double() - b.double()).norm() / b.double().norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("T,d,V", [(2048, 256, 4096), (2048, 1024, 256), (4096, 1024, 3072), (2000, 11008, 4096)])
+def test_a_weight_gradient_in_the_place_of_the_weights(T, d, V):
+    """dh reads the weights first, so dW may overwrite them: the products stay in their order, at sizes where one launch would take
+    both.  Bounds as above, which hold for logits of a few units: at a spread of 10 a label's 1 - p may be of the size of the logits' own
+    rounding, 2^-9 of 30."""
+    from olmax_amd import ops
+    print(f"[case] dW over W T{T} d{d} V{V}", flush=True)
+    h, W = rnd(T, d, seed=1), rnd(V, d, seed=2, scale=2 * d ** -0.5)
+    labels = torch.arange(T, device="cuda", dtype=torch.int32) * 7 % V
+    assert any(key >> 19 & 1 for key, *_ in recorded(lambda: ops.lmhead_ce(h, W, labels)))
+    kept, out = W.clone(), []
+    got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels, dW=W)))
+    assert not any(key >> 19 & 1 for key, *_ in got), got
+    check_gradients(h, kept, labels, *out[1:])
