@@ -786,10 +786,13 @@ static int64_t acts_bytes_of(const olmax_model_config* c) {
   carve_acts(c, a);
   return a.off;
 }
+static int64_t acts_room_of(const olmax_model_config* c) {
+  const Dims m = dims_of(c);
+  return std::min<int64_t>(256, (m.T + 255) / 256 * ((m.d + 255) / 256) * 8) << 18;
+}
 extern "C" int64_t olmax_block_acts_bytes(const olmax_model_config* c) {
   if (check_cfg(c)) return -1;
-  const Dims m = dims_of(c);
-  return acts_bytes_of(c) + (std::min<int64_t>(256, (m.T + 255) / 256 * ((m.d + 255) / 256) * 8) << 18);
+  return acts_bytes_of(c) + acts_room_of(c);
 }
 extern "C" int64_t olmax_block_tmp_bytes(const olmax_model_config* c) {
   if (check_cfg(c)) return -1;
@@ -813,7 +816,8 @@ extern "C" int32_t olmax_block_fwd(hipStream_t s, const olmax_model_config* c, c
               "olmax_block_fwd: activation buffer too small or not 256-byte aligned");
   Arena a(acts);
   Acts ac = carve_acts(c, a);
-  return block_forward(s, c, w, window, cos_t, sin_t, (const bf16*)x, (bf16*)y, ac, GemmScratch{a.base + a.off, acts_bytes - a.off});
+  const int64_t room = std::min(acts_bytes - a.off, acts_room_of(c));  // what lies behind it in a larger buffer is the caller's
+  return block_forward(s, c, w, window, cos_t, sin_t, (const bf16*)x, (bf16*)y, ac, GemmScratch{a.base + a.off, room});
 }
 
 extern "C" int32_t olmax_block_bwd(hipStream_t s, const olmax_model_config* c, const olmax_block_weights* w,
