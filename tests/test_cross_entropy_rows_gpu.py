@@ -103,3 +103,27 @@ def test_number_of_rows(V, cap, T):
     d = ref.cross_entropy_bwd(z, labels.long(), softcap=cap).cuda()
     for got, want in ((dW, d.t() @ h.double()), (dh, d @ W.double())):
         assert ((got.double() - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("V", [4096, 16392])
+@pytest.mark.parametrize("at", [20, 50, 250])
+def test_gradients_round_as_the_exact_ones(V, at):
+    """Rows about `at`: gradients that round to another bf16 than the exact ones (against the lse that the row has).  A relative error e of the
+    probability flips 185 |e| of them, the mean of p / ulp(p) over a binade: 4e-7, a few fp32 operations of 2^-24 each, 7e-5.  The
+    rounding of lse * log2(e), not taken back, would add half an ulp of it, 1e-6 at 20 and 1e-5 at 250."""
+    from olmax_amd import ops
+    print(f"[case] ce rounding V{V} at{at}", flush=True)
+    T = 8192  # a power of two: 1 / T is exact
+    g = torch.Generator(device="cuda").manual_seed(V)
+    z = (torch.randn(T, V, device="cuda", generator=g) * 4 + at - 12 + torch.rand(T, 1, device="cuda", generator=g) * 4).to(torch.bfloat16)
+    labels = torch.full((T,), V - 1, dtype=torch.int32, device="cuda")
+    d, lse = ops.cross_entropy(z, labels)[1:]
+    wrong = total = 0
+    for i in range(0, T, 1024):
+        p = (z[i:i + 1024, :-8].double() - lse.view(-1)[i:i + 1024, None].double()).exp() / T
+        big = p > 2 ** -100  # (no underflow)
+        # to bf16 by fp32 would round twice: half a unit added to the bits of the double, ties have no weight here
+        want = ((p.view(torch.int64) + (1 << 44)) >> 45 << 45).view(torch.float64)
+        wrong += int(((d[i:i + 1024, :-8].double() != want) & big).sum())
+        total += int(big.sum())
+    assert wrong / total < 1.25e-4, wrong / total
