@@ -178,7 +178,7 @@ __global__ __launch_bounds__(THREADS) void ce_row_kernel(
 // TAIL: a longer row; what the registers do not hold is reduced online and read a second time, right after
 // (4096 x 262144: 1.26 ms all read twice by 4 waves, 1.10 by 16, 1.04 with half of the row held).
 //
-// Bound by memory (8192 x 50304: 1.65 GB in 320 us = 5.1 TB/s) as long as the vector instructions stay below it,
+// Bound by memory (8192 x 50304: 1.65 GB in 316 us = 5.2 TB/s) as long as the vector instructions stay below it,
 // about 12 a logit: the maximum is taken of raw values, missing logits are minus infinity instead of a test in each pass,
 // only the one vector that holds the label looks for it, and the gradient's exponential is one fma and exp2.  The fma's
 // constant lse * log2(e) is rounded: half an ulp of it is a factor of exp(1.1e-5) at 256 (0.04 in the exponent at 1e6, and infinite at the type's
@@ -272,7 +272,8 @@ __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
   const float tmx = mx;
   float rmx = -INFINITY;  // of the raw logits: the soft-cap rises with them
   // each pass unpacks a vector when its turn comes: hidden from the compiler, which otherwise keeps all
-  // unpacked logits of a pass for the next and spills
+  // unpacked logits of a pass for the next and spills; so it did with the offsets of 25 vectors, loaded with and kept for the
+  // stores (13 to 18 registers, up to 76 bytes a lane: 8192 x 100352 715 us, 621 with the offsets computed again)
   auto keep = [](Pack8& v) {
     asm volatile("" : "+v"(v.u));
     __builtin_amdgcn_sched_barrier(0);
@@ -343,7 +344,9 @@ __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
   }
 #pragma unroll
   for (int i = 0; i < MAXV; i++) {
-    const int idx = i * THREADS + threadIdx.x;
+    int tid = threadIdx.x;
+    if (MAXV >= 25 || TAIL) asm volatile("" : "+v"(tid));
+    const int idx = i * THREADS + tid;
     keep(c[i]);
     if (idx < nvec) store(idx, c[i]);
   }
@@ -404,8 +407,8 @@ static int cross_entropy(hipStream_t stream, const void* logits, void* dlogits, 
     if (cap) CE_GO(float, true, 256); else CE_GO(float, false, 256);
   } else if (regs_ok && V <= 1024 * 8 * 20) {
     // The fewest threads that hold the row, so that as many rows as possible are on a CU in different phases: us with the
-    // workgroup below | the one of 512 threads x 26 vectors (1024 x 20) that held all rows: 2048 x 4096 20 | 46, 1500 x 16384 27 | 51, 8192 x 50304 320 | 425,
-    // 8192 x 100352 680 | 740, 4096 x 128256 424 | 493 (the last two only from the arithmetic).  Up to 256 rows each have a CU to
+    // workgroup below | the one of 512 threads x 26 vectors (1024 x 20) that held all rows: 2048 x 4096 20 | 46, 1500 x 16384 27 | 51, 8192 x 50304 316 | 425,
+    // 8192 x 100352 609 | 740, 4096 x 128256 424 | 493 (the last two only from the arithmetic).  Up to 256 rows each have a CU to
     // themselves and take twice the threads: 16 x 50304 12.6 | 16.4 (256 threads 16.9), 256 x 50304 17.6 | 20.9 (22.7),
     // 256 x 100352 29.7 | 32.9 (512 threads 34.7).
     if (V <= 256 * 8 * 2) CE_REGS(256, 2);
