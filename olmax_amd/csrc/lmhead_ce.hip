@@ -408,12 +408,12 @@ static int cross_entropy(hipStream_t stream, const void* logits, void* dlogits, 
   } else if (regs_ok && V <= 1024 * 8 * 20) {
     // The fewest threads that hold the row, so that as many rows as possible are on a CU in different phases: us with the
     // workgroup below | the one of 512 threads x 26 vectors (1024 x 20) that held all rows: 2048 x 4096 20 | 46, 1500 x 16384 27 | 51, 8192 x 50304 316 | 425,
-    // 8192 x 100352 609 | 740, 4096 x 128256 424 | 493 (the last two only from the arithmetic).  Up to 256 rows each have a CU to
-    // themselves and take twice the threads: 16 x 50304 12.6 | 16.4 (256 threads 16.9), 256 x 50304 17.6 | 20.9 (22.7),
-    // 256 x 100352 29.7 | 32.9 (512 threads 34.7).
+    // 8192 x 100352 609 | 740, 4096 x 128256 424 | 493 (the last two only from the arithmetic).  Rows that all find room
+    // at once, two workgroups of 512 threads (84 registers) or one of 1024 on a CU, take twice the threads: us with them | with half as many, 16 x 50304 12.6 | 16.9,
+    // 257 x 50304 20.3 | 21.7, 512 x 50304 25.3 | 26.9 (513: 31.5 | 29.0), 512 x 20000 16.8 | 18.3, 256 x 100352 29.7 | 34.7.
     if (V <= 256 * 8 * 2) CE_REGS(256, 2);
     else if (V <= 256 * 8 * 8) CE_REGS(256, 8);
-    else if (V <= 256 * 8 * 25 && T > 256) CE_REGS(256, 25);
+    else if (V <= 256 * 8 * 25 && T > 512) CE_REGS(256, 25);
     else if (V <= 256 * 8 * 25) CE_REGS(512, 13);
     else if (V <= 512 * 8 * 25 && T > 256) CE_REGS(512, 25);
     else CE_REGS(1024, 20);

@@ -127,3 +127,9 @@ def test_gradients_round_as_the_exact_ones(V, at):
         wrong += int(((d[i:i + 1024, :-8].double() != want) & big).sum())
         total += int(big.sum())
     assert wrong / total < 1.25e-4, wrong / total
+
+
+@pytest.mark.parametrize("T", [512, 513])
+@pytest.mark.parametrize("V,cap", [(16392, 0.0), (51200, 20.0), (51199, 0.0)])
+def test_number_of_rows_of_two_workgroups_to_a_cu(V, cap, T):
+    test_number_of_rows(V, cap, T)
