@@ -1328,7 +1328,6 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
   };
   float best = alone(T, in, out, true) + alone(out, in, T, false);
   int tile = 0;  // of the one launch, 0: two calls
-  // (bf16 gradients: the four waves' longer chains of fp32 additions are 1e-8 of the sum, and would show in an fp32 one)
   if (const float c = pair_small(T, in, out); c < best && !dw_f32 && out % 8 == 0 && in % 8 == 0 && T >= 64) best = c, tile = 64;
   // whole chunks and vector stores, whole k-tiles in the first product
   const bool direct = !dw_f32 && out % BK == 0 && in % 8 == 0 && lddy % 8 == 0 && ldw % 8 == 0 && ldx % 8 == 0 && lddx % 8 == 0 && lddw % 8 == 0 &&

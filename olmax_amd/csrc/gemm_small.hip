@@ -168,8 +168,9 @@ int tiles(const Problem& p) {
   return (int)((int64_t)((p.M + TS - 1) / TS) * ((p.N + TS - 1) / TS));
 }
 
-// Tile `pid` of `nwg` by the KG waves of a workgroup.
-template <int TS, int KG, bool A_KC, bool B_KC, Mode MODE>
+// Tile `pid` of `nwg` by the KG waves of a workgroup.  TWO: a wave's k-tiles go to two accumulators in turn, so that four waves have
+// the chains of fp32 additions of eight.
+template <int TS, int KG, bool A_KC, bool B_KC, Mode MODE, bool TWO = false>
 __device__ __forceinline__ void small_tile(const Problem& P, int pid, int nwg, unsigned char* smem) {
   const bf16 *A = P.A, *B = P.B, *R = P.R;
   void* Cv = P.C;
@@ -195,14 +196,16 @@ __device__ __forceinline__ void small_tile(const Problem& P, int pid, int nwg, u
   oa.init(A, lda, m0, M, lane);
   ob.init(B, ldb, n0, N, lane);
 
-  f32x4 acc[TF][TF];
+  f32x4 accs[1 + TWO][TF][TF];
 #pragma unroll
-  for (int i = 0; i < TF; i++)
+  for (int s = 0; s <= TWO; s++)
 #pragma unroll
-    for (int j = 0; j < TF; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TF; i++)
+#pragma unroll
+      for (int j = 0; j < TF; j++) accs[s][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // operands swapped, as in the large-tile kernel: an accumulator holds row l16, columns 4 g16 .. +3
-  auto multiply = [&]() {
+  auto multiply = [&](f32x4 (&acc)[TF][TF]) {
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
       bf16x8 fa[TF], fb[TF];
@@ -232,13 +235,26 @@ __device__ __forceinline__ void small_tile(const Problem& P, int pid, int nwg, u
   for (; kt < ktf; kt += KG) {
     park();
     if (kt + KG < ktf) load(kt + KG);
-    multiply();
+    multiply(accs[0]);
+    if (!TWO) continue;
+    kt += KG;
+    if (kt >= ktf) break;
+    park();
+    if (kt + KG < ktf) load(kt + KG);
+    multiply(accs[TWO]);
   }
   if (kt == ktf && ktf * BKS < K) {  // the ragged k-tile falls to the wave whose turn it is
     oa.load_tail(va, (int64_t)ktf * BKS, K, lane);
     ob.load_tail(vb, (int64_t)ktf * BKS, K, lane);
     park();
-    multiply();
+    multiply(accs[0]);
+  }
+  f32x4 (&acc)[TF][TF] = accs[0];
+  if (TWO) {
+#pragma unroll
+    for (int i = 0; i < TF; i++)
+#pragma unroll
+      for (int j = 0; j < TF; j++) acc[i][j] += accs[TWO][i][j];
   }
 
   // partial tiles into the waves' own regions, then every thread adds 8 columns of a row in wave order
@@ -305,13 +321,13 @@ __global__ __launch_bounds__(KG * 64, 2) void gemm_small_kernel(const Problem p)
 
 // dX = dY W (tiles of TSX) and dW = dY^T X (TSW) in one launch: neither fills the GPU, a launch alone is 3 us, and the second does not
 // need the first.  Workgroups of the longer reduction come first.  us, two launches -> one, T x in x out: 2048 x 256 x 2048
-// 22.4 -> 12.6, 2048 x 1024 x 256 17.1 -> 13.1, 2048 x 256 x 256 14.5 -> 6.4, 4096 x 256 x 768 24.9 -> 16.4, 100 x 1024 x 3072 19.8 -> 14.9.
-template <int TSX, int TSW>
-__global__ __launch_bounds__(256, 2) void gemm_small_pair_kernel(const Problem dx, const Problem dw, int n_dx, int n_dw, int dx_first) {
+// 22.4 -> 13.2, 2048 x 1024 x 256 17.1 -> 13.1, 2048 x 256 x 256 14.5 -> 6.7, 4096 x 256 x 768 24.9 -> 16.7, 130 x 1024 x 3072 15.0 -> 13.4.
+template <int TSX, int TSW, int KG, bool TWOX, bool TWOW>
+__global__ __launch_bounds__(KG * 64, 2) void gemm_small_pair_kernel(const Problem dx, const Problem dw, int n_dx, int n_dw, int dx_first) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int id = blockIdx.x;
-  if (dx_first ? id < n_dx : id >= n_dw) small_tile<TSX, 4, true, false, WHOLE>(dx, dx_first ? id : id - n_dw, n_dx, smem);
-  else small_tile<TSW, 4, false, false, WHOLE>(dw, dx_first ? id - n_dx : id, n_dw, smem);
+  if (dx_first ? id < n_dx : id >= n_dw) small_tile<TSX, KG, true, false, WHOLE, TWOX>(dx, dx_first ? id : id - n_dw, n_dx, smem);
+  else small_tile<TSW, KG, false, false, WHOLE, TWOW>(dw, dx_first ? id - n_dx : id, n_dw, smem);
 }
 
 template <typename K>
@@ -343,14 +359,14 @@ void dispatch(hipStream_t s, const Problem& p, bool a_kc, bool b_kc) {
   go(s, p);
 }
 
-template <int TSX, int TSW>
+template <int TSX, int TSW, int KG, bool TWOX = false, bool TWOW = false>
 void launch_pair(hipStream_t s, const Problem& dx, const Problem& dw) {
-  auto kern = gemm_small_pair_kernel<TSX, TSW>;
-  constexpr int SMEM = 4 * std::max(wave_lds(TSX), wave_lds(TSW));
+  auto kern = gemm_small_pair_kernel<TSX, TSW, KG, TWOX, TWOW>;
+  constexpr int SMEM = KG * std::max(wave_lds(TSX), wave_lds(TSW));
   static std::once_flag once;
   std::call_once(once, [&] { allow_lds(kern, SMEM); });
   const int n_dx = tiles<TSX>(dx), n_dw = tiles<TSW>(dw);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(n_dx + n_dw)), dim3(256), SMEM, s, dx, dw, n_dx, n_dw, (int)(dx.K > dw.K));
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_dx + n_dw)), dim3(KG * 64), SMEM, s, dx, dw, n_dx, n_dw, (int)(dx.K > dw.K));
 }
 
 }  // namespace
@@ -374,9 +390,28 @@ bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const b
   if (out % 8 || in % 8 || T < 64 || lddy >= (1 << 25) || ldw >= (1 << 25) || ldx >= (1 << 25)) return false;
   const Problem px = {dy, w, dx, r, T, in, out, lddy, ldw, lddx, ldr, 0};
   const Problem pw = {dy, x, dw, nullptr, out, in, T, lddy, ldx, lddw, 0, 0};
-  // tiles of 32 while they find a CU each
-  auto go = tiles<32>(px) <= 256 ? (tiles<32>(pw) <= 256 ? launch_pair<32, 32> : launch_pair<32, 64>)
-                                 : (tiles<32>(pw) <= 256 ? launch_pair<64, 32> : launch_pair<64, 64>);
-  go(s, px, pw);
+  // Tiles of 32 while they find a CU each.  Eight waves to a tile where all of them have a CU; else four, with two accumulators where the
+  // product alone would have eight (up to 256 tiles of 64, more than four k-tiles): no chain of additions is longer than in the two calls.
+  // us, eight waves | four, one accumulator | two: 1500 x 256 x 2048 12.0 | 11.8 | 13.3, 512 x 256 x 2048 7.1 | 7.0 | 7.6, 2048 x 256 x 256 6.8 | 6.6 | 6.9;
+  // more tiles than CUs, 2048 x 256 x 768 12.8 | 10.7 | 11.3, 1000 x 256 x 2048 13.6 | 11.8 | 12.2, 1500 x 512 x 512 11.4 | 9.1 | 9.6.
+  const int x32 = tiles<32>(px), w32 = tiles<32>(pw);
+  if ((x32 <= 256 ? x32 : tiles<64>(px)) + (w32 <= 256 ? w32 : tiles<64>(pw)) <= 256) {
+    auto go = x32 <= 256 ? (w32 <= 256 ? launch_pair<32, 32, 8> : launch_pair<32, 64, 8>)
+                         : (w32 <= 256 ? launch_pair<64, 32, 8> : launch_pair<64, 64, 8>);
+    go(s, px, pw);
+    return true;
+  }
+  auto form = [](const Problem& p) { return tiles<32>(p) <= 256 ? 0 : tiles<64>(p) > 256 || p.K <= 4 * BKS ? 1 : 2; };
+  switch (form(px) * 3 + form(pw)) {
+    case 0: launch_pair<32, 32, 4, true, true>(s, px, pw); break;
+    case 1: launch_pair<32, 64, 4, true, false>(s, px, pw); break;
+    case 2: launch_pair<32, 64, 4, true, true>(s, px, pw); break;
+    case 3: launch_pair<64, 32, 4, false, true>(s, px, pw); break;
+    case 4: launch_pair<64, 64, 4, false, false>(s, px, pw); break;
+    case 5: launch_pair<64, 64, 4, false, true>(s, px, pw); break;
+    case 6: launch_pair<64, 32, 4, true, true>(s, px, pw); break;
+    case 7: launch_pair<64, 64, 4, true, false>(s, px, pw); break;
+    default: launch_pair<64, 64, 4, true, true>(s, px, pw);
+  }
   return true;
 }

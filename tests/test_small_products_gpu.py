@@ -129,3 +129,35 @@ def test_a_weight_gradient_in_the_place_of_the_weights(T, d, V):
     got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels, dW=W)))
     assert not any(key >> 19 & 1 for key, *_ in got), got
     check_gradients(h, kept, labels, *out[1:])
+
+
+def head_sums(terms_h, terms_W, T, d, V):
+    """Gradients of the LM head whose logits are all zero, so that every dlogit but the labels' is one bf16 number c: rows of `terms` sit at
+    the first token (vocabulary entry) of their k-tile, and the gradient of the other operand is c times their sum.  Labels name the last
+    entry, whose row of W is zero."""
+    from olmax_amd import ops
+    h, W = (torch.zeros(n, d, device="cuda", dtype=torch.bfloat16) for n in (T, V))
+    for x, terms in ((h, terms_h), (W, terms_W)):
+        for kt, value in terms:
+            x[64 * kt] = value
+    labels = torch.full((T,), V - 1, device="cuda", dtype=torch.int32)
+    out = []
+    got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels)))
+    c = (torch.tensor(1.0, dtype=torch.float64) / V / T).to(torch.bfloat16)
+    return got, out[1], out[2][:-1], c
+
+
+@pytest.mark.parametrize("T,d,V", [
+    (1024, 256, 1024), (1536, 256, 2048),  # every tile finds a CU: eight waves to one
+    (1024, 512, 1024), (2048, 256, 4096), (2048, 512, 1024)])  # more tiles, of 32 and 64
+@pytest.mark.parametrize("which", ["dh", "dW"])
+def test_one_launch_keeps_eight_chains(T, d, V, which):
+    """A tile of the single product has eight waves, and wave w adds the k-tiles w, w + 8, ...: 2^24 and -2^24 meet there and a 1 from a
+    k-tile of another wave counts.  One chain for the k-tiles w, w + 4, ... would lose it: 2^24 + 1 = 2^24 in fp32."""
+    print(f"[case] chains T{T} d{d} V{V} {which}", flush=True)
+    n = (V if which == "dh" else T) // 64
+    terms = [(w, 2.0 ** 24) for w in range(4)] + [(4 + w, 1.0) for w in range(4)] + [(8 + w, -(2.0 ** 24)) for w in range(4)]
+    assert n > 12
+    got, dh, dW, c = head_sums(*(([], terms) if which == "dh" else (terms, [])), T, d, V)
+    assert (64 | 1 << 19, T, d, V, 1) in got, got
+    assert ((dh if which == "dh" else dW).float() == 4 * c.item()).all()
