@@ -1275,17 +1275,20 @@ struct Work {
   int64_t n;  // tiles
   int kt;
 };
-// 64 and 32 tiles in 4-wave workgroups, two of which fit a CU: their k-tiles with every CU busy, or the longer of the two chains
+// 64 and 32 tiles in 4-wave workgroups, two of which fit a CU: their k-tiles with every CU busy, or the longer of the two chains; 64 tiles alone
+// that need a few more than one round of them end unevenly (1700 x 1024 x 1024, 688 of them: 22.7 us, two calls 21.6)
 static float pair_small(int T, int in, int out) {
+  int64_t n64 = 0;
   auto part = [&](int M, int N, int K, float* chain) {
     const int kt = (K + BK - 1) / BK;
     const int64_t n32 = tiles_of(M, N, 32), n = n32 <= 256 ? n32 : tiles_of(M, N, 64);
+    n64 += n32 <= 256 ? 1024 : n;
     *chain = std::max(*chain, n32 <= 256 ? 3.6f + 0.165f * kt : 4.2f + 0.22f * kt);
     return n * ((n32 <= 256 ? 0.00046f : 0.00086f) * kt + 0.0047f);
   };
   float chain = 0.f;
   const float work = part(T, in, out, &chain) + part(out, in, T, &chain) + 3.5f;
-  return std::max(work, chain) / 0.9f;
+  return std::max(work, chain) / (n64 > 512 && n64 < 800 ? 0.82f : 0.9f);
 }
 // 128 tiles, 512 at a time: 1 us per k-tile of each, 17 % more where they end unevenly; or the long chains, beside the others and then alone
 static float pair_128(Work l, Work s) {
