@@ -172,8 +172,9 @@ int olmax_adamw_used_rows(hipStream_t stream, float* p, const float* g, float* m
 // gemm_small.hip: any M, N, K and alignment; `groups` (4 or 8) waves share a tile's reduction; tiles of 64 x 64 or 32 x 32
 void olmax_gemm_small(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N, int K, int64_t lda,
                       int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, int tile, int groups);
-// dX [T, in] = dY [T, out] W [out, in] (+ R) and dW [out, in] = dY^T X [T, in] in one launch; false: not these sizes, nothing was launched
-bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, bf16* dw, int T, int in,
+// dX [T, in] = dY [T, out] W [out, in] (+ R) and dW [out, in] = dY^T X [T, in] in one launch; wants in and out to be multiples of 8, T >= 64 and
+// row strides of dY, W and X below 2^25
+void olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, bf16* dw, int T, int in,
                            int out, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw);
 // memory a GEMM may use for partial results until it is done; what it holds before and after does not matter
 struct GemmScratch {

@@ -1127,19 +1127,25 @@ static int64_t tiles_of(int M, int N, int t) { return (int64_t)((M + t - 1) / t)
 static float cost_small(int M, int N, int kt, bool a_kc) { return std::min(cost_64(tiles_of(M, N, 64), kt), cost_32(tiles_of(M, N, 32), kt, a_kc)); }
 
 // Which kernel takes a problem.  0: gemm_small (any size and alignment), else the edge of the
-// direct-to-LDS kernel's tiles; *parts > 1: 256 tiles with that many workgroups to a reduction.
-static int pick_tile(int M, int N, int K, bool a_kc, bool b_kc, bool direct_ok, int64_t bytes, int* parts) {
+// direct-to-LDS kernel's tiles; *parts > 1: 256 tiles with that many workgroups to a reduction.  *cost: what it is expected to take.
+static int pick_tile(int M, int N, int K, bool a_kc, bool b_kc, bool direct_ok, int64_t bytes, int* parts, float* cost) {
   *parts = 1;
-  if (!direct_ok || M < 128 || N < 128 || K < BK) return 0;
   const int kt = (K + BK - 1) / BK;
+  float& best = *cost;
+  best = cost_small(M, N, kt, a_kc);
+  if (!direct_ok || M < 128 || N < 128 || K < BK) return 0;
   auto tiles = [&](int t) { return tiles_of(M, N, t); };
-  float best = cost_small(M, N, kt, a_kc);
   int tile = 0;
   if (const float c = cost_128(tiles(128), kt, b_kc); c < best) best = c, tile = 128;
   if (M < 256 || N < 256) return tile;
   if (const float c = cost_256(tiles(256), kt, bytes, b_kc); c < best) best = c, tile = 256;
   *parts = pick_parts(tiles(256), K / BK, bytes, &best);
   return *parts > 1 ? 256 : tile;
+}
+// Whether the direct-to-LDS kernels can take the operands: whole 16-byte chunks everywhere, i.e. aligned rows, and a chunk never crosses the end
+// of a row (a_padded: see olmax_gemm_padded).
+static bool direct(const bf16* a, const bf16* b, int M, int N, int K, int64_t lda, int64_t ldb, bool a_kc, bool b_kc, bool a_padded) {
+  return aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 && (a_padded || (a_kc ? K : M) % 8 == 0) && (b_kc ? K : N) % 8 == 0;
 }
 
 // Wave quantisation: with one 256x256 tile per CU per round, a last round that fills less
@@ -1188,13 +1194,12 @@ static bool glu_fused_wins(int M, int F, int K, GluForm form) {
 int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C, const bf16* r, int M, int N, int K,
                       int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, bool a_kc, bool b_kc, bool out_f32, bool a_padded,
                       GemmScratch scratch) {
-  // whole 16-byte chunks everywhere: aligned rows, and a chunk never crosses the end of a row
-  const bool direct_ok = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 && (a_padded || (a_kc ? K : M) % 8 == 0) &&
-                         (b_kc ? K : N) % 8 == 0;
+  const bool direct_ok = direct(a, b, M, N, K, lda, ldb, a_kc, b_kc, a_padded);
   const int force_tile = g_force_tile.load(std::memory_order_relaxed);
   int parts;
+  float cost;
   if ((b_kc && !a_kc) || force_tile || !aligned16(scratch.p)) scratch = GemmScratch();  // (no caller has that layout)
-  int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, scratch.bytes, &parts);
+  int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, scratch.bytes, &parts, &cost);
   if (parts > 1) {
     auto go = !a_kc ? launch_split<false, false> : b_kc ? launch_split<true, true> : launch_split<true, false>;
     return go(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts, (float*)scratch.p);
@@ -1317,26 +1322,23 @@ static float pair_256(Work l, Work s) {
 
 int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, void* dw, int T, int in, int out,
                      int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw, bool dw_f32, bool dy_padded, GemmScratch scratch) {
-  // what the better kernels take one after the other, as pick_tile sees them
+  // what the kernels that take the operands need one after the other
   const int64_t bytes = aligned16(scratch.p) ? scratch.bytes : 0;
-  auto alone = [&](int M, int N, int K, bool a_kc) {
-    const int kt = (K + BK - 1) / BK;
-    float c = cost_small(M, N, kt, a_kc);
-    if (M >= 128 && N >= 128) c = std::min(c, cost_128(tiles_of(M, N, 128), kt, false));
-    if (M >= 256 && N >= 256) {
-      c = std::min(c, cost_256(tiles_of(M, N, 256), kt, bytes, false));
-      (void)pick_parts(tiles_of(M, N, 256), K / BK, bytes, &c);
-    }
-    return c;
-  };
-  float best = alone(T, in, out, true) + alone(out, in, T, false);
+  const bool direct_x = direct(dy, w, T, in, out, lddy, ldw, true, false, dy_padded), direct_w = direct(dy, x, out, in, T, lddy, ldx, false, false, dy_padded);
+  int parts;
+  float best, best_w;
+  (void)pick_tile(T, in, out, true, false, direct_x, bytes, &parts, &best);
+  (void)pick_tile(out, in, T, false, false, direct_w, bytes, &parts, &best_w);
+  best += best_w;
   int tile = 0;  // of the one launch, 0: two calls
-  if (const float c = pair_small(T, in, out); c < best && !dw_f32 && out % 8 == 0 && in % 8 == 0 && T >= 64) best = c, tile = 64;
-  // whole chunks and vector stores, whole k-tiles in the first product
-  const bool direct = !dw_f32 && out % BK == 0 && in % 8 == 0 && lddy % 8 == 0 && ldw % 8 == 0 && ldx % 8 == 0 && lddx % 8 == 0 && lddw % 8 == 0 &&
-                      (!r || (ldr % 8 == 0 && aligned16(r))) && aligned16(dy) && aligned16(w) && aligned16(x) && aligned16(dx) && aligned16(dw);
+  // (the one form of the small kernel that is built: whole chunks, 32-bit line offsets and at least a tile of rows)
+  const bool small = !dw_f32 && out % 8 == 0 && in % 8 == 0 && T >= 64 && lddy < (1 << 25) && ldw < (1 << 25) && ldx < (1 << 25);
+  if (const float c = pair_small(T, in, out); small && c < best) best = c, tile = 64;
+  // vector stores, whole k-tiles in the first product
+  const bool large = !dw_f32 && direct_x && direct_w && out % BK == 0 && lddx % 8 == 0 && lddw % 8 == 0 && (!r || (ldr % 8 == 0 && aligned16(r))) &&
+                     aligned16(dx) && aligned16(dw);
   for (int t = 128; t <= 256; t *= 2) {
-    if (!direct || T < t || in < t || out < t) continue;
+    if (!large || T < t || in < t || out < t) continue;
     const Work wx = {tiles_of(T, in, t), out / BK}, ww = {tiles_of(out, in, t), (T + BK - 1) / BK};
     const Work &l = wx.kt > ww.kt ? wx : ww, &sh = wx.kt > ww.kt ? ww : wx;
     if (const float c = t == 128 ? pair_128(l, sh) : pair_256(l, sh); c < best) best = c, tile = t;
@@ -1352,9 +1354,8 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
       (void)hipEventCreate(&rec.e1);
       (void)hipEventRecord(rec.e0, s);
     }
-    bool done = true;
     if (tile == 64) {
-      done = olmax_gemm_small_pair(s, dy, w, x, dx, r, (bf16*)dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw);
+      olmax_gemm_small_pair(s, dy, w, x, dx, r, (bf16*)dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw);
     } else {
       const PairSide px = {dy, w, r, dx, T, in, out, lddy, ldw, lddx, ldr}, pw = {dy, x, nullptr, (bf16*)dw, out, in, T, lddy, ldx, lddw, 0};
       const bool rx = T % tile || in % tile;
@@ -1371,19 +1372,14 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
     if (g_prof_on) {
       (void)hipEventRecord(rec.e1, s);
       rec.flops = 4.0 * T * in * out;
-      rec.bytes = 2.0 * ((double)T * out + 2.0 * T * in + (r ? 1.0 * T * in : 0.0) + (dw_f32 ? 3.0 : 2.0) * in * out);
+      rec.bytes = 2.0 * ((double)T * out + 2.0 * T * in + (r ? 1.0 * T * in : 0.0) + 2.0 * in * out);
       rec.key = tile | (1 << 19);
       rec.M = T; rec.N = in; rec.K = out;
       std::lock_guard<std::mutex> lk(g_prof_mu);
-      if (done) {
-        g_prof.push_back(rec);
-      } else {
-        (void)hipEventDestroy(rec.e0);
-        (void)hipEventDestroy(rec.e1);
-      }
+      g_prof.push_back(rec);
     }
     OLMAX_LAUNCH_CHECK();
-    if (done) return OLMAX_OK;
+    return OLMAX_OK;
   }
   const int rc = olmax_gemm_padded(s, dy, w, dx, r, T, in, out, lddy, ldw, lddx, ldr, true, false, false, dy_padded, scratch);
   return rc ? rc : olmax_gemm_padded(s, dy, x, dw, nullptr, out, in, T, lddy, ldx, lddw, 0, false, false, dw_f32, dy_padded, scratch);

@@ -384,10 +384,8 @@ void olmax_gemm_small(hipStream_t s, const bf16* A, const bf16* B, void* C, cons
   }
 }
 
-bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, bf16* dw, int T, int in,
+void olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, bf16* dw, int T, int in,
                            int out, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw) {
-  // whole chunks, 32-bit line offsets and at least a tile of rows: the one mode that is built
-  if (out % 8 || in % 8 || T < 64 || lddy >= (1 << 25) || ldw >= (1 << 25) || ldx >= (1 << 25)) return false;
   const Problem px = {dy, w, dx, r, T, in, out, lddy, ldw, lddx, ldr, 0};
   const Problem pw = {dy, x, dw, nullptr, out, in, T, lddy, ldx, lddw, 0, 0};
   // Tiles of 32 while they find a CU each.  Eight waves to a tile where all of them have a CU; else four, with two accumulators where the
@@ -399,7 +397,7 @@ bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const b
     auto go = x32 <= 256 ? (w32 <= 256 ? launch_pair<32, 32, 8> : launch_pair<32, 64, 8>)
                          : (w32 <= 256 ? launch_pair<64, 32, 8> : launch_pair<64, 64, 8>);
     go(s, px, pw);
-    return true;
+    return;
   }
   auto form = [](const Problem& p) { return tiles<32>(p) <= 256 ? 0 : tiles<64>(p) > 256 || p.K <= 4 * BKS ? 1 : 2; };
   switch (form(px) * 3 + form(pw)) {
@@ -413,5 +411,4 @@ bool olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const b
     case 7: launch_pair<64, 64, 4, true, false>(s, px, pw); break;
     default: launch_pair<64, 64, 4, true, true>(s, px, pw);
   }
-  return true;
 }

@@ -161,3 +161,18 @@ def test_one_launch_keeps_eight_chains(T, d, V, which):
     got, dh, dW, c = head_sums(*(([], terms) if which == "dh" else (terms, [])), T, d, V)
     assert (64 | 1 << 19, T, d, V, 1) in got, got
     assert ((dh if which == "dh" else dW).float() == 4 * c.item()).all()
+
+
+@pytest.mark.parametrize("T,d,V", [(512, 1024, 4096), (2048, 2048, 256)])
+def test_one_launch_of_operands_that_only_the_small_kernel_takes(T, d, V):
+    """Rows that do not start on 16 bytes: the alternative is the small kernel twice, not the 128 tiles that aligned rows would take."""
+    from olmax_amd import ops
+    print(f"[case] pair of unaligned rows T{T} d{d} V{V}", flush=True)
+    h, W = (torch.empty(n * d + 4, device="cuda", dtype=torch.bfloat16)[4:].view(n, d) for n in (T, V))
+    h.copy_(rnd(T, d, seed=1))
+    W.copy_(rnd(V, d, seed=2, scale=0.1))
+    labels = torch.arange(T, device="cuda", dtype=torch.int32) * 7 % V
+    out = []
+    got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels)))
+    assert (64 | 1 << 19, T, d, V, 1) in got, got
+    check_gradients(h, W, labels, *out[1:])
