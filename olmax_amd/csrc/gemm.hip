@@ -91,8 +91,10 @@ std::mutex g_prof_mu;
 // that fetched a chunk past the end overwrites it with zeros in LDS once its own fetches have landed,
 // before the barrier that publishes the stage.  Wants M >= BM, N >= BN, K >= 64 and 16-byte chunks that do not cross the end of a row (see olmax_gemm_padded).
 //
-// The tile that workgroup `pid` of `nwg` takes; the residual of a HAS_RES form may be null.
-template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI, int RAG>
+// The tile that workgroup `pid` of `nwg` takes; the residual of a HAS_RES form may be null.  BLOCKS: the sums of every four k-tiles (below
+// 16 of them: two) are added up by themselves, so that a chain of fp32 additions is no longer than that of eight waves with every eighth k-tile each
+// (gemm_small.hip).  64 registers and 64 additions a block: 1 to 4 % (both gradients of 3000 x 1024 x 3072 47.5 -> 48.0 us, 512 x 4608 x 8192 86.2 -> 89.0).
+template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI, int RAG, bool BLOCKS = false>
 __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
     const bf16* __restrict__ R, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
@@ -497,11 +499,34 @@ __device__ __forceinline__ void gemm_tile(
       bp += b_step;
     }
   };
+  f32x4 sum[BLOCKS ? TM : 1][TN];
+  const int block = KT < 16 ? 0 : 2;
+  if (BLOCKS) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) sum[BLOCKS ? i : 0][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   for (int kt = 0; kt + 1 < KT; kt += 2) {
     k_tile(kt, std::integral_constant<int, 0>());
     k_tile(kt + 1, std::integral_constant<int, 1>());
+    if (BLOCKS && (kt & block) == block) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          sum[BLOCKS ? i : 0][j] += acc[i][j];
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
   }
   if (KT & 1) k_tile(KT - 1, std::integral_constant<int, 0>());
+  if (BLOCKS) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) acc[i][j] += sum[BLOCKS ? i : 0][j];
+  }
   dma_wait_all();  // the redundant tail DMAs must not outlive the workgroup's LDS allocation
   // The epilogue derives its addresses from a copy of the lane id that the compiler cannot see
   // through, so none of them is computed ahead of the loop and kept in registers across it.
@@ -762,18 +787,18 @@ struct PairSide {
   int64_t lda, ldb, ldc, ldr;
   int tiles_m, tiles_n, order, nwg;
 };
-template <int T, int W, int RAGX, int RAGW>
+template <int T, int W, int RAGX, int RAGW, bool BLOCKS>
 __global__ __launch_bounds__((T / W) * (T / 64) * 64) __attribute__((amdgpu_num_vgpr(120))) void gemm_pair_kernel(const PairSide x, const PairSide w, int x_first, int n_first) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const bool second = (int)blockIdx.x >= n_first;
   const int pid = second ? blockIdx.x - n_first : blockIdx.x;
   if (second != (x_first != 0)) {
     if (pid >= x.nwg) return;
-    gemm_tile<T, T, W, 64, true, false, true, false, 0, RAGX>(x.A, x.B, x.C, x.R, x.M, x.N, x.K, x.lda, x.ldb, x.ldc, x.ldr, x.tiles_m, x.tiles_n, 1,
+    gemm_tile<T, T, W, 64, true, false, true, false, 0, RAGX, BLOCKS>(x.A, x.B, x.C, x.R, x.M, x.N, x.K, x.lda, x.ldb, x.ldc, x.ldr, x.tiles_m, x.tiles_n, 1,
                                                               nullptr, nullptr, 1, 0, x.order, pid, x.nwg, smem);
   } else {
     if (pid >= w.nwg) return;
-    gemm_tile<T, T, W, 64, false, false, false, false, 0, RAGW>(w.A, w.B, w.C, nullptr, w.M, w.N, w.K, w.lda, w.ldb, w.ldc, 0, w.tiles_m, w.tiles_n, 1,
+    gemm_tile<T, T, W, 64, false, false, false, false, 0, RAGW, BLOCKS>(w.A, w.B, w.C, nullptr, w.M, w.N, w.K, w.lda, w.ldb, w.ldc, 0, w.tiles_m, w.tiles_n, 1,
                                                                 nullptr, nullptr, 1, 0, w.order, pid, w.nwg, smem);
   }
 }
@@ -874,9 +899,9 @@ int launch_glu(hipStream_t s, const bf16* A, const bf16* B, bf16* gu, bf16* act,
   return OLMAX_OK;
 }
 
-template <int T, int W, int RAGX, int RAGW>
+template <int T, int W, int RAGX, int RAGW, bool BLOCKS>
 void launch_pair(hipStream_t s, PairSide x, PairSide w) {
-  auto kern = gemm_pair_kernel<T, W, RAGX, RAGW>;
+  auto kern = gemm_pair_kernel<T, W, RAGX, RAGW, BLOCKS>;
   constexpr int SMEM = 4 * T * BK * 2;
   static std::once_flag attr_once;  // per instantiation
   std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM); });
@@ -1142,6 +1167,19 @@ static int pick_tile(int M, int N, int K, bool a_kc, bool b_kc, bool direct_ok, 
   *parts = pick_parts(tiles(256), K / BK, bytes, &best);
   return *parts > 1 ? 256 : tile;
 }
+// What gemm_small runs a problem in: the edge of its tiles and the waves that share a tile's reduction.
+struct SmallForm {
+  int edge, groups;
+};
+static SmallForm small_form(int M, int N, int K, bool a_kc, bool forced) {
+  const int64_t n64 = tiles_of(M, N, 64), n32 = tiles_of(M, N, 32);
+  const int kt = (K + BK - 1) / BK;
+  // (the 0.6 us: one round of 64 tiles, measured at 4 to 128 k-tiles; pick_tile's boundaries were measured without)
+  const int edge = !forced && cost_32(n32, kt, a_kc) < cost_64(n64, kt) + 0.6f ? 32 : 64;
+  // eight waves share a tile while there are not more 64 tiles than CUs, else two workgroups fit a CU.  (A 32 tile does as well with four, 300 x 1024 x 2816
+  // 11.0 us against 11.6, but a chain of fp32 additions twice as long is 7 to 29 % further from the exact sum; up to four k-tiles there is none.)
+  return {edge, n64 <= 256 && (edge == 64 || kt > 4) ? 8 : 4};
+}
 // Whether the direct-to-LDS kernels can take the operands: whole 16-byte chunks everywhere, i.e. aligned rows, and a chunk never crosses the end
 // of a row (a_padded: see olmax_gemm_padded).
 static bool direct(const bf16* a, const bf16* b, int M, int N, int K, int64_t lda, int64_t ldb, bool a_kc, bool b_kc, bool a_padded) {
@@ -1182,6 +1220,42 @@ static bool fused_wins(int M, int N, int K, float per_round, float passes) {
   plain = std::min(plain, cut.rm || cut.cn ? cost_256(n, kt, 0, true) : cost_rounds(n, kt));
   return cost_rounds(n, kt) + per_round * ((n + 255) / 256) <= plain + passes;
 }
+// Fp32 additions behind one another in a result, an MFMA counted as one: of n chains of `steps` k-tiles each that are added up,
+static int chain_of_parts(int n, int steps) { return 2 * steps + (n > 1 ? n : 0); }
+// of olmax_gemm_padded (the shortest of its parts where it cuts a problem),
+static int chain_of_product(int M, int N, int K, bool a_kc, bool b_kc, bool direct_ok, int64_t bytes) {
+  const int kt = (K + BK - 1) / BK;
+  int parts;
+  float cost;
+  const int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, bytes, &parts, &cost);
+  if (parts > 1) return chain_of_parts(parts, (kt + parts - 1) / parts);
+  if (tile == 0) {
+    const int g = std::min(kt, small_form(M, N, K, a_kc, false).groups);
+    return chain_of_parts(g, (kt + g - 1) / g);
+  }
+  if (tile == 256) {
+    const int tm = (M + 255) / 256, tn = (N + 255) / 256;
+    const Cut cut = find_cut(tm, tn);
+    auto part = [&](int m, int n) { return chain_of_product(m, n, K, a_kc, b_kc, direct_ok, bytes); };
+    if (cut.rm || cut.cn) {
+      const int m1 = cut.rm * 256, n1 = cut.cn * 256;
+      return (int64_t)cut.rm * tn >= (int64_t)cut.cn * tm ? std::min(part(m1, N), part(M - m1, N)) : std::min(part(M, n1), part(M, N - n1));
+    }
+  }
+  return chain_of_parts(1, kt);
+}
+// and of the forms of both gradients in one launch: small tiles (see olmax_gemm_small_pair), 128 ones, whose sums may be blocked, and 256 ones.
+static int chain_in_pair(int tile, bool blocks, int M, int N, int K) {
+  const int kt = (K + BK - 1) / BK;
+  if (tile >= 128 && !blocks) return chain_of_parts(1, kt);
+  if (tile == 128) {
+    const int steps = std::min(kt, kt < 16 ? 2 : 4);
+    return chain_of_parts((kt + steps - 1) / steps, steps);
+  }
+  const int g = std::min(kt, tiles_of(M, N, 64) <= 256 ? 8 : 4);
+  return chain_of_parts(g, (kt + g - 1) / g);
+}
+
 enum GluForm { GLU_SAVE, GLU_ONLY, GLU_BWD };
 static bool glu_fused_wins(int M, int F, int K, GluForm form) {
   const float e = (float)M * F;  // the elementwise passes move 6 (backward: 16) bytes an element at 5 TB/s
@@ -1236,14 +1310,8 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
       (void)hipEventCreate(&rec.e1);
       (void)hipEventRecord(rec.e0, stream);
     }
-    const int64_t n64 = tiles_of(M, N, 64), n32 = tiles_of(M, N, 32);
-    const int kt = (K + BK - 1) / BK;
-    // (the 0.6 us: one round of 64 tiles, measured at 4 to 128 k-tiles; pick_tile's boundaries were measured without)
-    const int edge = !force_tile && cost_32(n32, kt, a_kc) < cost_64(n64, kt) + 0.6f ? 32 : 64;
-    // eight waves share a tile while there are not more 64 tiles than CUs, else two workgroups fit a CU.  (A 32 tile does as well with four, 300 x 1024 x 2816
-    // 11.0 us against 11.6, but a chain of fp32 additions twice as long is 7 to 29 % further from the exact sum; up to four k-tiles there is none.)
-    const int groups = n64 <= 256 && (edge == 64 || kt > 4) ? 8 : 4;
-    olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, edge, groups);
+    const SmallForm f = small_form(M, N, K, a_kc, force_tile != 0);
+    olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, f.edge, f.groups);
     if (g_prof_on) {
       (void)hipEventRecord(rec.e1, stream);
       rec.flops = 2.0 * M * N * K;
@@ -1330,15 +1398,18 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
   (void)pick_tile(T, in, out, true, false, direct_x, bytes, &parts, &best);
   (void)pick_tile(out, in, T, false, false, direct_w, bytes, &parts, &best_w);
   best += best_w;
+  // One launch may not be less precise: no chain of additions longer than the calls'.
+  const int chain_x = chain_of_product(T, in, out, true, false, direct_x, bytes), chain_w = chain_of_product(out, in, T, false, false, direct_w, bytes);
+  auto precise = [&](int t, bool blocks) { return chain_in_pair(t, blocks, T, in, out) <= chain_x && chain_in_pair(t, blocks, out, in, T) <= chain_w; };
   int tile = 0;  // of the one launch, 0: two calls
   // (the one form of the small kernel that is built: whole chunks, 32-bit line offsets and at least a tile of rows)
   const bool small = !dw_f32 && out % 8 == 0 && in % 8 == 0 && T >= 64 && lddy < (1 << 25) && ldw < (1 << 25) && ldx < (1 << 25);
-  if (const float c = pair_small(T, in, out); small && c < best) best = c, tile = 64;
+  if (const float c = pair_small(T, in, out); small && c < best && precise(64, false)) best = c, tile = 64;
   // vector stores, whole k-tiles in the first product
   const bool large = !dw_f32 && direct_x && direct_w && out % BK == 0 && lddx % 8 == 0 && lddw % 8 == 0 && (!r || (ldr % 8 == 0 && aligned16(r))) &&
                      aligned16(dx) && aligned16(dw);
   for (int t = 128; t <= 256; t *= 2) {
-    if (!large || T < t || in < t || out < t) continue;
+    if (!large || T < t || in < t || out < t || !precise(t, t == 128)) continue;
     const Work wx = {tiles_of(T, in, t), out / BK}, ww = {tiles_of(out, in, t), (T + BK - 1) / BK};
     const Work &l = wx.kt > ww.kt ? wx : ww, &sh = wx.kt > ww.kt ? ww : wx;
     if (const float c = t == 128 ? pair_128(l, sh) : pair_256(l, sh); c < best) best = c, tile = t;
@@ -1360,13 +1431,14 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
       const PairSide px = {dy, w, r, dx, T, in, out, lddy, ldw, lddx, ldr}, pw = {dy, x, nullptr, (bf16*)dw, out, in, T, lddy, ldx, lddw, 0};
       const bool rx = T % tile || in % tile;
       const int rw = T % BK ? 2 : out % tile || in % tile;
-#define PAIR(E, W)                                                                                                              \
+#define PAIR(E, W, B)                                                                                                           \
   do {                                                                                                                          \
-    if (rx) rw == 2 ? launch_pair<E, W, 1, 2>(s, px, pw) : rw ? launch_pair<E, W, 1, 1>(s, px, pw) : launch_pair<E, W, 1, 0>(s, px, pw); \
-    else rw == 2 ? launch_pair<E, W, 0, 2>(s, px, pw) : rw ? launch_pair<E, W, 0, 1>(s, px, pw) : launch_pair<E, W, 0, 0>(s, px, pw);    \
+    if (rx) rw == 2 ? launch_pair<E, W, 1, 2, B>(s, px, pw) : rw ? launch_pair<E, W, 1, 1, B>(s, px, pw) : launch_pair<E, W, 1, 0, B>(s, px, pw); \
+    else rw == 2 ? launch_pair<E, W, 0, 2, B>(s, px, pw) : rw ? launch_pair<E, W, 0, 1, B>(s, px, pw) : launch_pair<E, W, 0, 0, B>(s, px, pw);    \
   } while (0)
-      if (tile == 128) PAIR(128, 64);
-      else PAIR(256, 128);
+      if (tile == 128 && !precise(128, false)) PAIR(128, 64, true);
+      else if (tile == 128) PAIR(128, 64, false);
+      else PAIR(256, 128, false);
 #undef PAIR
     }
     if (g_prof_on) {

@@ -176,3 +176,33 @@ def test_one_launch_of_operands_that_only_the_small_kernel_takes(T, d, V):
     got = recorded(lambda: out.extend(ops.lmhead_ce(h, W, labels)))
     assert (64 | 1 << 19, T, d, V, 1) in got, got
     check_gradients(h, W, labels, *out[1:])
+
+
+@pytest.mark.parametrize("T,d,V,which,block", [
+    (4096, 1024, 3072, "dh", 4), (4096, 1024, 3072, "dW", 4), (3000, 1024, 2880, "dh", 4), (3000, 1024, 2880, "dW", 4),  # partial k-tile and ragged edges
+    (512, 2816, 1024, "dh", 4), (512, 2816, 1024, "dW", 2)])
+def test_128_tiles_in_one_launch_add_in_blocks(T, d, V, which, block):
+    """1 in the first block of k-tiles, 2^24 and -2^24 in the second: one chain over all of them would lose the 1 (2^24 + 1 = 2^24 in fp32).  The
+    same in the last whole block."""
+    print(f"[case] blocks T{T} d{d} V{V} {which}", flush=True)
+    K = V if which == "dh" else T
+    n, first = -(-K // 64) // block * block, int(K % 64 != 0)  # (a partial k-tile comes before the whole ones)
+    for at in (block - first, n - block - first):
+        terms = [(0, 1.0), (at, 2.0 ** 24), (at + block - 1, -(2.0 ** 24))]
+        got, dh, dW, c = head_sums(*(([], terms) if which == "dh" else (terms, [])), T, d, V)
+        assert (128 | 1 << 19, T, d, V, 1) in got, got
+        assert ((dh if which == "dh" else dW).float() == c.item()).all()
+
+
+@pytest.mark.parametrize("seq", [1700, 2048])
+def test_one_launch_leaves_the_calls_their_shared_reductions(seq):
+    """The q|k|v gradients of a post-norm block: dX shares its 12288-long reduction between two workgroups, half the chain of the one launch's tiles."""
+    import dataclasses
+    from olmax_amd import TransformerRecipe
+    from olmax_amd.layer import TransformerBlock
+    print(f"[case] shared reductions S{seq}", flush=True)
+    block = TransformerBlock(dataclasses.replace(TransformerRecipe.olmo2_7B(), num_layers=1), batch_size=1, sequence_length=seq)
+    block.forward(rnd(seq, 4096, seed=1))
+    got = recorded(lambda: block.backward(rnd(seq, 4096, seed=2)))
+    assert any(key >> 18 & 1 and shape[:3] == [seq, 4096, 12288] for key, *shape in got), got
+    assert not any(key >> 19 & 1 and shape[:3] == [seq, 4096, 12288] for key, *shape in got), got
