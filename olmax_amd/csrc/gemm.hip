@@ -1171,11 +1171,15 @@ static int pick_tile(int M, int N, int K, bool a_kc, bool b_kc, bool direct_ok, 
 struct SmallForm {
   int edge, groups;
 };
-static SmallForm small_form(int M, int N, int K, bool a_kc, bool forced) {
+static SmallForm small_form(int M, int N, int K, bool a_kc, bool b_kc, bool forced) {
   const int64_t n64 = tiles_of(M, N, 64), n32 = tiles_of(M, N, 32);
   const int kt = (K + BK - 1) / BK;
   // (the 0.6 us: one round of 64 tiles, measured at 4 to 128 k-tiles; pick_tile's boundaries were measured without)
-  const int edge = !forced && cost_32(n32, kt, a_kc) < cost_64(n64, kt) + 0.6f ? 32 : 64;
+  // Part of one k-tile, 64 tiles that two workgroups a CU take in one round: 900 x 1800 x 16 5.8 us in 32 tiles, 5.1 in 64, 1200 x 1200 x 56 5.5 and 4.9.
+  // (With more or fewer of them 32 tiles win, 1500 x 1500 x 16 7.2 and 7.9, 1024 x 1024 x 16 3.8 and 4.4, and where chunks cross the end of a line,
+  // 1100 x 1100 x 56 with B [K, N] 6.6 and 7.6.)
+  const bool one_round = K < BK && n64 > 256 && n64 <= 512 && (a_kc || M % 8 == 0) && (b_kc || N % 8 == 0);
+  const int edge = !forced && !one_round && cost_32(n32, kt, a_kc) < cost_64(n64, kt) + 0.6f ? 32 : 64;
   // eight waves share a tile while there are not more 64 tiles than CUs, else two workgroups fit a CU.  (A 32 tile does as well with four, 300 x 1024 x 2816
   // 11.0 us against 11.6, but a chain of fp32 additions twice as long is 7 to 29 % further from the exact sum; up to four k-tiles there is none.)
   return {edge, n64 <= 256 && (edge == 64 || kt > 4) ? 8 : 4};
@@ -1230,7 +1234,7 @@ static int chain_of_product(int M, int N, int K, bool a_kc, bool b_kc, bool dire
   const int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, bytes, &parts, &cost);
   if (parts > 1) return chain_of_parts(parts, (kt + parts - 1) / parts);
   if (tile == 0) {
-    const int g = std::min(kt, small_form(M, N, K, a_kc, false).groups);
+    const int g = std::min(kt, small_form(M, N, K, a_kc, b_kc, false).groups);
     return chain_of_parts(g, (kt + g - 1) / g);
   }
   if (tile == 256) {
@@ -1310,7 +1314,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
       (void)hipEventCreate(&rec.e1);
       (void)hipEventRecord(rec.e0, stream);
     }
-    const SmallForm f = small_form(M, N, K, a_kc, force_tile != 0);
+    const SmallForm f = small_form(M, N, K, a_kc, b_kc, force_tile != 0);
     olmax_gemm_small(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, a_kc, b_kc, out_f32, f.edge, f.groups);
     if (g_prof_on) {
       (void)hipEventRecord(rec.e1, stream);

@@ -206,3 +206,9 @@ def test_one_launch_leaves_the_calls_their_shared_reductions(seq):
     got = recorded(lambda: block.backward(rnd(seq, 4096, seed=2)))
     assert any(key >> 18 & 1 and shape[:3] == [seq, 4096, 12288] for key, *shape in got), got
     assert not any(key >> 19 & 1 and shape[:3] == [seq, 4096, 12288] for key, *shape in got), got
+
+
+@pytest.mark.parametrize("al,bl", [(0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(900, 1800, 16), (1200, 1200, 40), (1024, 1040, 63), (1040, 1984, 8)])
+def test_part_of_a_k_tile_in_one_round_of_64_tiles(M, N, K, al, bl):
+    test_tiles_of_32(M, N, K, al, bl)
