@@ -1220,7 +1220,7 @@ static bool fused_wins(int M, int N, int K, float per_round, float passes) {
   const int64_t n = (int64_t)tm * tn;
   auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * (N / t); };
   const Cut cut = find_cut(tm, tn);
-  float plain = std::min(cost_64(tiles(64), kt), cost_128(tiles(128), kt, true));
+  float plain = std::min(cost_small(M, N, kt, true), cost_128(tiles(128), kt, true));
   plain = std::min(plain, cut.rm || cut.cn ? cost_256(n, kt, 0, true) : cost_rounds(n, kt));
   return cost_rounds(n, kt) + per_round * ((n + 255) / 256) <= plain + passes;
 }
