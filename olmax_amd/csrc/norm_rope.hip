@@ -642,9 +642,10 @@ extern "C" int32_t olmax_rmsnorm_bwd(hipStream_t stream, const void* x, const vo
                        dxp, dw, rows, d, ldx, lddy, lddres, lddx, eps);                                                           \
   } while (0)
   if (vec && d % 8 == 0 && d <= 256) {
-    // with dw few large workgroups, so that few atomics meet in a column: us with 32 lanes a row in 128 workgroups of 32 rows | 16 lanes in 256 of
-    // 16: 512 x 256 5.2 | 5.6, 2048 x 256 6.6 | 8.2, 8192 x 256 10.3 | 14.6 (without dw 5.0, 5.0, 8.7)
-    if (dw) OLMAX_NORM_BWD(32, 1024, 128, rmsnorm_bwd_kernel<32, 1, 1024>);
+    // with dw few large workgroups, so that few atomics meet in a column: us with 32 lanes a row in 128 (from 32768 rows on 256) workgroups of 32 rows | 16
+    // lanes in 256 of 16: 512 x 256 3.9 | 4.5, 8192 x 256 8.3 | 11.9, 65536 x 256 23.5 (in 128: 28.6) | 41.1, 16384 x 256 11.3 (in 256: 12.0) | 15.5.
+    // Up to 128 wide a row needs 16 lanes: 128 x 128 3.6 | 3.2, 512 x 64 3.9 | 3.75, but 1024 x 64 4.3 | 4.5, 8192 x 128 8.0 | 10.2, 65536 x 128 21.2 | 26.2.
+    if (dw && (d > 128 || rows > 512)) OLMAX_NORM_BWD(32, 1024, rows < 32768 ? 128 : 256, rmsnorm_bwd_kernel<32, 1, 1024>);
     else OLMAX_NORM_BWD(16, 256, 256, rmsnorm_bwd_kernel<16, 2, 256>);
   } else if (vec && d % 8 == 0 && d <= 1024) {
     // without dw nothing has to meet: small workgroups start sooner (512 x 512: 4.0 -> 3.2 us) and do as well on many rows
