@@ -377,13 +377,20 @@ Layout layout_of(const olmax_model_config* c) {
   return L;
 }
 
+// From this many parameters on the embedding's update takes two parts in the overlapped step (OverlapCtx): 0.4 ms or more at the end of a step.
+constexpr int64_t EARLY_EMBEDDING = 64 << 20;
+bool early_embedding(const olmax_model_config* c) {
+  const Dims m = dims_of(c);
+  return (int64_t)c->vocab * m.d >= EARLY_EMBEDDING && m.d >= 1024 && m.T < c->vocab && c->n_layers > 0 && c->checkpoint;
+}
+
 struct ModelWs {
   bf16* xs;       // [(L+1), T, d] layer inputs (xs[L] = final hidden state)
   bf16* hn;       // [T, d] final-normed hidden
   bf16 *da, *db;  // [T, d] gradient ping-pong
   void* head_ws;
   int64_t head_ws_bytes;
-  int32_t* first_use;  // [vocab], see EARLY_EMBEDDING
+  int32_t* first_use;  // [vocab], see early_embedding; else null
   Tmp tmp;
   char* acts_base;
   int64_t acts_stride;
@@ -397,7 +404,7 @@ ModelWs carve_model(const olmax_model_config* c, Arena& a, bool need_bwd) {
   w.db = a.take<bf16>(m.T * m.d);
   w.head_ws_bytes = olmax_lmhead_ce_workspace_bytes(m.T, c->vocab);
   w.head_ws = a.take<char>(w.head_ws_bytes);
-  w.first_use = a.take<int32_t>(c->vocab);
+  if (early_embedding(c)) w.first_use = a.take<int32_t>(c->vocab);
   if (need_bwd) w.tmp = carve_tmp(c, a);
   Arena probe(nullptr);
   carve_acts(c, probe);
@@ -619,8 +626,6 @@ struct OverlapCtx {
   float embed_wd = 0.f;
   bool tied = false;
 };
-// From this many parameters on the embedding's update takes the two parts: 0.4 ms or more at the end of a step.
-constexpr int64_t EARLY_EMBEDDING = 64 << 20;
 // AdamW launches the last olmax_model_train_step of this host thread put on its optimizer stream
 // (0: the step took the sequential branch); read back by tests through
 // olmax_model_last_step_overlapped_launches
@@ -1020,9 +1025,8 @@ extern "C" int32_t olmax_model_train_step(hipStream_t stream, hipStream_t opt_st
   if (hipEventRecord(ev, stream) != hipSuccess || hipStreamWaitEvent(opt_stream, ev, 0) != hipSuccess)
     rc = olmax_set_error(OLMAX_ERR_LAUNCH, "olmax_model_train_step: event record/wait failed");
   const Dims m = dims_of(c);
-  if (!rc && (int64_t)c->vocab * m.d >= EARLY_EMBEDDING && m.d >= 1024 && m.T < c->vocab && c->n_layers > 0 && ids && workspace &&
-      (((uintptr_t)workspace) & 255) == 0 && workspace_bytes >= olmax_model_workspace_bytes(c) && aligned16(master) && aligned16(mom) &&
-      aligned16(var) && aligned16(grad_f32) && aligned16(params_bf16)) {
+  if (!rc && early_embedding(c) && ids && workspace && (((uintptr_t)workspace) & 255) == 0 &&
+      workspace_bytes >= olmax_model_workspace_bytes(c) && aligned16(master) && aligned16(mom) && aligned16(var) && aligned16(grad_f32) && aligned16(params_bf16)) {
     Arena arena(workspace);
     int32_t* first_use = carve_model(c, arena, true).first_use;
     rc = olmax_first_use(stream, ids, first_use, m.T, c->vocab);
