@@ -661,8 +661,10 @@ int overlap_head_chunk(OverlapCtx* x, int64_t n, int grid_cap) {
 // up to n more elements of the embedding's unnamed rows
 int overlap_embed_chunk(OverlapCtx* x, int64_t n, int grid_cap) {
   n = std::min((n + 3) / 4 * 4, x->embed_numel - x->embed_done);
+  if (n <= 0) return OLMAX_OK;
   const int64_t at = x->embed_done;
   x->embed_done += n;
+  g_overlapped_launches++;
   return olmax_adamw_unused_rows(x->opt, x->master, x->tied ? x->grad_f32 : nullptr, x->mom, x->var, x->shadow, x->first_use, at, n, x->d, x->lr,
                                  x->b1, x->b2, x->eps, x->embed_wd, x->step, grid_cap, x->hyper_dev);
 }
