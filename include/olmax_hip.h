@@ -396,7 +396,7 @@ void olmax_gemm_set_order(int order);
 /* Record a HIP-event pair on the launch stream around every MFMA GEMM launch between begin and
  * end (allocates events).  end() waits for them and aggregates per kernel instantiation:
  * key = tile (64: 64 or 32, 128, 256) | a_kc<<12 | b_kc<<13 | has_res<<14 | out_f32<<15 | glu_epilogue<<16 |
- * rope_epilogue<<17 | shared_reduction<<18 | both_gradients<<19 (M, N, K: tokens, in, out); ms = summed durations, flops / bytes = summed algorithmic work (2MNK;
+ * rope_epilogue<<17 | shared_reduction<<18 | both_gradients<<19 (M, N, K: tokens, in, out; has_res: dX has one); ms = summed durations, flops / bytes = summed algorithmic work (2MNK;
  * operands and result moved once).  Returns the number of distinct keys written (at most cap). */
 void olmax_gemm_profile_begin(void);
 int32_t olmax_gemm_profile_end(int32_t* keys, double* ms, double* flops, double* bytes, int64_t* launches,

@@ -1449,7 +1449,7 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
       (void)hipEventRecord(rec.e1, s);
       rec.flops = 4.0 * T * in * out;
       rec.bytes = 2.0 * ((double)T * out + 2.0 * T * in + (r ? 1.0 * T * in : 0.0) + 2.0 * in * out);
-      rec.key = tile | (1 << 19);
+      rec.key = tile | ((r != nullptr) << 14) | (1 << 19);
       rec.M = T; rec.N = in; rec.K = out;
       std::lock_guard<std::mutex> lk(g_prof_mu);
       g_prof.push_back(rec);

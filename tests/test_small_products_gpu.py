@@ -85,10 +85,11 @@ def test_both_gradients_in_one_launch_of_large_tiles(T, d, V, tile):
     check_gradients(h, W, labels, *out[1:])
 
 
-@pytest.mark.parametrize("seq", [1500, 2048])
-def test_a_residual_joins_the_first_product(seq):
-    """Post-norm blocks add the residual's gradient in dX.  Against the two calls, which a forced tile brings back: the products are
-    rounded to bf16 (2^-9 each) and four of them follow one another."""
+@pytest.mark.parametrize("seq,tile,out", [(1500, 0, 0), (2048, 0, 0), (1000, 128, 22016), (2500, 256, 22016), (3000, 256, 12288)])
+def test_a_residual_joins_the_first_product(seq, tile, out):
+    """Post-norm blocks add the residual's gradient in dX, in one launch with dW in the last three cases (ragged rows, partial k-tiles); in the
+    others the products with a residual are two calls, beside those without.  Against the two calls, which a forced tile brings back: the products
+    are rounded to bf16 (2^-9 each) and four of them follow one another."""
     from olmax_amd import TransformerRecipe, _lib
     from olmax_amd.layer import TransformerBlock
     import dataclasses
@@ -102,6 +103,8 @@ def test_a_residual_joins_the_first_product(seq):
     res, dx = {}, []
     got = recorded(lambda: dx.append(block.backward(dy)))
     assert any(key >> 19 & 1 for key, *_ in got), got
+    assert any(key >> 19 & 1 and key >> 14 & 1 for key, *_ in got) == (tile != 0), got
+    assert not tile or (tile | 1 << 14 | 1 << 19, seq, 4096, out, 1) in got, got
     res[0] = [dx[0].clone()] + [v.clone() for v in block.grads.values()]
     for v in block.grads.values():
         v.zero_()
