@@ -190,6 +190,7 @@ __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
     float* __restrict__ row_loss, float* __restrict__ lse_out, const int32_t* __restrict__ n_counted,
     int V, int64_t ld, int64_t ldd, int32_t ignore_index, float cap, float dloss,
     const float* __restrict__ drow, int mean) {
+  static_assert(!(CAP && TAIL), "soft-capped rows beyond the registers take the streaming form");
   constexpr int NW = THREADS / 64;
   constexpr int HELD = MAXV * THREADS;  // vectors in registers
   constexpr uint32_t NEG_INF2 = 0xff80ff80u;
@@ -258,7 +259,6 @@ __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
       for (int u = 0; u < U; u++)
 #pragma unroll
         for (int e = 0; e < 8; e++) cm = fmaxf(cm, bf2f(t[u].e[e]));
-      if (CAP) cm = cap * soft(cm);
       if (cm > mx) {
         tsm *= __expf(mx - cm);
         mx = cm;
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(THREADS, 4) void ce_row_regs_kernel(
       const float ref = mx == -INFINITY ? 0.f : mx;  // nothing but minus infinity so far: the sum stays 0
 #pragma unroll
       for (int u = 0; u < U; u++)
-        if (!CAP || i0 + u * THREADS < nvec) tsm += exps(t[u], i0 + u * THREADS, ref);
+        tsm += exps(t[u], i0 + u * THREADS, ref);
     }
   }
   const float tmx = mx;

@@ -69,6 +69,11 @@ def test_rows_far_from_zero(V):
     zd = z.double()
     p = (zd - lse.cpu().double()[:, None]).exp()  # against the lse that the row has in fp32
     assert torch.isfinite(dz).all()
+    # sums of up to 2^18 terms, each off by a few 2^-24 for exponents up to 12; then the logarithm is added to the maximum in fp32
+    got = lse.cpu().double()
+    assert ((got - zd.logsumexp(1)).abs() <= 2 ** -23 * got.abs() + 2 ** -19).all()
+    want = (got - zd[torch.arange(4), labels.long()]).mean()
+    assert (loss.double().cpu() - want).abs() <= 2 ** -22 * want
     want = p / 4
     want[torch.arange(4), labels.long()] -= 0.25
     err = (dz.cpu().double() - want).abs() - (2 ** -8 * want.abs() + 2 ** -22 / 4)
