@@ -69,3 +69,14 @@ def test_ops_refuse_cpu_tensors():
     from olmax_amd import _lib, ops
     with pytest.raises(_lib.OlmaxHipError):
         ops.rms_norm_fwd(torch.zeros(2, 8, dtype=torch.bfloat16), None, 1e-6)
+
+
+def test_typed_entry_points_match_the_header():
+    """The argument types that _lib sets by hand, letter by letter: a wrong one would only show as a wrong argument on the GPU."""
+    from olmax_amd import _lib
+    text = re.sub(r"/\*.*?\*/", "", (ROOT / "include" / "olmax_hip.h").read_text(), flags=re.S)
+    for name, letters in _lib._SIGNATURES.items():
+        ret, args = re.search(r"(\w+)\s+" + name + r"\s*\(([^;]*)\)\s*;", text).groups()
+        kinds = ["P" if "*" in a or "olmax_stream_t" in a else {"int32_t": "I", "int": "I", "int64_t": "L", "float": "F"}[a.replace("const", "").split()[0]]
+                 for a in args.split(",")]
+        assert ret == "int32_t" and "".join(kinds) == letters, name
