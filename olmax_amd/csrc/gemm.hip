@@ -91,15 +91,16 @@ std::mutex g_prof_mu;
 // that fetched a chunk past the end overwrites it with zeros in LDS once its own fetches have landed,
 // before the barrier that publishes the stage.  Wants M >= BM, N >= BN, K >= 64 and 16-byte chunks that do not cross the end of a row (see olmax_gemm_padded).
 //
-// The tile that workgroup `pid` of `nwg` takes; the residual of a HAS_RES form may be null.  BLOCKS: the sums of every four k-tiles (below
-// 16 of them: two) are added up by themselves, so that a chain of fp32 additions is no longer than that of eight waves with every eighth k-tile each
-// (gemm_small.hip).  64 registers and 64 additions a block: 1 to 4 % (both gradients of 3000 x 1024 x 3072 47.5 -> 48.0 us, 512 x 4608 x 8192 86.2 -> 89.0).
-template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI, int RAG, bool BLOCKS = false>
+// The tile that workgroup `pid` of `nwg` takes; the residual of a HAS_RES form may be null.  BLOCKS: the sums of every `block` k-tiles (an
+// even number) are added up by themselves, for shorter chains of fp32 additions: 1 in registers, 2 (256 tiles, which have none left) parked
+// in `park`, 256 KB a tile and block.  us, both gradients with one chain -> with blocks: 3000 x 1024 x 3072 46.6 -> 46.6,
+// 4096 x 1024 x 3072 55.2 -> 55.7 (blocks of four k-tiles 56.3), 512 x 2816 x 1024 16.2 -> 16.6; 2048 x 4096 x 12288 305.8 -> 314.6.
+template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI, int RAG, int BLOCKS = 0>
 __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
     const bf16* __restrict__ R, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     int64_t ldr, int tiles_m, int tiles_n, int c_vec, const float* __restrict__ cos_t,
-    const float* __restrict__ sin_t, int seq_len, int rope_cols, int order, int pid, const int nwg, unsigned char* smem) {
+    const float* __restrict__ sin_t, int seq_len, int rope_cols, int order, int pid, const int nwg, unsigned char* smem, int block = 0, float* park = nullptr) {
   constexpr int GLU = (EPI == 1 || EPI == 2) ? EPI : (EPI == 4 ? 1 : (EPI == 5 ? 2 : 0));
   constexpr bool GLU_BWD = EPI == 4 || EPI == 5;
   constexpr bool ROPE = EPI == 3;
@@ -499,35 +500,58 @@ __device__ __forceinline__ void gemm_tile(
       bp += b_step;
     }
   };
-  f32x4 sum[BLOCKS ? TM : 1][TN];
-  const int block = KT < 16 ? 0 : 2;
-  if (BLOCKS) {
+  f32x4 sum[BLOCKS == 1 ? TM : 1][TN];
+  if (BLOCKS == 1) {
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-      for (int j = 0; j < TN; j++) sum[BLOCKS ? i : 0][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < TN; j++) sum[BLOCKS == 1 ? i : 0][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  int ends = block, parked = 0;  // of the block; blocks before it
+  auto parking = [&](int b) { return park + ((((int64_t)b * tiles_m + tile_m) * tiles_n + tile_n) * NW + wave) * (NM * 256); };  // of this wave
+  // (a copy of the lane id that the compiler cannot see through: no address of the rare accesses lives through the loop)
+  auto hidden_lane = [&]() {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l * 4;
+  };
   for (int kt = 0; kt + 1 < KT; kt += 2) {
     k_tile(kt, std::integral_constant<int, 0>());
     k_tile(kt + 1, std::integral_constant<int, 1>());
-    if (BLOCKS && (kt & block) == block) {
+    if (BLOCKS && kt + 2 == ends && ends < KT) {
+      ends += block;
+      float* q = parking(parked++);
+      const int at = hidden_lane();
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-          sum[BLOCKS ? i : 0][j] += acc[i][j];
+          if (BLOCKS == 1) sum[BLOCKS == 1 ? i : 0][j] += acc[i][j];
+          else *reinterpret_cast<f32x4*>(q + (i * TN + j) * 256 + at) = acc[i][j];
           acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
   }
   if (KT & 1) k_tile(KT - 1, std::integral_constant<int, 0>());
-  if (BLOCKS) {
+  if (BLOCKS == 1) {
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] += sum[BLOCKS ? i : 0][j];
+      for (int j = 0; j < TN; j++) acc[i][j] += sum[BLOCKS == 1 ? i : 0][j];
   }
   dma_wait_all();  // the redundant tail DMAs must not outlive the workgroup's LDS allocation
+  if (BLOCKS == 2) {  // (all that was parked has been written)
+    for (int b = 0; b < parked; b++) {
+      const float* q = parking(b);
+      const int at = hidden_lane();
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] += *reinterpret_cast<const f32x4*>(q + (i * TN + j) * 256 + at);
+        __builtin_amdgcn_sched_barrier(0);  // (the loads of all rows at once do not fit the registers)
+      }
+    }
+  }
   // The epilogue derives its addresses from a copy of the lane id that the compiler cannot see
   // through, so none of them is computed ahead of the loop and kept in registers across it.
   int lane_e = lane;
@@ -785,9 +809,10 @@ struct PairSide {
   bf16* C;
   int M, N, K;
   int64_t lda, ldb, ldc, ldr;
-  int tiles_m, tiles_n, order, nwg;
+  int tiles_m, tiles_n, order, nwg, block;
+  float* park;
 };
-template <int T, int W, int RAGX, int RAGW, bool BLOCKS>
+template <int T, int W, int RAGX, int RAGW, int BLOCKS>
 __global__ __launch_bounds__((T / W) * (T / 64) * 64) __attribute__((amdgpu_num_vgpr(120))) void gemm_pair_kernel(const PairSide x, const PairSide w, int x_first, int n_first) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const bool second = (int)blockIdx.x >= n_first;
@@ -795,11 +820,11 @@ __global__ __launch_bounds__((T / W) * (T / 64) * 64) __attribute__((amdgpu_num_
   if (second != (x_first != 0)) {
     if (pid >= x.nwg) return;
     gemm_tile<T, T, W, 64, true, false, true, false, 0, RAGX, BLOCKS>(x.A, x.B, x.C, x.R, x.M, x.N, x.K, x.lda, x.ldb, x.ldc, x.ldr, x.tiles_m, x.tiles_n, 1,
-                                                              nullptr, nullptr, 1, 0, x.order, pid, x.nwg, smem);
+                                                              nullptr, nullptr, 1, 0, x.order, pid, x.nwg, smem, x.block, x.park);
   } else {
     if (pid >= w.nwg) return;
-    gemm_tile<T, T, W, 64, false, false, false, false, 0, RAGW, BLOCKS>(w.A, w.B, w.C, nullptr, w.M, w.N, w.K, w.lda, w.ldb, w.ldc, 0, w.tiles_m, w.tiles_n, 1,
-                                                                nullptr, nullptr, 1, 0, w.order, pid, w.nwg, smem);
+    gemm_tile<T, T, W, 64, false, false, false, false, 0, RAGW, BLOCKS & 1>(w.A, w.B, w.C, nullptr, w.M, w.N, w.K, w.lda, w.ldb, w.ldc, 0, w.tiles_m, w.tiles_n, 1,
+                                                                nullptr, nullptr, 1, 0, w.order, pid, w.nwg, smem, w.block);
   }
 }
 
@@ -899,7 +924,7 @@ int launch_glu(hipStream_t s, const bf16* A, const bf16* B, bf16* gu, bf16* act,
   return OLMAX_OK;
 }
 
-template <int T, int W, int RAGX, int RAGW, bool BLOCKS>
+template <int T, int W, int RAGX, int RAGW, int BLOCKS>
 void launch_pair(hipStream_t s, PairSide x, PairSide w) {
   auto kern = gemm_pair_kernel<T, W, RAGX, RAGW, BLOCKS>;
   constexpr int SMEM = 4 * T * BK * 2;
@@ -1248,16 +1273,20 @@ static int chain_of_product(int M, int N, int K, bool a_kc, bool b_kc, bool dire
   }
   return chain_of_parts(1, kt);
 }
-// and of the forms of both gradients in one launch: small tiles (see olmax_gemm_small_pair), 128 ones, whose sums may be blocked, and 256 ones.
-static int chain_in_pair(int tile, bool blocks, int M, int N, int K) {
+// and of the small tiles in the one launch of both gradients (see olmax_gemm_small_pair).
+static int chain_of_small_pair(int M, int N, int K) {
   const int kt = (K + BK - 1) / BK;
-  if (tile >= 128 && !blocks) return chain_of_parts(1, kt);
-  if (tile == 128) {
-    const int steps = std::min(kt, kt < 16 ? 2 : 4);
-    return chain_of_parts((kt + steps - 1) / steps, steps);
-  }
   const int g = std::min(kt, tiles_of(M, N, 64) <= 256 ? 8 : 4);
   return chain_of_parts(g, (kt + g - 1) / g);
+}
+
+// Blocks of k-tiles (gemm_tile) that keep a chain to `most` additions: as few and large as that allows, of an even number of k-tiles; 0: none do.
+static int block_of(int kt, int most) {
+  for (int n = 1;; n++) {
+    const int b = ((kt + n - 1) / n + 1) & ~1;
+    if (chain_of_parts((kt + b - 1) / b, std::min(kt, b)) <= most) return b;
+    if (b == 2) return 0;
+  }
 }
 
 enum GluForm { GLU_SAVE, GLU_ONLY, GLU_BWD };
@@ -1402,19 +1431,24 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
   (void)pick_tile(T, in, out, true, false, direct_x, bytes, &parts, &best);
   (void)pick_tile(out, in, T, false, false, direct_w, bytes, &parts, &best_w);
   best += best_w;
-  // One launch may not be less precise: no chain of additions longer than the calls'.
+  // One launch may not be less precise: no chain of additions longer than the calls', which may have several waves or workgroups to a reduction.
   const int chain_x = chain_of_product(T, in, out, true, false, direct_x, bytes), chain_w = chain_of_product(out, in, T, false, false, direct_w, bytes);
-  auto precise = [&](int t, bool blocks) { return chain_in_pair(t, blocks, T, in, out) <= chain_x && chain_in_pair(t, blocks, out, in, T) <= chain_w; };
+  const int ktx = (out + BK - 1) / BK, ktw = (T + BK - 1) / BK, block_x = block_of(ktx, chain_x), block_w = block_of(ktw, chain_w);
+  const bool whole = block_x >= ktx && block_w >= ktw;
+  // what the blocks of dX take of the scratch memory in 256 tiles (dW has no registers left for the addresses)
+  const int64_t park = block_x ? ((ktx + block_x - 1) / block_x - 1) * tiles_of(T, in, 256) * 262144 : 0;
   int tile = 0;  // of the one launch, 0: two calls
   // (the one form of the small kernel that is built: whole chunks, 32-bit line offsets and at least a tile of rows)
   const bool small = !dw_f32 && out % 8 == 0 && in % 8 == 0 && T >= 64 && lddy < (1 << 25) && ldw < (1 << 25) && ldx < (1 << 25);
-  if (const float c = pair_small(T, in, out); small && c < best && precise(64, false)) best = c, tile = 64;
+  if (const float c = pair_small(T, in, out); small && c < best && chain_of_small_pair(T, in, out) <= chain_x && chain_of_small_pair(out, in, T) <= chain_w)
+    best = c, tile = 64;
   // vector stores, whole k-tiles in the first product
   const bool large = !dw_f32 && direct_x && direct_w && out % BK == 0 && lddx % 8 == 0 && lddw % 8 == 0 && (!r || (ldr % 8 == 0 && aligned16(r))) &&
                      aligned16(dx) && aligned16(dw);
   for (int t = 128; t <= 256; t *= 2) {
-    if (!large || T < t || in < t || out < t || !precise(t, t == 128)) continue;
-    const Work wx = {tiles_of(T, in, t), out / BK}, ww = {tiles_of(out, in, t), (T + BK - 1) / BK};
+    if (!large || T < t || in < t || out < t || !block_x || !block_w) continue;
+    if (t == 256 && (park > bytes || block_w < ktw)) continue;
+    const Work wx = {tiles_of(T, in, t), ktx}, ww = {tiles_of(out, in, t), ktw};
     const Work &l = wx.kt > ww.kt ? wx : ww, &sh = wx.kt > ww.kt ? ww : wx;
     if (const float c = t == 128 ? pair_128(l, sh) : pair_256(l, sh); c < best) best = c, tile = t;
   }
@@ -1432,7 +1466,10 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
     if (tile == 64) {
       olmax_gemm_small_pair(s, dy, w, x, dx, r, (bf16*)dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw);
     } else {
-      const PairSide px = {dy, w, r, dx, T, in, out, lddy, ldw, lddx, ldr}, pw = {dy, x, nullptr, (bf16*)dw, out, in, T, lddy, ldx, lddw, 0};
+      PairSide px = {dy, w, r, dx, T, in, out, lddy, ldw, lddx, ldr}, pw = {dy, x, nullptr, (bf16*)dw, out, in, T, lddy, ldx, lddw, 0};
+      px.block = block_x;
+      pw.block = block_w;
+      px.park = (float*)scratch.p;
       const bool rx = T % tile || in % tile;
       const int rw = T % BK ? 2 : out % tile || in % tile;
 #define PAIR(E, W, B)                                                                                                           \
@@ -1440,9 +1477,10 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
     if (rx) rw == 2 ? launch_pair<E, W, 1, 2, B>(s, px, pw) : rw ? launch_pair<E, W, 1, 1, B>(s, px, pw) : launch_pair<E, W, 1, 0, B>(s, px, pw); \
     else rw == 2 ? launch_pair<E, W, 0, 2, B>(s, px, pw) : rw ? launch_pair<E, W, 0, 1, B>(s, px, pw) : launch_pair<E, W, 0, 0, B>(s, px, pw);    \
   } while (0)
-      if (tile == 128 && !precise(128, false)) PAIR(128, 64, true);
-      else if (tile == 128) PAIR(128, 64, false);
-      else PAIR(256, 128, false);
+      if (tile == 128 && !whole) PAIR(128, 64, 1);
+      else if (tile == 128) PAIR(128, 64, 0);
+      else if (whole) PAIR(256, 128, 0);
+      else PAIR(256, 128, 2);
 #undef PAIR
     }
     if (g_prof_on) {

@@ -85,10 +85,10 @@ def test_both_gradients_in_one_launch_of_large_tiles(T, d, V, tile):
     check_gradients(h, W, labels, *out[1:])
 
 
-@pytest.mark.parametrize("seq,tile,out", [(1500, 0, 0), (2048, 0, 0), (1000, 128, 22016), (2500, 256, 22016), (3000, 256, 12288)])
+@pytest.mark.parametrize("seq,tile,out", [(1500, 0, 0), (2048, 256, 22016), (1000, 128, 22016), (2500, 256, 22016), (3000, 256, 12288)])
 def test_a_residual_joins_the_first_product(seq, tile, out):
-    """Post-norm blocks add the residual's gradient in dX, in one launch with dW in the last three cases (ragged rows, partial k-tiles); in the
-    others the products with a residual are two calls, beside those without.  Against the two calls, which a forced tile brings back: the products
+    """Post-norm blocks add the residual's gradient in dX, in one launch with dW, of whole and of ragged rows and k-tiles; at 1500 tokens
+    they are two calls, beside a launch of the products without a residual.  Against the two calls, which a forced tile brings back: the products
     are rounded to bf16 (2^-9 each) and four of them follow one another."""
     from olmax_amd import TransformerRecipe, _lib
     from olmax_amd.layer import TransformerBlock
@@ -182,11 +182,11 @@ def test_one_launch_of_operands_that_only_the_small_kernel_takes(T, d, V):
 
 
 @pytest.mark.parametrize("T,d,V,which,block", [
-    (4096, 1024, 3072, "dh", 4), (4096, 1024, 3072, "dW", 4), (3000, 1024, 2880, "dh", 4), (3000, 1024, 2880, "dW", 4),  # partial k-tile and ragged edges
-    (512, 2816, 1024, "dh", 4), (512, 2816, 1024, "dW", 2)])
+    (8192, 1024, 3072, "dW", 32), (4096, 1024, 3072, "dW", 16), (512, 2816, 1024, "dh", 4), (320, 2816, 320, "dh", 2), (320, 2816, 320, "dW", 2),
+    (3000, 1024, 2880, "dh", 12), (3000, 1024, 2880, "dW", 12)])  # partial k-tile and ragged edges
 def test_128_tiles_in_one_launch_add_in_blocks(T, d, V, which, block):
     """1 in the first block of k-tiles, 2^24 and -2^24 in the second: one chain over all of them would lose the 1 (2^24 + 1 = 2^24 in fp32).  The
-    same in the last whole block."""
+    same in the last whole block.  The blocks are as large as the chains of the two calls allow."""
     print(f"[case] blocks T{T} d{d} V{V} {which}", flush=True)
     K = V if which == "dh" else T
     n, first = -(-K // 64) // block * block, int(K % 64 != 0)  # (a partial k-tile comes before the whole ones)
@@ -198,17 +198,32 @@ def test_128_tiles_in_one_launch_add_in_blocks(T, d, V, which, block):
 
 
 @pytest.mark.parametrize("seq", [1700, 2048])
-def test_one_launch_leaves_the_calls_their_shared_reductions(seq):
-    """The q|k|v gradients of a post-norm block: dX shares its 12288-long reduction between two workgroups, half the chain of the one launch's tiles."""
+def test_one_launch_parks_the_sums_that_the_calls_share(seq, monkeypatch):
+    """dX of the q|k|v and the gate|up projections of a post-norm block: 12288 and 22016 long, each half a chain of its own as in the two calls, where
+    two workgroups share a reduction.  The calls, which gradients in the place of their weights bring back, add the same two sums: bit-equal."""
     import dataclasses
     from olmax_amd import TransformerRecipe
     from olmax_amd.layer import TransformerBlock
-    print(f"[case] shared reductions S{seq}", flush=True)
+    print(f"[case] parked sums S{seq}", flush=True)
     block = TransformerBlock(dataclasses.replace(TransformerRecipe.olmo2_7B(), num_layers=1), batch_size=1, sequence_length=seq)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for w in (block.wqkv, block.wo, block.wgu, block.wdown):
+        w.normal_(0.0, 0.02, generator=g)
     block.forward(rnd(seq, 4096, seed=1))
-    got = recorded(lambda: block.backward(rnd(seq, 4096, seed=2)))
-    assert any(key >> 18 & 1 and shape[:3] == [seq, 4096, 12288] for key, *shape in got), got
-    assert not any(key >> 19 & 1 and shape[:3] == [seq, 4096, 12288] for key, *shape in got), got
+    dy, res = rnd(seq, 4096, seed=2), []
+
+    def backward():
+        res.append([block.backward(dy)] + [block.grads[k].clone() for k in ("attention.q_proj.weight", "attention.v_proj.weight", "mlp.up_proj.weight")])
+    got = recorded(backward)
+    for out in (12288, 22016):
+        assert (256 | 1 << 14 | 1 << 19, seq, 4096, out, 1) in got, got
+    fresh = torch.empty_like
+    monkeypatch.setattr(torch, "empty_like", lambda t: t if t is block.wqkv or t is block.wgu else fresh(t))
+    got = recorded(backward)
+    for out in (12288, 22016):
+        assert any(key >> 18 & 1 and shape[:3] == [seq, 4096, out] for key, *shape in got), got
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("al,bl", [(0, 0), (0, 1), (1, 1)])
