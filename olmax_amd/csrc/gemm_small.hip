@@ -168,8 +168,9 @@ int tiles(const Problem& p) {
   return (int)((int64_t)((p.M + TS - 1) / TS) * ((p.N + TS - 1) / TS));
 }
 
-// Tile `pid` of `nwg` by the KG waves of a workgroup.  TWO: a wave's k-tiles go to two accumulators in turn, so that four waves have
-// the chains of fp32 additions of eight.
+// Tile `pid` of `nwg` by the KG waves of a workgroup.  TWO: the first half of a wave's k-tiles is added up by itself, so that four
+// waves have the chains of fp32 additions of eight.  (Two accumulators in turn, the loop's code twice: 2 % more time over 64 pairs of gradients,
+// 2048 x 256 x 768 9.66 us, 9.42 in halves, 512 x 1024 x 1024 9.42 and 8.91.)
 template <int TS, int KG, bool A_KC, bool B_KC, Mode MODE, bool TWO = false>
 __device__ __forceinline__ void small_tile(const Problem& P, int pid, int nwg, unsigned char* smem) {
   const bf16 *A = P.A, *B = P.B, *R = P.R;
@@ -232,16 +233,20 @@ __device__ __forceinline__ void small_tile(const Problem& P, int pid, int nwg, u
   const int ktf = K / BKS;  // whole k-tiles
   int kt = wave;
   if (kt < ktf) load(kt);
+  const int half = TWO ? wave + (ktf - wave + 2 * KG - 1) / (2 * KG) * KG : 0;  // first k-tile of the second half
   for (; kt < ktf; kt += KG) {
+    if (TWO && kt == half) {
+#pragma unroll
+      for (int i = 0; i < TF; i++)
+#pragma unroll
+        for (int j = 0; j < TF; j++) {
+          accs[TWO][i][j] = accs[0][i][j];
+          accs[0][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
     park();
     if (kt + KG < ktf) load(kt + KG);
     multiply(accs[0]);
-    if (!TWO) continue;
-    kt += KG;
-    if (kt >= ktf) break;
-    park();
-    if (kt + KG < ktf) load(kt + KG);
-    multiply(accs[TWO]);
   }
   if (kt == ktf && ktf * BKS < K) {  // the ragged k-tile falls to the wave whose turn it is
     oa.load_tail(va, (int64_t)ktf * BKS, K, lane);
@@ -388,9 +393,9 @@ void olmax_gemm_small_pair(hipStream_t s, const bf16* dy, const bf16* w, const b
                            int out, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw) {
   const Problem px = {dy, w, dx, r, T, in, out, lddy, ldw, lddx, ldr, 0};
   const Problem pw = {dy, x, dw, nullptr, out, in, T, lddy, ldx, lddw, 0, 0};
-  // Tiles of 32 while they find a CU each.  Eight waves to a tile where all of them have a CU; else four, with two accumulators where the
+  // Tiles of 32 while they find a CU each.  Eight waves to a tile where all of them have a CU; else four, with two chains each where the
   // product alone would have eight (up to 256 tiles of 64, more than four k-tiles): no chain of additions is longer than in the two calls.
-  // us, eight waves | four, one accumulator | two: 1500 x 256 x 2048 12.0 | 11.8 | 13.3, 512 x 256 x 2048 7.1 | 7.0 | 7.6, 2048 x 256 x 256 6.8 | 6.6 | 6.9;
+  // us, eight waves | four, one chain | two (in turn; halves 2 % less): 1500 x 256 x 2048 12.0 | 11.8 | 13.3, 512 x 256 x 2048 7.1 | 7.0 | 7.6, 2048 x 256 x 256 6.8 | 6.6 | 6.9;
   // more tiles than CUs, 2048 x 256 x 768 12.8 | 10.7 | 11.3, 1000 x 256 x 2048 13.6 | 11.8 | 12.2, 1500 x 512 x 512 11.4 | 9.1 | 9.6.
   const int x32 = tiles<32>(px), w32 = tiles<32>(pw);
   if ((x32 <= 256 ? x32 : tiles<64>(px)) + (w32 <= 256 ? w32 : tiles<64>(pw)) <= 256) {

@@ -150,16 +150,20 @@ def head_sums(terms_h, terms_W, T, d, V):
     return got, out[1], out[2][:-1], c
 
 
-@pytest.mark.parametrize("T,d,V", [
-    (1024, 256, 1024), (1536, 256, 2048),  # every tile finds a CU: eight waves to one
-    (1024, 512, 1024), (2048, 256, 4096), (2048, 512, 1024)])  # more tiles, of 32 and 64
+@pytest.mark.parametrize("T,d,V,waves", [
+    (1024, 512, 1024, 8), (1536, 256, 2048, 8),  # every tile finds a CU
+    (1024, 256, 1024, 4), (2048, 256, 4096, 4), (2048, 512, 1024, 4)])  # more tiles, of 32 and 64: two chains to a wave
 @pytest.mark.parametrize("which", ["dh", "dW"])
-def test_one_launch_keeps_eight_chains(T, d, V, which):
+def test_one_launch_keeps_eight_chains(T, d, V, waves, which):
     """A tile of the single product has eight waves, and wave w adds the k-tiles w, w + 8, ...: 2^24 and -2^24 meet there and a 1 from a
-    k-tile of another wave counts.  One chain for the k-tiles w, w + 4, ... would lose it: 2^24 + 1 = 2^24 in fp32."""
+    k-tile of another wave counts.  One chain for the k-tiles w, w + 4, ... would lose it: 2^24 + 1 = 2^24 in fp32.  Four waves have a chain for the
+    first half of these and one for the second: there the 1 comes first."""
     print(f"[case] chains T{T} d{d} V{V} {which}", flush=True)
     n = (V if which == "dh" else T) // 64
     terms = [(w, 2.0 ** 24) for w in range(4)] + [(4 + w, 1.0) for w in range(4)] + [(8 + w, -(2.0 ** 24)) for w in range(4)]
+    if waves == 4:
+        second = 4 * -(-n // 8)  # wave w's second half
+        terms = [(w, 1.0) for w in range(4)] + [(second + w, 2.0 ** 24) for w in range(4)] + [(second + 4 + w, -(2.0 ** 24)) for w in range(4)]
     assert n > 12
     got, dh, dW, c = head_sums(*(([], terms) if which == "dh" else (terms, [])), T, d, V)
     assert (64 | 1 << 19, T, d, V, 1) in got, got
