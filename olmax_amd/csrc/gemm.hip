@@ -14,7 +14,7 @@
 // Tiling: BM x BN x 64 block tile, 64-lane waves each owning a WM x WN sub-tile as
 // (WM/16) x (WN/16) v_mfma_f32_16x16x32_bf16 accumulators. Operand tiles stream from
 // global memory straight into LDS (global_load_lds_dwordx4, no VGPR staging, no LDS-write
-// phase) into the stage that is not being consumed; one barrier per k-tile. K-contiguous tiles live in LDS as [rows][64]; M/N-contiguous
+// phase) into what has been consumed of two stages. K-contiguous tiles live in LDS as [rows][64]; M/N-contiguous
 // tiles live as [64][rows] and are read with ds_read_b64_tr_b16, the gfx950 transposing
 // LDS load, which hands each lane 4 consecutive reduction-dim elements of its column.
 //
@@ -401,7 +401,27 @@ __device__ __forceinline__ void gemm_tile(
     }
   };
 
-  // ---- main loop.  Software pipeline, all of it in registers and the two LDS stages:
+  constexpr int NM = TM * TN, NF = TM + TN;
+  constexpr bool PINGPONG = BM == 256;
+  // ---- main loop of the 256 x 256 tiles: the two waves of a SIMD (w and w + 4) take turns.  A k-tile is two phases; in each a wave
+  // first fetches the fragments and issues DMA (memory part), then runs 32 MFMAs with nothing between them (matrix part), and a
+  // barrier after every part keeps waves 4-7 exactly one part behind waves 0-3: while one wave of the SIMD owns the matrix pipe, the
+  // other waits for its LDS reads, for the DMA queue and for the landing of the next k-tile, where it costs no MFMA time.  (Before, all
+  // eight waves issued reads and DMA between their own MFMAs and met at one barrier per k-tile: a full DMA queue or a late line stopped
+  // all of them, 61 % of the MFMA rate on operands of zeros, which leave the power limit out; now 80-86 %.)  us on random operands, before -> now:
+  //   NT 8192 x 12288 x 4096 558 -> 545, 8192 x 22016 x 4096 1067 -> 1004, 8192 x 4096 x 11008 514 -> 475, 8192 x 100352 x 4096 4895 -> 4529
+  //   NN 8192 x 4096 x 12288 565 -> 532, 8192 x 4096 x 22016 1028 -> 951;  TN 12288 x 4096 x 8192 581 -> 536, 22016 x 4096 x 8192 1096 -> 1011
+  // Bound by the board's power on such operands (zeros run 30 % faster).  Four phases of 16 MFMAs: NT 0 to -1 %, NN and TN +2 to +4 %;
+  // a higher wave priority in the matrix part +0.5 %; DMA ahead of the reads +0.3 to +2.5 %.
+  //   phases: by k-step where A is [64][rows] (a DMA instruction covers whole k-rows, so k-steps are what becomes free), else by half
+  //     of the wave's rows.  B's fragments of both k-steps are fetched in phase 0 and kept, but where both go by k-step;
+  //   DMA: in the memory part after the one that read it last a region is refilled for two k-tiles on: what phase 0 reads (d0)
+  //     in phase 1 of k-tile t for t + 2, what phase 1 reads (d1) in phase 0 of t + 1 for t + 2.  Past the end the last k-tile is fetched
+  //     again into a region nobody reads any more;
+  //   waits: every wave's LDS reads are complete before the barrier that ends its memory part, so no refill can overtake a read, and
+  //     vmcnt(8) there leaves only what was issued behind the d0 / d1 that the next phase of this kind reads.
+  //
+  // ---- main loop of the 128 x 128 tiles: software pipeline, all of it in registers and the two LDS stages:
   //   * fragments are double-buffered (fa/fb[0] = k-step 0, [1] = k-step 1 of a k-tile), and
   //     every LDS read is issued half a k-tile before the MFMAs that consume it;
   //   * the DMA of k-tile kt+2 goes into the stage k-tile kt occupied, right after the barrier
@@ -410,90 +430,128 @@ __device__ __forceinline__ void gemm_tile(
   //     wave never leaves the matrix pipe without work for longer than one MFMA;
   //   * the steady state has no branches: past the end the DMA re-fetches the last k-tile and
   //     the reads fetch a stage nobody uses any more.
-  constexpr int NM = TM * TN, NF = TM + TN;
-  // Register budget: B fragments are needed by every MFMA row of a half and are double-buffered;
-  // an A fragment dies after its row (i-major MFMA order), so the first ASB of them are
-  // single-buffered -- the next k-step's data is fetched into the same registers right behind the
-  // row's last MFMA, a whole half ahead of its first use.  The last TM - ASB rows stay
-  // double-buffered so that no fetch is issued within ~8 MFMAs of the barrier that waits for it.
-  constexpr int ASB = BM == 256 ? 6 : 0, ND = TM - ASB;
-  static_assert(2 * NINS <= NM && NF + 1 <= NM && NINS + NF <= NM, "not enough MFMA slots for the loads");
-  static_assert(ASB == 0 || (NM >= 3 * NINS - 2 && NM >= 4 * (TN + ND)), "slot layout of the single-buffered scheme");
-  bf16x8 fas[ASB > 0 ? ASB : 1], fad[2][ND], fb[2][TN];
+  static_assert(PINGPONG || (2 * NINS <= NM && NF + 1 <= NM && NINS + NF <= NM), "not enough MFMA slots for the loads");
+  static_assert(!PINGPONG || (NW == 8 && TM == 8 && TN == 4 && A_INS == 4 && B_INS == 4), "phases are laid out for 8 waves of 128 x 64");
+  constexpr bool BY_K = !A_KC, B_WHOLE = A_KC || B_KC;  // PINGPONG: phases by k-step; all of B is read in phase 0
+  constexpr int ND0 = B_WHOLE ? 6 : 4;                  // DMA instructions of d0
+  bf16x8 fa[2][PINGPONG ? 4 : TM], fb[2][TN];
+  // k-tiles t + 1 (PINGPONG) and t + 2 while they exist, then the last one
+  const bf16 *ap1 = a_panel + (int64_t)min(1, KT - 1) * a_step, *bp1 = b_panel + (int64_t)min(1, KT - 1) * b_step;
+  const bf16 *ap = a_panel + (int64_t)min(2, KT - 1) * a_step, *bp = b_panel + (int64_t)min(2, KT - 1) * b_step;
+  auto dma_a = [&](const bf16* p, int stage, int i) { dma16_s(p + i * a_istep, a_off, lds_base + stage * A_BYTES + (i * NW + wave) * 1024); };
+  auto dma_b = [&](const bf16* p, int stage, int i) { dma16_s(p + i * b_istep, b_off, lds_base + 2 * A_BYTES + stage * B_BYTES + (i * NW + wave) * 1024); };
+  // (instruction i holds rows 64i .. 64i+63 of a k-contiguous tile: i even, the first half of the rows of waves 0-3 / 4-7; k-rows 16i .. 16i+15 of the others)
+  auto d0 = [&](const bf16* pa, const bf16* pb, int stage) {
+    dma_a(pa, stage, 0);
+    dma_b(pb, stage, 0);
+    if (B_WHOLE) dma_b(pb, stage, 1);
+    dma_a(pa, stage, BY_K ? 1 : 2);
+    dma_b(pb, stage, B_WHOLE ? 2 : 1);
+    if (B_WHOLE) dma_b(pb, stage, 3);
+  };
+  auto d1 = [&](const bf16* pa, const bf16* pb, int stage) {
+    dma_a(pa, stage, BY_K ? 2 : 1);
+    if (!B_WHOLE) dma_b(pb, stage, 2);
+    dma_a(pa, stage, 3);
+    if (!B_WHOLE) dma_b(pb, stage, 3);
+  };
   if (KRAG) dma_tail(0);
   else dma(0, 0, 0, NINS);
-  if (KT > 1) {
-    dma(1, 1, 0, NINS);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NINS) : "memory");  // k-tile 0 has landed
+  if constexpr (PINGPONG) {
+    if (KRAG) {
+      dma_wait_all();
+      zero_tail(0);
+    }
+    d0(ap1, bp1, 1);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(ND0) : "memory");  // k-tile 0 has landed
+    __builtin_amdgcn_s_barrier();
+    if (wave >= 4) __builtin_amdgcn_s_barrier();  // one part behind (waves 0-3 make up for it after the loop)
   } else {
-    dma_wait_all();
-  }
-  if (KRAG) zero_tail(0);
-  __syncthreads();
+    if (KT > 1) {
+      dma(1, 1, 0, NINS);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NINS) : "memory");  // k-tile 0 has landed
+    } else {
+      dma_wait_all();
+    }
+    if (KRAG) zero_tail(0);
+    __syncthreads();
 #pragma unroll
-  for (int i = 0; i < TM; i++) {
-    if (i < ASB) fas[i] = load_a1(0, 0, i);
-    else fad[0][i - ASB] = load_a1(0, 0, i);
-  }
+    for (int i = 0; i < TM; i++) fa[0][i] = load_a1(0, 0, i);
 #pragma unroll
-  for (int j = 0; j < TN; j++) fb[0][j] = load_b1(0, 0, j);
-  // running DMA bases: k-tile kt+2 while it exists, then they stop advancing
-  const bf16* ap = a_panel + (int64_t)min(2, KT - 1) * a_step;
-  const bf16* bp = b_panel + (int64_t)min(2, KT - 1) * b_step;
-  // One k-tile.  The stage is a compile-time constant (the loop below is unrolled by two), so
-  // every LDS address is a loop-invariant per-lane register plus an immediate: no address
-  // arithmetic is left in the loop, where each vector instruction costs MFMA issue time.
+    for (int j = 0; j < TN; j++) fb[0][j] = load_b1(0, 0, j);
+  }
+  // One phase of a k-tile (PINGPONG); stage and phase are compile-time constants (the loop below is unrolled by two k-tiles), so every LDS address
+  // is a loop-invariant per-lane register plus an immediate: no address arithmetic is left in the loop.
+  auto phase = [&](auto cur_tag, auto ph_tag) {
+    constexpr int cur = decltype(cur_tag)::value, ph = decltype(ph_tag)::value;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < 8; x++)
+      if (B_WHOLE ? ph == 0 : x < 4) fb[x >> 2][x & 3] = load_b1(cur, B_WHOLE ? x >> 2 : ph, x & 3);
+#pragma unroll
+    for (int x = 0; x < 8; x++) fa[x >> 2][x & 3] = BY_K ? load_a1(cur, ph, x) : load_a1(cur, x >> 2, ph * 4 + (x & 3));
+    __builtin_amdgcn_sched_barrier(0);
+    if (ph == 0) d1(ap1, bp1, cur ^ 1);
+    else d0(ap, bp, cur);
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < 8; x++) {  // fragment x of A with all of B's that go with it
+      const int i = BY_K ? x : ph * 4 + (x & 3);
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[!B_WHOLE ? 0 : BY_K ? ph : x >> 2][j], fa[x >> 2][x & 3], acc[i][j], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
   auto k_tile = [&](int kt, auto cur_tag) {
     constexpr int cur = decltype(cur_tag)::value;
     constexpr int nxt = cur ^ 1;
-    const unsigned da = lds_base + cur * A_BYTES, db = lds_base + 2 * A_BYTES + cur * B_BYTES;
-    // ---- first half: k-step 0 from registers; the fragments of k-step 1 are fetched meanwhile
-    // (no fetch in slot 0: hoisted above the first MFMA it would make that MFMA's operand wait,
-    // an in-order counter, cover the new read's latency as well)
+    if constexpr (PINGPONG) {
+      phase(cur_tag, std::integral_constant<int, 0>());
+      phase(cur_tag, std::integral_constant<int, 1>());
+      ap1 = ap;
+      bp1 = bp;
+    } else {
+      // ---- first half: k-step 0 from registers; the fragments of k-step 1 are fetched meanwhile
+      // (no fetch in slot 0: hoisted above the first MFMA it would make that MFMA's operand wait,
+      // an in-order counter, cover the new read's latency as well)
 #pragma unroll
-    for (int m = 0; m < NM; m++) {
-      const int i = m / TN, j = m % TN;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], i < ASB ? fas[i] : fad[0][i < ASB ? 0 : i - ASB], acc[i][j], 0, 0, 0);
-      if (m >= 1 && m <= TN) fb[1][m - 1] = load_b1(cur, 1, m - 1);
-      if (m > TN && m <= TN + ND) fad[1][m - TN - 1] = load_a1(cur, 1, ASB + m - TN - 1);
-      if (j == TN - 1 && i < ASB) fas[i] = load_a1(cur, 1, i);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // k-tile kt+1 has landed (issued one k-tile ago); every wave is done reading k-tile kt
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __syncthreads();
-    // ---- second half: k-step 1 from registers; the slots issue the DMA of k-tile kt+2 into the
-    // retired stage and fetch k-step 0 of k-tile kt+1; the first MFMA goes out right behind the barrier
+      for (int m = 0; m < NM; m++) {
+        const int i = m / TN, j = m % TN;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[0][i], acc[i][j], 0, 0, 0);
+        if (m >= 1 && m <= TN) fb[1][m - 1] = load_b1(cur, 1, m - 1);
+        if (m > TN && m <= NF) fa[1][m - TN - 1] = load_a1(cur, 1, m - TN - 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // k-tile kt+1 has landed (issued one k-tile ago); every wave is done reading k-tile kt
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __syncthreads();
+      // ---- second half: k-step 1 from registers; the slots issue the DMA of k-tile kt+2 into the
+      // retired stage and fetch k-step 0 of k-tile kt+1; the first MFMA goes out right behind the barrier
 #pragma unroll
-    for (int m = 0; m < NM; m++) {
-      const int i = m / TN, j = m % TN;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], i < ASB ? fas[i] : fad[1][i < ASB ? 0 : i - ASB], acc[i][j], 0, 0, 0);
-      int q = -1, f = -1;  // DMA instruction / double-buffered fragment of this slot
-      if (ASB > 0) {
-        // every third slot from 0: DMA (measured on the 7B step: issued on even slots from 2 the
-        // step is 1.2 % slower, every 4th slot 0.6 %: the memory path likes an even request stream,
-        // but the last DMA still needs most of a k-tile to land); slots 1, 5, 9, ...: B then
-        // double-buffered A fragments
-        if (m % 3 == 0 && m / 3 < NINS) q = m / 3;
-        if ((m & 3) == 1 && (m >> 2) < TN + ND) f = m >> 2;
-      } else {
+      for (int m = 0; m < NM; m++) {
+        const int i = m / TN, j = m % TN;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], fa[1][i], acc[i][j], 0, 0, 0);
+        int q = -1, f = -1;  // DMA instruction / fragment of this slot
         // DMA issues and fragment reads alternate while both last, from slot 1 when they fit
         constexpr int FIRST = (NINS + NF <= NM - 1) ? 1 : 0;
         constexpr int BOTH = NINS < NF ? NINS : NF;
         const int k = m - FIRST;
         if (k >= 0 && k < 2 * BOTH) { if (k & 1) f = k >> 1; else q = k >> 1; }
         else if (k >= 2 * BOTH && k < NINS + NF) { if (NINS > NF) q = k - BOTH; else f = k - BOTH; }
+        if (q >= 0) {
+          if (q < A_INS) dma_a(ap, cur, q);
+          else dma_b(bp, cur, q - A_INS);
+        }
+        if (f >= 0) {
+          if (f < TN) fb[0][f] = load_b1(nxt, 0, f);
+          else fa[0][f - TN] = load_a1(nxt, 0, f - TN);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (q >= 0) {
-        if (q < A_INS) dma16_s(ap + q * a_istep, a_off, da + (q * NW + wave) * 1024);
-        else dma16_s(bp + (q - A_INS) * b_istep, b_off, db + ((q - A_INS) * NW + wave) * 1024);
-      }
-      if (f >= 0) {
-        if (f < TN) fb[0][f] = load_b1(nxt, 0, f);
-        else fad[0][f - TN] = load_a1(nxt, 0, ASB + f - TN);
-      }
-      if (j == TN - 1 && i < ASB) fas[i] = load_a1(nxt, 0, i);
-      __builtin_amdgcn_sched_barrier(0);
     }
     if (kt + 3 < KT) {
       ap += a_step;
@@ -533,6 +591,7 @@ __device__ __forceinline__ void gemm_tile(
     }
   }
   if (KT & 1) k_tile(KT - 1, std::integral_constant<int, 0>());
+  if (PINGPONG && wave < 4) __builtin_amdgcn_s_barrier();
   if (BLOCKS == 1) {
 #pragma unroll
     for (int i = 0; i < TM; i++)
