@@ -82,7 +82,8 @@ std::mutex g_prof_mu;
 //
 // EPI == 6 is one part of a reduction that several workgroups share (see olmax_gemm_padded): blockIdx.y
 // takes k in [y * seq_len, (y + 1) * seq_len), the last one the rest, and the accumulators leave as they
-// are, 1 KB per instruction, to Cv[part][tile][wave][i][j][lane] for gemm_split_sum_kernel.
+// are, 1 KB per instruction, to Cv[part][tile][wave][i][j][lane] for gemm_split_sum_kernel.  With `sums` (both gradients in one launch) the
+// operands are already those of a part, and its accumulators go there.
 //
 // RAG: 1 where M or N, 2 where K is not a multiple of the tile.  The last tile of a row or column is
 // moved back so that it ends with the matrix (the loop then reads nothing outside it and is the same
@@ -100,7 +101,8 @@ __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
     const bf16* __restrict__ R, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     int64_t ldr, int tiles_m, int tiles_n, int c_vec, const float* __restrict__ cos_t,
-    const float* __restrict__ sin_t, int seq_len, int rope_cols, int order, int pid, const int nwg, unsigned char* smem, int block = 0, float* park = nullptr) {
+    const float* __restrict__ sin_t, int seq_len, int rope_cols, int order, int pid, const int nwg, unsigned char* smem, int block = 0, float* park = nullptr,
+    float* sums = nullptr) {
   constexpr int GLU = (EPI == 1 || EPI == 2) ? EPI : (EPI == 4 ? 1 : (EPI == 5 ? 2 : 0));
   constexpr bool GLU_BWD = EPI == 4 || EPI == 5;
   constexpr bool ROPE = EPI == 3;
@@ -617,8 +619,9 @@ __device__ __forceinline__ void gemm_tile(
   asm volatile("" : "+v"(lane_e));
   const int l16e = lane_e & 15, g16e = lane_e >> 4;
 
-  if (SPLIT) {
-    float* part = reinterpret_cast<float*>(Cv) + ((((int64_t)blockIdx.y * tiles_m + tile_m) * tiles_n + tile_n) * NW + wave) * (NM * 256);
+  if (SPLIT || sums) {
+    float* part = SPLIT ? reinterpret_cast<float*>(Cv) + (int64_t)blockIdx.y * tiles_m * tiles_n * (NW * NM * 256) : sums;
+    part += (((int64_t)tile_m * tiles_n + tile_n) * NW + wave) * (NM * 256);
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -868,8 +871,9 @@ struct PairSide {
   bf16* C;
   int M, N, K;
   int64_t lda, ldb, ldc, ldr;
-  int tiles_m, tiles_n, order, nwg, block;
-  float* park;
+  int tiles_m, tiles_n, order, nwg, block;  // nwg: of one part
+  int parts = 1, chunk;                     // parts of dW's reduction in 256 tiles, k of all but the last
+  float* park;                              // parked blocks, or the sums of the parts
 };
 template <int T, int W, int RAGX, int RAGW, int BLOCKS>
 __global__ __launch_bounds__((T / W) * (T / 64) * 64) __attribute__((amdgpu_num_vgpr(120))) void gemm_pair_kernel(const PairSide x, const PairSide w, int x_first, int n_first) {
@@ -879,11 +883,14 @@ __global__ __launch_bounds__((T / W) * (T / 64) * 64) __attribute__((amdgpu_num_
   if (second != (x_first != 0)) {
     if (pid >= x.nwg) return;
     gemm_tile<T, T, W, 64, true, false, true, false, 0, RAGX, BLOCKS>(x.A, x.B, x.C, x.R, x.M, x.N, x.K, x.lda, x.ldb, x.ldc, x.ldr, x.tiles_m, x.tiles_n, 1,
-                                                              nullptr, nullptr, 1, 0, x.order, pid, x.nwg, smem, x.block, x.park);
+                                                                      nullptr, nullptr, 1, 0, x.order, pid, x.nwg, smem, x.block, x.park);
   } else {
-    if (pid >= w.nwg) return;
-    gemm_tile<T, T, W, 64, false, false, false, false, 0, RAGW, BLOCKS & 1>(w.A, w.B, w.C, nullptr, w.M, w.N, w.K, w.lda, w.ldb, w.ldc, 0, w.tiles_m, w.tiles_n, 1,
-                                                                nullptr, nullptr, 1, 0, w.order, pid, w.nwg, smem, w.block);
+    if (pid >= w.nwg * w.parts) return;
+    const int part = T == 256 ? pid / w.nwg : 0, k = part * w.chunk;
+    float* sums = T == 256 && w.parts > 1 ? w.park + (int64_t)part * w.tiles_m * w.tiles_n * 65536 : nullptr;
+    gemm_tile<T, T, W, 64, false, false, false, false, 0, RAGW, BLOCKS>(w.A + k * w.lda, w.B + k * w.ldb, w.C, nullptr, w.M, w.N, part + 1 < w.parts ? w.chunk : w.K - k,
+                                                                        w.lda, w.ldb, w.ldc, 0, w.tiles_m, w.tiles_n, 1, nullptr, nullptr, 1, 0, w.order,
+                                                                        pid - part * w.nwg, w.nwg, smem, w.block, w.park, sums);
   }
 }
 
@@ -992,11 +999,12 @@ void launch_pair(hipStream_t s, PairSide x, PairSide w) {
   for (auto p : {&x, &w}) {
     p->tiles_m = (p->M + T - 1) / T;
     p->tiles_n = (p->N + T - 1) / T;
-    p->order = tile_order(p->tiles_m, p->tiles_n, p == &x, false, p->N, p->K);
+    p->order = p->parts > 1 ? 0 : tile_order(p->tiles_m, p->tiles_n, p == &x, false, p->N, p->K);
     p->nwg = (int)order_grid(p->order, p->tiles_m, p->tiles_n);
   }
-  const int x_first = x.K > w.K, n_first = ((x_first ? x.nwg : w.nwg) + 7) & ~7;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(n_first + (x_first ? w.nwg : x.nwg))), dim3((T / W) * (T / 64) * 64), SMEM, s, x, w, x_first, n_first);
+  const bool x_first = x.K > (w.parts > 1 ? w.chunk : w.K);
+  const int nx = x.nwg, nw = w.nwg * w.parts, n_first = ((x_first ? nx : nw) + 7) & ~7;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_first + (x_first ? nw : nx))), dim3((T / W) * (T / 64) * 64), SMEM, s, x, w, (int)x_first, n_first);
 }
 
 template <bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32>
@@ -1063,6 +1071,13 @@ __global__ __launch_bounds__(256) void gemm_split_sum_kernel(const float* __rest
   }
 }
 
+void launch_split_sum(hipStream_t s, const float* sums, int parts, void* C, const bf16* R, int M, int N, int64_t ldc, int64_t ldr, bool a_kc, bool out_f32) {
+  const int tm = (M + 255) / 256, tn = (N + 255) / 256;
+  const int vec = N % 4 == 0 && ldc % 4 == 0 && !((uintptr_t)C & (out_f32 ? 15 : 7)) && (!R || (ldr % 4 == 0 && !((uintptr_t)R & 7)));
+  hipLaunchKernelGGL(gemm_split_sum_kernel, dim3((unsigned)(tm * tn * 16)), dim3(256), 0, s, sums, parts, C, R, M, N, ldc, ldr, a_kc ? M : (M + 7) & ~7, tn,
+                     tm * tn, (int)out_f32, vec);
+}
+
 template <bool A_KC, bool B_KC>
 int launch_split(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N, int K, int64_t lda, int64_t ldb,
                  int64_t ldc, int64_t ldr, bool out_f32, int parts, float* scratch) {
@@ -1087,10 +1102,7 @@ int launch_split(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf1
   // (run order: a round of windows is 256 tiles, and here there are fewer)
   hipLaunchKernelGGL(kern, dim3(tm * tn, parts), dim3(512), SMEM, s, A, B, (void*)scratch, (const bf16*)nullptr, M, N, K, lda,
                      ldb, (int64_t)0, (int64_t)0, tm, tn, 1, (const float*)nullptr, (const float*)nullptr, chunk * BK, 0, 0);
-  const uintptr_t mask = out_f32 ? 15 : 7;
-  const int vec = N % 4 == 0 && ldc % 4 == 0 && !((uintptr_t)C & mask) && (!R || (ldr % 4 == 0 && !((uintptr_t)R & 7)));
-  hipLaunchKernelGGL(gemm_split_sum_kernel, dim3((unsigned)(tm * tn * 16)), dim3(256), 0, s, (const float*)scratch, parts, C, R, M, N, ldc,
-                     ldr, A_KC ? M : (M + 7) & ~7, tn, tm * tn, (int)out_f32, vec);
+  launch_split_sum(s, scratch, parts, C, R, M, N, ldc, ldr, A_KC, out_f32);
   if (g_prof_on) {
     (void)hipEventRecord(rec.e1, s);
     rec.flops = 2.0 * M * N * K;
@@ -1482,6 +1494,31 @@ static float pair_256(Work l, Work s) {
   return t / 0.97f;
 }
 
+// Both products in 256 tiles.  The few tiles of a narrow layer's dW have long chains, which the calls share among workgroups: here dW's reduction comes in
+// `parts` (workgroups of their own, the sums added by a second kernel), or is whole and parks the sums of its blocks.  What costs the least among
+// those whose chains are as short as the calls' and whose sums fit.  us in a training step, the better of two calls and 128 tiles -> so: 8192 x 1024 x 5632 195 ->
+// 172 (parked), 8192 x 1024 x 3072 115 -> 104, 8192 x 2816 x 1024 117 -> 109 (five parts), 8192 x 1024 x 1024 61 -> 45 (eight).  dW of more tiles than CUs
+// fills the GPU by itself: parked, 8192 x 4096 x 22016 takes 2070 us, two calls 1930.  The 0.89: these forms beside the others, as measured there.
+struct PairPlan {
+  int parts = 1;
+  float cost = 1e30f;
+};
+static int64_t parked_of(Work v, int block) { return block >= v.kt ? 0 : ((v.kt + block - 1) / block - 1) * v.n; }  // of 256 KB
+static PairPlan plan_256(Work x, Work w, int whole_w, int chain_w, int block_x, int block_w, int64_t bytes) {
+  PairPlan best;
+  for (int p = 1; block_x && (p == 1 || (p <= 8 && w.n * p <= 256)); p++) {
+    const int chunk = (whole_w + p - 1) / p;  // every part has eight whole k-tiles or more (the last one a partial one too), and there are p of them
+    if (p == 1 ? !block_w || (block_w < w.kt && w.n > 256) : p * 8 > whole_w || (whole_w + chunk - 1) / chunk != p || chain_of_parts(p, chunk) > chain_w) continue;
+    const int64_t sums = p > 1 ? w.n * p : parked_of(w, block_w);
+    if ((sums + parked_of(x, block_x)) * 262144 > bytes) continue;
+    const Work part = {w.n * p, (w.kt + p - 1) / p};
+    float c = x.kt > part.kt ? pair_256(x, part) : pair_256(part, x);
+    if (sums) c = 0.89f * c + 0.1f * sums + (p > 1 ? 6.f : 0.f);
+    if (c < best.cost) best = {p, c};
+  }
+  return best;
+}
+
 int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x, bf16* dx, const bf16* r, void* dw, int T, int in, int out,
                      int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t ldr, int64_t lddw, bool dw_f32, bool dy_padded, GemmScratch scratch) {
   // what the kernels that take the operands need one after the other
@@ -1496,8 +1533,6 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
   const int chain_x = chain_of_product(T, in, out, true, false, direct_x, bytes), chain_w = chain_of_product(out, in, T, false, false, direct_w, bytes);
   const int ktx = (out + BK - 1) / BK, ktw = (T + BK - 1) / BK, block_x = block_of(ktx, chain_x), block_w = block_of(ktw, chain_w);
   const bool whole = block_x >= ktx && block_w >= ktw;
-  // what the blocks of dX take of the scratch memory in 256 tiles (dW has no registers left for the addresses)
-  const int64_t park = block_x ? ((ktx + block_x - 1) / block_x - 1) * tiles_of(T, in, 256) * 262144 : 0;
   int tile = 0;  // of the one launch, 0: two calls
   // (the one form of the small kernel that is built: whole chunks, 32-bit line offsets and at least a tile of rows)
   const bool small = !dw_f32 && out % 8 == 0 && in % 8 == 0 && T >= 64 && lddy < (1 << 25) && ldw < (1 << 25) && ldx < (1 << 25);
@@ -1506,12 +1541,14 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
   // vector stores, whole k-tiles in the first product
   const bool large = !dw_f32 && direct_x && direct_w && out % BK == 0 && lddx % 8 == 0 && lddw % 8 == 0 && (!r || (ldr % 8 == 0 && aligned16(r))) &&
                      aligned16(dx) && aligned16(dw);
-  for (int t = 128; t <= 256; t *= 2) {
-    if (!large || T < t || in < t || out < t || !block_x || !block_w) continue;
-    if (t == 256 && (park > bytes || block_w < ktw)) continue;
-    const Work wx = {tiles_of(T, in, t), ktx}, ww = {tiles_of(out, in, t), ktw};
-    const Work &l = wx.kt > ww.kt ? wx : ww, &sh = wx.kt > ww.kt ? ww : wx;
-    if (const float c = t == 128 ? pair_128(l, sh) : pair_256(l, sh); c < best) best = c, tile = t;
+  PairPlan plan;
+  if (large && T >= 128 && in >= 128 && out >= 128 && block_x && block_w) {
+    const Work wx = {tiles_of(T, in, 128), ktx}, ww = {tiles_of(out, in, 128), ktw};
+    if (const float c = wx.kt > ww.kt ? pair_128(wx, ww) : pair_128(ww, wx); c < best) best = c, tile = 128;
+  }
+  if (large && T >= 256 && in >= 256 && out >= 256) {
+    plan = plan_256({tiles_of(T, in, 256), ktx}, {tiles_of(out, in, 256), ktw}, T / BK, chain_w, block_x, block_w, bytes);
+    if (plan.cost < best) best = plan.cost, tile = 256;
   }
   // dW may take the place of W or of the residual, which the first product alone reads: not beside it
   auto meet = [](const void* p, int64_t n, const void* q, int64_t m) { return p && q && (uintptr_t)p < (uintptr_t)q + m && (uintptr_t)q < (uintptr_t)p + n; };
@@ -1524,13 +1561,17 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
       (void)hipEventCreate(&rec.e1);
       (void)hipEventRecord(rec.e0, s);
     }
+    if (tile != 256) plan.parts = 1;
     if (tile == 64) {
       olmax_gemm_small_pair(s, dy, w, x, dx, r, (bf16*)dw, T, in, out, lddy, ldw, ldx, lddx, ldr, lddw);
     } else {
       PairSide px = {dy, w, r, dx, T, in, out, lddy, ldw, lddx, ldr}, pw = {dy, x, nullptr, (bf16*)dw, out, in, T, lddy, ldx, lddw, 0};
       px.block = block_x;
-      pw.block = block_w;
+      pw.parts = plan.parts;  // (one in 128 tiles)
+      pw.chunk = (T / BK + pw.parts - 1) / pw.parts * BK;  // the last part takes what is left, at least a whole k-tile
+      pw.block = pw.parts > 1 ? ktw : block_w;
       px.park = (float*)scratch.p;
+      pw.park = px.park + parked_of({tiles_of(T, in, 256), ktx}, block_x) * 65536;
       const bool rx = T % tile || in % tile;
       const int rw = T % BK ? 2 : out % tile || in % tile;
 #define PAIR(E, W, B)                                                                                                           \
@@ -1540,9 +1581,10 @@ int olmax_gemm_grads(hipStream_t s, const bf16* dy, const bf16* w, const bf16* x
   } while (0)
       if (tile == 128 && !whole) PAIR(128, 64, 1);
       else if (tile == 128) PAIR(128, 64, 0);
-      else if (whole) PAIR(256, 128, 0);
+      else if (block_x >= ktx && pw.block >= ktw) PAIR(256, 128, 0);
       else PAIR(256, 128, 2);
 #undef PAIR
+      if (pw.parts > 1) launch_split_sum(s, pw.park, pw.parts, dw, nullptr, out, in, lddw, 0, false, false);
     }
     if (g_prof_on) {
       (void)hipEventRecord(rec.e1, s);

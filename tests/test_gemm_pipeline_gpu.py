@@ -21,3 +21,37 @@ def test_short_reductions_on_large_tiles_are_exact(M, N, al, bl):
             assert torch.equal(ops.gemm(a, b, a_layout=al, b_layout=bl, out_f32=True).double(), want)
     finally:
         _lib.load().olmax_gemm_set_tile(0)
+
+
+@pytest.mark.parametrize("seq", [8192, 7500])  # whole tiles; ragged rows and a partial k-tile at the end of dW's last part
+def test_a_narrow_layers_dw_shares_its_reduction_inside_the_one_launch(seq):
+    """Of a block of width 1024 the gate|up projection's dW parks its blocks and the q|k|v projection's comes in parts.  Against the two calls, which
+    a forced tile brings back: the products are rounded to bf16 (2^-9 each) and four of them follow one another."""
+    import dataclasses
+
+    from olmax_amd import TransformerRecipe, _lib
+    from olmax_amd.layer import TransformerBlock
+    from test_gemm_choice_gpu import recorded
+    print(f"[case] narrow block S{seq}", flush=True)
+    cfg = dataclasses.replace(TransformerRecipe.olmo2_7B(), num_layers=1, d_model=1024, hidden_size=2816, n_heads=8, n_kv_heads=8, head_dim=128)
+    block = TransformerBlock(cfg, batch_size=1, sequence_length=seq)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    for w in (block.wqkv, block.wo, block.wgu, block.wdown):
+        w.normal_(0.0, 0.02, generator=gen)
+    x, dy = (torch.empty(seq, 1024, device="cuda", dtype=torch.bfloat16).normal_(generator=gen) for _ in range(2))
+    block.forward(x)
+    dx = []
+    got = recorded(lambda: dx.append(block.backward(dy)))
+    for out in (3072, 5632):
+        assert any(key & 0xfff == (256 if out == 3072 or seq == 8192 else 128) and key >> 19 & 1 and (m, n, k) == (seq, 1024, out) for key, m, n, k, _ in got), got
+    res = [dx[0].clone()] + [v.clone() for v in block.grads.values()]
+    for v in block.grads.values():
+        v.zero_()
+    _lib.load().olmax_gemm_set_tile(256)
+    try:
+        got = recorded(lambda: dx.append(block.backward(dy)))
+    finally:
+        _lib.load().olmax_gemm_set_tile(0)
+    assert not any(key >> 19 & 1 for key, *_ in got), got
+    for a, b in zip(res, [dx[1]] + list(block.grads.values())):
+        assert ((a.double() - b.double()).norm() / b.double().norm()).item() < 2 ** -7
