@@ -15,8 +15,9 @@
 // prefetch of the next tile; 16-byte chunks are XOR-swizzled so that both ds_read_b128 and
 // the transposing reads are bank-conflict free.
 //
-// Backward is split in two deterministic kernels (no atomics): dK/dV with the key tile
-// stationary, dQ with the query tile stationary; each recomputes P from the saved LSE.
+// Backward is split in two deterministic halves (no atomics): dK/dV with the key tile
+// stationary, dQ with the query tile stationary; each recomputes P from the saved LSE.  They
+// are two kernels, or one launch where neither fills the GPU.
 #include "common.h"
 #include <algorithm>
 #include <mutex>
@@ -274,15 +275,15 @@ __device__ __forceinline__ void redo_dq(const bf16* q, const bf16* K, int64_t ld
   }
   if (lane >= lo && lane < hi) dq[lane] = f2bf(acc * scale);
 }
-// key j; Q, dO, lse, ndelta (minus delta) of the first of its rep query heads
+// key j; Q, dO, lse, ndelta (minus delta, nd_step to the next head's) of the first of its rep query heads
 template <bool CAP>
-__device__ __forceinline__ void redo_dkv(const bf16* Q, int64_t ldq, const bf16* dO, int64_t lddo, const float* lse, const float* ndelta,
+__device__ __forceinline__ void redo_dkv(const bf16* Q, int64_t ldq, const bf16* dO, int64_t lddo, const float* lse, const float* ndelta, int nd_step,
                                          const bf16* k, const bf16* v, bf16* dk, bf16* dv, int j, int S, int rep, int window, float scale,
                                          float cap, int lane, int lo, int hi) {
   const int last = window >= 0 ? min(S - 1, j + window) : S - 1;
   float ak = 0.f, av = 0.f;
 #pragma unroll 1
-  for (int r = 0; r < rep; r++, Q += 64, dO += 64, lse += S, ndelta += S)
+  for (int r = 0; r < rep; r++, Q += 64, dO += 64, lse += S, ndelta += nd_step)
 #pragma unroll 1
     for (int i0 = j; i0 <= last; i0 += 64) {
       const int n = min(64, last - i0 + 1);
@@ -561,184 +562,27 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_fwd_kernel(
 // dQ.  Same tiling and grid as the forward; K/V tiles stream through LDS.
 // ---------------------------------------------------------------------------------------
 template <int D, bool CAP, int QW, int KS>
+__device__ __forceinline__ void attn_dq(
+    const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
+    const bf16* __restrict__ O, const bf16* __restrict__ dO, const float* __restrict__ LSE,
+    float* __restrict__ DELTA, bf16* __restrict__ dQ, int S, int H, int KH, int64_t ldq, int64_t ldk,
+    int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, float scale, int window, float cap, unsigned id, unsigned nwg, unsigned char* smem) {
+#include "attn_dq.h"
+}
+
+template <int D, bool CAP, int QW, int KS>
 __global__ __launch_bounds__(QW * KS * 64, 2) void attn_bwd_dq_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     const bf16* __restrict__ O, const bf16* __restrict__ dO, const float* __restrict__ LSE,
     float* __restrict__ DELTA, bf16* __restrict__ dQ, int S, int H, int KH, int64_t ldq, int64_t ldk,
     int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, float scale, int window, float cap) {
-  constexpr int TILE = 64 * D * 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
-  const int l32 = lane & 31, lhi = lane >> 5;
-  const int qw = wave % QW, ks = wave / QW;
-  constexpr int QR = QW * 32;         // queries of the workgroup
-  constexpr int TEAMS = QW * KS / 4;  // tiles are fetched by teams of 4 waves
-  const int nqt = (S + QR - 1) / QR;
-  const WgCoord wg = decode_wg(blockIdx.x, (int)(gridDim.x / (nqt * (H / KH))), H / KH);
-  const int qt = nqt - 1 - wg.rank;  // longest rows first
-  const int b = wg.group / KH, kh = wg.group % KH;
-  const int h = kh * (H / KH) + wg.r;
-  const int i0 = qt * QR;
-  const int iw0 = i0 + qw * 32;
-  const int qi = iw0 + l32;
-  const int qic = min(qi, S - 1);
-
-  bf16x8 qf[D / 16], dof[D / 16];
-  // delta[b,h,i] = sum_d dO[i,h,d] * O[i,h,d]: the two lanes of a query each hold half of its dO
-  // row already, so the row sum costs one pass over O here; it is also written out for the dK/dV
-  // kernel, which runs after this one.
-  float dlt = 0.f;
-  {
-    const bf16* qp = Q + ((int64_t)b * S + qic) * ldq + h * D + lhi * 8;
-    const bf16* dp = dO + ((int64_t)b * S + qic) * lddo + h * D + lhi * 8;
-    const bf16* op = O + ((int64_t)b * S + qic) * ldo + h * D + lhi * 8;
-#pragma unroll
-    for (int s = 0; s < D / 16; s++) {
-      qf[s] = *reinterpret_cast<const bf16x8*>(qp + s * 16);
-      dof[s] = *reinterpret_cast<const bf16x8*>(dp + s * 16);
-      const bf16x8 of = *reinterpret_cast<const bf16x8*>(op + s * 16);
-#pragma unroll
-      for (int e = 0; e < 8; e++) dlt += bf2f(of[e]) * bf2f(dof[s][e]);
-    }
-  }
-  dlt = half_swap_sum(dlt);
-  // stored NEGATED: the dK/dV kernel starts its dP accumulators from it, so that dP - delta
-  // comes out of the MFMAs and costs that kernel no subtraction
-  if (lhi == 0 && ks == 0 && qi < S) DELTA[((int64_t)b * H + h) * S + qi] = -dlt;
-  const float lse2 = LSE[((int64_t)b * H + h) * S + qic] * LOG2E;
-  const int j_lo = window >= 0 ? max(0, i0 - window) : 0;
-  const int t_lo = j_lo >> 6;
-  const int t_hi = min(i0 + QR - 1, S - 1) >> 6;
-
-  f32x16 dq[D / 32];
-#pragma unroll
-  for (int dt = 0; dt < D / 32; dt++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) dq[dt][r] = 0.f;
-
-  const bf16* kbase = K + (int64_t)b * S * ldk + kh * D;
-  const bf16* vbase = V + (int64_t)b * S * ldv + kh * D;
-  const unsigned lds0 = lds_addr_of(smem);
-  const int wv = wave & 3, team = wave >> 2;
-  TileDma<64, D> dk, dv;
-  dk.init(ldk, wv, lane);
-  dv.init(ldv, wv, lane);
-  // K/V tiles of round r: tile t_lo + r KS + g for key group g
-  auto load_kv = [&](int round, int stage) {
-#pragma unroll
-    for (int g0 = 0; g0 < KS / TEAMS; g0++) {
-      const int g = g0 * TEAMS + team, t = t_lo + round * KS + g;
-      if (KS > 1 && t > t_hi) break;
-      const unsigned dst = lds0 + (g * 2 + stage) * (2 * TILE);
-      if (t * 64 + 64 <= S) {
-        dk.issue(kbase + (int64_t)t * 64 * ldk, dst, wv);
-        dv.issue(vbase + (int64_t)t * 64 * ldv, dst + TILE, wv);
-      } else {
-        dma_tile<64, D>(kbase, ldk, t * 64, S, dst, wv, lane);
-        dma_tile<64, D>(vbase, ldv, t * 64, S, dst + TILE, wv, lane);
-      }
-    }
-  };
-  const float sc2 = scale * LOG2E;
-  const float cap_c1 = CAP ? 2.f * sc2 / cap : 0.f, cap_l2 = cap * LOG2E;  // soft-cap: see cap_tanh
-
-  FragAddr<D, CAP && D == 128> fa;  // the soft-cap variant is the one short of registers
-  fa.init(lane);
-
-  load_kv(0, 0);
-  dma_wait_all();
-  __syncthreads();
-  const int rounds = (t_hi - t_lo + KS) / KS;
-  for (int r0 = 0; r0 < rounds; r0++) {
-    const int cur = r0 & 1;
-    if (r0 + 1 < rounds) load_kv(r0 + 1, cur ^ 1);
-    const int t = t_lo + r0 * KS + ks, j0 = t * 64;
-    const bool visible = (KS == 1 || t <= t_hi) && (j0 <= iw0 + 31) && (window < 0 || j0 + 63 >= iw0 - window);
-    if (visible) {
-      const unsigned char* sk = smem + (ks * 2 + cur) * (2 * TILE);
-      const unsigned char* sv = sk + TILE;
-      const bool need_mask = (j0 + 63 > iw0) || (window >= 0 && j0 < iw0 + 31 - window);
-      // dS of one 32-key half from its scores and dP, packed as the B operand of the dQ product
-      bf16x8 dsb[4];
-      auto finish_half = [&](int jt, f32x16& sj, const f32x16& dpj) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          float s = sj[r], chain = 1.f, p;
-          if (CAP) {
-            const float th = cap_tanh_of<D>(s, cap_c1, scale, cap);
-            p = fexp2(__builtin_fmaf(th, cap_l2, -lse2));
-            chain = 1.f - th * th;
-          } else {
-            p = fexp2(__builtin_fmaf(s, sc2, -lse2));
-          }
-          if (need_mask) {
-            const int j = j0 + jt * 32 + (r >> 2) * 8 + lhi * 4 + (r & 3);
-            const bool ok = (j <= qi) && (window < 0 || j >= qi - window);
-            p = ok ? p : 0.f;
-          }
-          sj[r] = p * (dpj[r] - dlt) * chain;
-        }
-        dsb[2 * jt] = pack_bf16x8(sj, 0);
-        dsb[2 * jt + 1] = pack_bf16x8(sj, 8);
-      };
-      f32x16 st[2], dpt[2];
-#pragma unroll
-      for (int jt = 0; jt < 2; jt++) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) { st[jt][r] = 0.f; dpt[jt][r] = 0.f; }
-#pragma unroll
-        for (int s = 0; s < D / 16; s++) {
-          st[jt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sk, jt * 32, s), qf[s], st[jt], 0, 0, 0);
-          dpt[jt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_kc(sv, jt * 32, s), dof[s], dpt[jt], 0, 0, 0);
-        }
-        // with the soft-cap's extra temporaries both halves do not fit the register file at once:
-        // finish each half before the next one's products start
-        if (CAP) finish_half(jt, st[jt], dpt[jt]);
-      }
-      if (!CAP) {
-#pragma unroll
-        for (int jt = 0; jt < 2; jt++) finish_half(jt, st[jt], dpt[jt]);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int dt = 0; dt < D / 32; dt++)
-          dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa.load_tr(sk, u * 16, dt), dsb[u], dq[dt], 0, 0, 0);
-    }
-    dma_wait_all();
-    __syncthreads();
-  }
-  float zeros = 0.f;  // see redo_rows
-  auto store4 = [&](int dt, int g, const f32x4& v) {
-    bf16* op = dQ + ((int64_t)b * S + qic) * lddq + h * D;
-    Pack4 pk;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float x = v[e] * scale;
-      if (D == 64) zeros = __builtin_fmaf(x, 0.f, zeros);
-      pk.e[e] = f2bf(x);
-    }
-    *reinterpret_cast<u32x2*>(op + dt * 32 + g * 8 + lhi * 4) = pk.u;
-  };
-  if constexpr (KS == 1) {
-    if (qi < S) {
-#pragma unroll
-      for (int dt = 0; dt < D / 32; dt++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) store4(dt, g, f32x4{dq[dt][g * 4], dq[dt][g * 4 + 1], dq[dt][g * 4 + 2], dq[dt][g * 4 + 3]});
-    }
+  const unsigned id = blockIdx.x, nwg = gridDim.x;
+  if constexpr (CAP && D == 128) {
+    attn_dq<D, CAP, QW, KS>(Q, K, V, O, dO, LSE, DELTA, dQ, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, cap, id, nwg, smem);
   } else {
-    add_partials<D, KS>(smem, dq, qw, ks, lane, [&](int u, const f32x4& v) {
-      if (qi < S) store4(u >> 2, u & 3, v);
-    });
+#include "attn_dq.h"
   }
-  if constexpr (D == 64)
-    redo_rows(zeros, [&](int r) {
-      const int64_t at = (int64_t)b * S + iw0 + r;
-      redo_dq<CAP>(Q + at * ldq + h * D, kbase, ldk, vbase, ldv, O + at * ldo + h * D, dO + at * lddo + h * D, LSE[((int64_t)b * H + h) * S + iw0 + r],
-                   dQ + at * lddq + h * D, iw0 + r, window, scale, cap, lane, ks * (D / KS), (ks + 1) * (D / KS));
-    });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -750,13 +594,40 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_bwd_dq_kernel(
 // KW = 2, QS = 4: one workgroup of eight waves per CU, half the keys and a quarter of the serial chain; the
 // four partial sums are added through LDS in group order.  See dkv_split.
 // ---------------------------------------------------------------------------------------
-template <int D, bool CAP, int KW, int QS>
+// dK/dV's LDS: stages and V tile, or the parked partial sums
+constexpr int smem_kv(int D, int KW, int QS) {
+  const int run = QS * 2 * (2 * 32 * D * 2 + 256) + KW * 32 * D * 2, sums = QS > 1 ? KW * QS * 32 * D * 4 : 0;
+  return run > sums ? run : sums;
+}
+// waves of the split forward and dQ kernels: what 160 KB of stages hold
+template <int D> constexpr int SPLIT_QW = D == 128 ? 4 : 2;
+template <int D> constexpr int SPLIT_KS = D == 128 ? 2 : 4;
+
+// BOTH: dQ in the same launch.  dK/dV's workgroups come first, longest first, then dQ's, longest first, so that the long ones of the second kind start where
+// the short ones of the first end.  Takes calls whose workgroups nearly all find room at once, where each kernel by itself waits for its longest chains (both_form).
+// Nobody hands delta over then: the workgroup forms that of all query rows it will meet itself, as dQ does, behind the rest of its LDS.
+template <int D, bool CAP, int KW, int QS, bool BOTH = false>
 __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V,
     const bf16* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ DELTA,
     bf16* __restrict__ dK, bf16* __restrict__ dV, int S, int H, int KH, int64_t ldq, int64_t ldk,
-    int64_t ldv, int64_t lddo, int64_t lddk, int64_t lddv, float scale, int window, float cap) {
+    int64_t ldv, int64_t lddo, int64_t lddk, int64_t lddv, float scale, int window, float cap,
+    const bf16* __restrict__ O, bf16* __restrict__ dQ, int64_t ldo, int64_t lddq, int nkv) {  // (BOTH)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  if constexpr (BOTH) {
+    if ((int)blockIdx.x >= nkv) {
+      constexpr int QW = QS > 1 ? SPLIT_QW<D> : 4, KS = QS > 1 ? SPLIT_KS<D> : 1;
+      const unsigned id = blockIdx.x - nkv, nwg = gridDim.x - nkv;
+      float* const DELTA = nullptr;
+      if constexpr (CAP && D == 128) {
+        attn_dq<D, CAP, QW, KS>(Q, K, V, O, dO, LSE, DELTA, dQ, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, cap, id, nwg, smem);
+      } else {
+#include "attn_dq.h"
+      }
+      return;
+    }
+  }
+  const unsigned nwg = BOTH ? nkv : gridDim.x;
   constexpr int QT = 32;                   // query rows per iteration
   constexpr int TILE = QT * D * 2;
   constexpr int STAGE = 2 * TILE + 256;  // Q | dO | lse, delta
@@ -767,7 +638,7 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
   const int l32 = lane & 31, lhi = lane >> 5;
   const int kw = wave % KW, qs = wave / KW;
   // key tile 0 is seen by every query: rank order is already longest first
-  const WgCoord wg = decode_wg(blockIdx.x, (int)(gridDim.x / ((S + KT - 1) / KT)), 1);
+  const WgCoord wg = decode_wg(blockIdx.x, (int)(nwg / ((S + KT - 1) / KT)), 1);
   const int kt = wg.rank;
   const int b = wg.group / KH, kh = wg.group % KH;
   const int rep = H / KH;
@@ -840,7 +711,7 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
     }
     if (kw == 0 && (QS == 1 || round * QS + qs < total)) {
       const int ii = min(own.t * QT + l32, S - 1);
-      const float* src = lane < QT ? LSE : DELTA;
+      const float* src = BOTH || lane < QT ? LSE : DELTA;
       sreg = src[((int64_t)b * H + own.h) * S + ii];  // consumed by store_stats a whole iteration later
     }
   };
@@ -850,11 +721,29 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
     if (kw == 0) reinterpret_cast<float*>(smem + (qs * 2 + stage) * STAGE + 2 * TILE)[lane] = lane < QT ? sreg * LOG2E : sreg;
   };
 
-  FragAddr<D> fa;
+  FragAddr<D, BOTH && CAP && D == 128> fa;  // (short of registers)
   fa.init(lane);
   const unsigned char* svt = smem + QS * 2 * STAGE;  // [KT keys][D] V tile
   if (team == 0) dma_tile<KT, D>(V + (int64_t)b * S * ldv + kh * D, ldv, j0, S, lds0 + QS * 2 * STAGE, wv, lane);
   load_tile(0, 0);
+  float* const own_delta = reinterpret_cast<float*>(smem + smem_kv(D, KW, QS));  // [head of the group][rows from t_lo QT]
+  if constexpr (BOTH) {
+    for (int u = wave; u < total; u += KW * QS) {
+      const int hq = u / ntile;
+      const int64_t row = (int64_t)b * S + min((t_lo + u - hq * ntile) * QT + l32, S - 1);
+      const bf16* op = O + row * ldo + (kh * rep + hq) * D + lhi * 8;
+      const bf16* dp = dO + row * lddo + (kh * rep + hq) * D + lhi * 8;
+      float dlt = 0.f;
+#pragma unroll
+      for (int s = 0; s < D / 16; s++) {
+        const bf16x8 of = *reinterpret_cast<const bf16x8*>(op + s * 16), df = *reinterpret_cast<const bf16x8*>(dp + s * 16);
+#pragma unroll
+        for (int e = 0; e < 8; e++) dlt += bf2f(of[e]) * bf2f(df[e]);
+      }
+      dlt = half_swap_sum(dlt);
+      if (lhi == 0) own_delta[u * QT + l32] = -dlt;
+    }
+  }
   store_stats(0);
   dma_wait_all();
   __syncthreads();
@@ -873,7 +762,7 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
       const unsigned char* sq = sgrp + CUR * STAGE;
       const unsigned char* so = sq + TILE;
       const float* slse = reinterpret_cast<const float*>(sq + 2 * TILE);
-      const float* sdel = slse + QT;
+      const float* sdel = BOTH ? own_delta + (round * QS + qs) * QT : slse + QT;
       // every (query, key) pair of the tile is visible unless the tile touches the diagonal, the
       // window edge or the end of the sequence
       const bool need_mask = (ib < jw0 + 31) || (ib + QT > S) || (window >= 0 && ib + QT - 1 > jw0 + window);
@@ -985,7 +874,8 @@ __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
   if constexpr (D == 64)
     redo_rows(zeros, [&](int r) {
       const int64_t seq = (int64_t)b * S, at = seq + jw0 + r, row = ((int64_t)b * H + kh * rep) * S;
-      redo_dkv<CAP>(Q + seq * ldq + kh * rep * D, ldq, dO + seq * lddo + kh * rep * D, lddo, LSE + row, DELTA + row, K + at * ldk + kh * D,
+      redo_dkv<CAP>(Q + seq * ldq + kh * rep * D, ldq, dO + seq * lddo + kh * rep * D, lddo, LSE + row, BOTH ? own_delta - t_lo * QT : DELTA + row,
+                    BOTH ? ntile * QT : S, K + at * ldk + kh * D,
                     V + at * ldv + kh * D, dK + at * lddk + kh * D, dV + at * lddv + kh * D, jw0 + r, S, rep, window, scale, cap, lane,
                     qs * (D / QS), (qs + 1) * (D / QS));
     });
@@ -1116,15 +1006,15 @@ bool bwd_fast_ok(const void* q, const void* k, const void* v, const void* o, con
 
 // forward, dQ: stages (the parked partial sums fit in their place), statistics of the forward's merge
 constexpr int smem_q(int D, int QW, int KS) { return KS * 2 * 2 * 64 * D * 2 + (KS > 1 ? QW * KS * 32 * 8 : 0); }
-// dK/dV: stages and V tile, or the parked partial sums
-constexpr int smem_kv(int D, int KW, int QS) {
-  const int run = QS * 2 * (2 * 32 * D * 2 + 256) + KW * 32 * D * 2, sums = QS > 1 ? KW * QS * 32 * D * 4 : 0;
-  return run > sums ? run : sums;
+// both in one launch; rows: query rows that the longest workgroup of dK/dV meets
+template <int D, int QW, int KS, int KW, int QS>
+constexpr int smem_both(int rows) {
+  const int q = smem_q(D, QW, KS), kv = smem_kv(D, KW, QS) + rows * 4;
+  return q > kv ? q : kv;
 }
 
-// waves of the split forward and dQ kernels: what 160 KB of stages hold
-template <int D> constexpr int SPLIT_QW = D == 128 ? 4 : 2;
-template <int D> constexpr int SPLIT_KS = D == 128 ? 2 : 4;
+// The most query rows that a workgroup of dK/dV meets where both run in one launch: their delta lies behind the 146 KB of its split form
+constexpr int BOTH_ROWS = 2112;
 
 // dynamic-LDS limits of the backward kernels, set once per process
 template <int D, bool CAP>
@@ -1135,6 +1025,8 @@ void bwd_fast_attributes_of() {
   (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, CAP, 2, 4>, ATTR, smem_kv(D, 2, 4));
   (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, CAP, 4, 1>, ATTR, smem_q(D, 4, 1));
   (void)hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, CAP, QW, KS>, ATTR, smem_q(D, QW, KS));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, CAP, 4, 1, true>, ATTR, smem_both<D, 4, 1, 4, 1>(BOTH_ROWS));
+  (void)hipFuncSetAttribute((const void*)attn_bwd_dkv_kernel<D, CAP, 2, 4, true>, ATTR, smem_both<D, QW, KS, 2, 4>(BOTH_ROWS));
 }
 void bwd_fast_attributes() {
   static std::once_flag once;
@@ -1192,6 +1084,40 @@ bool dkv_split(int B, int S, int H, int KH, int window) {
   return chain >= (n <= 256 ? base : base + (D == 128 ? 56 : 36) * (n - 256) / 256);
 }
 
+// Query rows (of all heads of a group) that a workgroup of dK/dV meets at most, in whole tiles of 32
+int both_rows(int S, int rep, int keys, int window) {
+  const int n = window >= 0 && window < S - keys ? window + keys : S;
+  return (int)std::min<int64_t>((int64_t)rep * ((n + 31) / 32 + 1) * 32, 1 << 30);
+}
+// Whether an output shares memory with an input: dK/dV may then leave only when dQ is done, and the other way round.
+bool meets_inputs(const bf16* const (&in)[5], const int64_t (&in_ld)[5], const int (&in_heads)[5], const bf16* const (&out)[3], const int64_t (&out_ld)[3],
+                  const int (&out_heads)[3], int64_t rows, int D) {
+  for (int i = 0; i < 5; i++)
+    for (int o = 0; o < 3; o++) {
+      const bf16 *ie = in[i] + (rows - 1) * in_ld[i] + in_heads[i] * D, *oe = out[o] + (rows - 1) * out_ld[o] + out_heads[o] * D;
+      if (in[i] < oe && out[o] < ie) return true;
+    }
+  return false;
+}
+// Whether dQ and dK/dV run in one launch: 2, both in their split forms (eight waves), 1, both in the plain ones (four waves), 0: two launches.
+// Each kernel by itself waits for its longest chains while the rest of the GPU idles, and a launch costs 2 us; but dK/dV has to form delta itself, about 1 us for
+// 256 query rows with eight waves.  us, two launches -> one (heads / K/V heads):
+// 2, by workgroups of both: 64 wide, 4 x 512 4/4 (256) 20.6 -> 14.9, 2 x 300 16/16 window 256 (320) 18.1 -> 14.2, 6 x 700 4/4 (528) 34 -> 25.7, 4 x 1024 4/4 (512) 31 -> 29.6;
+// 128 wide, 1 x 130 32/32 (160) 23.8 -> 14.8, 2 x 1024 8/8 (384) 57.5 -> 45.3, 1 x 2000 8/8 soft-cap (384) 114 -> 80, 1 x 1024 32/16 (512) 77 -> 70; 3 x 1000 8/8 (576)
+// 62.4 -> 64.3, 1 x 1000 32/32 (768) 70 -> 80, 8 x 1024 4/4 64 wide (1024) 44 -> 49; with equal chains (even_chains) 1 x 1024 16/16 window 256 (512) 19.6 -> 20.9.
+// Rows to form delta of: 1 x 256 32/8 (1152) 40.6 -> 39.1, 1 x 400 40/8 (2240) 63 -> 72, 64 wide 2 x 500 16/4 (2176) 39.6 -> 43.9, 1 x 3000 8/8 135 -> 149.
+// 1, by workgroups of 128 queries: 64 wide, 4 x 500 16/16 (256) 35 -> 30.6; 128 wide, 3 x 512 32/32 (384) 67 -> 57, 3 x 1000 16/16 (384) 108 -> 84, 8 x 1024 8/8 (512)
+// 112 -> 103, 5 x 1600 8/8 (520) 156 -> 137; 8 x 256 32/32 (512) 54 -> 59, 10 x 1024 8/8 (640) 120 -> 128, 1 x 2000 32/32 window 1024 (512) 129 -> 147, 2 x 1000 32/16 (512) 101 -> 136.
+template <int D>
+int both_form(int B, int S, int H, int KH, int window, bool split_q) {
+  const int rep = H / KH;
+  const bool even = even_chains(S, window);
+  const int64_t split = (int64_t)((S + 32 * SPLIT_QW<D> - 1) / (32 * SPLIT_QW<D>)) * H * B + (int64_t)((S + 63) / 64) * KH * B;
+  if (split <= (even ? 448 : 544) && both_rows(S, rep, 64, window) <= (rep <= 2 ? BOTH_ROWS : 1280)) return 2;
+  const int64_t n = (int64_t)((S + 127) / 128) * H * B;
+  return rep == 1 && !even && !split_q && n >= 256 && n <= (S >= 512 ? 528 : 448) && both_rows(S, 1, 128, window) <= BOTH_ROWS ? 1 : 0;
+}
+
 // The two MFMA kernels of the backward pass; delta: fp32 [B, H, S] scratch, fully
 // written by the dQ kernel (each workgroup computes the entries of its own queries) before the
 // dK/dV kernel, launched after it, reads them.
@@ -1203,15 +1129,25 @@ void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const b
   const float scale = 1.f / sqrtf((float)D);
   bwd_fast_attributes();
   const bool split_q = q_split<D>(B, S, H, window), split_kv = dkv_split<D>(B, S, H, KH, window);
+  const bool apart = meets_inputs({qp, kp, vp, op, gop}, {ldq, ldk, ldv, ldo, lddo}, {H, KH, KH, H, H}, {dq, dk, dv}, {lddq, lddk, lddv}, {H, KH, KH}, (int64_t)B * S, D);
+  const int both = apart ? 0 : both_form<D>(B, S, H, KH, window, split_q);
   auto go = [&](auto cap) {
     constexpr bool CAP = decltype(cap)::value;
+    auto one = [&](auto kern, int qr, int kr, int threads, int smem) {
+      const int nkv = (S + kr - 1) / kr * KH * B;
+      hipLaunchKernelGGL(kern, dim3((unsigned)(nkv + (S + qr - 1) / qr * H * B)), dim3(threads), smem, stream, qp, kp, vp, gop, lse, (const float*)nullptr, dk, dv, S, H, KH,
+                         ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap, op, dq, ldo, lddq, nkv);
+    };
+    constexpr int QW = SPLIT_QW<D>, KS = SPLIT_KS<D>;
+    if (both == 1) return one(attn_bwd_dkv_kernel<D, CAP, 4, 1, true>, 128, 128, 256, smem_both<D, 4, 1, 4, 1>(both_rows(S, H / KH, 128, window)));
+    if (both == 2) return one(attn_bwd_dkv_kernel<D, CAP, 2, 4, true>, QW * 32, 64, 512, smem_both<D, QW, KS, 2, 4>(both_rows(S, H / KH, 64, window)));
     auto qk = [&](auto kern, int qw, int ks) {
       hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * qw - 1) / (32 * qw)) * H * B)), dim3(qw * ks * 64), smem_q(D, qw, ks), stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
     };
     if (split_q) qk(attn_bwd_dq_kernel<D, CAP, SPLIT_QW<D>, SPLIT_KS<D>>, SPLIT_QW<D>, SPLIT_KS<D>);
     else qk(attn_bwd_dq_kernel<D, CAP, 4, 1>, 4, 1);
     auto kv = [&](auto kern, int kw, int nqs) {
-      hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * kw - 1) / (32 * kw)) * KH * B)), dim3(kw * nqs * 64), smem_kv(D, kw, nqs), stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap);
+      hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * kw - 1) / (32 * kw)) * KH * B)), dim3(kw * nqs * 64), smem_kv(D, kw, nqs), stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap, (const bf16*)nullptr, (bf16*)nullptr, (int64_t)0, (int64_t)0, 0);
     };
     if (split_kv) kv(attn_bwd_dkv_kernel<D, CAP, 2, 4>, 2, 4);
     else kv(attn_bwd_dkv_kernel<D, CAP, 4, 1>, 4, 1);
