@@ -386,8 +386,8 @@ int32_t olmax_block_bwd(olmax_stream_t stream, const olmax_model_config* cfg, co
  * are meant for tests, tuning and profiling runs, and are not for use while other threads are
  * inside the library or under graph capture.
  * ===================================================================================== */
-/* Force the MFMA tile variant of olmax_gemm_bf16 (0 = automatic, 128, 256).  While set, the
- * fused GLU / RoPE projections take their unfused paths (same results). */
+/* Force the MFMA tile variant of olmax_gemm_bf16 (0 = automatic, 128, 256; 384: 256 x 128, bf16 results of
+ * two reduction-contiguous operands).  While set, the fused GLU / RoPE projections take their unfused paths (same results). */
 void olmax_gemm_set_tile(int tile);
 /* Order in which the MFMA GEMM's workgroups take their tiles: 0 = automatic (per shape and operand
  * layout), -1 = one contiguous run of tiles per XCD, n > 0 = windows of 8 x 4 tiles per XCD whose 8
@@ -395,7 +395,7 @@ void olmax_gemm_set_tile(int tile);
 void olmax_gemm_set_order(int order);
 /* Record a HIP-event pair on the launch stream around every MFMA GEMM launch between begin and
  * end (allocates events).  end() waits for them and aggregates per kernel instantiation:
- * key = tile (64: 64 or 32, 128, 256) | a_kc<<12 | b_kc<<13 | has_res<<14 | out_f32<<15 | glu_epilogue<<16 |
+ * key = tile (64: 64 or 32, 128, 256, 384: 256 x 128) | a_kc<<12 | b_kc<<13 | has_res<<14 | out_f32<<15 | glu_epilogue<<16 |
  * rope_epilogue<<17 | shared_reduction<<18 | both_gradients<<19 (M, N, K: tokens, in, out; has_res: dX has one); ms = summed durations, flops / bytes = summed algorithmic work (2MNK;
  * operands and result moved once).  Returns the number of distinct keys written (at most cap). */
 void olmax_gemm_profile_begin(void);

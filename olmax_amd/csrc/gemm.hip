@@ -41,6 +41,7 @@
 namespace {
 
 constexpr int BK = 64;
+constexpr int THIN_TILE = 256 + 128;  // 256 rows x 128 columns
 typedef u32x4 __attribute__((aligned(2))) u32x4_u;  // 16 bytes at any element (ragged column edges)
 typedef f32x4 __attribute__((aligned(4))) f32x4_u;
 
@@ -116,9 +117,10 @@ __device__ __forceinline__ void gemm_tile(
   constexpr int B_INS = B_BYTES / 1024 / NW;
   static_assert(A_INS >= 1 && B_INS >= 1, "tile too small for the wave count");
   constexpr int NINS = A_INS + B_INS;
-  constexpr int STAGE = A_BYTES + B_BYTES;
+  constexpr bool THIN = BM == 256 && BN == 128;
+  constexpr int STAGES = THIN ? 3 : 2;  // of LDS
 
-  // LDS: [A stage 0 | A stage 1 | B stage 0 | B stage 1]
+  // LDS: [A stage 0 | A stage 1 | .. | B stage 0 | B stage 1 | ..]
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -254,7 +256,7 @@ __device__ __forceinline__ void gemm_tile(
   // issue DMA instructions [lo, hi) of the combined A+B list of k-tile kt into `stage`
   auto dma = [&](int kt, int stage, int lo, int hi) {
     const unsigned sa = lds_base + stage * A_BYTES;
-    const unsigned sb = lds_base + 2 * A_BYTES + stage * B_BYTES;
+    const unsigned sb = lds_base + STAGES * A_BYTES + stage * B_BYTES;
 #pragma unroll
     for (int i = 0; i < NINS; i++) {
       if (i < lo || i >= hi) continue;
@@ -295,7 +297,7 @@ __device__ __forceinline__ void gemm_tile(
   };
   auto tail_lds = [&](int i, int stage) -> unsigned {
     return i < A_INS ? lds_base + stage * A_BYTES + (i * NW + wave) * 1024
-                     : lds_base + 2 * A_BYTES + stage * B_BYTES + ((i - A_INS) * NW + wave) * 1024;
+                     : lds_base + STAGES * A_BYTES + stage * B_BYTES + ((i - A_INS) * NW + wave) * 1024;
   };
   auto dma_tail = [&](int stage) {
 #pragma unroll 1
@@ -334,7 +336,7 @@ __device__ __forceinline__ void gemm_tile(
   // lane, which it does: k-row = 32*kk + 8*(lane/16) + 4*h + lane%16/4.)
   constexpr int NA_BASE = A_KC ? 2 : TM, NB_BASE = B_KC ? 2 : TN;
   static_assert(A_BYTES + 36 * (BM > BN ? BM : BN) * 2 < 65536, "fragment immediates must fit 16 bits");
-  unsigned a_base[NA_BASE], b_base[NB_BASE];
+  unsigned a_base[NA_BASE], b_base[NB_BASE], a_base2[THIN ? NA_BASE : 1];  // (A's third stage is out of the immediates' reach)
 #pragma unroll
   for (int x = 0; x < NA_BASE; x++) {
     unsigned v;
@@ -349,6 +351,11 @@ __device__ __forceinline__ void gemm_tile(
     v += lds_base;
     asm volatile("" : "+v"(v));
     a_base[x] = v;
+    if (THIN) {
+      v += 2 * A_BYTES;
+      asm volatile("" : "+v"(v));
+      a_base2[THIN ? x : 0] = v;
+    }
   }
 #pragma unroll
   for (int x = 0; x < NB_BASE; x++) {
@@ -361,7 +368,7 @@ __device__ __forceinline__ void gemm_tile(
       const int kr = g16 * 8 + (l16 >> 2);
       v = kr * (BN * 2) + (((col >> 3) ^ tswz(kr)) << 4) + ((col & 7) << 1);
     }
-    v += lds_base + 2 * A_BYTES;
+    v += lds_base + STAGES * A_BYTES;
     asm volatile("" : "+v"(v));
     b_base[x] = v;
   }
@@ -375,13 +382,13 @@ __device__ __forceinline__ void gemm_tile(
   // one operand fragment (16 rows x 32 k) of k-step kk (0 or 1) of stage st (all compile-time)
   auto load_a1 = [&](int st, int kk, int i) -> bf16x8 {
     if (A_KC) {
-      return lds_b128(a_base[kk] + st * A_BYTES + i * 2048);
+      return lds_b128(THIN && st == 2 ? a_base2[THIN ? kk : 0] + i * 2048 : a_base[kk] + st * A_BYTES + i * 2048);
     } else {
       // transposing read: the 16-lane group g16 fetches k-rows kk*32 + 8*g16 + {0..3, 4..7}
       Pack8 p;
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        const u32x2 t = lds_tr64(a_base[i] + st * A_BYTES + (kk * 32 + h * 4) * (BM * 2));
+        const u32x2 t = lds_tr64((THIN && st == 2 ? a_base2[THIN ? i : 0] : a_base[i] + st * A_BYTES) + (kk * 32 + h * 4) * (BM * 2));
         p.u[h * 2 + 0] = t[0];
         p.u[h * 2 + 1] = t[1];
       }
@@ -423,6 +430,9 @@ __device__ __forceinline__ void gemm_tile(
   //   waits: every wave's LDS reads are complete before the barrier that ends its memory part, so no refill can overtake a read, and
   //     vmcnt(8) there leaves only what was issued behind the d0 / d1 that the next phase of this kind reads.
   //
+  // 256 x 128 tiles (THIN): as above, but a k-tile is one phase (64 registers of fragments, 32 MFMAs) and LDS has three stages, so that k-tile t + 2 is fetched
+  // into the stage of t - 1 while t is worked on.  They move 25 % less than four waves' 128 x 128 tiles, two of which share a CU (see thin_takes).
+  //
   // ---- main loop of the 128 x 128 tiles: software pipeline, all of it in registers and the two LDS stages:
   //   * fragments are double-buffered (fa/fb[0] = k-step 0, [1] = k-step 1 of a k-tile), and
   //     every LDS read is issued half a k-tile before the MFMAs that consume it;
@@ -433,7 +443,8 @@ __device__ __forceinline__ void gemm_tile(
   //   * the steady state has no branches: past the end the DMA re-fetches the last k-tile and
   //     the reads fetch a stage nobody uses any more.
   static_assert(PINGPONG || (2 * NINS <= NM && NF + 1 <= NM && NINS + NF <= NM), "not enough MFMA slots for the loads");
-  static_assert(!PINGPONG || (NW == 8 && TM == 8 && TN == 4 && A_INS == 4 && B_INS == 4), "phases are laid out for 8 waves of 128 x 64");
+  static_assert(!PINGPONG || THIN || (NW == 8 && TM == 8 && TN == 4 && A_INS == 4 && B_INS == 4), "phases are laid out for 8 waves of 128 x 64");
+  static_assert(!THIN || (NW == 8 && TM == 4 && TN == 4), "8 waves of 64 x 64");
   constexpr bool BY_K = !A_KC, B_WHOLE = A_KC || B_KC;  // PINGPONG: phases by k-step; all of B is read in phase 0
   constexpr int ND0 = B_WHOLE ? 6 : 4;                  // DMA instructions of d0
   bf16x8 fa[2][PINGPONG ? 4 : TM], fb[2][TN];
@@ -441,7 +452,7 @@ __device__ __forceinline__ void gemm_tile(
   const bf16 *ap1 = a_panel + (int64_t)min(1, KT - 1) * a_step, *bp1 = b_panel + (int64_t)min(1, KT - 1) * b_step;
   const bf16 *ap = a_panel + (int64_t)min(2, KT - 1) * a_step, *bp = b_panel + (int64_t)min(2, KT - 1) * b_step;
   auto dma_a = [&](const bf16* p, int stage, int i) { dma16_s(p + i * a_istep, a_off, lds_base + stage * A_BYTES + (i * NW + wave) * 1024); };
-  auto dma_b = [&](const bf16* p, int stage, int i) { dma16_s(p + i * b_istep, b_off, lds_base + 2 * A_BYTES + stage * B_BYTES + (i * NW + wave) * 1024); };
+  auto dma_b = [&](const bf16* p, int stage, int i) { dma16_s(p + i * b_istep, b_off, lds_base + STAGES * A_BYTES + stage * B_BYTES + (i * NW + wave) * 1024); };
   // (instruction i holds rows 64i .. 64i+63 of a k-contiguous tile: i even, the first half of the rows of waves 0-3 / 4-7; k-rows 16i .. 16i+15 of the others)
   auto d0 = [&](const bf16* pa, const bf16* pb, int stage) {
     dma_a(pa, stage, 0);
@@ -457,6 +468,12 @@ __device__ __forceinline__ void gemm_tile(
     dma_a(pa, stage, 3);
     if (!B_WHOLE) dma_b(pb, stage, 3);
   };
+  auto d_all = [&](const bf16* pa, const bf16* pb, int stage) {
+#pragma unroll
+    for (int i = 0; i < A_INS; i++) dma_a(pa, stage, i);
+#pragma unroll
+    for (int i = 0; i < B_INS; i++) dma_b(pb, stage, i);
+  };
   if (KRAG) dma_tail(0);
   else dma(0, 0, 0, NINS);
   if constexpr (PINGPONG) {
@@ -464,8 +481,9 @@ __device__ __forceinline__ void gemm_tile(
       dma_wait_all();
       zero_tail(0);
     }
-    d0(ap1, bp1, 1);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(ND0) : "memory");  // k-tile 0 has landed
+    if (THIN) d_all(ap1, bp1, 1);
+    else d0(ap1, bp1, 1);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(THIN ? NINS : ND0) : "memory");  // k-tile 0 has landed
     __builtin_amdgcn_s_barrier();
     if (wave >= 4) __builtin_amdgcn_s_barrier();  // one part behind (waves 0-3 make up for it after the loop)
   } else {
@@ -511,7 +529,25 @@ __device__ __forceinline__ void gemm_tile(
   auto k_tile = [&](int kt, auto cur_tag) {
     constexpr int cur = decltype(cur_tag)::value;
     constexpr int nxt = cur ^ 1;
-    if constexpr (PINGPONG) {
+    if constexpr (THIN) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 8; x++) fb[x >> 2][x & 3] = load_b1(cur, x >> 2, x & 3);
+#pragma unroll
+      for (int x = 0; x < 8; x++) fa[x >> 2][x & 3] = load_a1(cur, x >> 2, x & 3);
+      __builtin_amdgcn_sched_barrier(0);
+      d_all(ap, bp, (cur + 2) % 3);
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NINS) : "memory");  // k-tile kt+1 has landed
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 8; x++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[x & 3][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[x >> 2][j], fa[x >> 2][x & 3], acc[x & 3][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    } else if constexpr (PINGPONG) {
       phase(cur_tag, std::integral_constant<int, 0>());
       phase(cur_tag, std::integral_constant<int, 1>());
       ap1 = ap;
@@ -575,10 +611,12 @@ __device__ __forceinline__ void gemm_tile(
     asm volatile("" : "+v"(l));
     return l * 4;
   };
-  for (int kt = 0; kt + 1 < KT; kt += 2) {
+  int kt = 0;
+  for (; kt + STAGES <= KT; kt += STAGES) {
     k_tile(kt, std::integral_constant<int, 0>());
     k_tile(kt + 1, std::integral_constant<int, 1>());
-    if (BLOCKS && kt + 2 == ends && ends < KT) {
+    if constexpr (THIN) k_tile(kt + 2, std::integral_constant<int, 2>());
+    if (BLOCKS && kt + STAGES == ends && ends < KT) {
       ends += block;
       float* q = parking(parked++);
       const int at = hidden_lane();
@@ -592,7 +630,9 @@ __device__ __forceinline__ void gemm_tile(
         }
     }
   }
-  if (KT & 1) k_tile(KT - 1, std::integral_constant<int, 0>());
+  if (kt < KT) k_tile(kt, std::integral_constant<int, 0>());
+  if constexpr (THIN)
+    if (kt + 1 < KT) k_tile(kt + 1, std::integral_constant<int, 1>());
   if (PINGPONG && wave < 4) __builtin_amdgcn_s_barrier();
   if (BLOCKS == 1) {
 #pragma unroll
@@ -927,7 +967,7 @@ template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bo
 int launch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N,
                 int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr) {
   constexpr int NT = (BM / WM) * (BN / WN) * 64;
-  constexpr int SMEM = 2 * (BM + BN) * BK * 2;
+  constexpr int SMEM = (BM != BN ? 3 : 2) * (BM + BN) * BK * 2;
   auto kern = gemm_bf16_kernel<BM, BN, WM, WN, A_KC, B_KC, HAS_RES, OUT_F32, 0, RAG>;
   static std::once_flag attr_once;  // per instantiation
   std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM); });
@@ -947,7 +987,7 @@ int launch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16
     (void)hipEventRecord(rec.e1, s);
     rec.flops = 2.0 * M * N * K;
     rec.bytes = 2.0 * ((double)M * K + (double)N * K + (double)M * N * (HAS_RES ? 2 : 1) * (OUT_F32 ? 2 : 1));
-    rec.key = (BM == 256 ? 256 : 128) | (A_KC << 12) | (B_KC << 13) | (HAS_RES << 14) | (OUT_F32 << 15);
+    rec.key = (BM != BN ? BM + BN : BM) | (A_KC << 12) | (B_KC << 13) | (HAS_RES << 14) | (OUT_F32 << 15);
     rec.M = M; rec.N = N; rec.K = K;
     std::lock_guard<std::mutex> lk(g_prof_mu);
     g_prof.push_back(rec);
@@ -1010,6 +1050,13 @@ void launch_pair(hipStream_t s, PairSide x, PairSide w) {
 template <bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32>
 int dispatch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf16* R, int M, int N,
                   int K, int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, int tile) {
+  if constexpr (A_KC && B_KC && !OUT_F32) {
+    if (tile == THIN_TILE) {
+#define TILE(RAG) launch_tile<256, 128, 64, 64, A_KC, B_KC, HAS_RES, OUT_F32, RAG>(s, A, B, C, R, M, N, K, lda, ldb, ldc, ldr)
+      return K % BK ? TILE(2) : M % 256 || N % 128 ? TILE(1) : TILE(0);
+#undef TILE
+    }
+  }
   const bool rag = M % tile || N % tile;
 #define TILE(T, W, RAG) launch_tile<T, T, W, 64, A_KC, B_KC, HAS_RES, OUT_F32, RAG>(s, A, B, C, R, M, N, K, lda, ldb, ldc, ldr)
   if (tile == 256) return K % BK ? TILE(256, 128, 2) : rag ? TILE(256, 128, 1) : TILE(256, 128, 0);
@@ -1360,6 +1407,18 @@ static int block_of(int kt, int most) {
   }
 }
 
+// Whether a forward product that pick_tile gave to 128 tiles runs in 256 x 128 ones instead, while each of these has a CU of its own (the chains of additions are
+// the same).  Both are bound by operand delivery, 17 TB/s with 256 in flight.  us in a training step, 128 tiles -> so: 2048 x 4096 x 4096 70 -> 62,
+// 1500 x 4096 x 4096 70 -> 60, 8192 x 1024 x 2816 56 -> 51.5, 4096 x 1280 x 4096 129 -> 98 (beside the update); alone, with fewer tiles or short reductions: 512 x 4096
+// x 4096 39.0 -> 37.0 (64 tiles 29.7), 3000 x 1024 x 1024 14.0 -> 14.2.  (B stored [K, N]: 8 % at best; both operands so: up to 20 % slower, as the transposing
+// reads fill LDS.)
+static float cost_thin(int64_t n, int kt) { return (n <= 128 ? 0.52f : 0.52f + 0.24f * (n - 128) / 128.f) * kt + 8.f; }
+static bool thin_takes(int M, int N, int K, int tile, float cost) {
+  const int kt = (K + BK - 1) / BK;
+  const int64_t n = (int64_t)((M + 255) / 256) * ((N + 127) / 128);
+  return tile == 128 && M >= 256 && n >= 96 && n <= 256 && kt >= 32 && cost_thin(n, kt) < cost;
+}
+
 enum GluForm { GLU_SAVE, GLU_ONLY, GLU_BWD };
 static bool glu_fused_wins(int M, int F, int K, GluForm form) {
   const float e = (float)M * F;  // the elementwise passes move 6 (backward: 16) bytes an element at 5 TB/s
@@ -1378,6 +1437,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   float cost;
   if ((b_kc && !a_kc) || force_tile || !aligned16(scratch.p)) scratch = GemmScratch();  // (no caller has that layout)
   int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, scratch.bytes, &parts, &cost);
+  if (a_kc && b_kc && !out_f32 && !force_tile && thin_takes(M, N, K, tile, cost)) tile = THIN_TILE;
   if (parts > 1) {
     auto go = !a_kc ? launch_split<false, false> : b_kc ? launch_split<true, true> : launch_split<true, false>;
     return go(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts, (float*)scratch.p);
@@ -1385,6 +1445,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   if (force_tile && direct_ok && K >= BK) {  // whatever the rule chose, if the problem has a tile of that size
     if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
     if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;
+    if (force_tile == THIN_TILE && M >= 256 && N >= 128 && a_kc && b_kc && !out_f32) tile = THIN_TILE;
   }
   if (tile == 256 && !force_tile) {
     const Cut cut = find_cut((M + 255) / 256, (N + 255) / 256);

@@ -23,6 +23,33 @@ def test_short_reductions_on_large_tiles_are_exact(M, N, al, bl):
         _lib.load().olmax_gemm_set_tile(0)
 
 
+@pytest.mark.parametrize("M,N", [(256, 128), (300, 200), (520, 768)])
+def test_short_reductions_on_256_x_128_tiles_are_exact(M, N):
+    """Products of -1, 0 and 1: sums and residuals stay below 256, whole numbers that bf16 holds.  One k-tile to seven: the three stages twice over."""
+    from olmax_amd import _lib, ops
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    ints = lambda *s: torch.randint(-1, 2, s, device="cuda", generator=gen).bfloat16()  # noqa: E731
+    _lib.load().olmax_gemm_set_tile(384)
+    try:
+        for K in (64, 72, 128, 136, 192, 256, 264, 320, 384, 448):
+            print(f"[case] 256 x 128 tiles M{M} N{N} K{K}", flush=True)
+            a, b, r = ints(M, K), ints(N, K), ints(M, N)
+            want = a.double() @ b.t().double()
+            assert want.abs().max() < 255
+            assert torch.equal(ops.gemm(a, b).double(), want)
+            assert torch.equal(ops.gemm(a, b, residual=r).double(), want + r.double())
+    finally:
+        _lib.load().olmax_gemm_set_tile(0)
+
+
+def test_forward_products_of_few_128_tiles_take_256_x_128_ones():
+    from olmax_amd import ops
+    from test_gemm_choice_gpu import operands, recorded
+    a, b = operands(1500, 4096, 4096, 0, 0)
+    print("[case] 256 x 128 tiles chosen", flush=True)
+    assert [(key & 0xfff, m, n, k) for key, m, n, k, _ in recorded(lambda: ops.gemm(a, b))] == [(384, 1500, 4096, 4096)]
+
+
 @pytest.mark.parametrize("seq", [8192, 7500])  # whole tiles; ragged rows and a partial k-tile at the end of dW's last part
 def test_a_narrow_layers_dw_shares_its_reduction_inside_the_one_launch(seq):
     """Of a block of width 1024 the gate|up projection's dW parks its blocks and the q|k|v projection's comes in parts.  Against the two calls, which
