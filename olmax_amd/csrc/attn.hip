@@ -578,11 +578,7 @@ __global__ __launch_bounds__(QW * KS * 64, 2) void attn_bwd_dq_kernel(
     int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, float scale, int window, float cap) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const unsigned id = blockIdx.x, nwg = gridDim.x;
-  if constexpr (CAP && D == 128) {
-    attn_dq<D, CAP, QW, KS>(Q, K, V, O, dO, LSE, DELTA, dQ, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, cap, id, nwg, smem);
-  } else {
 #include "attn_dq.h"
-  }
 }
 
 // ---------------------------------------------------------------------------------------

@@ -1,6 +1,7 @@
-// Body of dQ, taken in by its kernel, by the one that runs it beside dK/dV and by the function of that name in attn.hip.  (Text where there is no soft-cap:
-// as an inlined function it takes four registers and 7 % more time, 2 x 4096, 32 heads 965 -> 1016 us a backward pass.  With the soft-cap at head_dim 128
-// the function takes 18 registers less, and the time falls by 1 to 2 %.)  Expects the kernel's arguments, smem, and the workgroup's id among nwg; DELTA may be null.
+// Body of dQ, taken in by its kernel, by the one that runs it beside dK/dV and by the function of that name in attn.hip.  (Text, because as an inlined function
+// it takes four registers and 7 % more time, 2 x 4096, 32 heads 965 -> 1016 us a backward pass.  With the soft-cap at head_dim 128 the function takes 18 registers
+// less, which the launch of both needs; by itself it is as fast, 2 x 4096, 32/16 heads 1144 -> 1128, 2 x 1777, 32/8 heads 267 -> 269.)
+// Expects the kernel's arguments, smem, and the workgroup's id among nwg; DELTA may be null.
   constexpr int TILE = 64 * D * 2;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler too
