@@ -999,7 +999,8 @@ extern "C" int32_t olmax_model_train_step(hipStream_t stream, hipStream_t opt_st
   if (hyper_dev) step = 1;
   g_overlapped_launches = 0;
   // Without recompute the optimizer would share the GPU with the backward GEMMs only (no
-  // forward GEMMs in between), which measured 4 % slower than running it afterwards.
+  // forward GEMMs in between), which gains next to nothing over running it afterwards (four
+  // layers of width 1024, 8192 tokens: 7.04 -> 6.99 ms; more workgroups or fewer lose).
   if (!opt_stream || opt_stream == stream || max_grad_norm > 0.f || !c->checkpoint) {
     RC(model_run(stream, c, windows, cos_tables, sin_tables, params_bf16, ids, labels, loss, grad_bf16, grad_f32, workspace,
                  workspace_bytes, true));
@@ -1018,9 +1019,8 @@ extern "C" int32_t olmax_model_train_step(hipStream_t stream, hipStream_t opt_st
   x.head_windows = c->n_layers;  // one recompute window per layer
   x.layer_numel = per_layer_params(c);
   // Pre-norm blocks open their backward with the d act GEMM (dY Wdown, hoisted in front of the
-  // recompute): its waves fill the register file, so an update running beside it would keep
-  // its workgroups off the CUs (measured: 1.9 ms instead of 0.5).  The update of the layer
-  // above therefore starts right behind that GEMM, beside the recompute's forward kernels.
+  // recompute).  The update of the layer above starts right behind it, beside the recompute's
+  // forward kernels: launched at once, two layers of the 7B step take 40.9 ms instead of 40.2.
   if (c->layer_type == 0) x.flush_point = POINT_AFTER_DACT;
   // the optimizer stream must not run ahead of work already queued on the main stream
   int rc = OLMAX_OK;
