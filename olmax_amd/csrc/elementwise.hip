@@ -394,37 +394,46 @@ __global__ __launch_bounds__(256) void adamw_used_rows_kernel(
 }
 
 // sum of squares of a gradient leaf, accumulated (fp32 atomics) into *out
-// (four or eight elements per load where the alignment allows it, two loads in flight: 155 M fp32 188 -> 157 us)
+// Bound by HBM at large sizes (4 TB/s), by what meets at one address at small ones: all workgroups end together and their atomics take 13 ns each.  So few and
+// large ones, 512 of sixteen waves at most, eight loads of a lane in flight over a contiguous span.  us, up to 2048 workgroups of four waves with two
+// loads -> so: fp32 in the cache 1 M 17.0 -> 7.0, 6.3 M 30.6 -> 9.7, 60 M 54 -> 37, from HBM 6.3 M 35 -> 15, 60 M 92 -> 89, 155 M 164 -> 162; bf16 6.3 M 30.2 -> 7.2.  A step
+// with clipping: 6.3 M parameters 690 -> 622, 155 M 6917 -> 6807.  (Non-temporal loads read 155 M in 97 us, but then the update that follows
+// writes back what they leave in the cache, 503 -> 546: nothing gained.)
 template <bool G_BF16>
-__global__ __launch_bounds__(256) void sumsq_kernel(const void* __restrict__ gv, int64_t n, int vec, float* __restrict__ out) {
-  constexpr int VEC = G_BF16 ? 8 : 4;
-  __shared__ float red[4];
-  float s0 = 0.f, s1 = 0.f;
-  auto load = [&](int64_t i) { return reinterpret_cast<const u32x4*>(gv)[i]; };
-  auto add = [&](const u32x4& q) {
-    Pack8 b;
-    b.u = q;
-    const f32x4 f = (const f32x4&)q;
-#pragma unroll
-    for (int e = 0; e < VEC; e++) {
-      const float g = G_BF16 ? bf2f(b.e[e]) : f[e & 3];
-      (e & 1 ? s1 : s0) += g * g;
-    }
+__global__ __launch_bounds__(1024) void sumsq_kernel(const void* __restrict__ gv, int64_t n, int64_t head, int width, float* __restrict__ out) {
+  constexpr int VEC = G_BF16 ? 8 : 4, U = 8;
+  __shared__ float red[16];
+  float s[U] = {};
+  auto element = [&](int64_t j) {
+    const float x = G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[j]) : reinterpret_cast<const float*>(gv)[j];
+    s[0] += x * x;
   };
-  const int64_t nv = vec ? n / VEC : 0, step = (int64_t)gridDim.x * 256;
-  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  for (; i + step < nv; i += 2 * step) {
-    const u32x4 a = load(i), b = load(i + step);
-    add(a);
-    add(b);
+  const u32x4* g = reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(gv) + head * (16 / VEC));
+  const int64_t nv = (n - head) / VEC;
+  for (int64_t b = blockIdx.x; b * 1024 * width < nv; b += gridDim.x) {
+    const int64_t i = b * 1024 * width + threadIdx.x;
+    u32x4 q[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      q[u] = u32x4{0, 0, 0, 0};
+      if (u < width && i + u * 1024 < nv) q[u] = g[i + u * 1024];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      Pack8 b8;
+      b8.u = q[u];
+      const f32x4 f = (const f32x4&)q[u];
+#pragma unroll
+      for (int e = 0; e < VEC; e++) {
+        const float x = G_BF16 ? bf2f(b8.e[e]) : f[e & 3];
+        s[u] += x * x;
+      }
+    }
   }
-  if (i < nv) add(load(i));
-  for (int64_t j = nv * VEC + (int64_t)blockIdx.x * 256 + threadIdx.x; j < n; j += step) {
-    const float g = G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[j]) : reinterpret_cast<const float*>(gv)[j];
-    s0 += g * g;
-  }
-  const float s = block_sum<4>(s0 + s1, red);
-  if (threadIdx.x == 0) atomicAdd(out, s);
+  for (int64_t j = (int64_t)blockIdx.x * 1024 + threadIdx.x; j < head; j += (int64_t)gridDim.x * 1024) element(j);
+  if (const int64_t at = head + nv * VEC + threadIdx.x; blockIdx.x == 0 && at < n) element(at);
+  const float t = block_sum<16>(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])), red);
+  if (threadIdx.x == 0) atomicAdd(out, t);
 }
 
 __global__ void cast_f32_bf16_kernel(const float* __restrict__ in, bf16* __restrict__ out, int64_t n) {
@@ -670,10 +679,13 @@ extern "C" int32_t olmax_adamw(hipStream_t stream, float* p, const void* g, floa
 extern "C" int32_t olmax_sumsq(hipStream_t stream, const void* g, int64_t n, int32_t is_bf16, float* out) {
   if (n == 0) return OLMAX_OK;
   OLMAX_CHECK(g && out && n >= 0, OLMAX_ERR_ARG, "olmax_sumsq: bad argument");
-  const int vec = aligned16(g);
-  const int grid = grid_1d(vec ? (n + 3) / 4 : n, 2048);
-  if (is_bf16) hipLaunchKernelGGL(sumsq_kernel<true>, dim3(grid), dim3(256), 0, stream, g, n, vec, out);
-  else hipLaunchKernelGGL(sumsq_kernel<false>, dim3(grid), dim3(256), 0, stream, g, n, vec, out);
+  const int size = is_bf16 ? 2 : 4;
+  // elements before the first aligned vector (all of them where they are not aligned to their size)
+  const int64_t head = (uintptr_t)g % size ? n : std::min<int64_t>(n, (-(uintptr_t)g & 15) / size), nv = n * size / 16;
+  const int width = (int)std::min<int64_t>(std::max<int64_t>(nv / (1024 * 64), 1), 8);  // loads of a lane: 64 workgroups before they grow
+  const dim3 grid((unsigned)std::min<int64_t>(std::max<int64_t>((nv + 1024 * width - 1) / (1024 * width), 1), 512));
+  if (is_bf16) hipLaunchKernelGGL(sumsq_kernel<true>, grid, dim3(1024), 0, stream, g, n, head, width, out);
+  else hipLaunchKernelGGL(sumsq_kernel<false>, grid, dim3(1024), 0, stream, g, n, head, width, out);
   OLMAX_LAUNCH_CHECK();
   return OLMAX_OK;
 }

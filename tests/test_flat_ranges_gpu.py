@@ -81,3 +81,18 @@ def test_sum_of_squares(n, shift, dtype):
     x = torch.randn(n + shift, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).to(dtype)[shift:]
     want = x.double().square().sum().item()
     assert abs(ops.sumsq(x).item() - want) < 2 ** -12 * want
+
+
+@pytest.mark.parametrize("n", [8, 1023, 8192, 65536 * 4 + 4, 65536 * 8 * 8 + 9, 512 * 65536 + 3, (128 << 20) + 40])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sum_of_squares_by_spans(n, shift, dtype):
+    """Ends of spans, of the elements before the first aligned vector and of the last one, one load of a lane to eight, several spans a workgroup, leaves beyond the
+    cache.  Whole numbers: exact below 2^24, whatever the order; above it no chain has more than 712 additions (8 lanes' loads of 25 spans, 512 workgroups), 2^-24 each."""
+    from olmax_amd import ops
+    print(f"[case] sumsq spans n{n} shift{shift} {dtype}", flush=True)
+    x = torch.randint(-3, 4, (n + shift,), device="cuda", generator=torch.Generator(device="cuda").manual_seed(2), dtype=torch.int8).to(dtype)[shift:]
+    x[0] = x[-1] = 64.0
+    want = sum(c.double().square().sum().item() for c in x.split(1 << 20))
+    got = ops.sumsq(x).item()
+    assert got == want if want < 2 ** 24 else abs(got - want) < 712 * 2 ** -24 * want
