@@ -403,6 +403,9 @@ int32_t olmax_gemm_profile_end(int32_t* keys, double* ms, double* flops, double*
                                int32_t cap);
 /* The same, aggregated per (key, M, N, K): mnk receives three ints per entry. */
 int32_t olmax_gemm_profile_end_shapes(int32_t* keys, int32_t* mnk, double* ms, int64_t* launches, int32_t cap);
+/* How olmax_attn_bwd runs on 16-byte aligned operands whose outputs share no memory with its inputs: bit 0 dQ, bit 1 dK/dV
+ * with a workgroup's chain split over its waves, bit 2 both in one launch; -1: neither (another head_dim).  Host only. */
+int32_t olmax_attn_bwd_form(int32_t B, int32_t S, int32_t H, int32_t KH, int32_t D, int32_t window);
 /* Profiler ranges: the counterpart of the reference's jax.named_scope annotations and
  * ProfilerCallback (src/olmax/train/callbacks/profiler.py:33-50).  on != 0: the whole-model entry
  * points emit roctx ranges ("olmax.layers.<l>.forward" / ".backward", "olmax.lm_head_and_loss")

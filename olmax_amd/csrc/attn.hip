@@ -600,7 +600,7 @@ template <int D> constexpr int SPLIT_QW = D == 128 ? 4 : 2;
 template <int D> constexpr int SPLIT_KS = D == 128 ? 2 : 4;
 
 // BOTH: dQ in the same launch.  dK/dV's workgroups come first, longest first, then dQ's, longest first, so that the long ones of the second kind start where
-// the short ones of the first end.  Takes calls whose workgroups nearly all find room at once, where each kernel by itself waits for its longest chains (both_form).
+// the short ones of the first end.  Takes calls whose workgroups nearly all find room at once, where each kernel by itself waits for its longest chains (bwd_form).
 // Nobody hands delta over then: the workgroup forms that of all query rows it will meet itself, as dQ does, behind the rest of its LDS.
 template <int D, bool CAP, int KW, int QS, bool BOTH = false>
 __global__ __launch_bounds__(KW * QS * 64, 2) void attn_bwd_dkv_kernel(
@@ -1095,28 +1095,48 @@ bool meets_inputs(const bf16* const (&in)[5], const int64_t (&in_ld)[5], const i
     }
   return false;
 }
-// Whether dQ and dK/dV run in one launch: 2, both in their split forms (eight waves), 1, both in the plain ones (four waves), 0: two launches.
+// How dQ and dK/dV run: each plain or split, in a launch of its own, or both in one, where both are split (eight waves) or both plain (four).
+struct BwdForm {
+  bool split_q, split_kv, one;
+};
 // Each kernel by itself waits for its longest chains while the rest of the GPU idles, and a launch costs 2 us; but dK/dV has to form delta itself, about 1 us for
 // 256 query rows with eight waves.  us, two launches -> one (heads / K/V heads):
-// 2, by workgroups of both: 64 wide, 4 x 512 4/4 (256) 20.6 -> 14.9, 2 x 300 16/16 window 256 (320) 18.1 -> 14.2, 6 x 700 4/4 (528) 34 -> 25.7, 4 x 1024 4/4 (512) 31 -> 29.6;
+// split, by workgroups of both: 64 wide, 4 x 512 4/4 (256) 20.6 -> 14.9, 2 x 300 16/16 window 256 (320) 18.1 -> 14.2, 6 x 700 4/4 (528) 34 -> 25.7, 4 x 1024 4/4 (512) 31 -> 29.6;
 // 128 wide, 1 x 130 32/32 (160) 23.8 -> 14.8, 2 x 1024 8/8 (384) 57.5 -> 45.3, 1 x 2000 8/8 soft-cap (384) 114 -> 80, 1 x 1024 32/16 (512) 77 -> 70; 3 x 1000 8/8 (576)
 // 62.4 -> 64.3, 1 x 1000 32/32 (768) 70 -> 80, 8 x 1024 4/4 64 wide (1024) 44 -> 49; with equal chains (even_chains) 1 x 1024 16/16 window 256 (512) 19.6 -> 20.9.
 // Rows to form delta of: 1 x 256 32/8 (1152) 40.6 -> 39.1, 1 x 400 40/8 (2240) 63 -> 72, 64 wide 2 x 500 16/4 (2176) 39.6 -> 43.9, 1 x 3000 8/8 135 -> 149.
-// 1, by workgroups of 128 queries: 64 wide, 4 x 500 16/16 (256) 35 -> 30.6; 128 wide, 3 x 512 32/32 (384) 67 -> 57, 3 x 1000 16/16 (384) 108 -> 84, 8 x 1024 8/8 (512)
+// Up to 256 workgroups each has a CU of its own.  Beyond, the rest comes in a second round (and a third), which only long chains are worth.  By 32-row tiles of one
+// query head's chain, 128 wide, one query head to a K/V head: 1 tile 4 x 30 48/48 (384) 13.9 -> 16.7, 11 x 31 24/24 (528) 16.9 -> 23.7; 2 tiles 8 x 55 24/24 (384) 17.6 -> 19.4;
+// 3 tiles 8 x 86 16/16 (384) 22.1 -> 19.3, 11 x 68 16/16 (528) 22.9 -> 24.7; 14 tiles 3 x 437 16/16 (528) 42.2 -> 37.9.  Two to one: 2 tiles 9 x 34 32/16 (432) 21.8 -> 18.6;
+// 4 tiles 8 x 113 32/16 (512) 27.5 -> 29.7; 10 tiles 3 x 312 32/16 (528) 40.3 -> 42.8; 16 tiles 2 x 492 32/16 soft-cap (512) 56.8 -> 53.9.  More: 1 tile
+// 8 x 28 40/8 (384) 19.8 -> 16.0; 2 tiles 9 x 54 40/8 (432) 25.5 -> 26.7; 4 tiles 10 x 127 32/8 soft-cap (480) 40.9 -> 42.3; 5 tiles 10 x 156 16/4 (440) 36.1 -> 33.4.  64 wide:
+// 1 tile 11 x 32 40/8 (528) 14.9 -> 17.3; 5 tiles 9 x 151 16/4 (540) 25.0 -> 20.6.  Equal chains: 2 x 1590 8/4 window 64 (408) 28.9 -> 31.9.
+// plain, by workgroups of 128 queries: 64 wide, 4 x 500 16/16 (256) 35 -> 30.6; 128 wide, 3 x 512 32/32 (384) 67 -> 57, 3 x 1000 16/16 (384) 108 -> 84, 8 x 1024 8/8 (512)
 // 112 -> 103, 5 x 1600 8/8 (520) 156 -> 137; 8 x 256 32/32 (512) 54 -> 59, 10 x 1024 8/8 (640) 120 -> 128, 1 x 2000 32/32 window 1024 (512) 129 -> 147, 2 x 1000 32/16 (512) 101 -> 136.
+// (Also where dK/dV by itself would be split, 64 wide 4 x 709 16/16 soft-cap 92 -> 64, 3 x 282 32/32 28.4 -> 21.6: one fp32 chain in the place of four added up.  What P, dS and the
+// results lose as bf16 hides that: the error of dK and dV against float64, 0.24 to 0.25 % over twenty such shapes, is 0.9995 to 1.0001 of the split form's.)
 template <int D>
-int both_form(int B, int S, int H, int KH, int window, bool split_q) {
+BwdForm bwd_form(int B, int S, int H, int KH, int window, bool apart) {
+  const BwdForm two = {q_split<D>(B, S, H, window), dkv_split<D>(B, S, H, KH, window), false};
+  if (apart) return two;
   const int rep = H / KH;
   const bool even = even_chains(S, window);
+  const int tiles = ((window >= 0 && window < S - 64 ? window + 64 : S) + 31) / 32;
+  int room = tiles < 5 ? 512 : 544;  // workgroups of both
+  if (D == 128 && rep == 1 && tiles < 3) room = 256;
+  if (D == 128 && rep == 2 && tiles < 16) room = tiles < 3 ? 480 : 400;
+  if (D == 128 && rep > 2 && tiles < 5) room = tiles < 3 ? 400 : 448;
+  if (even) room = std::min(room, D == 128 && rep == 2 ? 360 : 448);
   const int64_t split = (int64_t)((S + 32 * SPLIT_QW<D> - 1) / (32 * SPLIT_QW<D>)) * H * B + (int64_t)((S + 63) / 64) * KH * B;
-  if (split <= (even ? 448 : 544) && both_rows(S, rep, 64, window) <= (rep <= 2 ? BOTH_ROWS : 1280)) return 2;
+  if (split <= room && both_rows(S, rep, 64, window) <= (rep <= 2 ? BOTH_ROWS : 1280)) return {true, true, true};
   const int64_t n = (int64_t)((S + 127) / 128) * H * B;
-  return rep == 1 && !even && !split_q && n >= 256 && n <= (S >= 512 ? 528 : 448) && both_rows(S, 1, 128, window) <= BOTH_ROWS ? 1 : 0;
+  if (rep == 1 && !even && !two.split_q && n >= 256 && n <= (S >= 512 ? 528 : 448) && both_rows(S, 1, 128, window) <= BOTH_ROWS) return {false, false, true};
+  return two;
 }
 
 // The two MFMA kernels of the backward pass; delta: fp32 [B, H, S] scratch, fully
 // written by the dQ kernel (each workgroup computes the entries of its own queries) before the
-// dK/dV kernel, launched after it, reads them.
+// dK/dV kernel, launched after it, reads them (one launch of both leaves it as it is).
 template <int D>
 void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const bf16* vp, const bf16* op, const float* lse,
                      const bf16* gop, bf16* dq, bf16* dk, bf16* dv, float* delta, int B, int S, int H, int KH, int64_t ldq,
@@ -1124,9 +1144,8 @@ void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const b
                      float softcap) {
   const float scale = 1.f / sqrtf((float)D);
   bwd_fast_attributes();
-  const bool split_q = q_split<D>(B, S, H, window), split_kv = dkv_split<D>(B, S, H, KH, window);
   const bool apart = meets_inputs({qp, kp, vp, op, gop}, {ldq, ldk, ldv, ldo, lddo}, {H, KH, KH, H, H}, {dq, dk, dv}, {lddq, lddk, lddv}, {H, KH, KH}, (int64_t)B * S, D);
-  const int both = apart ? 0 : both_form<D>(B, S, H, KH, window, split_q);
+  const BwdForm form = bwd_form<D>(B, S, H, KH, window, apart);
   auto go = [&](auto cap) {
     constexpr bool CAP = decltype(cap)::value;
     auto one = [&](auto kern, int qr, int kr, int threads, int smem) {
@@ -1135,17 +1154,17 @@ void launch_bwd_fast(hipStream_t stream, const bf16* qp, const bf16* kp, const b
                          ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap, op, dq, ldo, lddq, nkv);
     };
     constexpr int QW = SPLIT_QW<D>, KS = SPLIT_KS<D>;
-    if (both == 1) return one(attn_bwd_dkv_kernel<D, CAP, 4, 1, true>, 128, 128, 256, smem_both<D, 4, 1, 4, 1>(both_rows(S, H / KH, 128, window)));
-    if (both == 2) return one(attn_bwd_dkv_kernel<D, CAP, 2, 4, true>, QW * 32, 64, 512, smem_both<D, QW, KS, 2, 4>(both_rows(S, H / KH, 64, window)));
+    if (form.one && !form.split_q) return one(attn_bwd_dkv_kernel<D, CAP, 4, 1, true>, 128, 128, 256, smem_both<D, 4, 1, 4, 1>(both_rows(S, H / KH, 128, window)));
+    if (form.one) return one(attn_bwd_dkv_kernel<D, CAP, 2, 4, true>, QW * 32, 64, 512, smem_both<D, QW, KS, 2, 4>(both_rows(S, H / KH, 64, window)));
     auto qk = [&](auto kern, int qw, int ks) {
       hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * qw - 1) / (32 * qw)) * H * B)), dim3(qw * ks * 64), smem_q(D, qw, ks), stream, qp, kp, vp, op, gop, lse, delta, dq, S, H, KH, ldq, ldk, ldv, ldo, lddo, lddq, scale, window, softcap);
     };
-    if (split_q) qk(attn_bwd_dq_kernel<D, CAP, SPLIT_QW<D>, SPLIT_KS<D>>, SPLIT_QW<D>, SPLIT_KS<D>);
+    if (form.split_q) qk(attn_bwd_dq_kernel<D, CAP, SPLIT_QW<D>, SPLIT_KS<D>>, SPLIT_QW<D>, SPLIT_KS<D>);
     else qk(attn_bwd_dq_kernel<D, CAP, 4, 1>, 4, 1);
     auto kv = [&](auto kern, int kw, int nqs) {
       hipLaunchKernelGGL(kern, dim3((unsigned)(((S + 32 * kw - 1) / (32 * kw)) * KH * B)), dim3(kw * nqs * 64), smem_kv(D, kw, nqs), stream, qp, kp, vp, gop, lse, delta, dk, dv, S, H, KH, ldq, ldk, ldv, lddo, lddk, lddv, scale, window, softcap, (const bf16*)nullptr, (bf16*)nullptr, (int64_t)0, (int64_t)0, 0);
     };
-    if (split_kv) kv(attn_bwd_dkv_kernel<D, CAP, 2, 4>, 2, 4);
+    if (form.split_kv) kv(attn_bwd_dkv_kernel<D, CAP, 2, 4>, 2, 4);
     else kv(attn_bwd_dkv_kernel<D, CAP, 4, 1>, 4, 1);
   };
   if (softcap > 0.f) go(std::true_type());
@@ -1216,6 +1235,13 @@ extern "C" int64_t olmax_attn_bwd_workspace_bytes(int32_t B, int32_t S, int32_t 
 // What the MFMA path alone needs (delta only): for callers that KNOW head_dim is 128 and every
 // operand is 16-byte aligned with row strides that are multiples of 8.
 extern "C" int64_t olmax_attn_bwd_workspace_bytes_aligned(int32_t B, int32_t S, int32_t H) { return attn_delta_bytes(B, S, H); }
+
+// Which kernels the backward takes for operands that need no others (aligned, outputs apart from inputs): see the header.
+extern "C" int32_t olmax_attn_bwd_form(int32_t B, int32_t S, int32_t H, int32_t KH, int32_t D, int32_t window) {
+  if (B <= 0 || S <= 0 || H <= 0 || KH <= 0 || H % KH || !(D == 128 || (D == 64 && S <= GENERIC_MAX_S_BWD))) return -1;
+  const BwdForm f = (D == 128 ? bwd_form<128> : bwd_form<64>)(B, S, H, KH, reach(window, S), false);
+  return (f.split_q ? 1 : 0) | (f.split_kv ? 2 : 0) | (f.one ? 4 : 0);
+}
 
 extern "C" int32_t olmax_attn_bwd(hipStream_t stream, const void* q, const void* k, const void* v,
                                   const void* o, const float* lse, const void* d_o, void* dq, void* dk,

@@ -21,8 +21,8 @@
 
   bf16x8 qf[D / 16], dof[D / 16];
   // delta[b,h,i] = sum_d dO[i,h,d] * O[i,h,d]: the two lanes of a query each hold half of its dO
-  // row already, so the row sum costs one pass over O here; it is also written out for the dK/dV
-  // kernel, which runs after this one.
+  // row already, so the row sum costs one pass over O here; it is also written out (DELTA) for a
+  // dK/dV kernel that runs after this one.  In one launch dK/dV forms its own and DELTA is null.
   float dlt = 0.f;
   {
     const bf16* qp = Q + ((int64_t)b * S + qic) * ldq + h * D + lhi * 8;
