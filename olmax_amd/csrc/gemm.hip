@@ -1053,7 +1053,7 @@ int dispatch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf
   if constexpr (A_KC && B_KC && !OUT_F32) {
     if (tile == THIN_TILE) {
 #define TILE(RAG) launch_tile<256, 128, 64, 64, A_KC, B_KC, HAS_RES, OUT_F32, RAG>(s, A, B, C, R, M, N, K, lda, ldb, ldc, ldr)
-      return K % BK ? TILE(2) : M % 256 || N % 128 ? TILE(1) : TILE(0);
+      return M % 256 || N % 128 ? TILE(1) : TILE(0);  // (whole k-tiles: see thin_takes)
 #undef TILE
     }
   }
@@ -1408,15 +1408,13 @@ static int block_of(int kt, int most) {
 }
 
 // Whether a forward product that pick_tile gave to 128 tiles runs in 256 x 128 ones instead, while each of these has a CU of its own (the chains of additions are
-// the same).  Both are bound by operand delivery, 17 TB/s with 256 in flight.  us in a training step, 128 tiles -> so: 2048 x 4096 x 4096 70 -> 62,
-// 1500 x 4096 x 4096 70 -> 60, 8192 x 1024 x 2816 56 -> 51.5, 4096 x 1280 x 4096 129 -> 98 (beside the update); alone, with fewer tiles or short reductions: 512 x 4096
-// x 4096 39.0 -> 37.0 (64 tiles 29.7), 3000 x 1024 x 1024 14.0 -> 14.2.  (B stored [K, N]: 8 % at best; both operands so: up to 20 % slower, as the transposing
-// reads fill LDS.)
-static float cost_thin(int64_t n, int kt) { return (n <= 128 ? 0.52f : 0.52f + 0.24f * (n - 128) / 128.f) * kt + 8.f; }
-static bool thin_takes(int M, int N, int K, int tile, float cost) {
-  const int kt = (K + BK - 1) / BK;
-  const int64_t n = (int64_t)((M + 255) / 256) * ((N + 127) / 128);
-  return tile == 128 && M >= 256 && n >= 96 && n <= 256 && kt >= 32 && cost_thin(n, kt) < cost;
+// the same).  Both are bound by operand delivery.  us, 128 tiles -> so, behind another product and with operands from HBM, with more than 288 tiles of 128 (two on
+// many CUs): 8192 x 1024 x 2816 59.5 -> 48.6, 1000 x 6144 x 4096 76 -> 58, 1500 x 4096 x 4096 64 -> 58, 4096 x 1280 x 4096 62 -> 59, 260 x 14336 x 4096 66 -> 61, 3000 x 2048 x
+// 9216 133 -> 128; with fewer, half of the CUs have nothing to do: 2048 x 2048 x 2816 43.6 -> 45.0, x 5120 6 % slower, 2048 x 2304 x 3072 3 %.  A partial k-tile costs what they
+// gain: 1500 x 4096 x 4104 84.5 -> 89.7, x 2056 47.9 -> 50.0.  Longer reductions gain or lose: x 11008 1000 x 6144 202 -> 157, 6000 x 1024 163 -> 169; 2500 x 2304 x 16384 225 -> 262;
+// of short ones 3000 x 1024 x 1024 14.0 -> 14.2.  (B stored [K, N]: 8 % at best; both operands so: up to 20 % slower, as the transposing reads fill LDS.)
+static bool thin_takes(int M, int N, int K, int tile) {
+  return tile == 128 && M >= 256 && K % BK == 0 && K >= 32 * BK && K <= 144 * BK && (int64_t)((M + 255) / 256) * ((N + 127) / 128) <= 256 && tiles_of(M, N, 128) > 288;
 }
 
 enum GluForm { GLU_SAVE, GLU_ONLY, GLU_BWD };
@@ -1437,7 +1435,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   float cost;
   if ((b_kc && !a_kc) || force_tile || !aligned16(scratch.p)) scratch = GemmScratch();  // (no caller has that layout)
   int tile = pick_tile(M, N, K, a_kc, b_kc, direct_ok, scratch.bytes, &parts, &cost);
-  if (a_kc && b_kc && !out_f32 && !force_tile && thin_takes(M, N, K, tile, cost)) tile = THIN_TILE;
+  if (a_kc && b_kc && !out_f32 && !force_tile && thin_takes(M, N, K, tile)) tile = THIN_TILE;
   if (parts > 1) {
     auto go = !a_kc ? launch_split<false, false> : b_kc ? launch_split<true, true> : launch_split<true, false>;
     return go(stream, a, b, C, r, M, N, K, lda, ldb, ldc, ldr, out_f32, parts, (float*)scratch.p);
@@ -1445,7 +1443,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   if (force_tile && direct_ok && K >= BK) {  // whatever the rule chose, if the problem has a tile of that size
     if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
     if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;
-    if (force_tile == THIN_TILE && M >= 256 && N >= 128 && a_kc && b_kc && !out_f32) tile = THIN_TILE;
+    if (force_tile == THIN_TILE && M >= 256 && N >= 128 && K % BK == 0 && a_kc && b_kc && !out_f32) tile = THIN_TILE;
   }
   if (tile == 256 && !force_tile) {
     const Cut cut = find_cut((M + 255) / 256, (N + 255) / 256);

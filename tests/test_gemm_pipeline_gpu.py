@@ -50,6 +50,21 @@ def test_forward_products_of_few_128_tiles_take_256_x_128_ones():
     assert [(key & 0xfff, m, n, k) for key, m, n, k, _ in recorded(lambda: ops.gemm(a, b))] == [(384, 1500, 4096, 4096)]
 
 
+@pytest.mark.parametrize("M,N,K,tile", [
+    (260, 14336, 4096, 384), (4096, 1280, 4096, 384), (8192, 1024, 2816, 384), (1000, 6144, 9216, 384),
+    (2048, 2048, 2816, 128), (2048, 2304, 3072, 128), (1500, 4096, 4104, 128), (6000, 1024, 11008, 128), (2500, 2304, 16384, 128), (2048, 4096, 1984, 128)])
+def test_256_x_128_tiles_take_what_they_are_faster_on(M, N, K, tile):
+    """Not with 288 tiles of 128 or fewer, part of a k-tile, very long or short reductions.  Against float64: 2^-9 for the rounding to bf16, as much again for the sums."""
+    from olmax_amd import ops
+    from test_gemm_choice_gpu import operands, recorded
+    a, b = operands(M, N, K, 0, 0)
+    print(f"[case] 256 x 128 or 128 tiles M{M} N{N} K{K}", flush=True)
+    out = []
+    assert [(key & 0xfff, m, n, k) for key, m, n, k, _ in recorded(lambda: out.append(ops.gemm(a, b)))] == [(tile, M, N, K)]
+    want = a[-300:].double() @ b[-300:].double().t()
+    assert (out[0][-300:, -300:].double() - want).norm() < 2 ** -8 * want.norm()
+
+
 @pytest.mark.parametrize("seq", [8192, 7500])  # whole tiles; ragged rows and a partial k-tile at the end of dW's last part
 def test_a_narrow_layers_dw_shares_its_reduction_inside_the_one_launch(seq):
     """Of a block of width 1024 the gate|up projection's dW parks its blocks and the q|k|v projection's comes in parts.  Against the two calls, which
