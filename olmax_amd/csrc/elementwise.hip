@@ -399,24 +399,26 @@ __global__ __launch_bounds__(256) void adamw_used_rows_kernel(
 // loads -> so: fp32 in the cache 1 M 17.0 -> 7.0, 6.3 M 30.6 -> 9.7, 60 M 54 -> 37, from HBM 6.3 M 35 -> 15, 60 M 92 -> 89, 155 M 164 -> 162; bf16 6.3 M 30.2 -> 7.2.  A step
 // with clipping: 6.3 M parameters 690 -> 622, 155 M 6917 -> 6807.  (Non-temporal loads read 155 M in 97 us, but then the update that follows
 // writes back what they leave in the cache, 503 -> 546: nothing gained.)
-template <bool G_BF16>
-__global__ __launch_bounds__(1024) void sumsq_kernel(const void* __restrict__ gv, int64_t n, int64_t head, int width, float* __restrict__ out) {
-  constexpr int VEC = G_BF16 ? 8 : 4, U = 8;
-  __shared__ float red[16];
-  float s[U] = {};
+// Up to 16384 vectors workgroups of four waves, with one load a lane up to 1024 and four beyond: sixteen waves and code for eight loads take 0.5 to 0.8 us more (a call on cold fp32, with
+// the events around it, 4096 9.4 -> 8.8, 65536 9.4 -> 9.2).  A vector is two chains of additions: as one, 4096 numbers were 1.28 times as far from the exact sum.
+template <bool G_BF16, int NT, int U>
+__global__ __launch_bounds__(NT) void sumsq_kernel(const void* __restrict__ gv, int64_t n, int64_t head, int width, float* __restrict__ out) {
+  constexpr int VEC = G_BF16 ? 8 : 4;
+  __shared__ float red[NT / 64];
+  float s[8] = {};
   auto element = [&](int64_t j) {
     const float x = G_BF16 ? bf2f(reinterpret_cast<const bf16*>(gv)[j]) : reinterpret_cast<const float*>(gv)[j];
     s[0] += x * x;
   };
   const u32x4* g = reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(gv) + head * (16 / VEC));
   const int64_t nv = (n - head) / VEC;
-  for (int64_t b = blockIdx.x; b * 1024 * width < nv; b += gridDim.x) {
-    const int64_t i = b * 1024 * width + threadIdx.x;
+  for (int64_t b = blockIdx.x; b * NT * width < nv; b += gridDim.x) {
+    const int64_t i = b * NT * width + threadIdx.x;
     u32x4 q[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
       q[u] = u32x4{0, 0, 0, 0};
-      if (u < width && i + u * 1024 < nv) q[u] = g[i + u * 1024];
+      if (u < width && i + u * NT < nv) q[u] = g[i + u * NT];
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -426,13 +428,13 @@ __global__ __launch_bounds__(1024) void sumsq_kernel(const void* __restrict__ gv
 #pragma unroll
       for (int e = 0; e < VEC; e++) {
         const float x = G_BF16 ? bf2f(b8.e[e]) : f[e & 3];
-        s[u] += x * x;
+        s[(u + (e & 1) * 4) % 8] += x * x;  // (two chains to a vector)
       }
     }
   }
-  for (int64_t j = (int64_t)blockIdx.x * 1024 + threadIdx.x; j < head; j += (int64_t)gridDim.x * 1024) element(j);
+  for (int64_t j = (int64_t)blockIdx.x * NT + threadIdx.x; j < head; j += (int64_t)gridDim.x * NT) element(j);
   if (const int64_t at = head + nv * VEC + threadIdx.x; blockIdx.x == 0 && at < n) element(at);
-  const float t = block_sum<16>(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])), red);
+  const float t = block_sum<NT / 64>(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])), red);
   if (threadIdx.x == 0) atomicAdd(out, t);
 }
 
@@ -682,10 +684,13 @@ extern "C" int32_t olmax_sumsq(hipStream_t stream, const void* g, int64_t n, int
   const int size = is_bf16 ? 2 : 4;
   // elements before the first aligned vector (all of them where they are not aligned to their size)
   const int64_t head = (uintptr_t)g % size ? n : std::min<int64_t>(n, (-(uintptr_t)g & 15) / size), nv = n * size / 16;
-  const int width = (int)std::min<int64_t>(std::max<int64_t>(nv / (1024 * 64), 1), 8);  // loads of a lane: 64 workgroups before they grow
-  const dim3 grid((unsigned)std::min<int64_t>(std::max<int64_t>((nv + 1024 * width - 1) / (1024 * width), 1), 512));
-  if (is_bf16) hipLaunchKernelGGL(sumsq_kernel<true>, grid, dim3(1024), 0, stream, g, n, head, width, out);
-  else hipLaunchKernelGGL(sumsq_kernel<false>, grid, dim3(1024), 0, stream, g, n, head, width, out);
+  const int nt = nv <= 16384 ? 256 : 1024, most = nv <= 1024 ? 1 : nv <= 16384 ? 4 : 8;
+  const int width = (int)std::min<int64_t>(std::max<int64_t>(nv / (nt == 256 ? 1024 : 65536), 1), most);  // loads of a lane: 4 or 64 workgroups before they grow
+  const dim3 grid((unsigned)std::min<int64_t>(std::max<int64_t>((nv + nt * width - 1) / (nt * width), 1), 512));
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(nt), 0, stream, g, n, head, width, out); };
+  if (most == 1) go(is_bf16 ? sumsq_kernel<true, 256, 1> : sumsq_kernel<false, 256, 1>);
+  else if (most == 4) go(is_bf16 ? sumsq_kernel<true, 256, 4> : sumsq_kernel<false, 256, 4>);
+  else go(is_bf16 ? sumsq_kernel<true, 1024, 8> : sumsq_kernel<false, 1024, 8>);
   OLMAX_LAUNCH_CHECK();
   return OLMAX_OK;
 }

@@ -88,7 +88,8 @@ def test_sum_of_squares(n, shift, dtype):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_sum_of_squares_by_spans(n, shift, dtype):
     """Ends of spans, of the elements before the first aligned vector and of the last one, one load of a lane to eight, several spans a workgroup, leaves beyond the
-    cache.  Whole numbers: exact below 2^24, whatever the order; above it no chain has more than 712 additions (8 lanes' loads of 25 spans, 512 workgroups), 2^-24 each."""
+    cache.  Whole numbers: exact below 2^24, whatever the order; above it no chain has more than 573 additions (4 elements of each of
+    9 spans, 3 + 6 + 16 in the workgroup, 512 workgroups), 2^-24 each; the test below is the exact one there."""
     from olmax_amd import ops
     print(f"[case] sumsq spans n{n} shift{shift} {dtype}", flush=True)
     x = torch.randint(-3, 4, (n + shift,), device="cuda", generator=torch.Generator(device="cuda").manual_seed(2), dtype=torch.int8).to(dtype)[shift:]
@@ -96,3 +97,37 @@ def test_sum_of_squares_by_spans(n, shift, dtype):
     want = sum(c.double().square().sum().item() for c in x.split(1 << 20))
     got = ops.sumsq(x).item()
     assert got == want if want < 2 ** 24 else abs(got - want) < 712 * 2 ** -24 * want
+
+
+@pytest.mark.parametrize("n", [8, 1000, 4096, 8192 + 5, 65536, 65536 * 4 + 4, 65536 * 8 * 8 + 9, 512 * 65536 + 3, (128 << 20) + 40])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sum_of_squares_counts_every_element_once(n, shift, dtype):
+    """Zeros but for whole numbers around every power of two, the ends of all spans of 1024 to 65536 elements that the sizes above meet first and last, and both ends of the
+    leaf: a sum below 2^24, exact in any order, to which each adds a share of its own."""
+    from olmax_amd import ops
+    print(f"[case] sumsq sparse n{n} shift{shift} {dtype}", flush=True)
+    at = {0, 1, 2, 7, 8, n - 1, n - 2, n - 7, n - 8, n - 9}
+    for span in [1 << i for i in range(2, 28)] + [n // 2, n // 3]:
+        at |= {span + d for d in (-9, -8, -1, 0, 1, 7, 8)} | {n // span * span + d for d in (-1, 0, 1)}
+    at = sorted(i for i in at if 0 <= i < n)
+    x = torch.zeros(n + shift, device="cuda", dtype=dtype)[shift:]
+    value = torch.arange(1, len(at) + 1, device="cuda") % 240 + 1  # whole numbers that bf16 holds
+    x[torch.tensor(at, device="cuda")] = value.to(dtype)
+    want = value.square().sum().item()
+    assert want < 2 ** 24
+    assert ops.sumsq(x).item() == want
+
+
+@pytest.mark.parametrize("n", [8, 1000, 4096, 10000, 65536, 1 << 20])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sum_of_squares_adds_a_vector_as_two_chains(n, dtype):
+    """2^24 and a 1 in every other place of the same 16 bytes: behind it in one chain the ones would be lost, 2^24 + 1 = 2^24 in fp32."""
+    from olmax_amd import ops
+    vec = 16 // dtype.itemsize
+    for first in (0, (n // vec // 2) * vec, n // vec * vec - vec):
+        print(f"[case] sumsq chains n{n} at {first} {dtype}", flush=True)
+        x = torch.zeros(n, device="cuda", dtype=dtype)
+        x[first] = 4096.0
+        x[first + 1:first + vec:2] = 1.0
+        assert ops.sumsq(x).item() == 2 ** 24 + vec // 2
