@@ -1566,11 +1566,12 @@ static int64_t parked_of(Work v, int block) { return block >= v.kt ? 0 : ((v.kt 
 static PairPlan plan_256(Work x, Work w, int whole_w, int chain_w, int block_x, int block_w, int64_t bytes) {
   PairPlan best;
   for (int p = 1; block_x && (p == 1 || (p <= 8 && w.n * p <= 256)); p++) {
-    const int chunk = (whole_w + p - 1) / p;  // every part has eight whole k-tiles or more (the last one a partial one too), and there are p of them
-    if (p == 1 ? !block_w || (block_w < w.kt && w.n > 256) : p * 8 > whole_w || (whole_w + chunk - 1) / chunk != p || chain_of_parts(p, chunk) > chain_w) continue;
+    const int chunk = (whole_w + p - 1) / p;  // whole k-tiles of a part, eight or more; the last one takes what is left, one at least, and a partial one
+    const int longest = (w.kt + p - 1) / p;   // that partial one counted: chunk, or one more where the parts come out even
+    if (p == 1 ? !block_w || (block_w < w.kt && w.n > 256) : p * 8 > whole_w || (whole_w + chunk - 1) / chunk != p || chain_of_parts(p, longest) > chain_w) continue;
     const int64_t sums = p > 1 ? w.n * p : parked_of(w, block_w);
     if ((sums + parked_of(x, block_x)) * 262144 > bytes) continue;
-    const Work part = {w.n * p, (w.kt + p - 1) / p};
+    const Work part = {w.n * p, longest};
     float c = x.kt > part.kt ? pair_256(x, part) : pair_256(part, x);
     if (sums) c = 0.89f * c + 0.1f * sums + (p > 1 ? 6.f : 0.f);
     if (c < best.cost) best = {p, c};
