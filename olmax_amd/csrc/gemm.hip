@@ -1408,13 +1408,13 @@ static int block_of(int kt, int most) {
 }
 
 // Whether a forward product that pick_tile gave to 128 tiles runs in 256 x 128 ones instead, while each of these has a CU of its own (the chains of additions are
-// the same).  Both are bound by operand delivery.  us, 128 tiles -> so, behind another product and with operands from HBM, with more than 288 tiles of 128 (two on
-// many CUs): 8192 x 1024 x 2816 59.5 -> 48.6, 1000 x 6144 x 4096 76 -> 58, 1500 x 4096 x 4096 64 -> 58, 4096 x 1280 x 4096 62 -> 59, 260 x 14336 x 4096 66 -> 61, 3000 x 2048 x
-// 9216 133 -> 128; with fewer, half of the CUs have nothing to do: 2048 x 2048 x 2816 43.6 -> 45.0, x 5120 6 % slower, 2048 x 2304 x 3072 3 %.  A partial k-tile costs what they
-// gain: 1500 x 4096 x 4104 84.5 -> 89.7, x 2056 47.9 -> 50.0.  Longer reductions gain or lose: x 11008 1000 x 6144 202 -> 157, 6000 x 1024 163 -> 169; 2500 x 2304 x 16384 225 -> 262;
-// of short ones 3000 x 1024 x 1024 14.0 -> 14.2.  (B stored [K, N]: 8 % at best; both operands so: up to 20 % slower, as the transposing reads fill LDS.)
+// the same).  Both are bound by operand delivery.  us, 128 tiles -> so, behind another product and with operands from HBM, where some CUs get two tiles of 128: 8192 x 1024 x
+// 2816 59.5 -> 48.6, 1000 x 6144 x 4096 76 -> 58, 1500 x 4096 x 4096 64 -> 58, 4096 x 1280 x 4096 62 -> 59, 448 x 9152 x 9152 240 -> 196; of 650 such measurements, K 2048 to 16384,
+// the mean is 8 % less, 17 are 3 to 6 % more and one 14 % (2500 x 2304 x 16384 225 -> 262).  Where each has one, half of the CUs are left with nothing: 2048 x 2048 x 2816 43.6 ->
+// 45.0, x 5120 6 % slower, x 4096 59.1 -> 57.2; and a partial k-tile costs what they gain: 1500 x 4096 x 4104 84.5 -> 89.7, x 2056 47.9 -> 50.0.  Of short reductions 3000 x 1024 x
+// 1024 14.0 -> 14.2.  (B stored [K, N]: 8 % at best; both operands so: up to 20 % slower, as the transposing reads fill LDS.)
 static bool thin_takes(int M, int N, int K, int tile) {
-  return tile == 128 && M >= 256 && K % BK == 0 && K >= 32 * BK && K <= 144 * BK && (int64_t)((M + 255) / 256) * ((N + 127) / 128) <= 256 && tiles_of(M, N, 128) > 288;
+  return tile == 128 && M >= 256 && K % BK == 0 && K >= 32 * BK && (int64_t)((M + 255) / 256) * ((N + 127) / 128) <= 256 && tiles_of(M, N, 128) > 256;
 }
 
 enum GluForm { GLU_SAVE, GLU_ONLY, GLU_BWD };
