@@ -1,5 +1,5 @@
 // Body of dQ, taken in by its kernel, by the one that runs it beside dK/dV and by the function of that name in attn.hip.  (Text, because as an inlined function
-// it takes four registers and 7 % more time, 2 x 4096, 32 heads 965 -> 1016 us a backward pass.  With the soft-cap at head_dim 128 the function takes 18 registers
+// it takes four registers and 7 % more time, 2 x 4096, 32 heads 965 -> 1016 us a backward pass: the mask of each score becomes a compare and a select that every tile pays, here a branch around it.  With the soft-cap at head_dim 128 the function takes 18 registers
 // less, which the launch of both needs; by itself it would be 1 % faster on some lengths and 1 % slower on others, 2 x 4096, 32/16 heads 1144 -> 1128, 2 x 1777, 32/8 heads 267 -> 269.)
 // Expects the kernel's arguments, smem, and the workgroup's id among nwg; DELTA may be null.
   constexpr int TILE = 64 * D * 2;

@@ -95,8 +95,8 @@ std::mutex g_prof_mu;
 //
 // The tile that workgroup `pid` of `nwg` takes; the residual of a HAS_RES form may be null.  BLOCKS: the sums of every `block` k-tiles (an
 // even number) are added up by themselves, for shorter chains of fp32 additions: 1 in registers, 2 (256 tiles, which have none left) parked
-// in `park`, 256 KB a tile and block.  us, both gradients with one chain -> with blocks: 3000 x 1024 x 3072 46.6 -> 46.6,
-// 4096 x 1024 x 3072 55.2 -> 55.7 (blocks of four k-tiles 56.3), 512 x 2816 x 1024 16.2 -> 16.6; 2048 x 4096 x 12288 305.8 -> 314.6.
+// in `park`, 256 KB a tile and block.  us in a block's backward pass, both gradients with one chain -> with blocks: 3000 x 1024 x 3072 44.6 -> 46.6,
+// 4096 x 1024 x 3072 59.8 -> 60.4, 512 x 2816 x 1024 16.8 -> 17.6; 2048 x 4096 x 12288 302 -> 308, x 22016 540 -> 555.
 template <int BM, int BN, int WM, int WN, bool A_KC, bool B_KC, bool HAS_RES, bool OUT_F32, int EPI, int RAG, int BLOCKS = 0>
 __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ A, const bf16* __restrict__ B, void* __restrict__ Cv,
@@ -903,8 +903,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) GEMM_VGPR_CAP void gemm
 
 // dX = dY W (+ R) and dW = dY^T X in one launch of T x T tiles: the second starts on the CUs that the first's last round of tiles
 // leaves idle.  Workgroups [0, n_first) are the product with the longer reduction (and padding up to a whole number of XCDs).
-// us, two calls -> one, T x in x out: tiles of 128: 3000 x 1024 x 3072 76 -> 54, 3000 x 2816 x 1024 63 -> 41, 1024 x 4096 x 4096 79 -> 71;
-// tiles of 256: 2048 x 11008 x 4096 343 -> 306, 1500 x 14336 x 4096 368 -> 316, 8192 x 11008 x 4096 1141 -> 1091.
+// us in a block's backward pass, two calls -> one, T x in x out: tiles of 128: 3000 x 1024 x 3072 76 -> 47, 3000 x 2816 x 1024 65 -> 42, 4096 x 1024 x 3072 92 -> 60;
+// tiles of 256: 2048 x 4096 x 12288 339 -> 308, 1500 x 4096 x 28672 706 -> 601, 8192 x 1024 x 5632 199 -> 178, 8192 x 11008 x 4096 1066 -> 1008; no longer 2048 x 4096 x 22016 549 -> 555.
 // 240 registers (the cap counts pairs): as in the single kernels a wave of the overlapped update fits beside two of these.
 struct PairSide {
   const bf16 *A, *B, *R;
@@ -1241,8 +1241,10 @@ static int device_cu_count() {
 }
 
 // Estimated time (us) of each kernel on a problem of kt k-tiles, from measurements at 16 to 8192 rows
-// and 256 to 11008 columns (every layout; within about 15 %) on the 256 CUs of this GPU.  A k-tile costs a 256 tile 1.05 us with
-// few tiles in flight and 1.52 us with one on every CU (both bound by operand delivery), a 128 tile
+// and 256 to 11008 columns (every layout; within about 15 %) on the 256 CUs of this GPU, on warm operands: with operands from HBM and behind another product all
+// of them take a quarter to a half more.  What counts is how they compare.  A k-tile costs a 256 tile 1.05 us with few tiles in flight and 1.52 us with one on every CU, and a
+// round 6 us beside: the figures of the loop before its waves took turns, which every choice below was compared with.  Now it is 1.27 to 1.35 and 9.5, so that
+// long reductions take up to 12 % less than priced (8192 x 22016 x 4096 1130, 1004 measured) and short ones more.  A 128 tile costs
 // 0.57 us alone, 0.83 us with one on every CU and 1.08 us with the two that fit, a 64 tile 0.22 us
 // per round.  Up to 32 k-tiles and one 128 tile per CU the operands of a whole product stay near: 0.40 us up to 8 k-tiles, rising to 0.6,
 // sooner where B is [K, N].  us of 128 tiles | 64 tiles: 384 x 2816 x 512 6.8 | 7.6, 512 x 4096 x 1024 10.3 | 11.5 ([K, N]: 10.6 | 11.3), 256 x 5632 x 1024
@@ -1557,7 +1559,9 @@ static float pair_256(Work l, Work s) {
 // `parts` (workgroups of their own, the sums added by a second kernel), or is whole and parks the sums of its blocks.  What costs the least among
 // those whose chains are as short as the calls' and whose sums fit.  us in a training step, the better of two calls and 128 tiles -> so: 8192 x 1024 x 5632 195 ->
 // 172 (parked), 8192 x 1024 x 3072 115 -> 104, 8192 x 2816 x 1024 117 -> 109 (five parts), 8192 x 1024 x 1024 61 -> 45 (eight).  dW of more tiles than CUs
-// fills the GPU by itself: parked, 8192 x 4096 x 22016 takes 2070 us, two calls 1930.  The 0.89: these forms beside the others, as measured there.
+// fills the GPU by itself: parked, 8192 x 4096 x 22016 takes 2070 us, two calls 1930.  The 0.89 is the present loop against the one that pair_256 prices (see cost_128): it
+// is here, where the forms with sums were fitted, and not in the price of the form without, which was compared as it is.  Of 58 products of drawn blocks that take a form
+// with sums 54 are faster than in the form they would take else, 11 % less time on average, two are 7 % slower (6528 x 1024 x 4096 114 -> 122, 6283 x 2816 x 1024 81 -> 87).
 struct PairPlan {
   int parts = 1;
   float cost = 1e30f;
