@@ -1560,8 +1560,9 @@ static float pair_256(Work l, Work s) {
 // those whose chains are as short as the calls' and whose sums fit.  us in a training step, the better of two calls and 128 tiles -> so: 8192 x 1024 x 5632 195 ->
 // 172 (parked), 8192 x 1024 x 3072 115 -> 104, 8192 x 2816 x 1024 117 -> 109 (five parts), 8192 x 1024 x 1024 61 -> 45 (eight).  dW of more tiles than CUs
 // fills the GPU by itself: parked, 8192 x 4096 x 22016 takes 2070 us, two calls 1930.  The 0.89 is the present loop against the one that pair_256 prices (see cost_128): it
-// is here, where the forms with sums were fitted, and not in the price of the form without, which was compared as it is.  Of 58 products of drawn blocks that take a form
-// with sums 54 are faster than in the form they would take else, 11 % less time on average, two are 7 % slower (6528 x 1024 x 4096 114 -> 122, 6283 x 2816 x 1024 81 -> 87).
+// is here, where the forms with sums were fitted, and not in the price of the form without, which was compared as it is.  Against 128 tiles in one launch, 230 products of drawn blocks (width
+// 512 to 2560, 2000 to 8300 tokens) that take 256 tiles: 16 % less time on average, 208 faster, 15 slower by 2 to 14 %, half of them T x 2816 x 1024 of 5100 to 7800 tokens (6272: 79 -> 84).  T x 512 x
+// 4096 varies with where the buffers lie (8027: 128 tiles 88 to 92, this 91 to 107, once 150).
 struct PairPlan {
   int parts = 1;
   float cost = 1e30f;
