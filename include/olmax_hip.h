@@ -387,7 +387,7 @@ int32_t olmax_block_bwd(olmax_stream_t stream, const olmax_model_config* cfg, co
  * inside the library or under graph capture.
  * ===================================================================================== */
 /* Force the MFMA tile variant of olmax_gemm_bf16 (0 = automatic, 128, 256; 384: 256 x 128, bf16 results of
- * two reduction-contiguous operands, K a multiple of 64).  While set, the fused GLU / RoPE projections take their unfused paths (same results). */
+ * two reduction-contiguous operands).  While set, the fused GLU / RoPE projections take their unfused paths (same results). */
 void olmax_gemm_set_tile(int tile);
 /* Order in which the MFMA GEMM's workgroups take their tiles: 0 = automatic (per shape and operand
  * layout), -1 = one contiguous run of tiles per XCD, n > 0 = windows of 8 x 4 tiles per XCD whose 8

@@ -1053,7 +1053,7 @@ int dispatch_tile(hipStream_t s, const bf16* A, const bf16* B, void* C, const bf
   if constexpr (A_KC && B_KC && !OUT_F32) {
     if (tile == THIN_TILE) {
 #define TILE(RAG) launch_tile<256, 128, 64, 64, A_KC, B_KC, HAS_RES, OUT_F32, RAG>(s, A, B, C, R, M, N, K, lda, ldb, ldc, ldr)
-      return M % 256 || N % 128 ? TILE(1) : TILE(0);  // (whole k-tiles: see thin_takes)
+      return K % BK ? TILE(2) : M % 256 || N % 128 ? TILE(1) : TILE(0);
 #undef TILE
     }
   }
@@ -1412,11 +1412,17 @@ static int block_of(int kt, int most) {
 // Whether a forward product that pick_tile gave to 128 tiles runs in 256 x 128 ones instead, while each of these has a CU of its own (the chains of additions are
 // the same).  Both are bound by operand delivery.  us, 128 tiles -> so, behind another product and with operands from HBM, where some CUs get two tiles of 128: 8192 x 1024 x
 // 2816 59.5 -> 48.6, 1000 x 6144 x 4096 76 -> 58, 1500 x 4096 x 4096 64 -> 58, 4096 x 1280 x 4096 62 -> 59, 448 x 9152 x 9152 240 -> 196; of 650 such measurements, K 2048 to 16384,
-// the mean is 8 % less, 17 are 3 to 6 % more and one 14 % (2500 x 2304 x 16384 225 -> 262).  Where each has one, half of the CUs are left with nothing: 2048 x 2048 x 2816 43.6 ->
-// 45.0, x 5120 6 % slower, x 4096 59.1 -> 57.2; and a partial k-tile costs what they gain: 1500 x 4096 x 4104 84.5 -> 89.7, x 2056 47.9 -> 50.0.  Of short reductions 3000 x 1024 x
-// 1024 14.0 -> 14.2.  (B stored [K, N]: 8 % at best; both operands so: up to 20 % slower, as the transposing reads fill LDS.)
+// the mean is 8 % less, 17 are 3 to 6 % more and one 14 % (2500 x 2304 x 16384 225 -> 262).  Where each has one, half of the CUs are left with
+// nothing, and only a wide product, whose weights are then read half as often, is worth that: N >= 2 M and 96 such tiles or more 1000 x 4096 x 4096 59.7 -> 56.6, 768 x 5248 x 6336 105
+// -> 91, 300 sizes 5 % less on average, 5 % more at most; others 2048 x 2048 x 2816 43.6 -> 45.0, 8192 x 512 x 11008 157 -> 166, 2048 x 2048 x 4096 59.1 -> 57.2, 2 % more on average.  A partial
+// k-tile costs more here: 1500 x 4096 x 4104 84.5 -> 89.7, x 2056 47.9 -> 50.0, narrow products 8 % on average, wide ones with up to 288 tiles of 128 3 %; beyond they still gain 9 %
+// (1064 x 5504 x 9144 213 -> 195).  Of short reductions 3000 x 1024 x 1024 14.0 -> 14.2.  (B stored [K, N]: 8 % at best; both operands so: up to 20 % slower, as the transposing reads
+// fill LDS.)
 static bool thin_takes(int M, int N, int K, int tile) {
-  return tile == 128 && M >= 256 && K % BK == 0 && K >= 32 * BK && (int64_t)((M + 255) / 256) * ((N + 127) / 128) <= 256 && tiles_of(M, N, 128) > 256;
+  const int64_t n = (int64_t)((M + 255) / 256) * ((N + 127) / 128), n128 = tiles_of(M, N, 128);
+  if (tile != 128 || M < 256 || K < 32 * BK || n > 256) return false;
+  const bool wide = N >= 2 * (int64_t)M;
+  return K % BK ? wide && n128 > 288 : n128 > 256 || (wide && n >= 96);
 }
 
 enum GluForm { GLU_SAVE, GLU_ONLY, GLU_BWD };
@@ -1445,7 +1451,7 @@ int olmax_gemm_padded(hipStream_t stream, const bf16* a, const bf16* b, void* C,
   if (force_tile && direct_ok && K >= BK) {  // whatever the rule chose, if the problem has a tile of that size
     if (force_tile == 256 && M >= 256 && N >= 256) tile = 256;
     if (force_tile == 128 && M >= 128 && N >= 128) tile = 128;
-    if (force_tile == THIN_TILE && M >= 256 && N >= 128 && K % BK == 0 && a_kc && b_kc && !out_f32) tile = THIN_TILE;
+    if (force_tile == THIN_TILE && M >= 256 && N >= 128 && a_kc && b_kc && !out_f32) tile = THIN_TILE;
   }
   if (tile == 256 && !force_tile) {
     const Cut cut = find_cut((M + 255) / 256, (N + 255) / 256);

@@ -52,9 +52,10 @@ def test_forward_products_of_few_128_tiles_take_256_x_128_ones():
 
 @pytest.mark.parametrize("M,N,K,tile", [
     (260, 14336, 4096, 384), (4096, 1280, 4096, 384), (8192, 1024, 2816, 384), (1000, 6144, 9216, 384), (448, 9152, 9152, 384), (1500, 2816, 2048, 384),
-    (2048, 2048, 2816, 128), (1024, 4096, 5120, 128), (700, 4608, 11008, 128), (1500, 4096, 4104, 128), (1500, 4096, 2056, 128), (2048, 4096, 1984, 128)])
+    (512, 8064, 4096, 384), (768, 5248, 6336, 384), (2048, 2048, 2816, 128), (4096, 1024, 5120, 128), (8192, 512, 11008, 128),
+    (1500, 2816, 4104, 128), (768, 5120, 6960, 128), (1064, 5504, 4104, 384), (498, 11896, 2056, 384), (2048, 4096, 1984, 128)])
 def test_256_x_128_tiles_take_what_they_are_faster_on(M, N, K, tile):
-    """Not while a tile of 128 has a CU to itself, part of a k-tile, or short reductions.  Against float64: 2^-9 for the rounding to bf16, as much again for the sums."""
+    """While a tile of 128 has a CU to itself only wide products; part of a k-tile only in wide ones of more; no short reductions.  Against float64: 2^-9 for the rounding to bf16, as much again for the sums."""
     from olmax_amd import ops
     from test_gemm_choice_gpu import operands, recorded
     a, b = operands(M, N, K, 0, 0)
